@@ -26,8 +26,7 @@
 namespace {
 
 // forward scratch of one step: predictor, predictor corner emf, corrector fluxes
-const int kSeqForwardScratch[] = {SK_BEGIN_ONCE, SK_PRED_X1_SAVE, SK_PRED_X2_SAVE, SK_CORNER_P, SK_CORR,
-                                  SK_CORR2};
+const int kSeqForwardScratch[] = {SK_BEGIN_ONCE, SK_PRED_SAVE, SK_CORNER_P, SK_CORR_BOTH};
 // the rest of integrate_2d after kSeqForwardScratch, and the set_bvals that
 // follows it. integrate_2d leaves the ghost cells as they were (the drop-in's
 // carry copies them into the new buffer), but the set_bvals right after it
@@ -36,8 +35,8 @@ const int kSeqForwardScratch[] = {SK_BEGIN_ONCE, SK_PRED_X1_SAVE, SK_PRED_X2_SAV
 const int kSeqFinishStep[] = {SK_CORNER_C, SK_FINAL, SK_END_ONCE};
 const int kSeqGhostCur[] = {SK_GHOST_CUR};
 // a whole step so: integrate_2d without the carry (then set_bvals)
-const int kSeqRolloutStep[] = {SK_BEGIN_ONCE, SK_PRED_X1, SK_PRED_X2, SK_CORNER_P, SK_CORR,
-                               SK_CORR2,      SK_CORNER_C, SK_FINAL,  SK_END_ONCE};
+const int kSeqRolloutStep[] = {SK_BEGIN_ONCE, SK_PRED,  SK_CORNER_P, SK_CORR_BOTH,
+                               SK_CORNER_C,   SK_FINAL, SK_END_ONCE};
 // the reverse of one step on two streams: the x1 and x2 halves of Steps 8
 // and 1-2 are independent (their adjoints meet in ain through atomic adds)
 const int kRevHead[] = {AK_FOLD_OUT, AK_ZERO, AK_UPDATE, AK_CORNER_C};  // then fork

@@ -409,7 +409,7 @@ int athmi_profile_steps(athmi_grid* g, int nsteps, double* avg_ms, int nslots) {
   for (int s = 0; s < nsteps; s++) {
     HIP_TRY(hipEventRecord(ev[0], g->stream));
     for (int k = 0; k < kStepLen; k++) {
-      HIP_TRY(g->launch(&g->bl, kSeqStep[k], g->stream));
+      HIP_TRY(g->launch(&g->bl, kSeqProfile[k], g->stream));
       HIP_TRY(hipEventRecord(ev[k + 1], g->stream));
     }
     HIP_TRY(hipEventSynchronize(ev[kStepLen]));

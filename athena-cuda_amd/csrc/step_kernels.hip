@@ -4,10 +4,12 @@
 //
 // Pipeline of one step (all state in SoA planes, ping-pong buffers):
 //   k_begin      clock: limits, tlim clamp of dt, reset of dt partials
-//   k_pred_x1    Steps 1a-1e: x1 sweep, PLM via an LDS neighbour exchange
-//   k_pred_x2    Steps 2a-2e: x2 sweep, each lane marches down a column
+//   k_pred       both sweeps' predictors in one launch: the tiles of
+//     k_pred_x1  Steps 1a-1e: x1 sweep, PLM via an LDS neighbour exchange
+//     k_pred_x2l Steps 2a-2e: x2 sweep, each lane marches down a column
 //   k_corner<P>  Step 4 corner emf (and Step 3 emf3_cc comes from k_pred_x1)
-//   k_corr       Steps 4 (half-step face B), 5, 6, 7, 8b, 8c
+//   k_corr_both  Steps 4 (half-step face B), 5, 6, 7, 8b, 8c: the tiles of both
+//                parts of k_corr in one launch
 //   k_corner<C>  Step 9 corner emf
 //   k_final      Steps 9 (face B), 11a/11b, 13 and the new_dt max, fused
 //   k_ghost      set_bvals on the new state
@@ -193,83 +195,88 @@ struct RowStencil {
 // solver; a launch takes only the tiles of instances that use it, and with one
 // solver per kernel the predictor fits two waves per SIMD.
 template <bool SAVE, int FLUX>
+__device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int ninst, int t,
+                                             double (*sw)[kX1Block], double (*swl)[kX1Block],
+                                             double (*swr)[kX1Block]) {
+  const int tid = threadIdx.x;
+  const Inst& g = insts[find_inst(insts, ninst, K_PRED_X1, t)];
+  const Clock* clk = g.clk;
+  if (!clk->active || g.flux != FLUX) return;
+  const int local = uni(t - g.tile0[K_PRED_X1]);
+  const int gis = uni(g.is), gie = uni(g.ie);
+  const int nseg = dcdiv(uni(g.nx1) + 4, kX1Faces);
+  const int row = local / nseg, seg = local - row * nseg;
+  const int j = uni(g.js) - 2 + row;
+  const int f0 = gis - 1 + seg * kX1Faces;
+  const int cell = f0 - 2 + tid;
+  const double dt = uni(clk->dt);
+  const double dx1 = uni(g.dx1);
+  const double dtodx1 = dt / dx1;
+  const double hdt = 0.5 * dt;
+  const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
+  const double* __restrict__ st = uni(g.state[clk->cur]);
+  double* __restrict__ sc = uni(g.scratch);
+  double* __restrict__ pw = uni(g.prims);
+  const size_t ps = (size_t)uni((int)g.ps);
+  const uint32_t rk = (uint32_t)(j * uni(g.pitch));
+  double bxc = 0.0;
+  if (cell >= gis - 3 && cell <= gie + 3) {
+    const uint32_t k = rk + (uint32_t)cell;
+    const double d = LD(st + F_D * ps, k), m1 = LD(st + F_M1 * ps, k), m2 = LD(st + F_M2 * ps, k);
+    const double b1c = LD(st + F_B1C * ps, k), b2c = LD(st + F_B2C * ps, k);
+    const Cons7 u{d, m1, m2, LD(st + F_M3 * ps, k), LD(st + F_E * ps, k), b2c, LD(st + F_B3C * ps, k)};
+    bxc = b1c;
+    lds_put(sw, tid, cons_to_prim(u, bxc, eos));
+    // Step 3 (:249-255): emf3 at t^n over [jl,ju] x [il,iu]
+    if (cell >= gis - 2 && cell <= gie + 2 && tid >= 1 && tid <= kX1Block - 2)
+      ST(sc + S_ECC * ps, k, (b1c * m2 - b2c * m1) / d);
+  }
+  __syncthreads();
+  if (tid >= 1 && tid <= kX1Block - 2 && cell >= gis - 2 && cell <= gie + 2) {
+    Prim7 wl, wr;
+    plm_cell_s(RowStencil{sw, tid}, bxc, dtodx1, eos, wl, wr);
+    lds_put(swl, tid + 1, wl);
+    lds_put(swr, tid, wr);
+  }
+  __syncthreads();
+  if (tid >= 2 && tid <= kX1Block - 2 && cell <= gie + 2) {
+    const uint32_t k = rk + (uint32_t)cell;
+    // face states: PLM output + MHD source terms for 1/2 dt (:156-164) +
+    // prim->cons (:175-176); rebuilt from LDS and memory for the HLLE fallback
+    auto build = [&](Cons7& ul, Cons7& ur, Prim7& wl, Prim7& wr, double& b0) {
+      compiler_fence();
+      wl = lds_prim(swl, tid);
+      wr = lds_prim(swr, tid);
+      const double bm = LD(st + F_B1I * ps, k - 1), bp = LD(st + F_B1I * ps, k + 1);
+      b0 = LD(st + F_B1I * ps, k);
+      double src = (LD(st + F_M2 * ps, k - 1) / LD(st + F_D * ps, k - 1)) * (b0 - bm) / dx1;
+      wl.by = wl.by + hdt * src;
+      src = (LD(st + F_M2 * ps, k) / LD(st + F_D * ps, k)) * (bp - b0) / dx1;
+      wr.by = wr.by + hdt * src;
+      ul = prim_to_cons(wl, b0, eos);
+      ur = prim_to_cons(wr, b0, eos);
+    };
+    Cons7 ul, ur;
+    Prim7 wl, wr;
+    double b0;
+    build(ul, ur, wl, wr, b0);
+    if (SAVE) {
+      put7(pw + P_WL1 * ps, ps, k, wl);
+      put7(pw + P_WR1 * ps, ps, k, wr);
+    }
+    put7(sc + S_UL1 * ps, ps, k, ul);
+    put7(sc + S_UR1 * ps, ps, k, ur);
+    put7(sc + S_F1 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
+  }
+}
+template <bool SAVE, int FLUX>
 __global__ void __launch_bounds__(kX1Block, 2) k_pred_x1(const Inst* __restrict__ insts,
                                                          int ninst, int ntiles, int remap) {
   __shared__ double sw[7][kX1Block];
   __shared__ double swl[7][kX1Block];
   __shared__ double swr[7][kX1Block];
-  const int tid = threadIdx.x;
   for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x) {
-    const int t = xcd_tile(t0, ntiles, remap);
-    const Inst& g = insts[find_inst(insts, ninst, K_PRED_X1, t)];
-    const Clock* clk = g.clk;
-    if (!clk->active || g.flux != FLUX) continue;
-    const int local = uni(t - g.tile0[K_PRED_X1]);
-    const int gis = uni(g.is), gie = uni(g.ie);
-    const int nseg = dcdiv(uni(g.nx1) + 4, kX1Faces);
-    const int row = local / nseg, seg = local - row * nseg;
-    const int j = uni(g.js) - 2 + row;
-    const int f0 = gis - 1 + seg * kX1Faces;
-    const int cell = f0 - 2 + tid;
-    const double dt = uni(clk->dt);
-    const double dx1 = uni(g.dx1);
-    const double dtodx1 = dt / dx1;
-    const double hdt = 0.5 * dt;
-    const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
-    const double* __restrict__ st = uni(g.state[clk->cur]);
-    double* __restrict__ sc = uni(g.scratch);
-    double* __restrict__ pw = uni(g.prims);
-    const size_t ps = (size_t)uni((int)g.ps);
-    const uint32_t rk = (uint32_t)(j * uni(g.pitch));
-    double bxc = 0.0;
-    if (cell >= gis - 3 && cell <= gie + 3) {
-      const uint32_t k = rk + (uint32_t)cell;
-      const double d = LD(st + F_D * ps, k), m1 = LD(st + F_M1 * ps, k), m2 = LD(st + F_M2 * ps, k);
-      const double b1c = LD(st + F_B1C * ps, k), b2c = LD(st + F_B2C * ps, k);
-      const Cons7 u{d, m1, m2, LD(st + F_M3 * ps, k), LD(st + F_E * ps, k), b2c, LD(st + F_B3C * ps, k)};
-      bxc = b1c;
-      lds_put(sw, tid, cons_to_prim(u, bxc, eos));
-      // Step 3 (:249-255): emf3 at t^n over [jl,ju] x [il,iu]
-      if (cell >= gis - 2 && cell <= gie + 2 && tid >= 1 && tid <= kX1Block - 2)
-        ST(sc + S_ECC * ps, k, (b1c * m2 - b2c * m1) / d);
-    }
-    __syncthreads();
-    if (tid >= 1 && tid <= kX1Block - 2 && cell >= gis - 2 && cell <= gie + 2) {
-      Prim7 wl, wr;
-      plm_cell_s(RowStencil{sw, tid}, bxc, dtodx1, eos, wl, wr);
-      lds_put(swl, tid + 1, wl);
-      lds_put(swr, tid, wr);
-    }
-    __syncthreads();
-    if (tid >= 2 && tid <= kX1Block - 2 && cell <= gie + 2) {
-      const uint32_t k = rk + (uint32_t)cell;
-      // face states: PLM output + MHD source terms for 1/2 dt (:156-164) +
-      // prim->cons (:175-176); rebuilt from LDS and memory for the HLLE fallback
-      auto build = [&](Cons7& ul, Cons7& ur, Prim7& wl, Prim7& wr, double& b0) {
-        compiler_fence();
-        wl = lds_prim(swl, tid);
-        wr = lds_prim(swr, tid);
-        const double bm = LD(st + F_B1I * ps, k - 1), bp = LD(st + F_B1I * ps, k + 1);
-        b0 = LD(st + F_B1I * ps, k);
-        double src = (LD(st + F_M2 * ps, k - 1) / LD(st + F_D * ps, k - 1)) * (b0 - bm) / dx1;
-        wl.by = wl.by + hdt * src;
-        src = (LD(st + F_M2 * ps, k) / LD(st + F_D * ps, k)) * (bp - b0) / dx1;
-        wr.by = wr.by + hdt * src;
-        ul = prim_to_cons(wl, b0, eos);
-        ur = prim_to_cons(wr, b0, eos);
-      };
-      Cons7 ul, ur;
-      Prim7 wl, wr;
-      double b0;
-      build(ul, ur, wl, wr, b0);
-      if (SAVE) {
-        put7(pw + P_WL1 * ps, ps, k, wl);
-        put7(pw + P_WR1 * ps, ps, k, wr);
-      }
-      put7(sc + S_UL1 * ps, ps, k, ul);
-      put7(sc + S_UR1 * ps, ps, k, ur);
-      put7(sc + S_F1 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
-    }
+    pred_x1_tile<SAVE, FLUX>(insts, ninst, xcd_tile(t0, ntiles, remap), sw, swl, swr);
     __syncthreads();
   }
 }
@@ -395,13 +402,11 @@ __global__ void __launch_bounds__(kX2Block) k_pred_x2(const Inst* __restrict__ i
 // 160 KiB.
 constexpr int kX2Slots = 5;  // 4 rotating + the Wr slot
 constexpr int kX2Aux = 5;    // B2i ring (2), s ring (2), M1/d carry
+typedef double X2Slots[7][kX2Block];
 template <bool SAVE, int FLUX>
-__global__ void __launch_bounds__(kX2Block, 2) k_pred_x2l(const Inst* __restrict__ insts,
-                                                          int ninst, int ntiles, int seg_len,
-                                                          int remap) {
-  __shared__ double slots[kX2Slots][7][kX2Block];
-  __shared__ double aux[kX2Aux][kX2Block];
-  const int lane = threadIdx.x;
+__device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int ninst, int t,
+                                             int seg_len, X2Slots* slots,
+                                             double (*aux)[kX2Block], int lane) {
   // aux rows: B2i of row r at r & 1, s(r) at 2 + (r & 1), M1/d of the newest row
   auto b2i_slot = [&](int r) -> double& { return aux[r & 1][lane]; };
   auto src_slot = [&](int r) -> double& { return aux[2 + (r & 1)][lane]; };
@@ -426,109 +431,144 @@ __global__ void __launch_bounds__(kX2Block, 2) k_pred_x2l(const Inst* __restrict
     }
     __device__ void fence() const { compiler_fence(); }
   };
-  for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x) {
-    const int t = xcd_tile(t0, ntiles, remap);
-    const Inst& g = insts[find_inst(insts, ninst, K_PRED_X2, t)];
-    const Clock* clk = g.clk;
-    if (!clk->active || g.flux != FLUX) continue;
-    const int local = uni(t - g.tile0[K_PRED_X2]);
-    // chunks from column 0: each row segment starts on a cache line
-    const int ncb = dcdiv(uni(g.nx1) + 6, kX2Block);
-    const int sg = local / ncb, cb = local - sg * ncb;
-    const int i = cb * kX2Block + lane;
-    if (i < uni(g.is) - 2) continue;
-    if (i > uni(g.ie) + 2) continue;
-    const int jf0 = uni(g.js) - 1 + sg * seg_len;
-    const int jf1 = min(jf0 + seg_len - 1, uni(g.je) + 2);
-    const double dt = uni(clk->dt);
-    const double dx2 = uni(g.dx2);
-    const double dtodx2 = dt / dx2;
-    const double hdt = 0.5 * dt;
-    const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
-    const double* __restrict__ st = uni(g.state[clk->cur]);
-    double* __restrict__ sc = uni(g.scratch);
-    double* __restrict__ pw = uni(g.prims);
-    const size_t ps = (size_t)uni((int)g.ps);
-    const int pitch = uni(g.pitch);
-    // cons->prim of row jj in the permuted order (d, M2, M3, M1, E, B3c, B1c), Bx = B2c;
-    // with M1/d (the source term's division form) and B2i of the row
-    auto load_row = [&](int jj, int slot, double& v1, double& b2i) {
-      const uint32_t k = (uint32_t)(jj * pitch + i);
-      const double d = LD(st + F_D * ps, k), m1 = LD(st + F_M1 * ps, k);
-      const Cons7 u{d, LD(st + F_M2 * ps, k), LD(st + F_M3 * ps, k), m1,
-                    LD(st + F_E * ps, k), LD(st + F_B3C * ps, k), LD(st + F_B1C * ps, k)};
-      put(slot, cons_to_prim(u, LD(st + F_B2C * ps, k), eos));
-      v1 = m1 / d;
-      b2i = LD(st + F_B2I * ps, k);
-    };
-    auto bx_at = [&](int jj) { return LD(st + F_B2C * ps, (uint32_t)(jj * pitch + i)); };
-    // start of the march: rows jf0-2, jf0-1, jf0, the source s(jf0-1) and
-    // the PLM of cell jf0-1
+  const Inst& g = insts[find_inst(insts, ninst, K_PRED_X2, t)];
+  const Clock* clk = g.clk;
+  if (!clk->active || g.flux != FLUX) return;
+  const int local = uni(t - g.tile0[K_PRED_X2]);
+  // chunks from column 0: each row segment starts on a cache line
+  const int ncb = dcdiv(uni(g.nx1) + 6, kX2Block);
+  const int sg = local / ncb, cb = local - sg * ncb;
+  const int i = cb * kX2Block + lane;
+  if (i < uni(g.is) - 2) return;
+  if (i > uni(g.ie) + 2) return;
+  const int jf0 = uni(g.js) - 1 + sg * seg_len;
+  const int jf1 = min(jf0 + seg_len - 1, uni(g.je) + 2);
+  const double dt = uni(clk->dt);
+  const double dx2 = uni(g.dx2);
+  const double dtodx2 = dt / dx2;
+  const double hdt = 0.5 * dt;
+  const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
+  const double* __restrict__ st = uni(g.state[clk->cur]);
+  double* __restrict__ sc = uni(g.scratch);
+  double* __restrict__ pw = uni(g.prims);
+  const size_t ps = (size_t)uni((int)g.ps);
+  const int pitch = uni(g.pitch);
+  // cons->prim of row jj in the permuted order (d, M2, M3, M1, E, B3c, B1c), Bx = B2c;
+  // with M1/d (the source term's division form) and B2i of the row
+  auto load_row = [&](int jj, int slot, double& v1, double& b2i) {
+    const uint32_t k = (uint32_t)(jj * pitch + i);
+    const double d = LD(st + F_D * ps, k), m1 = LD(st + F_M1 * ps, k);
+    const Cons7 u{d, LD(st + F_M2 * ps, k), LD(st + F_M3 * ps, k), m1,
+                  LD(st + F_E * ps, k), LD(st + F_B3C * ps, k), LD(st + F_B1C * ps, k)};
+    put(slot, cons_to_prim(u, LD(st + F_B2C * ps, k), eos));
+    v1 = m1 / d;
+    b2i = LD(st + F_B2I * ps, k);
+  };
+  auto bx_at = [&](int jj) { return LD(st + F_B2C * ps, (uint32_t)(jj * pitch + i)); };
+  // start of the march: rows jf0-2, jf0-1, jf0, the source s(jf0-1) and
+  // the PLM of cell jf0-1
+  {
+    double v1m, b2m, v10, b20, v1u, b2u;
+    load_row(jf0 - 2, 0, v1u, b2u);
+    load_row(jf0 - 1, 1, v1m, b2m);
+    load_row(jf0, 2, v10, b20);
+    src_slot(jf0 - 1) = v1m * (b20 - b2m) / dx2;
+    b2i_slot(jf0) = b20;
+    v1_carry = v10;
+  }
+  {
+    Prim7 wl, wr_unused;
+    plm_cell_s(LdsStencil{&get, 0, 1, 2}, bx_at(jf0 - 1), dtodx2, eos, wl, wr_unused);
+    compiler_fence();
+    put(0, wl);
+  }
+  int sP = 1, sQ = 2, sW = 0, sF = 3;  // rows j-1, j; pending Wl(j); free
+  for (int j = jf0; j <= jf1; j++) {
+    phase_fence();
     {
-      double v1m, b2m, v10, b20, v1u, b2u;
-      load_row(jf0 - 2, 0, v1u, b2u);
-      load_row(jf0 - 1, 1, v1m, b2m);
-      load_row(jf0, 2, v10, b20);
-      src_slot(jf0 - 1) = v1m * (b20 - b2m) / dx2;
-      b2i_slot(jf0) = b20;
-      v1_carry = v10;
+      // row j+1; then s(j) = (M1/d)(j) (B2i(j+1) - B2i(j)) / dx2 (:216-224)
+      double v1n, b2n;
+      load_row(j + 1, sF, v1n, b2n);
+      src_slot(j) = v1_carry * (b2n - b2i_slot(j)) / dx2;
+      b2i_slot(j + 1) = b2n;
+      v1_carry = v1n;
     }
+    phase_fence();
     {
-      Prim7 wl, wr_unused;
-      plm_cell_s(LdsStencil{&get, 0, 1, 2}, bx_at(jf0 - 1), dtodx2, eos, wl, wr_unused);
+      Prim7 wl_next, wr_cur;
+      const LdsStencil sten{&get, sP, sQ, sF};
+      plm_cell_s(sten, bx_at(j), dtodx2, eos, wl_next, wr_cur);
       compiler_fence();
-      put(0, wl);
+      put(kWr, wr_cur);
+      put(sP, wl_next);
     }
-    int sP = 1, sQ = 2, sW = 0, sF = 3;  // rows j-1, j; pending Wl(j); free
-    for (int j = jf0; j <= jf1; j++) {
-      phase_fence();
-      {
-        // row j+1; then s(j) = (M1/d)(j) (B2i(j+1) - B2i(j)) / dx2 (:216-224)
-        double v1n, b2n;
-        load_row(j + 1, sF, v1n, b2n);
-        src_slot(j) = v1_carry * (b2n - b2i_slot(j)) / dx2;
-        b2i_slot(j + 1) = b2n;
-        v1_carry = v1n;
-      }
-      phase_fence();
-      {
-        Prim7 wl_next, wr_cur;
-        const LdsStencil sten{&get, sP, sQ, sF};
-        plm_cell_s(sten, bx_at(j), dtodx2, eos, wl_next, wr_cur);
-        compiler_fence();
-        put(kWr, wr_cur);
-        put(sP, wl_next);
-      }
-      phase_fence();
-      const uint32_t k = (uint32_t)(j * pitch + i);
-      const int sw = sW;
-      // face states: PLM output + MHD source terms for 1/2 dt (:216-224) +
-      // prim->cons (:235-236); rebuilt from LDS for the HLLE fallback
-      auto build = [&](Cons7& ul, Cons7& ur, Prim7& wl, Prim7& wr, double& b0) {
-        compiler_fence();
-        wl = get(sw);
-        wr = get(kWr);
-        b0 = b2i_slot(j);
-        wl.bz = wl.bz + hdt * src_slot(j - 1);
-        wr.bz = wr.bz + hdt * src_slot(j);
-        ul = prim_to_cons(wl, b0, eos);
-        ur = prim_to_cons(wr, b0, eos);
-      };
-      Cons7 ul, ur;
-      Prim7 wl, wr;
-      double b0;
-      build(ul, ur, wl, wr, b0);
-      if (SAVE) {
-        put7(pw + P_WL2 * ps, ps, k, wl);
-        put7(pw + P_WR2 * ps, ps, k, wr);
-      }
-      put7(sc + S_UL2 * ps, ps, k, ul);
-      put7(sc + S_UR2 * ps, ps, k, ur);
-      put7(sc + S_F2 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
-      // rotate: row j -> j-1, row j+1 -> j, Wl(j+1) pending, Wl(j)'s slot free
-      const int nP = sQ, nQ = sF, nW = sP, nF = sW;
-      sP = nP; sQ = nQ; sW = nW; sF = nF;
+    phase_fence();
+    const uint32_t k = (uint32_t)(j * pitch + i);
+    const int sw = sW;
+    // face states: PLM output + MHD source terms for 1/2 dt (:216-224) +
+    // prim->cons (:235-236); rebuilt from LDS for the HLLE fallback
+    auto build = [&](Cons7& ul, Cons7& ur, Prim7& wl, Prim7& wr, double& b0) {
+      compiler_fence();
+      wl = get(sw);
+      wr = get(kWr);
+      b0 = b2i_slot(j);
+      wl.bz = wl.bz + hdt * src_slot(j - 1);
+      wr.bz = wr.bz + hdt * src_slot(j);
+      ul = prim_to_cons(wl, b0, eos);
+      ur = prim_to_cons(wr, b0, eos);
+    };
+    Cons7 ul, ur;
+    Prim7 wl, wr;
+    double b0;
+    build(ul, ur, wl, wr, b0);
+    if (SAVE) {
+      put7(pw + P_WL2 * ps, ps, k, wl);
+      put7(pw + P_WR2 * ps, ps, k, wr);
     }
+    put7(sc + S_UL2 * ps, ps, k, ul);
+    put7(sc + S_UR2 * ps, ps, k, ur);
+    put7(sc + S_F2 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
+    // rotate: row j -> j-1, row j+1 -> j, Wl(j+1) pending, Wl(j)'s slot free
+    const int nP = sQ, nQ = sF, nW = sP, nF = sW;
+    sP = nP; sQ = nQ; sW = nW; sF = nF;
+  }
+}
+template <bool SAVE, int FLUX>
+__global__ void __launch_bounds__(kX2Block, 2) k_pred_x2l(const Inst* __restrict__ insts,
+                                                          int ninst, int ntiles, int seg_len,
+                                                          int remap) {
+  __shared__ X2Slots slots[kX2Slots];
+  __shared__ double aux[kX2Aux][kX2Block];
+  for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x)
+    pred_x2_tile<SAVE, FLUX>(insts, ninst, xcd_tile(t0, ntiles, remap), seg_len, slots, aux,
+                             threadIdx.x);
+}
+
+// Both predictors in one launch (they write disjoint planes). Workgroups
+// [0, nb2) hold two x2 tiles each, one per wave -- the longer marches start
+// first -- and the rest one x1 tile each; both kinds take the 20 KiB of LDS
+// and the registers per wave of two waves per SIMD.
+constexpr int kX2Lds = (kX2Slots * 7 + kX2Aux) * kX2Block;  // doubles of a wave's x2 tile
+constexpr int kX2PerBlock = kX1Block / kX2Block;
+template <bool SAVE, int FLUX>
+__global__ void __launch_bounds__(kX1Block, 2) k_pred(const Inst* __restrict__ insts, int ninst,
+                                                      int n1, int n2, int nb2, int seg_len,
+                                                      int remap) {
+  __shared__ double lds[kX2PerBlock * kX2Lds];
+  static_assert(kX2PerBlock * kX2Lds >= 21 * kX1Block, "the x1 tile's LDS fits the x2 tiles'");
+  const int b = blockIdx.x;
+  if (b < nb2) {
+    const int w = threadIdx.x / kX2Block;
+    const int t = uni(kX2PerBlock * xcd_tile(b, nb2, remap) + w);
+    if (t >= n2) return;
+    double* mine = lds + w * kX2Lds;
+    pred_x2_tile<SAVE, FLUX>(insts, ninst, t, seg_len, (X2Slots*)mine,
+                             (double (*)[kX2Block])(mine + kX2Slots * 7 * kX2Block),
+                             threadIdx.x % kX2Block);
+  } else {
+    double (*const s)[kX1Block] = (double (*)[kX1Block])lds;
+    pred_x1_tile<SAVE, FLUX>(insts, ninst, xcd_tile(b - nb2, n1, remap), s, s + 7,
+                             s + 14);
   }
 }
 
@@ -612,185 +652,204 @@ __global__ void __launch_bounds__(kTileX* kTileY) k_corner(const Inst* __restric
 // stores the corners it owns -- together the range [js-1,je+2]x[is-1,ie+2] --
 // in the corner plane for the x2 part (no k_corner<pred> launch).
 constexpr int kCornerCols = kTileX + 1;
-template <int PART, int TY, int FLUX, bool CP = false>  // TY: rows of a tile of kTileX x TY faces
+template <int PART, int TY, int FLUX, bool CP>  // TY: rows of a tile of kTileX x TY faces
+__device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ninst, int t,
+                                          int strip, const LdsPark& park, double* cemf) {
+  static_assert(!CP || PART == 1, "the corner phase belongs to the x1 part");
+  const Inst& g = insts[find_inst(insts, ninst, K_CORR, t)];
+  const Clock* clk = g.clk;
+  if (!clk->active || g.flux != FLUX) return;
+  const int local = uni(t - g.tile0[K_CORR]);
+  const int gis = uni(g.is), gjs = uni(g.js);
+  int tx, ty;
+  tile_pos(local, dcdiv(uni(g.nx1) + 3, kTileX), dcdiv(uni(g.nx2) + 3, TY), strip, tx, ty);
+  const int i0 = gis - 1 + tx * kTileX, j0 = gjs - 1 + ty * TY;
+  const int i = i0 + threadIdx.x;
+  const int j = j0 + threadIdx.y;
+  if (CP) {
+    // every thread of the block reaches both barriers: the one before the
+    // fill keeps the previous tile's readers ahead of it
+    __syncthreads();
+    double* __restrict__ scw = uni(g.scratch);
+    const size_t psw = (size_t)uni((int)g.ps);
+    const int pw = uni(g.pitch);
+    const int je2 = uni(g.je) + 2, ie2 = uni(g.ie) + 2;
+    for (int c = threadIdx.y * kTileX + threadIdx.x; c < (TY + 1) * kCornerCols;
+         c += kTileX * TY) {
+      const int cr = c / kCornerCols, cl = c - cr * kCornerCols;
+      const int cj = j0 + cr, ci = i0 + cl;
+      double e = 0.0;
+      if (cj <= je2 && ci <= ie2) {
+        e = corner_emf(scw + S_F1 * psw, scw + S_F2 * psw, scw + S_ECC * psw, psw, pw, cj, ci);
+        // owned: the tile's own rows and columns, and the last row and
+        // column of the range where they fall just outside them
+        if ((cr < TY || cj == je2) && (cl < kTileX || ci == ie2))
+          ST(scw + S_EMF * psw, (uint32_t)(cj * pw + ci), e);
+      }
+      cemf[c] = e;
+    }
+    __syncthreads();
+  }
+  if (i > uni(g.ie) + 1 || j > uni(g.je) + 1) return;
+  const double dt = uni(clk->dt);
+  const double dtodx1 = dt / uni(g.dx1), dtodx2 = dt / uni(g.dx2);
+  const double hdtodx1 = 0.5 * dtodx1, hdtodx2 = 0.5 * dtodx2;
+  const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
+  const double* __restrict__ st = uni(g.state[clk->cur]);
+  double* __restrict__ sc = uni(g.scratch);
+  const size_t ps = (size_t)uni((int)g.ps);
+  const int pitch = uni(g.pitch);
+  const uint32_t k = (uint32_t)(j * pitch + i);
+  const double* emf = sc + S_EMF * ps;
+  const double* B1i = st + F_B1I * ps;
+  const double* B2i = st + F_B2I * ps;
+  auto b1h = [&](uint32_t kk) { return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk)); };
+  auto b2h = [&](uint32_t kk) { return LD(B2i, kk) + hdtodx1 * (LD(emf, kk + 1) - LD(emf, kk)); };
+  const double* F1 = sc + S_F1 * ps;
+  const double* F2 = sc + S_F2 * ps;
+  if (PART == 1 && i >= gis) {
+    // corrected x1-face states (Steps 5a, 5b) at the half-step face field;
+    // rebuilt from memory for the HLLE fallback
+    auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
+      compiler_fence();
+      L = get7(sc + S_UL1 * ps, ps, k);
+      R = get7(sc + S_UR1 * ps, ps, k);
+      {  // Step 5a: x2 fluxes at (j+1,i-1),(j,i-1) for L and (j+1,i),(j,i) for R
+        const uint32_t a1 = k + pitch - 1, a0 = k - 1, c1 = k + pitch, c0 = k;
+        L.d = L.d - hdtodx2 * (LD(F2, a1) - LD(F2, a0));
+        L.mx = L.mx - hdtodx2 * (LD(F2 + 3 * ps, a1) - LD(F2 + 3 * ps, a0));
+        L.my = L.my - hdtodx2 * (LD(F2 + 1 * ps, a1) - LD(F2 + 1 * ps, a0));
+        L.mz = L.mz - hdtodx2 * (LD(F2 + 2 * ps, a1) - LD(F2 + 2 * ps, a0));
+        L.e = L.e - hdtodx2 * (LD(F2 + 4 * ps, a1) - LD(F2 + 4 * ps, a0));
+        L.bz = L.bz - hdtodx2 * (LD(F2 + 5 * ps, a1) - LD(F2 + 5 * ps, a0));
+        R.d = R.d - hdtodx2 * (LD(F2, c1) - LD(F2, c0));
+        R.mx = R.mx - hdtodx2 * (LD(F2 + 3 * ps, c1) - LD(F2 + 3 * ps, c0));
+        R.my = R.my - hdtodx2 * (LD(F2 + 1 * ps, c1) - LD(F2 + 1 * ps, c0));
+        R.mz = R.mz - hdtodx2 * (LD(F2 + 2 * ps, c1) - LD(F2 + 2 * ps, c0));
+        R.e = R.e - hdtodx2 * (LD(F2 + 4 * ps, c1) - LD(F2 + 4 * ps, c0));
+        R.bz = R.bz - hdtodx2 * (LD(F2 + 5 * ps, c1) - LD(F2 + 5 * ps, c0));
+      }
+      {  // Step 5b: MHD source terms with the cell-centred field of cells i-1, i
+        double dbx = LD(B1i, k) - LD(B1i, k - 1);
+        double b1 = LD(st + F_B1C * ps, k - 1), b2 = LD(st + F_B2C * ps, k - 1);
+        double b3 = LD(st + F_B3C * ps, k - 1);
+        double v3 = LD(st + F_M3 * ps, k - 1) / LD(st + F_D * ps, k - 1);
+        L.mx = L.mx + hdtodx1 * b1 * dbx;
+        L.my = L.my + hdtodx1 * b2 * dbx;
+        L.mz = L.mz + hdtodx1 * b3 * dbx;
+        L.bz = L.bz + hdtodx1 * v3 * dbx;
+        L.e = L.e + hdtodx1 * b3 * v3 * dbx;
+        dbx = LD(B1i, k + 1) - LD(B1i, k);
+        b1 = LD(st + F_B1C * ps, k); b2 = LD(st + F_B2C * ps, k); b3 = LD(st + F_B3C * ps, k);
+        v3 = LD(st + F_M3 * ps, k) / LD(st + F_D * ps, k);
+        R.mx = R.mx + hdtodx1 * b1 * dbx;
+        R.my = R.my + hdtodx1 * b2 * dbx;
+        R.mz = R.mz + hdtodx1 * b3 * dbx;
+        R.bz = R.bz + hdtodx1 * v3 * dbx;
+        R.e = R.e + hdtodx1 * b3 * v3 * dbx;
+      }
+      if (CP) {
+        const int cc = threadIdx.y * kCornerCols + threadIdx.x;
+        bx = LD(B1i, k) - hdtodx2 * (cemf[cc + kCornerCols] - cemf[cc]);
+      } else {
+        bx = b1h(k);
+      }
+      wl = cons_to_prim(L, bx, eos);
+      wr = cons_to_prim(R, bx, eos);
+    };
+    Cons7 L, R;
+    Prim7 wl, wr;
+    double bx;
+    build(L, R, wl, wr, bx);
+    put7(sc + S_F1C * ps, ps, k, riemann_of<FLUX>(L, R, wl, wr, bx, eos, build, park));
+  }
+  if (PART == 1) return;
+  if (j >= gjs) {
+    // corrected x2-face states (Steps 6a, 6b) at the half-step face field
+    auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
+      compiler_fence();
+      L = get7(sc + S_UL2 * ps, ps, k);
+      R = get7(sc + S_UR2 * ps, ps, k);
+      {  // Step 6a: x1 fluxes at (j-1,i+1),(j-1,i) for L and (j,i+1),(j,i) for R
+        const uint32_t a1 = k - pitch + 1, a0 = k - pitch, c1 = k + 1, c0 = k;
+        L.d = L.d - hdtodx1 * (LD(F1, a1) - LD(F1, a0));
+        L.mx = L.mx - hdtodx1 * (LD(F1 + 2 * ps, a1) - LD(F1 + 2 * ps, a0));
+        L.my = L.my - hdtodx1 * (LD(F1 + 3 * ps, a1) - LD(F1 + 3 * ps, a0));
+        L.mz = L.mz - hdtodx1 * (LD(F1 + 1 * ps, a1) - LD(F1 + 1 * ps, a0));
+        L.e = L.e - hdtodx1 * (LD(F1 + 4 * ps, a1) - LD(F1 + 4 * ps, a0));
+        L.by = L.by - hdtodx1 * (LD(F1 + 6 * ps, a1) - LD(F1 + 6 * ps, a0));
+        R.d = R.d - hdtodx1 * (LD(F1, c1) - LD(F1, c0));
+        R.mx = R.mx - hdtodx1 * (LD(F1 + 2 * ps, c1) - LD(F1 + 2 * ps, c0));
+        R.my = R.my - hdtodx1 * (LD(F1 + 3 * ps, c1) - LD(F1 + 3 * ps, c0));
+        R.mz = R.mz - hdtodx1 * (LD(F1 + 1 * ps, c1) - LD(F1 + 1 * ps, c0));
+        R.e = R.e - hdtodx1 * (LD(F1 + 4 * ps, c1) - LD(F1 + 4 * ps, c0));
+        R.by = R.by - hdtodx1 * (LD(F1 + 6 * ps, c1) - LD(F1 + 6 * ps, c0));
+      }
+      {  // Step 6b: MHD source terms with the cell-centred field of cells j-1, j
+        const uint32_t km = k - pitch;
+        double dby = LD(B2i, k) - LD(B2i, km);
+        double b1 = LD(st + F_B1C * ps, km), b2 = LD(st + F_B2C * ps, km), b3 = LD(st + F_B3C * ps, km);
+        double v3 = LD(st + F_M3 * ps, km) / LD(st + F_D * ps, km);
+        L.mz = L.mz + hdtodx2 * b1 * dby;
+        L.mx = L.mx + hdtodx2 * b2 * dby;
+        L.my = L.my + hdtodx2 * b3 * dby;
+        L.by = L.by + hdtodx2 * v3 * dby;
+        L.e = L.e + hdtodx2 * b3 * v3 * dby;
+        dby = LD(B2i, k + pitch) - LD(B2i, k);
+        b1 = LD(st + F_B1C * ps, k); b2 = LD(st + F_B2C * ps, k); b3 = LD(st + F_B3C * ps, k);
+        v3 = LD(st + F_M3 * ps, k) / LD(st + F_D * ps, k);
+        R.mz = R.mz + hdtodx2 * b1 * dby;
+        R.mx = R.mx + hdtodx2 * b2 * dby;
+        R.my = R.my + hdtodx2 * b3 * dby;
+        R.by = R.by + hdtodx2 * v3 * dby;
+        R.e = R.e + hdtodx2 * b3 * v3 * dby;
+      }
+      bx = b2h(k);
+      wl = cons_to_prim(L, bx, eos);
+      wr = cons_to_prim(R, bx, eos);
+    };
+    Cons7 L, R;
+    Prim7 wl, wr;
+    double bx;
+    build(L, R, wl, wr, bx);
+    put7(sc + S_F2C * ps, ps, k, riemann_of<FLUX>(L, R, wl, wr, bx, eos, build, park));
+  }
+  // Step 7
+  const double dhalf = LD(st + F_D * ps, k) - hdtodx1 * (LD(F1, k + 1) - LD(F1, k)) -
+                       hdtodx2 * (LD(F2, k + pitch) - LD(F2, k));
+  const double m1 = LD(st + F_M1 * ps, k) - hdtodx1 * (LD(F1 + 1 * ps, k + 1) - LD(F1 + 1 * ps, k)) -
+                    hdtodx2 * (LD(F2 + 3 * ps, k + pitch) - LD(F2 + 3 * ps, k));
+  const double m2 = LD(st + F_M2 * ps, k) - hdtodx1 * (LD(F1 + 2 * ps, k + 1) - LD(F1 + 2 * ps, k)) -
+                    hdtodx2 * (LD(F2 + 1 * ps, k + pitch) - LD(F2 + 1 * ps, k));
+  const double b1c = 0.5 * (b1h(k) + b1h(k + 1));
+  const double b2c = 0.5 * (b2h(k) + b2h(k + pitch));
+  ST(sc + S_ECH * ps, k, (b1c * m2 - b2c * m1) / dhalf);
+}
+template <int PART, int TY, int FLUX, bool CP = false>
 __global__ void __launch_bounds__(kTileX* TY, 2) k_corr(const Inst* __restrict__ insts,
                                                             int ninst, int ntiles, int remap,
                                                             int strip) {
-  static_assert(!CP || PART == 1, "the corner phase belongs to the x1 part");
   __shared__ double park_lds[14 * kTileX * TY];
   __shared__ double cemf[CP ? (TY + 1) * kCornerCols : 1];
   const LdsPark park{park_lds, kTileX * TY, (int)(threadIdx.y * kTileX + threadIdx.x)};
-  for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x) {
-    const int t = xcd_tile(t0, ntiles, remap);
-    const Inst& g = insts[find_inst(insts, ninst, K_CORR, t)];
-    const Clock* clk = g.clk;
-    if (!clk->active || g.flux != FLUX) continue;
-    const int local = uni(t - g.tile0[K_CORR]);
-    const int gis = uni(g.is), gjs = uni(g.js);
-    int tx, ty;
-    tile_pos(local, dcdiv(uni(g.nx1) + 3, kTileX), dcdiv(uni(g.nx2) + 3, TY), strip, tx, ty);
-    const int i0 = gis - 1 + tx * kTileX, j0 = gjs - 1 + ty * TY;
-    const int i = i0 + threadIdx.x;
-    const int j = j0 + threadIdx.y;
-    if (CP) {
-      // every thread of the block reaches both barriers: the one before the
-      // fill keeps the previous tile's readers ahead of it
-      __syncthreads();
-      double* __restrict__ scw = uni(g.scratch);
-      const size_t psw = (size_t)uni((int)g.ps);
-      const int pw = uni(g.pitch);
-      const int je2 = uni(g.je) + 2, ie2 = uni(g.ie) + 2;
-      for (int c = threadIdx.y * kTileX + threadIdx.x; c < (TY + 1) * kCornerCols;
-           c += kTileX * TY) {
-        const int cr = c / kCornerCols, cl = c - cr * kCornerCols;
-        const int cj = j0 + cr, ci = i0 + cl;
-        double e = 0.0;
-        if (cj <= je2 && ci <= ie2) {
-          e = corner_emf(scw + S_F1 * psw, scw + S_F2 * psw, scw + S_ECC * psw, psw, pw, cj, ci);
-          // owned: the tile's own rows and columns, and the last row and
-          // column of the range where they fall just outside them
-          if ((cr < TY || cj == je2) && (cl < kTileX || ci == ie2))
-            ST(scw + S_EMF * psw, (uint32_t)(cj * pw + ci), e);
-        }
-        cemf[c] = e;
-      }
-      __syncthreads();
-    }
-    if (i > uni(g.ie) + 1 || j > uni(g.je) + 1) continue;
-    const double dt = uni(clk->dt);
-    const double dtodx1 = dt / uni(g.dx1), dtodx2 = dt / uni(g.dx2);
-    const double hdtodx1 = 0.5 * dtodx1, hdtodx2 = 0.5 * dtodx2;
-    const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
-    const double* __restrict__ st = uni(g.state[clk->cur]);
-    double* __restrict__ sc = uni(g.scratch);
-    const size_t ps = (size_t)uni((int)g.ps);
-    const int pitch = uni(g.pitch);
-    const uint32_t k = (uint32_t)(j * pitch + i);
-    const double* emf = sc + S_EMF * ps;
-    const double* B1i = st + F_B1I * ps;
-    const double* B2i = st + F_B2I * ps;
-    auto b1h = [&](uint32_t kk) { return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk)); };
-    auto b2h = [&](uint32_t kk) { return LD(B2i, kk) + hdtodx1 * (LD(emf, kk + 1) - LD(emf, kk)); };
-    const double* F1 = sc + S_F1 * ps;
-    const double* F2 = sc + S_F2 * ps;
-    if (PART == 1 && i >= gis) {
-      // corrected x1-face states (Steps 5a, 5b) at the half-step face field;
-      // rebuilt from memory for the HLLE fallback
-      auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
-        compiler_fence();
-        L = get7(sc + S_UL1 * ps, ps, k);
-        R = get7(sc + S_UR1 * ps, ps, k);
-        {  // Step 5a: x2 fluxes at (j+1,i-1),(j,i-1) for L and (j+1,i),(j,i) for R
-          const uint32_t a1 = k + pitch - 1, a0 = k - 1, c1 = k + pitch, c0 = k;
-          L.d = L.d - hdtodx2 * (LD(F2, a1) - LD(F2, a0));
-          L.mx = L.mx - hdtodx2 * (LD(F2 + 3 * ps, a1) - LD(F2 + 3 * ps, a0));
-          L.my = L.my - hdtodx2 * (LD(F2 + 1 * ps, a1) - LD(F2 + 1 * ps, a0));
-          L.mz = L.mz - hdtodx2 * (LD(F2 + 2 * ps, a1) - LD(F2 + 2 * ps, a0));
-          L.e = L.e - hdtodx2 * (LD(F2 + 4 * ps, a1) - LD(F2 + 4 * ps, a0));
-          L.bz = L.bz - hdtodx2 * (LD(F2 + 5 * ps, a1) - LD(F2 + 5 * ps, a0));
-          R.d = R.d - hdtodx2 * (LD(F2, c1) - LD(F2, c0));
-          R.mx = R.mx - hdtodx2 * (LD(F2 + 3 * ps, c1) - LD(F2 + 3 * ps, c0));
-          R.my = R.my - hdtodx2 * (LD(F2 + 1 * ps, c1) - LD(F2 + 1 * ps, c0));
-          R.mz = R.mz - hdtodx2 * (LD(F2 + 2 * ps, c1) - LD(F2 + 2 * ps, c0));
-          R.e = R.e - hdtodx2 * (LD(F2 + 4 * ps, c1) - LD(F2 + 4 * ps, c0));
-          R.bz = R.bz - hdtodx2 * (LD(F2 + 5 * ps, c1) - LD(F2 + 5 * ps, c0));
-        }
-        {  // Step 5b: MHD source terms with the cell-centred field of cells i-1, i
-          double dbx = LD(B1i, k) - LD(B1i, k - 1);
-          double b1 = LD(st + F_B1C * ps, k - 1), b2 = LD(st + F_B2C * ps, k - 1);
-          double b3 = LD(st + F_B3C * ps, k - 1);
-          double v3 = LD(st + F_M3 * ps, k - 1) / LD(st + F_D * ps, k - 1);
-          L.mx = L.mx + hdtodx1 * b1 * dbx;
-          L.my = L.my + hdtodx1 * b2 * dbx;
-          L.mz = L.mz + hdtodx1 * b3 * dbx;
-          L.bz = L.bz + hdtodx1 * v3 * dbx;
-          L.e = L.e + hdtodx1 * b3 * v3 * dbx;
-          dbx = LD(B1i, k + 1) - LD(B1i, k);
-          b1 = LD(st + F_B1C * ps, k); b2 = LD(st + F_B2C * ps, k); b3 = LD(st + F_B3C * ps, k);
-          v3 = LD(st + F_M3 * ps, k) / LD(st + F_D * ps, k);
-          R.mx = R.mx + hdtodx1 * b1 * dbx;
-          R.my = R.my + hdtodx1 * b2 * dbx;
-          R.mz = R.mz + hdtodx1 * b3 * dbx;
-          R.bz = R.bz + hdtodx1 * v3 * dbx;
-          R.e = R.e + hdtodx1 * b3 * v3 * dbx;
-        }
-        if (CP) {
-          const int cc = threadIdx.y * kCornerCols + threadIdx.x;
-          bx = LD(B1i, k) - hdtodx2 * (cemf[cc + kCornerCols] - cemf[cc]);
-        } else {
-          bx = b1h(k);
-        }
-        wl = cons_to_prim(L, bx, eos);
-        wr = cons_to_prim(R, bx, eos);
-      };
-      Cons7 L, R;
-      Prim7 wl, wr;
-      double bx;
-      build(L, R, wl, wr, bx);
-      put7(sc + S_F1C * ps, ps, k, riemann_of<FLUX>(L, R, wl, wr, bx, eos, build, park));
-    }
-    if (PART == 1) continue;
-    if (j >= gjs) {
-      // corrected x2-face states (Steps 6a, 6b) at the half-step face field
-      auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
-        compiler_fence();
-        L = get7(sc + S_UL2 * ps, ps, k);
-        R = get7(sc + S_UR2 * ps, ps, k);
-        {  // Step 6a: x1 fluxes at (j-1,i+1),(j-1,i) for L and (j,i+1),(j,i) for R
-          const uint32_t a1 = k - pitch + 1, a0 = k - pitch, c1 = k + 1, c0 = k;
-          L.d = L.d - hdtodx1 * (LD(F1, a1) - LD(F1, a0));
-          L.mx = L.mx - hdtodx1 * (LD(F1 + 2 * ps, a1) - LD(F1 + 2 * ps, a0));
-          L.my = L.my - hdtodx1 * (LD(F1 + 3 * ps, a1) - LD(F1 + 3 * ps, a0));
-          L.mz = L.mz - hdtodx1 * (LD(F1 + 1 * ps, a1) - LD(F1 + 1 * ps, a0));
-          L.e = L.e - hdtodx1 * (LD(F1 + 4 * ps, a1) - LD(F1 + 4 * ps, a0));
-          L.by = L.by - hdtodx1 * (LD(F1 + 6 * ps, a1) - LD(F1 + 6 * ps, a0));
-          R.d = R.d - hdtodx1 * (LD(F1, c1) - LD(F1, c0));
-          R.mx = R.mx - hdtodx1 * (LD(F1 + 2 * ps, c1) - LD(F1 + 2 * ps, c0));
-          R.my = R.my - hdtodx1 * (LD(F1 + 3 * ps, c1) - LD(F1 + 3 * ps, c0));
-          R.mz = R.mz - hdtodx1 * (LD(F1 + 1 * ps, c1) - LD(F1 + 1 * ps, c0));
-          R.e = R.e - hdtodx1 * (LD(F1 + 4 * ps, c1) - LD(F1 + 4 * ps, c0));
-          R.by = R.by - hdtodx1 * (LD(F1 + 6 * ps, c1) - LD(F1 + 6 * ps, c0));
-        }
-        {  // Step 6b: MHD source terms with the cell-centred field of cells j-1, j
-          const uint32_t km = k - pitch;
-          double dby = LD(B2i, k) - LD(B2i, km);
-          double b1 = LD(st + F_B1C * ps, km), b2 = LD(st + F_B2C * ps, km), b3 = LD(st + F_B3C * ps, km);
-          double v3 = LD(st + F_M3 * ps, km) / LD(st + F_D * ps, km);
-          L.mz = L.mz + hdtodx2 * b1 * dby;
-          L.mx = L.mx + hdtodx2 * b2 * dby;
-          L.my = L.my + hdtodx2 * b3 * dby;
-          L.by = L.by + hdtodx2 * v3 * dby;
-          L.e = L.e + hdtodx2 * b3 * v3 * dby;
-          dby = LD(B2i, k + pitch) - LD(B2i, k);
-          b1 = LD(st + F_B1C * ps, k); b2 = LD(st + F_B2C * ps, k); b3 = LD(st + F_B3C * ps, k);
-          v3 = LD(st + F_M3 * ps, k) / LD(st + F_D * ps, k);
-          R.mz = R.mz + hdtodx2 * b1 * dby;
-          R.mx = R.mx + hdtodx2 * b2 * dby;
-          R.my = R.my + hdtodx2 * b3 * dby;
-          R.by = R.by + hdtodx2 * v3 * dby;
-          R.e = R.e + hdtodx2 * b3 * v3 * dby;
-        }
-        bx = b2h(k);
-        wl = cons_to_prim(L, bx, eos);
-        wr = cons_to_prim(R, bx, eos);
-      };
-      Cons7 L, R;
-      Prim7 wl, wr;
-      double bx;
-      build(L, R, wl, wr, bx);
-      put7(sc + S_F2C * ps, ps, k, riemann_of<FLUX>(L, R, wl, wr, bx, eos, build, park));
-    }
-    // Step 7
-    const double dhalf = LD(st + F_D * ps, k) - hdtodx1 * (LD(F1, k + 1) - LD(F1, k)) -
-                         hdtodx2 * (LD(F2, k + pitch) - LD(F2, k));
-    const double m1 = LD(st + F_M1 * ps, k) - hdtodx1 * (LD(F1 + 1 * ps, k + 1) - LD(F1 + 1 * ps, k)) -
-                      hdtodx2 * (LD(F2 + 3 * ps, k + pitch) - LD(F2 + 3 * ps, k));
-    const double m2 = LD(st + F_M2 * ps, k) - hdtodx1 * (LD(F1 + 2 * ps, k + 1) - LD(F1 + 2 * ps, k)) -
-                      hdtodx2 * (LD(F2 + 1 * ps, k + pitch) - LD(F2 + 1 * ps, k));
-    const double b1c = 0.5 * (b1h(k) + b1h(k + 1));
-    const double b2c = 0.5 * (b2h(k) + b2h(k + pitch));
-    ST(sc + S_ECH * ps, k, (b1c * m2 - b2c * m1) / dhalf);
-  }
+  for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x)
+    corr_tile<PART, TY, FLUX, CP>(insts, ninst, xcd_tile(t0, ntiles, remap), strip, park, cemf);
+}
+
+// Both parts in one launch (they read the same planes and write disjoint
+// ones): workgroups [0, ntiles) the x2 part with Step 7, the rest the x1 part.
+template <int TY, int FLUX>
+__global__ void __launch_bounds__(kTileX* TY, 2) k_corr_both(const Inst* __restrict__ insts,
+                                                             int ninst, int ntiles, int remap,
+                                                             int strip) {
+  __shared__ double park_lds[14 * kTileX * TY];
+  const LdsPark park{park_lds, kTileX * TY, (int)(threadIdx.y * kTileX + threadIdx.x)};
+  const int b = blockIdx.x;
+  if (b < ntiles)
+    corr_tile<2, TY, FLUX, false>(insts, ninst, xcd_tile(b, ntiles, remap), strip, park, nullptr);
+  else
+    corr_tile<1, TY, FLUX, false>(insts, ninst, xcd_tile(b - ntiles, ntiles, remap), strip, park,
+                                  nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1154,6 +1213,18 @@ static CorrKernel corr_kernel(int part, int ty, int flux, bool cp) {
 }
 
 // persistent grids: persist x per_cu workgroups per CU (persist 0: one per tile)
+// Whether the two sweeps share a launch: everywhere but on persistent grids
+// (their workgroups loop over one tile kind) and with the register form of the
+// x2 predictor (another workgroup shape). A small grid's step is the sum of its
+// launches' latencies (64^2 Roe 79 -> 58 us), a middle one saves the nearly empty last
+// round of waves of one launch (512^2 182 -> 162 us, 1024^2 557 -> 521), and 4096^2
+// goes 7.34 -> 7.06 ms. Ordering the two kinds in turns instead of one after the
+// other, so that they share their planes in L2, was slower (predictors 4-8%,
+// correctors 1-2% of the step): the mixed kernels miss the instruction cache.
+static bool merge_sweeps(const BatchLaunch& b) {
+  return b.shape.persist <= 0 && b.shape.x2_kind == 1;
+}
+
 static int grid_of(const BatchLaunch& b, int kind, int per_cu) {
   const int n = b.ntiles[kind];
   if (b.shape.persist <= 0) return n;
@@ -1203,6 +1274,26 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
                            b.ninst, b.ntiles[K_PRED_X2], b.shape.x2_seg, b.shape.xcd_remap);
       }
       break;
+    case SK_PRED:
+    case SK_PRED_SAVE: {
+      const bool save = kernel == SK_PRED_SAVE;
+      if (!merge_sweeps(b)) {
+        const hipError_t e =
+            ATHMI_FN(launch)(bl, save ? SK_PRED_X1_SAVE : SK_PRED_X1, s);
+        if (e != hipSuccess) return e;
+        return ATHMI_FN(launch)(bl, save ? SK_PRED_X2_SAVE : SK_PRED_X2, s);
+      }
+      const int n1 = b.ntiles[K_PRED_X1], n2 = b.ntiles[K_PRED_X2];
+      const int nb2 = cdiv(n2, kX2PerBlock);
+      for (int f = 0; f < 2; f++) {
+        if (!(b.flux_mask & (1 << f))) continue;
+        const auto fn = f == kFluxHlle ? (save ? k_pred<true, kFluxHlle> : k_pred<false, kFluxHlle>)
+                                       : (save ? k_pred<true, kFluxRoe> : k_pred<false, kFluxRoe>);
+        hipLaunchKernelGGL(fn, dim3(n1 + nb2), dim3(kX1Block), 0, s, b.insts, b.ninst, n1, n2, nb2,
+                           b.shape.x2_seg, b.shape.xcd_remap);
+      }
+      break;
+    }
     case SK_CORNER_P:
       // at fusion depth 2 the x1 corrector computes these corners
       if (b.shape.fuse_corner >= 2) break;
@@ -1220,6 +1311,26 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         if (!(b.flux_mask & (1 << f))) continue;
         const CorrKernel fn = corr_kernel(x1 ? 1 : 2, ty, f, b.shape.fuse_corner >= 2);
         hipLaunchKernelGGL(fn, grid, blk, 0, s, b.insts, b.ninst, b.ntiles[K_CORR],
+                           b.shape.xcd_remap, b.shape.strip);
+      }
+      break;
+    }
+    case SK_CORR_BOTH: {
+      if (!merge_sweeps(b) || b.shape.fuse_corner >= 2) {
+        const hipError_t e = ATHMI_FN(launch)(bl, SK_CORR, s);
+        if (e != hipSuccess) return e;
+        return ATHMI_FN(launch)(bl, SK_CORR2, s);
+      }
+      const int ty = b.shape.corr_rows, n = b.ntiles[K_CORR];
+      for (int f = 0; f < 2; f++) {
+        if (!(b.flux_mask & (1 << f))) continue;
+        const CorrKernel fn =
+            f == kFluxHlle
+                ? (ty == 1 ? k_corr_both<1, kFluxHlle>
+                           : ty == 2 ? k_corr_both<2, kFluxHlle> : k_corr_both<4, kFluxHlle>)
+                : (ty == 1 ? k_corr_both<1, kFluxRoe>
+                           : ty == 2 ? k_corr_both<2, kFluxRoe> : k_corr_both<4, kFluxRoe>);
+        hipLaunchKernelGGL(fn, dim3(2 * n), dim3(kTileX, ty), 0, s, b.insts, b.ninst, n,
                            b.shape.xcd_remap, b.shape.strip);
       }
       break;

@@ -188,6 +188,9 @@ enum StepKernel {
   SK_DIVB,
   SK_PRED_X1_SAVE,    // predictors that also store their primitive face states
   SK_PRED_X2_SAVE,    // (Inst::prims), for the adjoint's re-run
+  SK_PRED,            // both predictors, both corrector parts: one launch or two, by the
+  SK_PRED_SAVE,       // batch's size
+  SK_CORR_BOTH,
   SK_COUNT
 };
 
