@@ -26,17 +26,19 @@
 namespace {
 
 // forward scratch of one step: predictor, predictor corner emf, corrector fluxes
-const int kSeqForwardScratch[] = {SK_BEGIN_ONCE, SK_PRED_SAVE, SK_CORNER_P, SK_CORR_BOTH};
-// the rest of integrate_2d after kSeqForwardScratch, and the set_bvals that
+const int kSeqForwardScratch[] = {SK_PRED_SAVE, SK_CORNER_P, SK_CORR_BOTH};
+// the rest of integrate_2d after kSeqForwardScratch and the set_bvals that
 // follows it. integrate_2d leaves the ghost cells as they were (the drop-in's
 // carry copies them into the new buffer), but the set_bvals right after it
 // writes every ghost cell from non-ghost ones when Nx1, Nx2 >= 4, which the
-// adjoint requires: its steps skip the carry
-const int kSeqFinishStep[] = {SK_CORNER_C, SK_FINAL, SK_END_ONCE};
-const int kSeqGhostCur[] = {SK_GHOST_CUR};
-// a whole step so: integrate_2d without the carry (then set_bvals)
-const int kSeqRolloutStep[] = {SK_BEGIN_ONCE, SK_PRED,  SK_CORNER_P, SK_CORR_BOTH,
-                               SK_CORNER_C,   SK_FINAL, SK_END_ONCE};
+// adjoint requires: its steps skip the carry, and the final kernel fills the
+// ghosts
+const int kSeqFinishStep[] = {SK_CORNER_C, SK_FINAL_GHOST, SK_END_ONCE};
+// a whole step so: integrate_2d without the carry, and set_bvals
+const int kSeqRolloutStep[] = {SK_PRED,     SK_CORNER_P,    SK_CORR_BOTH,
+                               SK_CORNER_C, SK_FINAL_GHOST, SK_END_ONCE};
+// dt never changes along a rollout: the clock is started once per run of steps
+const int kSeqStart[] = {SK_BEGIN_ONCE};
 // the reverse of one step on two streams: the x1 and x2 halves of Steps 8
 // and 1-2 are independent (their adjoints meet in ain through atomic adds)
 const int kRevHead[] = {AK_FOLD_OUT, AK_ZERO, AK_UPDATE, AK_CORNER_C};  // then fork
@@ -103,7 +105,6 @@ static int rollout_step(athmi_adjoint* h) {
   int rc = adj_issue(h, kSeqRolloutStep, sizeof(kSeqRolloutStep) / sizeof(int));
   if (rc) return rc;
   h->cur ^= 1;  // k_end swaps the buffers
-  HIP_TRY(h->g->launch(&h->g->bl, SK_GHOST_CUR, h->g->stream));
   return ATHMI_OK;
 }
 
@@ -143,6 +144,7 @@ static int rerun_segment(athmi_adjoint* h, int s, int b, bool finish_last = fals
   const Inst* slots = h->dslot + (size_t)(2 * b + h->cur) * h->every;
   int rc;
   if ((rc = copy_state(h, h->seg_state(b, 0), h->ck + (size_t)s * h->state_doubles))) return rc;
+  if ((rc = adj_issue(h, kSeqStart, 1))) return rc;
   for (int m = n0; m < n1; m++) {
     const Inst* ins = slots + (m - n0);
     double* sc = h->slot(b, m - n0);
@@ -157,7 +159,6 @@ static int rerun_segment(athmi_adjoint* h, int s, int b, bool finish_last = fals
     if (m + 1 < n1 || finish_last) {
       if ((rc = issue_on(h, ins, kSeqFinishStep, sizeof(kSeqFinishStep) / sizeof(int)))) return rc;
       h->cur ^= 1;  // k_end swaps the buffers: the output is seg[b][m + 1]
-      if ((rc = issue_on(h, ins, kSeqGhostCur, 1))) return rc;
     }
   }
   return ATHMI_OK;
@@ -290,6 +291,7 @@ int athmi_adjoint_forward(athmi_adjoint* h, const double* state0, double* stateN
   h->last_filled = false;
   if ((rc = dense_to_planes(h, live_state(h), state0, h->g->stream))) return rc;
   HIP_TRY(h->g->launch(&h->g->bl, SK_GHOST_CUR, h->g->stream));
+  if ((rc = adj_issue(h, kSeqStart, 1))) return rc;
   const int slast = h->nck - 1, blast = slast % h->nbank;
   for (int n = 0; n < slast * h->every; n++) {
     if (n % h->every == 0 &&

@@ -324,6 +324,7 @@ int athmi_set_bvals(athmi_grid* g) {
 
 int athmi_new_dt(athmi_grid* g) {
   if (!g) return fail(ATHMI_EINVAL, "null handle");
+  g->clock_written = true;  // by the device
   int rc = issue(g, kSeqNewDt);
   if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(g->stream));
@@ -334,6 +335,7 @@ int athmi_new_dt(athmi_grid* g) {
 // buffer carry the current values, as an in-place update would leave them
 int athmi_integrate(athmi_grid* g) {
   if (!g) return fail(ATHMI_EINVAL, "null handle");
+  g->clock_written = true;  // SK_BEGIN_ONCE
   return issue(g, kSeqIntegrate);
 }
 
@@ -341,6 +343,12 @@ static int issue_step(athmi_grid* g) { return issue(g, kSeqStep); }
 
 int athmi_step(athmi_grid* g) {
   if (!g) return fail(ATHMI_EINVAL, "null handle");
+  // without the graph every step starts itself: its launches may be captured
+  // by the caller and replayed after the host has written the clock
+  if (g->clock_written || !g->use_graph) {
+    HIP_TRY(g->launch(&g->bl, SK_BEGIN_STEP, g->stream));
+    g->clock_written = !g->use_graph;
+  }
   if (!g->use_graph) return issue_step(g);
   if (!g->graph) {
     hipGraph_t graph;
@@ -406,6 +414,7 @@ int athmi_profile_steps(athmi_grid* g, int nsteps, double* avg_ms, int nslots) {
   std::vector<hipEvent_t> ev(kStepLen + 1);
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
   for (int k = 0; k < kStepLen; k++) avg_ms[k] = 0.0;
+  g->clock_written = true;
   for (int s = 0; s < nsteps; s++) {
     HIP_TRY(hipEventRecord(ev[0], g->stream));
     for (int k = 0; k < kStepLen; k++) {
@@ -490,6 +499,7 @@ int athmi_autotune(athmi_grid* g, int steps, int* x2_seg, int* persist, int* xcd
     }
     HIP_TRY(hipMemcpyAsync(g->dclk, hc.data(), sizeof(Clock) * g->n, hipMemcpyHostToDevice,
                            g->stream));
+    g->clock_written = true;
     HIP_TRY(hipStreamSynchronize(g->stream));
     return ATHMI_OK;
   };

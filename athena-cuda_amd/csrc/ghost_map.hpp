@@ -141,4 +141,40 @@ __device__ __forceinline__ bool ghost_src(const Inst& g, int f, int j, int i, in
   return ghost_src(g, f, j, i, sj, si, neg, stale);
 }
 
+// The same map from the source's side, for Nx1, Nx2 >= 4 (every ghost copies
+// one non-ghost cell): the ghosts along one direction that copy index c of an
+// interior lo..hi, as a mask -- bit k-1: index lo - k, bit 3+k: hi + k, for
+// k = 1..4. face: a plane whose index hi + 1 is not a ghost.
+__device__ __forceinline__ unsigned ghost_images(int c, int lo, int hi, int bc_lo, int bc_hi,
+                                                 bool face) {
+  unsigned m = 0;
+#pragma unroll
+  for (int k = 1; k <= 4; k++) {
+    const int a = bc_lo == BC_PERIODIC ? hi - (k - 1) : (bc_lo == BC_OUTFLOW ? lo : lo + (k - 1));
+    if (a == c) m |= 1u << (k - 1);
+    if (face && k == 1) continue;
+    const int b = bc_hi == BC_PERIODIC ? lo + (k - 1)
+                                       : (bc_hi == BC_OUTFLOW ? hi : hi - (k - (face ? 2 : 1)));
+    if (b == c) m |= 1u << (3 + k);
+  }
+  return m;
+}
+
+// calls put(row, column, nx, ny) for every ghost that copies cell (j, i), given
+// its image masks along x1 and x2; nx, ny: the x1 / x2 fill reflects
+template <class Put>
+__device__ __forceinline__ void for_ghost_images(const Inst& g, int j, int i, unsigned mx,
+                                                 unsigned my, Put put) {
+  for (unsigned ry = (my << 1) | 1u; ry; ry &= ry - 1) {
+    const int b = __builtin_ctz(ry);  // 0: row j itself
+    const int r = b == 0 ? j : (b <= 4 ? g.js - b : g.je + (b - 4));
+    const bool ny = b > 0 && (b <= 4 ? g.bc[2] : g.bc[3]) == BC_REFLECT;
+    for (unsigned rx = (mx << 1) | (b ? 1u : 0u); rx; rx &= rx - 1) {
+      const int a = __builtin_ctz(rx);
+      const int c = a == 0 ? i : (a <= 4 ? g.is - a : g.ie + (a - 4));
+      put(r, c, a > 0 && (a <= 4 ? g.bc[0] : g.bc[1]) == BC_REFLECT, ny);
+    }
+  }
+}
+
 }  // namespace athmi

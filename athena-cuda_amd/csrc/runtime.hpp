@@ -48,10 +48,12 @@ hipError_t launch_state_pack(const double* st, double* stage, size_t ps, int pit
 namespace athmi_rt {
 
 // kernel sequences of the reference's routines
-const int kSeqStep[] = {SK_BEGIN_STEP, SK_PRED,  SK_CORNER_P,   SK_CORR_BOTH,
-                        SK_CORNER_C,   SK_FINAL, SK_GHOST_NEXT, SK_END_STEP};
-const int kSeqIntegrate[] = {SK_BEGIN_ONCE, SK_PRED,  SK_CORNER_P,    SK_CORR_BOTH,
-                             SK_CORNER_C,   SK_FINAL, SK_GHOST_CARRY, SK_END_ONCE};
+// (a main-loop step is started by the k_end before it, or by SK_BEGIN_STEP
+// once the host has written the clock: athmi_grid::clock_written)
+const int kSeqStep[] = {SK_PRED, SK_CORNER_P, SK_CORR_BOTH, SK_CORNER_C, SK_FINAL_GHOST,
+                        SK_END_STEP};
+const int kSeqIntegrate[] = {SK_BEGIN_ONCE, SK_PRED,  SK_CORNER_P_CARRY, SK_CORR_BOTH,
+                             SK_CORNER_C,   SK_FINAL, SK_END_ONCE};
 // the step one kernel at a time, as athmi_profile_steps times it
 const int kSeqProfile[] = {SK_BEGIN_STEP, SK_PRED_X1, SK_PRED_X2, SK_CORNER_P,   SK_CORR,
                            SK_CORR2,      SK_CORNER_C, SK_FINAL,  SK_GHOST_NEXT, SK_END_STEP};
@@ -83,6 +85,7 @@ struct athmi_grid {
   bool own_stream = false;
   bool use_graph = true;
   hipGraphExec_t graph = nullptr;
+  bool clock_written = true;  // the host wrote a clock since the last main-loop step
   std::vector<std::vector<double>> cpaw_soln;  // initial cpaw2d states (8 planes)
   void* outbuf = nullptr;                      // device staging of the output formats
   size_t outbuf_bytes = 0;
@@ -104,7 +107,9 @@ struct athmi_grid {
     for (int kind = 0; kind < NKINDS; kind++) bl.ntiles[kind] = tot[kind];
     bl.flux_mask = 0;
     bl.stale_ghosts = 0;
+    bl.thin = 0;
     for (int k = 0; k < n; k++) {
+      if (hinst[k].nx1 < 4 || hinst[k].nx2 < 4) bl.thin = 1;
       bl.flux_mask |= 1 << hinst[k].flux;
       if (ghost_fill_reads_stale(hinst[k])) bl.stale_ghosts = 1;
     }
@@ -119,6 +124,7 @@ struct athmi_grid {
     return ATHMI_OK;
   }
   int write_clock_head(int k, const Clock& c) {
+    clock_written = true;
     HIP_TRY(hipMemcpy(dclk + k, &c, offsetof(Clock, divb_bits), hipMemcpyHostToDevice));
     return ATHMI_OK;
   }

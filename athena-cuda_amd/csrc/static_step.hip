@@ -45,6 +45,7 @@ __global__ void k_static_head(athmi::Inst inst, athmi::Clock* clk_dst, athmi::In
   __syncthreads();
   if (threadIdx.x == 0) {
     clk_dst->dt = dt;
+    clk_dst->dts = dt;
     clk_dst->cour_no = cour_no;
     clk_dst->tlim = HUGE_VAL;
     clk_dst->tpause = HUGE_VAL;
@@ -55,12 +56,11 @@ __global__ void k_static_head(athmi::Inst inst, athmi::Clock* clk_dst, athmi::In
   }
 }
 
-// zero n doubles (the scratch planes this call uses keep no earlier call's data)
-__global__ void __launch_bounds__(256) k_static_clear(double* p, size_t n) {
-  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (size_t)gridDim.x * blockDim.x)
-    p[e] = 0.0;
-}
+// integrate_2d after the head kernel has started the clock; the ping-pong
+// index and the dt reduction are not read back, so no clock kernel follows.
+// The scratch planes keep earlier calls' data: every plane is written by this
+// call over the range its readers cover.
+const int kSeqStatic[] = {SK_PRED, SK_CORNER_P_CARRY, SK_CORR_BOTH, SK_FINAL};
 
 int resolve(int dev, unsigned char** ptr, int* ncu) {
   if (dev < 0 || dev >= kMaxDevices)
@@ -153,8 +153,7 @@ int athmi_integrate_static(const athmi_desc* desc, double dt, const double* stat
   I.gamma = d.gamma;
   I.g1 = d.gamma - 1.0;  // main.c:93-94
   I.g2 = d.gamma - 2.0;
-  // state[cur = 0] is read, state[1] receives the integrated state (k_end's
-  // swap of the clock's index is not read back)
+  // state[cur = 0] is read, state[1] receives the integrated state
   I.state[0] = const_cast<double*>(state_in);
   I.state[1] = state_out;
   I.scratch = dscratch;
@@ -173,6 +172,7 @@ int athmi_integrate_static(const athmi_desc* desc, double dt, const double* stat
   bl.shape.corr_rows = 2;
   bl.shape.final_rows = 8;
   bl.shape.x2_kind = 1;
+  bl.shape.fuse_corner = 1;
   for (int kind = 0; kind < NKINDS; kind++) {
     I.tile0[kind] = 0;
     bl.ntiles[kind] = tiles_of(kind, d.nx1, d.nx2, bl.shape.x2_seg, bl.shape.corr_rows,
@@ -183,13 +183,8 @@ int athmi_integrate_static(const athmi_desc* desc, double dt, const double* stat
   const hipStream_t s = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(k_static_head, dim3(1), dim3(256), 0, s, I, dclk, dinst, dt, d.cour_no);
   HIP_TRY(hipGetLastError());
-  const size_t nclear = (size_t)NSCRATCH * plane_stride;
-  const size_t blocks = (nclear + 255) / 256;
-  hipLaunchKernelGGL(k_static_clear, dim3(blocks < 8192 ? (unsigned)blocks : 8192u), dim3(256),
-                     0, s, dscratch, nclear);
-  HIP_TRY(hipGetLastError());
   const LaunchFn launch = (d.variant == ATHMI_FAST) ? athmi_fast_launch : athmi_exact_launch;
-  for (int k : athmi_rt::kSeqIntegrate) HIP_TRY(launch(&bl, k, s));
+  for (int k : kSeqStatic) HIP_TRY(launch(&bl, k, s));
   return ATHMI_OK;
 }
 

@@ -3,7 +3,8 @@
 // gfx950 over a tile work-list spanning one or many grid instances.
 //
 // Pipeline of one step (all state in SoA planes, ping-pong buffers):
-//   k_begin      clock: limits, tlim clamp of dt, reset of dt partials
+//   k_begin      clock: limits, tlim clamp of dt, reset of dt partials (only when the
+//                host has written the clock: k_end starts the next step)
 //   k_pred       both sweeps' predictors in one launch: the tiles of
 //     k_pred_x1  Steps 1a-1e: x1 sweep, PLM via an LDS neighbour exchange
 //     k_pred_x2l Steps 2a-2e: x2 sweep, each lane marches down a column
@@ -12,8 +13,10 @@
 //                parts of k_corr in one launch
 //   k_corner<C>  Step 9 corner emf
 //   k_final      Steps 9 (face B), 11a/11b, 13 and the new_dt max, fused
-//   k_ghost      set_bvals on the new state
-//   k_end        nstep++, time += dt, dt = min(2 dt, CourNo/max_dti), swap
+//                and, from the source's side, set_bvals on the new state
+//   k_ghost      set_bvals by itself (a standalone call, grids under 4 cells)
+//   k_end        nstep++, time += dt, dt = min(2 dt, CourNo/max_dti), swap, and the
+//                limits and dt of the next step
 //
 // This file is compiled twice: ATHMI_VARIANT=exact with -ffp-contract=off
 // (one rounding per operation, as the reference CPU build) and
@@ -209,7 +212,7 @@ __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int
   const int j = uni(g.js) - 2 + row;
   const int f0 = gis - 1 + seg * kX1Faces;
   const int cell = f0 - 2 + tid;
-  const double dt = uni(clk->dt);
+  const double dt = uni(clk->dts);
   const double dx1 = uni(g.dx1);
   const double dtodx1 = dt / dx1;
   const double hdt = 0.5 * dt;
@@ -308,7 +311,7 @@ __global__ void __launch_bounds__(kX2Block) k_pred_x2(const Inst* __restrict__ i
     if (i > g.ie + 2) continue;
     const int jf0 = g.js - 1 + sg * seg_len;
     const int jf1 = min(jf0 + seg_len - 1, g.je + 2);
-    const double dt = clk->dt;
+    const double dt = clk->dts;
     const double dtodx2 = dt / g.dx2;
     const double hdt = 0.5 * dt;
     const EosC eos{g.gamma, g.g1, g.g2};
@@ -443,7 +446,7 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
   if (i > uni(g.ie) + 2) return;
   const int jf0 = uni(g.js) - 1 + sg * seg_len;
   const int jf1 = min(jf0 + seg_len - 1, uni(g.je) + 2);
-  const double dt = uni(clk->dt);
+  const double dt = uni(clk->dts);
   const double dx2 = uni(g.dx2);
   const double dtodx2 = dt / dx2;
   const double hdt = 0.5 * dt;
@@ -604,15 +607,68 @@ __device__ __forceinline__ double corner_emf(const double* F1, const double* F2,
 }
 
 // ---------------------------------------------------------------------------
+// cell (j, i) of thread `tid` of ghost tile t: the ghost rows, then the ghost
+// columns of the other rows (both ends, and the face row / column past them)
+__device__ __forceinline__ bool ghost_cell(const Inst& g, int t, int tid, int& j, int& i) {
+  const int e = (t - g.tile0[K_GHOST]) * kGhostBlock + tid;
+  const int nrow = 8 * g.sx;
+  if (e >= nrow + (g.nx2 + 1) * 8) return false;
+  if (e < nrow) {
+    const int r = e / g.sx;
+    i = e - r * g.sx;
+    j = (r < 4) ? r : g.je + 1 + (r - 4);
+  } else {
+    const int e2 = e - nrow;
+    const int r = e2 >> 3, c = e2 & 7;
+    j = g.js + r;
+    i = (c < 4) ? c : g.ie + 1 + (c - 4);
+  }
+  return true;
+}
+
+// ghost tile t of buffer cur carried unchanged into the other one (an
+// in-place integrate_2d leaves the ghost zones as they were)
+__device__ __forceinline__ void ghost_carry(const Inst& g, int cur, int t) {
+  int j, i;
+  if (!ghost_cell(g, t, threadIdx.x + threadIdx.y * blockDim.x, j, i)) return;
+  const double* __restrict__ src = g.state[cur];
+  double* __restrict__ dst = g.state[cur ^ 1];
+  const size_t ps = g.ps;
+  const uint32_t k = (uint32_t)(j * g.pitch + i);
+  const bool gx = i < g.is || i > g.ie, gy = j < g.js || j > g.je;
+  double v[NSTATE];
+#pragma unroll
+  for (int f = 0; f < NSTATE; f++) v[f] = LD(src + f * ps, k);
+#pragma unroll
+  for (int f = 0; f < NSTATE; f++) {
+    // the face at ie+1 of B1i (je+1 of B2i) is not a ghost
+    const bool ghost = f == F_B1I   ? (gy || i < g.is || i > g.ie + 1)
+                       : f == F_B2I ? (gx || j < g.js || j > g.je + 1)
+                                    : (gx || gy);
+    if (ghost) ST(dst + f * ps, k, v[f]);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // integrate_emf3_corner (__integrate_2d__.c:632-702): upwinded corner emf from
 // the face fluxes (x1-flux of B2 is -E3, x2-flux of B1 is +E3) and the
 // cell-centred emf3. PRED: Step 4 over [js-1,je+2]x[is-1,ie+2] from predictor
 // fluxes; otherwise Step 9 over [js,je+1]x[is,ie+1], the corners Step 9 uses.
+// The first ncarry workgroups (PRED) carry the ghost zones of an in-place
+// integrate_2d into the produced buffer, which no kernel of the step reads.
 template <bool PRED>
 __global__ void __launch_bounds__(kTileX* kTileY) k_corner(const Inst* __restrict__ insts,
-                                                            int ninst, int ntiles, int remap) {
+                                                            int ninst, int ntiles, int remap,
+                                                            int ncarry) {
   const int kind = PRED ? K_CORNER_P : K_CORNER_C;
-  for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x) {
+  static_assert(kTileX * kTileY == kGhostBlock, "a workgroup also fits a ghost tile");
+  if (PRED && (int)blockIdx.x < ncarry) {
+    const int t = blockIdx.x;
+    const Inst& g = insts[find_inst(insts, ninst, K_GHOST, t)];
+    ghost_carry(g, g.clk->cur, t);
+    return;
+  }
+  for (int t0 = blockIdx.x - ncarry; t0 < ntiles; t0 += gridDim.x - ncarry) {
     const int t = xcd_tile(t0, ntiles, remap);
     const Inst& g = insts[find_inst(insts, ninst, kind, t)];
     if (!g.clk->active) continue;
@@ -691,7 +747,7 @@ __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ni
     __syncthreads();
   }
   if (i > uni(g.ie) + 1 || j > uni(g.je) + 1) return;
-  const double dt = uni(clk->dt);
+  const double dt = uni(clk->dts);
   const double dtodx1 = dt / uni(g.dx1), dtodx2 = dt / uni(g.dx2);
   const double hdtodx1 = 0.5 * dtodx1, hdtodx2 = 0.5 * dtodx2;
   const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
@@ -893,10 +949,15 @@ __device__ __forceinline__ int cell_fail_bits(const Inst& g, double d, double M1
 // write and read fewer). TY: rows of a tile of kTileX x TY cells; the taller,
 // the smaller the share of halo rows (corners and x2 fluxes of the row below)
 // that the tile reads a second time.
+// fill: each cell is also stored into the ghosts that copy it (set_bvals,
+// grids of at least 4 x 4 cells). A ghost launch of its own is a chain of
+// dependent loads of 8-15 us at any size that re-reads what this kernel holds
+// in registers; without it and the clock launch at the step's start 64^2 takes
+// 58 -> 49 us a step, 512^2 162 -> 151, 1024^2 521 -> 512, 4096^2 7.06 -> 7.05 ms.
 template <bool FUSED, int TY>
 __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ insts,
                                                        int ninst, int ntiles, int remap,
-                                                       int strip) {
+                                                       int strip, int fill) {
   __shared__ double red[TY];  // kTileX x TY threads: TY waves
   __shared__ double cemf[FUSED ? (TY + 1) * kCornerCols : 1];
   for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x) {
@@ -927,7 +988,7 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
     }
     double dti = 0.0;
     if (i <= g.ie + 1 && j <= g.je + 1) {
-      const double dt = clk->dt;
+      const double dt = clk->dts;
       const double dtodx1 = dt / g.dx1, dtodx2 = dt / g.dx2;
       const int cur = clk->cur;
       const double* __restrict__ st = g.state[cur];
@@ -943,13 +1004,32 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
       };
       const double e00 = corner(0, 0), e10 = corner(1, 0), e01 = corner(0, 1);
       double b1n = 0.0, b2n = 0.0;
+      // set_bvals from the source's side: only a tile that reaches the five
+      // cells at an edge (four, and the face past them) has ghost images
+      const bool edge = fill && (i0 <= g.is + 4 || i0 + kTileX > g.ie - 4 || j0 <= g.js + 4 ||
+                                 j0 + TY > g.je - 4);
+      unsigned ix = 0, iy = 0;
+      if (edge) {
+        ix = ghost_images(i, g.is, g.ie, g.bc[0], g.bc[1], false);
+        iy = ghost_images(j, g.js, g.je, g.bc[2], g.bc[3], false);
+      }
       if (j <= g.je) {
         b1n = LD(st + F_B1I * ps, k) - dtodx2 * (e10 - e00);
         ST(out + F_B1I * ps, k, b1n);
+        if (edge)
+          for_ghost_images(g, j, i, ghost_images(i, g.is, g.ie, g.bc[0], g.bc[1], true), iy,
+                           [&](int r, int c, bool, bool) {
+                             ST(out + F_B1I * ps, (uint32_t)(r * pitch + c), b1n);
+                           });
       }
       if (i <= g.ie) {
         b2n = LD(st + F_B2I * ps, k) + dtodx1 * (e01 - e00);
         ST(out + F_B2I * ps, k, b2n);
+        if (edge)
+          for_ghost_images(g, j, i, ix, ghost_images(j, g.js, g.je, g.bc[2], g.bc[3], true),
+                           [&](int r, int c, bool, bool) {
+                             ST(out + F_B2I * ps, (uint32_t)(r * pitch + c), b2n);
+                           });
       }
       if (j <= g.je && i <= g.ie) {
         const double e11 = corner(1, 1);
@@ -982,6 +1062,19 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
         ST(out + F_B2C * ps, k, B2c);
         ST(out + F_B3C * ps, k, B3c);
         ST(out + F_B3I * ps, k, B3c);
+        if (edge)
+          for_ghost_images(g, j, i, ix, iy, [&](int r, int c, bool nx, bool ny) {
+            const uint32_t kg = (uint32_t)(r * pitch + c);
+            ST(out + F_D * ps, kg, d);
+            ST(out + F_M1 * ps, kg, nx ? -M1 : M1);
+            ST(out + F_M2 * ps, kg, ny ? -M2 : M2);
+            ST(out + F_M3 * ps, kg, M3);
+            ST(out + F_E * ps, kg, E);
+            ST(out + F_B1C * ps, kg, B1c);
+            ST(out + F_B2C * ps, kg, B2c);
+            ST(out + F_B3C * ps, kg, B3c);
+            ST(out + F_B3I * ps, kg, B3c);
+          });
         dti = inverse_dt(g, d, M1, M2, M3, E);
         const int bits = cell_fail_bits(g, d, M1, M2, M3, E, B1c, B2c, B3c);
         if (bits) atomicOr(&clk->fail, bits);
@@ -1004,22 +1097,13 @@ __global__ void __launch_bounds__(kGhostBlock) k_ghost(const Inst* __restrict__ 
     const Inst& g = insts[find_inst(insts, ninst, K_GHOST, t)];
     const Clock* clk = g.clk;
     if (respect_active && !clk->active) continue;
-    const int e = (t - g.tile0[K_GHOST]) * kGhostBlock + threadIdx.x;
-    const int nrow = 8 * g.sx;
-    if (e >= nrow + (g.nx2 + 1) * 8) continue;
-    int j, i;
-    if (e < nrow) {
-      const int r = e / g.sx;
-      i = e - r * g.sx;
-      j = (r < 4) ? r : g.je + 1 + (r - 4);
-    } else {
-      const int e2 = e - nrow;
-      const int r = e2 >> 3, c = e2 & 7;
-      j = g.js + r;
-      i = (c < 4) ? c : g.ie + 1 + (c - 4);
+    if (which == 2) {
+      ghost_carry(g, clk->cur, t);
+      continue;
     }
+    int j, i;
+    if (!ghost_cell(g, t, threadIdx.x, j, i)) continue;
     double* buf = g.state[which ? (clk->cur ^ 1) : clk->cur];
-    const double* src = (which == 2) ? g.state[clk->cur] : buf;
     // where a stale source (a ghost's value before this fill, grids thinner
     // than the ghost layers) is read: filling the other buffer, the current
     // one holds the last fill's ghosts; filling in place, the launcher has
@@ -1043,12 +1127,8 @@ __global__ void __launch_bounds__(kGhostBlock) k_ghost(const Inst* __restrict__ 
       const int c = ghost_class(f);
       v[f] = 0.0;
       if (gh[c]) {
-        if (which == 2) {
-          v[f] = LD(src + f * ps, k);
-        } else {
-          const double x = LD((stale[c] ? pre : src) + f * ps, (size_t)sj[c] * g.pitch + si[c]);
-          v[f] = ghost_negates(f, nx[c], ny[c]) ? -x : x;
-        }
+        const double x = LD((stale[c] ? pre : buf) + f * ps, (size_t)sj[c] * g.pitch + si[c]);
+        v[f] = ghost_negates(f, nx[c], ny[c]) ? -x : x;
       }
     }
 #pragma unroll
@@ -1059,34 +1139,47 @@ __global__ void __launch_bounds__(kGhostBlock) k_ghost(const Inst* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // Clock kernels: one workgroup of 256 threads per instance.
-// mode 0: main-loop step (main.c:221-232): run while time < tlim and
-//         (nlim < 0 or nstep < nlim) and no failure bit of fail_stop is set;
-//         clamp dt to reach tlim exactly. The
-//         step also waits (does not run) once time >= tpause, so that the
-//         host can write the outputs due at the top of the iteration
-//         (main.c:226, output.c:372-376) before it runs.
-// mode 1: unconditional single integration (drop-in integrate_2d).
-__global__ void __launch_bounds__(256) k_begin(const Inst* __restrict__ insts, int mode) {
+// The start of a main-loop step (main.c:221-232): run while time < tlim and
+// (nlim < 0 or nstep < nlim) and no failure bit of fail_stop is set, with dt
+// clamped to reach tlim exactly. The step also waits (does not run) once
+// time >= tpause, so that the host can write the outputs due at the top of the
+// iteration (main.c:226, output.c:372-376) before it runs. The clamp goes to
+// dts only, so it can be taken as soon as the step before has ended: dt itself
+// stays as new_dt left it until the step runs.
+__device__ __forceinline__ void start_step(Clock* c, double dt, double time, int nstep,
+                                           int fail) {
+  const int act = (time < c->tlim) && (c->nlim < 0 || nstep < c->nlim) && (time < c->tpause) &&
+                  ((fail & c->fail_stop) == 0);
+  c->dts = (act && (c->tlim - time) < dt) ? (c->tlim - time) : dt;
+  c->active = act;
+}
+
+// mode 0: main-loop step; mode 1: unconditional single integration (drop-in
+// integrate_2d). Needed before the first step after the host has written the
+// clock; later steps are started by k_end.
+__global__ void __launch_bounds__(kDtSlots) k_begin(const Inst* __restrict__ insts, int mode) {
   Clock* c = insts[blockIdx.x].clk;
-  for (int s = threadIdx.x; s < kDtSlots; s += blockDim.x) c->dti_slot[s] = 0ull;
+  c->dti_slot[threadIdx.x] = 0ull;
   if (threadIdx.x == 0) {
-    int act = 1;
     if (mode == 0) {
-      act = (c->time < c->tlim) && (c->nlim < 0 || c->nstep < c->nlim) &&
-            (c->time < c->tpause) && ((c->fail & c->fail_stop) == 0);
-      if (act && (c->tlim - c->time) < c->dt) c->dt = (c->tlim - c->time);
+      start_step(c, c->dt, c->time, c->nstep, c->fail);
+    } else {
+      c->dts = c->dt;
+      c->active = 1;
     }
-    c->active = act;
   }
 }
 
-__device__ __forceinline__ double reduce_slots(const Clock* c, double* red) {
-  double m = __longlong_as_double((long long)c->dti_slot[threadIdx.x]);
+// the maximum of the dt slots, which are cleared for the next reduction
+__device__ __forceinline__ double reduce_slots(Clock* c, double* red) {
+  const double m = __longlong_as_double((long long)c->dti_slot[threadIdx.x]);
+  c->dti_slot[threadIdx.x] = 0ull;
   return block_max(m, red);
 }
 
 // mode 0 (end of a main-loop step, main.c:289-292 + new_dt.c:93-97):
-//   nstep++, time += dt, dt = MIN(2 dt, CourNo/max_dti), swap buffers
+//   nstep++, time += dt, dt = MIN(2 dt, CourNo/max_dti), swap buffers, and the
+//   start of the next step
 // mode 1 (end of an unconditional integration): swap buffers only
 // Both record the step number of the first state that raised a failure bit.
 __global__ void __launch_bounds__(kDtSlots) k_end(const Inst* __restrict__ insts, int mode) {
@@ -1094,14 +1187,20 @@ __global__ void __launch_bounds__(kDtSlots) k_end(const Inst* __restrict__ insts
   Clock* c = insts[blockIdx.x].clk;
   const double max_dti = reduce_slots(c, red);
   if (threadIdx.x == 0 && c->active) {
+    const int fail = c->fail;
+    int nstep = c->nstep;
     if (mode == 0) {
-      c->nstep = c->nstep + 1;
-      c->time = c->time + c->dt;
-      const double a = 2.0 * c->dt, b = c->cour_no / max_dti;
-      c->dt = (c->nstep == 0) ? b : dmin(a, b);
+      nstep = nstep + 1;
+      const double time = c->time + c->dts;
+      const double a = 2.0 * c->dts, b = c->cour_no / max_dti;
+      const double dt = (nstep == 0) ? b : dmin(a, b);
+      c->nstep = nstep;
+      c->time = time;
+      c->dt = dt;
       c->steps_run = c->steps_run + 1;
+      start_step(c, dt, time, nstep, fail);
     }
-    if (c->fail != 0 && c->fail_nstep < 0) c->fail_nstep = mode == 0 ? c->nstep : c->nstep + 1;
+    if (fail != 0 && c->fail_nstep < 0) c->fail_nstep = mode == 0 ? nstep : nstep + 1;
     c->cur = c->cur ^ 1;
   }
 }
@@ -1195,7 +1294,7 @@ static PredX2Kernel pred_x2_kernel(bool save, int flux, int kind) {
   return save ? k_pred_x2<true, kFluxRoe> : k_pred_x2<false, kFluxRoe>;
 }
 typedef void (*CorrKernel)(const Inst*, int, int, int, int);
-typedef void (*FinalKernel)(const Inst*, int, int, int, int);
+typedef void (*FinalKernel)(const Inst*, int, int, int, int, int);
 // the corrector instantiation for a part (1: x1 faces, 2: x2 faces and Step
 // 7), tile height and Riemann solver
 template <int PART, bool CP>
@@ -1251,7 +1350,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
   switch (kernel) {
     case SK_BEGIN_STEP:
     case SK_BEGIN_ONCE:
-      hipLaunchKernelGGL(k_begin, dim3(b.ninst), dim3(256), 0, s, b.insts,
+      hipLaunchKernelGGL(k_begin, dim3(b.ninst), dim3(kDtSlots), 0, s, b.insts,
                          kernel == SK_BEGIN_STEP ? 0 : 1);
       break;
     case SK_PRED_X1:
@@ -1298,7 +1397,13 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       // at fusion depth 2 the x1 corrector computes these corners
       if (b.shape.fuse_corner >= 2) break;
       hipLaunchKernelGGL(k_corner<true>, dim3(grid_of(b, K_CORNER_P, 8)), b2, 0, s, b.insts,
-                         b.ninst, b.ntiles[K_CORNER_P], b.shape.xcd_remap);
+                         b.ninst, b.ntiles[K_CORNER_P], b.shape.xcd_remap, 0);
+      break;
+    case SK_CORNER_P_CARRY:
+      if (b.shape.fuse_corner >= 2) return ATHMI_FN(launch)(bl, SK_GHOST_CARRY, s);
+      hipLaunchKernelGGL(k_corner<true>, dim3(b.ntiles[K_GHOST] + grid_of(b, K_CORNER_P, 8)), b2,
+                         0, s, b.insts, b.ninst, b.ntiles[K_CORNER_P], b.shape.xcd_remap,
+                         b.ntiles[K_GHOST]);
       break;
     case SK_CORR:
     case SK_CORR2: {
@@ -1339,9 +1444,15 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       // with the fused final kernel the corners are computed there
       if (b.shape.fuse_corner) break;
       hipLaunchKernelGGL(k_corner<false>, dim3(grid_of(b, K_CORNER_C, 8)), b2, 0, s, b.insts,
-                         b.ninst, b.ntiles[K_CORNER_C], b.shape.xcd_remap);
+                         b.ninst, b.ntiles[K_CORNER_C], b.shape.xcd_remap, 0);
       break;
-    case SK_FINAL: {
+    case SK_FINAL:
+    case SK_FINAL_GHOST: {
+      const int fill = kernel == SK_FINAL_GHOST;
+      if (fill && b.thin) {
+        const hipError_t e = ATHMI_FN(launch)(bl, SK_FINAL, s);
+        return e != hipSuccess ? e : ATHMI_FN(launch)(bl, SK_GHOST_NEXT, s);
+      }
       // 32 waves per CU whatever the tile height
       const int ty = final_rows_of(b.shape.final_rows);
       const bool f = b.shape.fuse_corner != 0;
@@ -1349,7 +1460,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
                              : ty == 8 ? (f ? k_final<true, 8> : k_final<false, 8>)
                                        : (f ? k_final<true, 4> : k_final<false, 4>);
       hipLaunchKernelGGL(fn, dim3(grid_of(b, K_FINAL, 32 / ty)), dim3(kTileX, ty), 0, s, b.insts,
-                         b.ninst, b.ntiles[K_FINAL], b.shape.xcd_remap, b.shape.strip);
+                         b.ninst, b.ntiles[K_FINAL], b.shape.xcd_remap, b.shape.strip, fill);
       break;
     }
     case SK_GHOST_CUR:

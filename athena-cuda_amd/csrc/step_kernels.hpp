@@ -48,6 +48,7 @@ enum FailBits {
 // plus the main-loop limits of main.c:217-218).
 struct Clock {
   double dt, time, tlim, cour_no;
+  double dts;  // dt of the step under way or next: dt, clamped to reach tlim exactly
   double tpause;  // the main-loop step does not run once time >= tpause (an output is due)
   int nstep, nlim, active, cur;  // cur: which ping-pong state buffer holds the state
   int fail;        // FailBits of the states produced so far (0: healthy)
@@ -161,6 +162,7 @@ struct BatchLaunch {
   int ninst;
   int ntiles[NKINDS];
   int stale_ghosts;  // some instance's ghost fill reads stale ghosts (ghost_map.hpp)
+  int thin;          // some instance has Nx1 or Nx2 < 4: ghosts may copy ghosts
   LaunchShape shape;
   int ncu;
   int flux_mask;  // bit f set: some instance uses Riemann solver f (kFluxRoe, kFluxHlle)
@@ -180,7 +182,7 @@ enum StepKernel {
   SK_GHOST_CUR,       // set_bvals on the current buffer
   SK_GHOST_NEXT,      // set_bvals on the buffer this step produces (respects the clock)
   SK_GHOST_CARRY,     // carry current ghost values into the produced buffer
-  SK_END_STEP,        // k_end, main-loop mode
+  SK_END_STEP,        // k_end, main-loop mode: the clock of this step, and the next one's start
   SK_END_ONCE,        // k_end, swap only
   SK_CLEAR,           // reset reduction slots
   SK_DTI,             // new_dt partial maxima
@@ -191,6 +193,9 @@ enum StepKernel {
   SK_PRED,            // both predictors, both corrector parts: one launch or two, by the
   SK_PRED_SAVE,       // batch's size
   SK_CORR_BOTH,
+  SK_FINAL_GHOST,     // SK_FINAL and SK_GHOST_NEXT: one launch where every ghost copies a
+                      // non-ghost cell
+  SK_CORNER_P_CARRY,  // SK_CORNER_P and SK_GHOST_CARRY, in one launch where both are launched
   SK_COUNT
 };
 
