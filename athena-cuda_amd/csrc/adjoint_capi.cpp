@@ -91,7 +91,7 @@ struct athmi_adjoint {
 // launch a kernel sequence of the instance through the descriptor ins
 static int issue_on(athmi_adjoint* h, const Inst* ins, const int* seq, size_t n) {
   BatchLaunch bl = h->g->bl;
-  bl.insts = ins;
+  bl.single(ins, h->g->hinst[0].flux);
   for (size_t k = 0; k < n; k++) HIP_TRY(h->g->launch(&bl, seq[k], h->g->stream));
   return ATHMI_OK;
 }

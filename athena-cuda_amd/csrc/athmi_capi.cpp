@@ -55,7 +55,6 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
   g->desc.assign(desc, desc + n);
   g->hinst.resize(n);
   g->cpaw_soln.resize(n);
-  g->bl.ninst = n;
   g->bl.ncu = prop.multiProcessorCount;
   // faces marched per lane by the x2 predictor (1..16)
   long cols = 0;
@@ -115,7 +114,7 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
     return fail(ATHMI_EHIP, "athmi_create: clearing the state failed");
   }
   if (hipMalloc(&g->dclk, sizeof(Clock) * n) != hipSuccess ||
-      hipMalloc(&g->dinst, sizeof(Inst) * n) != hipSuccess) {
+      hipMalloc(&g->dinst, 2 * inst_list_bytes(n)) != hipSuccess) {
     athmi_destroy(g);
     return fail(ATHMI_ENOMEM, "athmi_create: hipMalloc of the descriptors failed");
   }
@@ -145,7 +144,6 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
     return fail(ATHMI_EHIP, "athmi_create: stream creation failed");
   }
   g->own_stream = true;
-  g->bl.insts = g->dinst;
   int rc = g->refresh_tiles();
   if (rc != ATHMI_OK) {
     athmi_destroy(g);

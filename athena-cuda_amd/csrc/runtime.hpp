@@ -75,7 +75,7 @@ struct athmi_grid {
   int variant = ATHMI_EXACT;
   std::vector<athmi_desc> desc;
   std::vector<Inst> hinst;
-  Inst* dinst = nullptr;
+  Inst* dinst = nullptr;  // the device lists of bl
   Clock* dclk = nullptr;
   double* dmem = nullptr;
   size_t dmem_bytes = 0;
@@ -94,26 +94,44 @@ struct athmi_grid {
     if (graph) (void)hipGraphExecDestroy(graph);
     graph = nullptr;
   }
+  // the device lists: every instance, and (a batch that mixes the solvers)
+  // those of each solver, each with its own tile numbering
   int refresh_tiles() {
-    int tot[NKINDS] = {0};
-    for (int k = 0; k < n; k++) {
-      Inst& I = hinst[k];
-      for (int kind = 0; kind < NKINDS; kind++) {
-        I.tile0[kind] = tot[kind];
-        tot[kind] += tiles_of(kind, I.nx1, I.nx2, bl.shape.x2_seg, bl.shape.corr_rows,
-                              bl.shape.final_rows);
-      }
-    }
-    for (int kind = 0; kind < NKINDS; kind++) bl.ntiles[kind] = tot[kind];
-    bl.flux_mask = 0;
+    std::vector<unsigned char> img(2 * inst_list_bytes(n));
+    unsigned char* base = reinterpret_cast<unsigned char*>(dinst);
+    size_t used = 0;
+    auto add = [&](InstList& L, int flux) {
+      Inst* I = reinterpret_cast<Inst*>(img.data() + used);
+      int m = 0, tot[NKINDS] = {0};
+      for (int k = 0; k < n; k++)
+        if (flux < 0 || hinst[k].flux == flux) I[m++] = hinst[k];
+      int* first = reinterpret_cast<int*>(I + m);
+      for (int k = 0; k < m; k++)
+        for (int kind = 0; kind < NKINDS; kind++) {
+          first[kind * m + k] = I[k].tile0[kind] = tot[kind];
+          tot[kind] += tiles_of(kind, I[k].nx1, I[k].nx2, bl.shape.x2_seg, bl.shape.corr_rows,
+                                bl.shape.final_rows);
+        }
+      L.insts = reinterpret_cast<const Inst*>(base + used);
+      L.ninst = m;
+      for (int kind = 0; kind < NKINDS; kind++) L.ntiles[kind] = tot[kind];
+      used += inst_list_bytes(m);
+    };
+    int count[2] = {0, 0};
     bl.stale_ghosts = 0;
     bl.thin = 0;
-    for (int k = 0; k < n; k++) {
-      if (hinst[k].nx1 < 4 || hinst[k].nx2 < 4) bl.thin = 1;
-      bl.flux_mask |= 1 << hinst[k].flux;
-      if (ghost_fill_reads_stale(hinst[k])) bl.stale_ghosts = 1;
+    for (const Inst& I : hinst) {
+      count[I.flux]++;
+      if (I.nx1 < 4 || I.nx2 < 4) bl.thin = 1;
+      if (ghost_fill_reads_stale(I)) bl.stale_ghosts = 1;
     }
-    HIP_TRY(hipMemcpy(dinst, hinst.data(), sizeof(Inst) * n, hipMemcpyHostToDevice));
+    add(bl.all, -1);
+    for (int f = 0; f < 2; f++) {
+      if (count[f] == n) bl.of_flux[f] = bl.all;
+      else if (count[f] == 0) bl.of_flux[f] = InstList{};
+      else add(bl.of_flux[f], f);
+    }
+    HIP_TRY(hipMemcpy(dinst, img.data(), used, hipMemcpyHostToDevice));
     drop_graph();
     return ATHMI_OK;
   }

@@ -162,8 +162,7 @@ int athmi_integrate_static(const athmi_desc* desc, double dt, const double* stat
   I.clk = dclk;
 
   BatchLaunch bl{};
-  bl.insts = dinst;
-  bl.ninst = 1;
+  bl.all.ninst = 1;
   bl.ncu = ncu;
   // the handle's default launch shape for one grid
   bl.shape.x2_seg = default_x2_seg((long)cdiv(d.nx1 + 6, kX2Block) * (d.nx2 + 4));
@@ -175,10 +174,10 @@ int athmi_integrate_static(const athmi_desc* desc, double dt, const double* stat
   bl.shape.fuse_corner = 1;
   for (int kind = 0; kind < NKINDS; kind++) {
     I.tile0[kind] = 0;
-    bl.ntiles[kind] = tiles_of(kind, d.nx1, d.nx2, bl.shape.x2_seg, bl.shape.corr_rows,
+    bl.all.ntiles[kind] = tiles_of(kind, d.nx1, d.nx2, bl.shape.x2_seg, bl.shape.corr_rows,
                               bl.shape.final_rows);
   }
-  bl.flux_mask = 1 << d.flux;
+  bl.single(dinst, d.flux);
 
   const hipStream_t s = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(k_static_head, dim3(1), dim3(256), 0, s, I, dclk, dinst, dt, d.cour_no);

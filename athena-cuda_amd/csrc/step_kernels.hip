@@ -85,13 +85,22 @@ __device__ __forceinline__ void tile_pos(int local, int ntx, int nty, int strip,
   tx = sidx * strip + (r - ty * w);
 }
 
-// instance owning global tile t of kernel kind `kind` (tile0 ascending)
+// Instance of the list that owns its tile t (first tiles ascending; t the same
+// in every lane of the wave). The lanes search together: 64 first tiles of the
+// dense table per load, so 64 instances take one load and 4096 two, where a
+// binary search by the wave as a whole chains 6 and 12 of them -- up to 2 us
+// before a tile's own loads can start, which two waves per SIMD do not hide.
 __device__ __forceinline__ int find_inst(const Inst* __restrict__ in, int n, int kind, int t) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (in[mid].tile0[kind] <= t) lo = mid;
-    else hi = mid - 1;
+  if (n == 1) return 0;
+  const int* __restrict__ first = reinterpret_cast<const int*>(in + n) + kind * n;
+  const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  int lo = 0, len = n;
+  while (len > 1) {
+    const int step = (len + 63) >> 6, at = lane * step;
+    const bool below = at < len && first[lo + at] <= t;
+    const int c = __popcll(__ballot(below)) - 1;
+    lo += c * step;
+    len = min(step, len - c * step);
   }
   return lo;
 }
@@ -195,7 +204,9 @@ struct RowStencil {
 };
 
 // SAVE: also store the primitive face states (Inst::prims). FLUX: the Riemann
-// solver; a launch takes only the tiles of instances that use it, and with one
+// solver; a launch takes the list of the instances that use it (a batch that
+// mixes the solvers no longer launches every tile for both: with the search
+// above, 40 mixed instances of 64^2..1024^2 6.5 -> 5.6 ms a step), and with one
 // solver per kernel the predictor fits two waves per SIMD.
 template <bool SAVE, int FLUX>
 __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int ninst, int t,
@@ -204,7 +215,7 @@ __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int
   const int tid = threadIdx.x;
   const Inst& g = insts[find_inst(insts, ninst, K_PRED_X1, t)];
   const Clock* clk = g.clk;
-  if (!clk->active || g.flux != FLUX) return;
+  if (!clk->active) return;
   const int local = uni(t - g.tile0[K_PRED_X1]);
   const int gis = uni(g.is), gie = uni(g.ie);
   const int nseg = dcdiv(uni(g.nx1) + 4, kX1Faces);
@@ -301,7 +312,7 @@ __global__ void __launch_bounds__(kX2Block) k_pred_x2(const Inst* __restrict__ i
     const int t = xcd_tile(t0, ntiles, remap);
     const Inst& g = insts[find_inst(insts, ninst, K_PRED_X2, t)];
     const Clock* clk = g.clk;
-    if (!clk->active || g.flux != FLUX) continue;
+    if (!clk->active) continue;
     const int local = t - g.tile0[K_PRED_X2];
     // chunks from column 0: each row segment starts on a cache line
     const int ncb = dcdiv(g.nx1 + 6, kX2Block);
@@ -436,7 +447,7 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
   };
   const Inst& g = insts[find_inst(insts, ninst, K_PRED_X2, t)];
   const Clock* clk = g.clk;
-  if (!clk->active || g.flux != FLUX) return;
+  if (!clk->active) return;
   const int local = uni(t - g.tile0[K_PRED_X2]);
   // chunks from column 0: each row segment starts on a cache line
   const int ncb = dcdiv(uni(g.nx1) + 6, kX2Block);
@@ -700,7 +711,7 @@ __global__ void __launch_bounds__(kTileX* kTileY) k_corner(const Inst* __restric
 // PART 1: the x1 faces (Steps 5, 8b); PART 2: the x2 faces and Step 7 (6, 8c, 7).
 // Split so that each thread evaluates one Riemann flux: the loads of the second
 // face no longer compete for registers with the first face's flux.
-// FLUX: the Riemann solver; a launch takes only the tiles of instances that use
+// FLUX: the Riemann solver; a launch takes the list of the instances that use
 // it. With one solver per kernel (the Roe one keeps its HLLE fallback) the
 // corrector fits two waves per SIMD.
 // CP (x1 part only): the tile first computes the Step 4 corner emf of its rows
@@ -714,7 +725,7 @@ __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ni
   static_assert(!CP || PART == 1, "the corner phase belongs to the x1 part");
   const Inst& g = insts[find_inst(insts, ninst, K_CORR, t)];
   const Clock* clk = g.clk;
-  if (!clk->active || g.flux != FLUX) return;
+  if (!clk->active) return;
   const int local = uni(t - g.tile0[K_CORR]);
   const int gis = uni(g.is), gjs = uni(g.js);
   int tx, ty;
@@ -894,8 +905,9 @@ __global__ void __launch_bounds__(kTileX* TY, 2) k_corr(const Inst* __restrict__
 
 // Both parts in one launch (they read the same planes and write disjoint
 // ones): workgroups [0, ntiles) the x2 part with Step 7, the rest the x1 part.
+// HLLE: 132 registers left three waves per SIMD; 128 hold four without spills.
 template <int TY, int FLUX>
-__global__ void __launch_bounds__(kTileX* TY, 2) k_corr_both(const Inst* __restrict__ insts,
+__global__ void __launch_bounds__(kTileX* TY, FLUX == kFluxHlle ? 4 : 2) k_corr_both(const Inst* __restrict__ insts,
                                                              int ninst, int ntiles, int remap,
                                                              int strip) {
   __shared__ double park_lds[14 * kTileX * TY];
@@ -1324,8 +1336,8 @@ static bool merge_sweeps(const BatchLaunch& b) {
   return b.shape.persist <= 0 && b.shape.x2_kind == 1;
 }
 
-static int grid_of(const BatchLaunch& b, int kind, int per_cu) {
-  const int n = b.ntiles[kind];
+static int grid_of(const BatchLaunch& b, const InstList& list, int kind, int per_cu) {
+  const int n = list.ntiles[kind];
   if (b.shape.persist <= 0) return n;
   const int cap = b.ncu * b.shape.persist * per_cu;
   return n < cap ? n : cap;
@@ -1346,31 +1358,34 @@ extern "C" {
 // Launch one kernel of the pipeline for every instance of the batch.
 hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
   const BatchLaunch& b = *static_cast<const BatchLaunch*>(bl);
+  const InstList& a = b.all;
   const dim3 b2(kTileX, kTileY);
   switch (kernel) {
     case SK_BEGIN_STEP:
     case SK_BEGIN_ONCE:
-      hipLaunchKernelGGL(k_begin, dim3(b.ninst), dim3(kDtSlots), 0, s, b.insts,
+      hipLaunchKernelGGL(k_begin, dim3(a.ninst), dim3(kDtSlots), 0, s, a.insts,
                          kernel == SK_BEGIN_STEP ? 0 : 1);
       break;
     case SK_PRED_X1:
     case SK_PRED_X1_SAVE:
       for (int f = 0; f < 2; f++) {
-        if (!(b.flux_mask & (1 << f))) continue;
+        const InstList& l = b.of_flux[f];
+        if (!l.ninst) continue;
         const PredX1Kernel fn = pred_x1_kernel(kernel == SK_PRED_X1_SAVE, f);
-        hipLaunchKernelGGL(fn, dim3(grid_of(b, K_PRED_X1, kX1PerCu)), dim3(kX1Block), 0, s,
-                           b.insts, b.ninst, b.ntiles[K_PRED_X1], b.shape.xcd_remap);
+        hipLaunchKernelGGL(fn, dim3(grid_of(b, l, K_PRED_X1, kX1PerCu)), dim3(kX1Block), 0, s,
+                           l.insts, l.ninst, l.ntiles[K_PRED_X1], b.shape.xcd_remap);
       }
       break;
     case SK_PRED_X2:
     case SK_PRED_X2_SAVE:
       for (int f = 0; f < 2; f++) {
-        if (!(b.flux_mask & (1 << f))) continue;
+        const InstList& l = b.of_flux[f];
+        if (!l.ninst) continue;
         const int kind = b.shape.x2_kind;
         const PredX2Kernel fn = pred_x2_kernel(kernel == SK_PRED_X2_SAVE, f, kind);
-        hipLaunchKernelGGL(fn, dim3(grid_of(b, K_PRED_X2, kind == 1 ? 8 : 16)), dim3(kX2Block),
-                           0, s, b.insts,
-                           b.ninst, b.ntiles[K_PRED_X2], b.shape.x2_seg, b.shape.xcd_remap);
+        hipLaunchKernelGGL(fn, dim3(grid_of(b, l, K_PRED_X2, kind == 1 ? 8 : 16)), dim3(kX2Block),
+                           0, s, l.insts,
+                           l.ninst, l.ntiles[K_PRED_X2], b.shape.x2_seg, b.shape.xcd_remap);
       }
       break;
     case SK_PRED:
@@ -1382,13 +1397,14 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         if (e != hipSuccess) return e;
         return ATHMI_FN(launch)(bl, save ? SK_PRED_X2_SAVE : SK_PRED_X2, s);
       }
-      const int n1 = b.ntiles[K_PRED_X1], n2 = b.ntiles[K_PRED_X2];
-      const int nb2 = cdiv(n2, kX2PerBlock);
       for (int f = 0; f < 2; f++) {
-        if (!(b.flux_mask & (1 << f))) continue;
+        const InstList& l = b.of_flux[f];
+        if (!l.ninst) continue;
         const auto fn = f == kFluxHlle ? (save ? k_pred<true, kFluxHlle> : k_pred<false, kFluxHlle>)
                                        : (save ? k_pred<true, kFluxRoe> : k_pred<false, kFluxRoe>);
-        hipLaunchKernelGGL(fn, dim3(n1 + nb2), dim3(kX1Block), 0, s, b.insts, b.ninst, n1, n2, nb2,
+        const int n1 = l.ntiles[K_PRED_X1], n2 = l.ntiles[K_PRED_X2];
+        const int nb2 = cdiv(n2, kX2PerBlock);
+        hipLaunchKernelGGL(fn, dim3(n1 + nb2), dim3(kX1Block), 0, s, l.insts, l.ninst, n1, n2, nb2,
                            b.shape.x2_seg, b.shape.xcd_remap);
       }
       break;
@@ -1396,26 +1412,28 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
     case SK_CORNER_P:
       // at fusion depth 2 the x1 corrector computes these corners
       if (b.shape.fuse_corner >= 2) break;
-      hipLaunchKernelGGL(k_corner<true>, dim3(grid_of(b, K_CORNER_P, 8)), b2, 0, s, b.insts,
-                         b.ninst, b.ntiles[K_CORNER_P], b.shape.xcd_remap, 0);
+      hipLaunchKernelGGL(k_corner<true>, dim3(grid_of(b, a, K_CORNER_P, 8)), b2, 0, s, a.insts,
+                         a.ninst, a.ntiles[K_CORNER_P], b.shape.xcd_remap, 0);
       break;
     case SK_CORNER_P_CARRY:
       if (b.shape.fuse_corner >= 2) return ATHMI_FN(launch)(bl, SK_GHOST_CARRY, s);
-      hipLaunchKernelGGL(k_corner<true>, dim3(b.ntiles[K_GHOST] + grid_of(b, K_CORNER_P, 8)), b2,
-                         0, s, b.insts, b.ninst, b.ntiles[K_CORNER_P], b.shape.xcd_remap,
-                         b.ntiles[K_GHOST]);
+      hipLaunchKernelGGL(k_corner<true>, dim3(a.ntiles[K_GHOST] + grid_of(b, a, K_CORNER_P, 8)),
+                         b2, 0, s, a.insts, a.ninst, a.ntiles[K_CORNER_P], b.shape.xcd_remap,
+                         a.ntiles[K_GHOST]);
       break;
     case SK_CORR:
     case SK_CORR2: {
       // the same threads in flight per CU whatever the tile height; one launch
       // per Riemann solver in use
       const int ty = b.shape.corr_rows;
-      const dim3 grid(grid_of(b, K_CORR, 4 * (kTileY / ty))), blk(kTileX, ty);
+      const dim3 blk(kTileX, ty);
       const bool x1 = (kernel == SK_CORR);
       for (int f = 0; f < 2; f++) {
-        if (!(b.flux_mask & (1 << f))) continue;
+        const InstList& l = b.of_flux[f];
+        if (!l.ninst) continue;
         const CorrKernel fn = corr_kernel(x1 ? 1 : 2, ty, f, b.shape.fuse_corner >= 2);
-        hipLaunchKernelGGL(fn, grid, blk, 0, s, b.insts, b.ninst, b.ntiles[K_CORR],
+        hipLaunchKernelGGL(fn, dim3(grid_of(b, l, K_CORR, 4 * (kTileY / ty))), blk, 0, s,
+                           l.insts, l.ninst, l.ntiles[K_CORR],
                            b.shape.xcd_remap, b.shape.strip);
       }
       break;
@@ -1426,16 +1444,18 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         if (e != hipSuccess) return e;
         return ATHMI_FN(launch)(bl, SK_CORR2, s);
       }
-      const int ty = b.shape.corr_rows, n = b.ntiles[K_CORR];
+      const int ty = b.shape.corr_rows;
       for (int f = 0; f < 2; f++) {
-        if (!(b.flux_mask & (1 << f))) continue;
+        const InstList& l = b.of_flux[f];
+        if (!l.ninst) continue;
         const CorrKernel fn =
             f == kFluxHlle
                 ? (ty == 1 ? k_corr_both<1, kFluxHlle>
                            : ty == 2 ? k_corr_both<2, kFluxHlle> : k_corr_both<4, kFluxHlle>)
                 : (ty == 1 ? k_corr_both<1, kFluxRoe>
                            : ty == 2 ? k_corr_both<2, kFluxRoe> : k_corr_both<4, kFluxRoe>);
-        hipLaunchKernelGGL(fn, dim3(2 * n), dim3(kTileX, ty), 0, s, b.insts, b.ninst, n,
+        const int n = l.ntiles[K_CORR];
+        hipLaunchKernelGGL(fn, dim3(2 * n), dim3(kTileX, ty), 0, s, l.insts, l.ninst, n,
                            b.shape.xcd_remap, b.shape.strip);
       }
       break;
@@ -1443,8 +1463,8 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
     case SK_CORNER_C:
       // with the fused final kernel the corners are computed there
       if (b.shape.fuse_corner) break;
-      hipLaunchKernelGGL(k_corner<false>, dim3(grid_of(b, K_CORNER_C, 8)), b2, 0, s, b.insts,
-                         b.ninst, b.ntiles[K_CORNER_C], b.shape.xcd_remap, 0);
+      hipLaunchKernelGGL(k_corner<false>, dim3(grid_of(b, a, K_CORNER_C, 8)), b2, 0, s, a.insts,
+                         a.ninst, a.ntiles[K_CORNER_C], b.shape.xcd_remap, 0);
       break;
     case SK_FINAL:
     case SK_FINAL_GHOST: {
@@ -1459,8 +1479,8 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       const FinalKernel fn = ty == 16 ? (f ? k_final<true, 16> : k_final<false, 16>)
                              : ty == 8 ? (f ? k_final<true, 8> : k_final<false, 8>)
                                        : (f ? k_final<true, 4> : k_final<false, 4>);
-      hipLaunchKernelGGL(fn, dim3(grid_of(b, K_FINAL, 32 / ty)), dim3(kTileX, ty), 0, s, b.insts,
-                         b.ninst, b.ntiles[K_FINAL], b.shape.xcd_remap, b.shape.strip, fill);
+      hipLaunchKernelGGL(fn, dim3(grid_of(b, a, K_FINAL, 32 / ty)), dim3(kTileX, ty), 0, s, a.insts,
+                         a.ninst, a.ntiles[K_FINAL], b.shape.xcd_remap, b.shape.strip, fill);
       break;
     }
     case SK_GHOST_CUR:
@@ -1470,31 +1490,31 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       // an in-place fill that reads stale ghosts reads them from the other
       // buffer: carry them there first
       if (which == 0 && b.stale_ghosts)
-        hipLaunchKernelGGL(k_ghost, dim3(grid_of(b, K_GHOST, 8)), dim3(kGhostBlock), 0, s,
-                           b.insts, b.ninst, b.ntiles[K_GHOST], 2, 0, b.shape.xcd_remap);
-      hipLaunchKernelGGL(k_ghost, dim3(grid_of(b, K_GHOST, 8)), dim3(kGhostBlock), 0, s, b.insts,
-                         b.ninst, b.ntiles[K_GHOST], which, kernel == SK_GHOST_NEXT ? 1 : 0,
+        hipLaunchKernelGGL(k_ghost, dim3(grid_of(b, a, K_GHOST, 8)), dim3(kGhostBlock), 0, s,
+                           a.insts, a.ninst, a.ntiles[K_GHOST], 2, 0, b.shape.xcd_remap);
+      hipLaunchKernelGGL(k_ghost, dim3(grid_of(b, a, K_GHOST, 8)), dim3(kGhostBlock), 0, s, a.insts,
+                         a.ninst, a.ntiles[K_GHOST], which, kernel == SK_GHOST_NEXT ? 1 : 0,
                          b.shape.xcd_remap);
       break;
     }
     case SK_END_STEP:
     case SK_END_ONCE:
-      hipLaunchKernelGGL(k_end, dim3(b.ninst), dim3(kDtSlots), 0, s, b.insts,
+      hipLaunchKernelGGL(k_end, dim3(a.ninst), dim3(kDtSlots), 0, s, a.insts,
                          kernel == SK_END_STEP ? 0 : 1);
       break;
     case SK_CLEAR:
-      hipLaunchKernelGGL(k_clear_slots, dim3(b.ninst), dim3(256), 0, s, b.insts);
+      hipLaunchKernelGGL(k_clear_slots, dim3(a.ninst), dim3(256), 0, s, a.insts);
       break;
     case SK_DTI:
-      hipLaunchKernelGGL(k_dti, dim3(grid_of(b, K_INTERIOR, 8)), b2, 0, s, b.insts, b.ninst,
-                         b.ntiles[K_INTERIOR], b.shape.xcd_remap);
+      hipLaunchKernelGGL(k_dti, dim3(grid_of(b, a, K_INTERIOR, 8)), b2, 0, s, a.insts, a.ninst,
+                         a.ntiles[K_INTERIOR], b.shape.xcd_remap);
       break;
     case SK_DT_FINAL:
-      hipLaunchKernelGGL(k_dt_final, dim3(b.ninst), dim3(kDtSlots), 0, s, b.insts);
+      hipLaunchKernelGGL(k_dt_final, dim3(a.ninst), dim3(kDtSlots), 0, s, a.insts);
       break;
     case SK_DIVB:
-      hipLaunchKernelGGL(k_divb, dim3(grid_of(b, K_INTERIOR, 8)), b2, 0, s, b.insts, b.ninst,
-                         b.ntiles[K_INTERIOR], b.shape.xcd_remap);
+      hipLaunchKernelGGL(k_divb, dim3(grid_of(b, a, K_INTERIOR, 8)), b2, 0, s, a.insts, a.ninst,
+                         a.ntiles[K_INTERIOR], b.shape.xcd_remap);
       break;
     default:
       return hipErrorInvalidValue;

@@ -155,17 +155,32 @@ struct LaunchShape {
   int final_rows;    // rows of a final-update tile: 4, 8 or 16 (final_rows_of)
 };
 
-// Everything a launcher needs for one batch (device descriptor array, tile
-// totals per kernel kind, the tuned shape and the CU count)
-struct BatchLaunch {
+// A list of instances on the device and its tile totals per kernel kind. In
+// device memory the descriptors are followed by the first tiles again, as a
+// dense table [NKINDS][ninst] that find_inst searches (a list of one has none).
+struct InstList {
   const Inst* insts;
   int ninst;
   int ntiles[NKINDS];
+};
+inline size_t inst_list_bytes(size_t n) { return n * (sizeof(Inst) + sizeof(int) * NKINDS); }
+
+// Everything a launcher needs for one batch (the instances, the tuned shape
+// and the CU count). The kernels that are compiled per Riemann solver take the
+// list of the instances that use it; the others take them all.
+struct BatchLaunch {
+  InstList all;
+  InstList of_flux[2];  // by solver (kFluxRoe, kFluxHlle); ninst = 0: not in use
   int stale_ghosts;  // some instance's ghost fill reads stale ghosts (ghost_map.hpp)
   int thin;          // some instance has Nx1 or Nx2 < 4: ghosts may copy ghosts
   LaunchShape shape;
   int ncu;
-  int flux_mask;  // bit f set: some instance uses Riemann solver f (kFluxRoe, kFluxHlle)
+  // a batch of one: its only list, read through descriptor `ins`
+  void single(const Inst* ins, int flux) {
+    all.insts = ins;
+    of_flux[flux] = all;
+    of_flux[1 - flux] = InstList{};
+  }
 };
 
 // Kernels of the pipeline, launched one at a time by athmi_<variant>_launch
