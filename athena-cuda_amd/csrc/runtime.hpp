@@ -117,6 +117,7 @@ struct athmi_grid {
       for (int kind = 0; kind < NKINDS; kind++) L.ntiles[kind] = tot[kind];
       used += inst_list_bytes(m);
     };
+    bl.outgrows_cache = dmem_bytes > kInfinityCacheBytes;
     int count[2] = {0, 0};
     bl.stale_ghosts = 0;
     bl.thin = 0;

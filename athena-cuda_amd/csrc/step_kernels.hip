@@ -124,6 +124,13 @@ __device__ __forceinline__ void ST(double* plane, uint32_t k, double v) {
   *(__attribute__((address_space(1))) double*)((gbytes*)plane + k * 8u) = v;
 }
 
+// A store that leaves the line behind the lines already in the caches (the
+// caches, the 256 MB Infinity Cache among them, then keep what is read again)
+__device__ __forceinline__ void ST_STREAM(double* plane, uint32_t k, double v) {
+  __builtin_nontemporal_store(
+      v, (__attribute__((address_space(1))) double*)((gbytes*)plane + k * 8u));
+}
+
 __device__ __forceinline__ Prim7 lds_prim64(double (*s)[kX2Block], int t) {
   return Prim7{s[0][t], s[1][t], s[2][t], s[3][t], s[4][t], s[5][t], s[6][t]};
 }
@@ -142,7 +149,14 @@ __device__ __forceinline__ void phase_fence() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+template <bool STREAM = false>
 __device__ __forceinline__ void put7(double* base, size_t ps, uint32_t k, const Cons7& u) {
+  if constexpr (STREAM) {
+    const double* v = &u.d;
+#pragma unroll
+    for (int n = 0; n < 7; n++) ST_STREAM(base + n * ps, k, v[n]);
+    return;
+  }
   ST(base + 0 * ps, k, u.d); ST(base + 1 * ps, k, u.mx); ST(base + 2 * ps, k, u.my);
   ST(base + 3 * ps, k, u.mz); ST(base + 4 * ps, k, u.e); ST(base + 5 * ps, k, u.by);
   ST(base + 6 * ps, k, u.bz);
@@ -208,7 +222,7 @@ struct RowStencil {
 // mixes the solvers no longer launches every tile for both: with the search
 // above, 40 mixed instances of 64^2..1024^2 6.5 -> 5.6 ms a step), and with one
 // solver per kernel the predictor fits two waves per SIMD.
-template <bool SAVE, int FLUX>
+template <bool SAVE, int FLUX, bool STREAM = false>
 __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int ninst, int t,
                                              double (*sw)[kX1Block], double (*swl)[kX1Block],
                                              double (*swr)[kX1Block]) {
@@ -278,9 +292,9 @@ __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int
       put7(pw + P_WL1 * ps, ps, k, wl);
       put7(pw + P_WR1 * ps, ps, k, wr);
     }
-    put7(sc + S_UL1 * ps, ps, k, ul);
-    put7(sc + S_UR1 * ps, ps, k, ur);
-    put7(sc + S_F1 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
+    put7<STREAM>(sc + S_UL1 * ps, ps, k, ul);
+    put7<STREAM>(sc + S_UR1 * ps, ps, k, ur);
+    put7<STREAM>(sc + S_F1 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
   }
 }
 template <bool SAVE, int FLUX>
@@ -417,7 +431,7 @@ __global__ void __launch_bounds__(kX2Block) k_pred_x2(const Inst* __restrict__ i
 constexpr int kX2Slots = 5;  // 4 rotating + the Wr slot
 constexpr int kX2Aux = 5;    // B2i ring (2), s ring (2), M1/d carry
 typedef double X2Slots[7][kX2Block];
-template <bool SAVE, int FLUX>
+template <bool SAVE, int FLUX, bool STREAM = false>
 __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int ninst, int t,
                                              int seg_len, X2Slots* slots,
                                              double (*aux)[kX2Block], int lane) {
@@ -539,9 +553,9 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
       put7(pw + P_WL2 * ps, ps, k, wl);
       put7(pw + P_WR2 * ps, ps, k, wr);
     }
-    put7(sc + S_UL2 * ps, ps, k, ul);
-    put7(sc + S_UR2 * ps, ps, k, ur);
-    put7(sc + S_F2 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
+    put7<STREAM>(sc + S_UL2 * ps, ps, k, ul);
+    put7<STREAM>(sc + S_UR2 * ps, ps, k, ur);
+    put7<STREAM>(sc + S_F2 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
     // rotate: row j -> j-1, row j+1 -> j, Wl(j+1) pending, Wl(j)'s slot free
     const int nP = sQ, nQ = sF, nW = sP, nF = sW;
     sP = nP; sQ = nQ; sW = nW; sF = nF;
@@ -562,9 +576,15 @@ __global__ void __launch_bounds__(kX2Block, 2) k_pred_x2l(const Inst* __restrict
 // [0, nb2) hold two x2 tiles each, one per wave -- the longer marches start
 // first -- and the rest one x1 tile each; both kinds take the 20 KiB of LDS
 // and the registers per wave of two waves per SIMD.
+// STREAM: the 42 output planes are stored past the caches. Where a step's
+// planes outgrow the Infinity Cache the corrector finds them in HBM anyway, and
+// 344 B per cell of stores only push out the state the other sweep and the
+// corrector still read: a step of 1024^2 takes 510 -> 485 us (HLLE 446 -> 411),
+// 2048x1536 1388 -> 1347 (1224 -> 1172), 4096^2 7.07 -> 6.99 ms. Where they fit,
+// the corrector reads them from the cache and streaming costs (512^2 151 -> 157 us).
 constexpr int kX2Lds = (kX2Slots * 7 + kX2Aux) * kX2Block;  // doubles of a wave's x2 tile
 constexpr int kX2PerBlock = kX1Block / kX2Block;
-template <bool SAVE, int FLUX>
+template <bool SAVE, int FLUX, bool STREAM>
 __global__ void __launch_bounds__(kX1Block, 2) k_pred(const Inst* __restrict__ insts, int ninst,
                                                       int n1, int n2, int nb2, int seg_len,
                                                       int remap) {
@@ -576,12 +596,12 @@ __global__ void __launch_bounds__(kX1Block, 2) k_pred(const Inst* __restrict__ i
     const int t = uni(kX2PerBlock * xcd_tile(b, nb2, remap) + w);
     if (t >= n2) return;
     double* mine = lds + w * kX2Lds;
-    pred_x2_tile<SAVE, FLUX>(insts, ninst, t, seg_len, (X2Slots*)mine,
+    pred_x2_tile<SAVE, FLUX, STREAM>(insts, ninst, t, seg_len, (X2Slots*)mine,
                              (double (*)[kX2Block])(mine + kX2Slots * 7 * kX2Block),
                              threadIdx.x % kX2Block);
   } else {
     double (*const s)[kX1Block] = (double (*)[kX1Block])lds;
-    pred_x1_tile<SAVE, FLUX>(insts, ninst, xcd_tile(b - nb2, n1, remap), s, s + 7,
+    pred_x1_tile<SAVE, FLUX, STREAM>(insts, ninst, xcd_tile(b - nb2, n1, remap), s, s + 7,
                              s + 14);
   }
 }
@@ -1400,8 +1420,12 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       for (int f = 0; f < 2; f++) {
         const InstList& l = b.of_flux[f];
         if (!l.ninst) continue;
-        const auto fn = f == kFluxHlle ? (save ? k_pred<true, kFluxHlle> : k_pred<false, kFluxHlle>)
-                                       : (save ? k_pred<true, kFluxRoe> : k_pred<false, kFluxRoe>);
+        const auto fn = save ? (f == kFluxHlle ? k_pred<true, kFluxHlle, false>
+                                               : k_pred<true, kFluxRoe, false>)
+                        : b.outgrows_cache ? (f == kFluxHlle ? k_pred<false, kFluxHlle, true>
+                                                             : k_pred<false, kFluxRoe, true>)
+                                           : (f == kFluxHlle ? k_pred<false, kFluxHlle, false>
+                                                             : k_pred<false, kFluxRoe, false>);
         const int n1 = l.ntiles[K_PRED_X1], n2 = l.ntiles[K_PRED_X2];
         const int nb2 = cdiv(n2, kX2PerBlock);
         hipLaunchKernelGGL(fn, dim3(n1 + nb2), dim3(kX1Block), 0, s, l.insts, l.ninst, n1, n2, nb2,

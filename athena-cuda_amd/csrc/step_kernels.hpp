@@ -33,6 +33,8 @@ enum PrimSave { P_WL1 = 0, P_WR1 = 7, P_WL2 = 14, P_WR2 = 21, NPRIMS = 28 };
 
 enum BcKind { BC_REFLECT = 1, BC_OUTFLOW = 2, BC_PERIODIC = 4 };
 
+constexpr size_t kInfinityCacheBytes = (size_t)256 << 20;
+
 constexpr int kDtSlots = 256;  // partial max slots of the fused dt reduction
 
 // Failure bits of an instance, raised by the step on the state it produces
@@ -173,6 +175,10 @@ struct BatchLaunch {
   InstList of_flux[2];  // by solver (kFluxRoe, kFluxHlle); ninst = 0: not in use
   int stale_ghosts;  // some instance's ghost fill reads stale ghosts (ghost_map.hpp)
   int thin;          // some instance has Nx1 or Nx2 < 4: ghosts may copy ghosts
+  // the batch's state and scratch planes outgrow the Infinity Cache: the
+  // predictors store past it (measured: 600^2, 247 MB, is slower so, 700^2,
+  // 330 MB, faster)
+  bool outgrows_cache;
   LaunchShape shape;
   int ncu;
   // a batch of one: its only list, read through descriptor `ins`
