@@ -1562,31 +1562,36 @@ ATHMI_HD int flux_roe_b(const Cons7& Ul, const Cons7& Ur, const Prim7& Wl, const
     Wrb.bz += pbrb * Wr.bz;
     return 0;
   }
+  // every loop over the seven waves is unrolled: a matrix entry is then one
+  // of the record's expressions and the vectors stay in registers (left as
+  // loops, each entry was a 49-way switch and the vectors sat in scratch)
   double dU[7], a[7];
+#pragma unroll
   for (int n = 0; n < 7; n++) dU[n] = arr(Ur)[n] - arr(Ul)[n];
+#pragma unroll
   for (int n = 0; n < 7; n++) {
     double acc = 0.0;
+#pragma unroll
     for (int m = 0; m < 7; m++)
       if (roe_Lnz(n, m)) acc = acc + e.L(n, m) * dU[m];
     a[n] = acc;
   }
-  // intermediate-state positivity test (:212-237)
+  // intermediate-state positivity test (:212-237); a state after the first
+  // failure is never used
   int flag = 0;
   {
     double ui[7];
+#pragma unroll
     for (int n = 0; n < 7; n++) ui[n] = arr(Ul)[n];
-    for (int n = 0; n < 6 && !flag; n++) {
+#pragma unroll
+    for (int n = 0; n < 6; n++) {
+#pragma unroll
       for (int m = 0; m < 7; m++)
         if (roe_Rnz(m, n)) ui[m] = ui[m] + a[n] * e.R(m, n);
-      if (e.ev[n + 1] > e.ev[n]) {
-        if (ui[0] <= 0.0) {
-          flag = 1;
-          break;
-        }
-        double pi = ui[4] - 0.5 * (sqr(ui[1]) + sqr(ui[2]) + sqr(ui[3])) / ui[0];
-        pi = pi - 0.5 * (sqr(ui[5]) + sqr(ui[6]) + sqr(Bxi));
-        if (pi < 0.0) flag = 2;
-      }
+      double pi = ui[4] - 0.5 * (sqr(ui[1]) + sqr(ui[2]) + sqr(ui[3])) / ui[0];
+      pi = pi - 0.5 * (sqr(ui[5]) + sqr(ui[6]) + sqr(Bxi));
+      const int f = (ui[0] <= 0.0) ? 1 : ((pi < 0.0) ? 2 : 0);
+      if (flag == 0 && e.ev[n + 1] > e.ev[n]) flag = f;
     }
   }
   if (flag) {
@@ -1594,9 +1599,12 @@ ATHMI_HD int flux_roe_b(const Cons7& Ul, const Cons7& Ur, const Prim7& Wl, const
     return flag;
   }
   double coeff[7], coeffb[7], ab[7], evb[7];
+#pragma unroll
   for (int m = 0; m < 7; m++) coeff[m] = 0.5 * dmax(fabs(e.ev[m]), 0.0) * a[m];
+#pragma unroll
   for (int m = 0; m < 7; m++) {
     double acc = 0.0;
+#pragma unroll
     for (int n = 0; n < 7; n++)
       if (roe_Rnz(n, m)) acc -= arr(Fb)[n] * e.R(n, m);
     coeffb[m] = acc;
@@ -1604,8 +1612,10 @@ ATHMI_HD int flux_roe_b(const Cons7& Ul, const Cons7& Ur, const Prim7& Wl, const
     ab[m] = coeffb[m] * 0.5 * mag;
     evb[m] = (fabs(e.ev[m]) > 0.0) ? coeffb[m] * 0.5 * a[m] * sgnabs(e.ev[m]) : 0.0;
   }
+#pragma unroll
   for (int m = 0; m < 7; m++) {
     double acc = 0.0;
+#pragma unroll
     for (int n = 0; n < 7; n++)
       if (roe_Lnz(n, m)) acc += ab[n] * e.L(n, m);
     arr(Urb)[m] += acc;
@@ -1615,6 +1625,7 @@ ATHMI_HD int flux_roe_b(const Cons7& Ul, const Cons7& Ur, const Prim7& Wl, const
   e.back([&](int n, int m) { return -arr(Fb)[n] * coeff[m]; },
          [&](int n, int m) { return ab[n] * dU[m]; }, evb, inb);
   Cons7 Fhb;
+#pragma unroll
   for (int n = 0; n < 7; n++) arr(Fhb)[n] = 0.5 * arr(Fb)[n];
   roe_side_b(Ul, Wl, Bxi, r.pbl, Fhb, Ulb, Wlb, Bxib, pblb);
   roe_side_b(Ur, Wr, Bxi, r.pbr, Fhb, Urb, Wrb, Bxib, pbrb);
