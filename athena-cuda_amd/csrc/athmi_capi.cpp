@@ -62,7 +62,7 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
   g->bl.shape.x2_seg = default_x2_seg(cols);
   g->bl.shape.persist = 0;
   g->bl.shape.xcd_remap = 1;
-  g->bl.shape.corr_rows = 2;  // 64 x 2 corrector tiles (at 4096^2: 1.46 against 1.60 ms for 64 x 4)
+  g->bl.shape.corr_rows = 1;  // one-row corrector tiles, which follow each other across row ends
   g->bl.shape.x2_kind = 1;  // the two-wave x2 predictor (1.79 against 2.05 ms at 4096^2)
   g->bl.shape.fuse_corner = 1;  // Step 9 corners inside k_final (the autotuner's pick at 4096^2)
   g->bl.shape.strip = 0;        // corrector and final tiles row by row

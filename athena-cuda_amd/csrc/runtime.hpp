@@ -109,8 +109,7 @@ struct athmi_grid {
       for (int k = 0; k < m; k++)
         for (int kind = 0; kind < NKINDS; kind++) {
           first[kind * m + k] = I[k].tile0[kind] = tot[kind];
-          tot[kind] += tiles_of(kind, I[k].nx1, I[k].nx2, bl.shape.x2_seg, bl.shape.corr_rows,
-                                bl.shape.final_rows);
+          tot[kind] += tiles_of(kind, I[k].nx1, I[k].nx2, bl.shape);
         }
       L.insts = reinterpret_cast<const Inst*>(base + used);
       L.ninst = m;

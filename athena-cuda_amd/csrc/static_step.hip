@@ -168,14 +168,13 @@ int athmi_integrate_static(const athmi_desc* desc, double dt, const double* stat
   bl.shape.x2_seg = default_x2_seg((long)cdiv(d.nx1 + 6, kX2Block) * (d.nx2 + 4));
   bl.shape.persist = 0;
   bl.shape.xcd_remap = 1;
-  bl.shape.corr_rows = 2;
+  bl.shape.corr_rows = 1;
   bl.shape.final_rows = 8;
   bl.shape.x2_kind = 1;
   bl.shape.fuse_corner = 1;
   for (int kind = 0; kind < NKINDS; kind++) {
     I.tile0[kind] = 0;
-    bl.all.ntiles[kind] = tiles_of(kind, d.nx1, d.nx2, bl.shape.x2_seg, bl.shape.corr_rows,
-                              bl.shape.final_rows);
+    bl.all.ntiles[kind] = tiles_of(kind, d.nx1, d.nx2, bl.shape);
   }
   bl.single(dinst, d.flux);
 

@@ -231,12 +231,13 @@ __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int
   const Clock* clk = g.clk;
   if (!clk->active) return;
   const int local = uni(t - g.tile0[K_PRED_X1]);
-  const int gis = uni(g.is), gie = uni(g.ie);
-  const int nseg = dcdiv(uni(g.nx1) + 4, kX1Faces);
-  const int row = local / nseg, seg = local - row * nseg;
-  const int j = uni(g.js) - 2 + row;
-  const int f0 = gis - 1 + seg * kX1Faces;
-  const int cell = f0 - 2 + tid;
+  // the tile's 128 cells in the row-after-row order of the cells is-3..ie+3 of
+  // rows js-2..je+2 (tiles overlap by the three halo cells; a tile may end one row
+  // and start the next: whole tiles per row left 19% of the lanes idle at 512^2)
+  const int w = uni(g.nx1) + 6;
+  const int q = local * kX1Faces + tid;
+  const int row = q / w, col = q - row * w;
+  const bool in = row < uni(g.nx2) + 4;
   const double dt = uni(clk->dts);
   const double dx1 = uni(g.dx1);
   const double dtodx1 = dt / dx1;
@@ -246,29 +247,28 @@ __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int
   double* __restrict__ sc = uni(g.scratch);
   double* __restrict__ pw = uni(g.prims);
   const size_t ps = (size_t)uni((int)g.ps);
-  const uint32_t rk = (uint32_t)(j * uni(g.pitch));
+  const uint32_t k = (uint32_t)((uni(g.js) - 2 + row) * uni(g.pitch) + uni(g.is) - 3 + col);
+  // cells with both neighbours (is-2..ie+2) in the tile
+  const bool mid = in && col >= 1 && col <= w - 2 && tid >= 1 && tid <= kX1Block - 2;
   double bxc = 0.0;
-  if (cell >= gis - 3 && cell <= gie + 3) {
-    const uint32_t k = rk + (uint32_t)cell;
+  if (in) {
     const double d = LD(st + F_D * ps, k), m1 = LD(st + F_M1 * ps, k), m2 = LD(st + F_M2 * ps, k);
     const double b1c = LD(st + F_B1C * ps, k), b2c = LD(st + F_B2C * ps, k);
     const Cons7 u{d, m1, m2, LD(st + F_M3 * ps, k), LD(st + F_E * ps, k), b2c, LD(st + F_B3C * ps, k)};
     bxc = b1c;
     lds_put(sw, tid, cons_to_prim(u, bxc, eos));
     // Step 3 (:249-255): emf3 at t^n over [jl,ju] x [il,iu]
-    if (cell >= gis - 2 && cell <= gie + 2 && tid >= 1 && tid <= kX1Block - 2)
-      ST(sc + S_ECC * ps, k, (b1c * m2 - b2c * m1) / d);
+    if (mid) ST(sc + S_ECC * ps, k, (b1c * m2 - b2c * m1) / d);
   }
   __syncthreads();
-  if (tid >= 1 && tid <= kX1Block - 2 && cell >= gis - 2 && cell <= gie + 2) {
+  if (mid) {
     Prim7 wl, wr;
     plm_cell_s(RowStencil{sw, tid}, bxc, dtodx1, eos, wl, wr);
     lds_put(swl, tid + 1, wl);
     lds_put(swr, tid, wr);
   }
   __syncthreads();
-  if (tid >= 2 && tid <= kX1Block - 2 && cell <= gie + 2) {
-    const uint32_t k = rk + (uint32_t)cell;
+  if (mid && tid >= 2 && col >= 2) {
     // face states: PLM output + MHD source terms for 1/2 dt (:156-164) +
     // prim->cons (:175-176); rebuilt from LDS and memory for the HLLE fallback
     auto build = [&](Cons7& ul, Cons7& ur, Prim7& wl, Prim7& wr, double& b0) {
@@ -309,6 +309,26 @@ __global__ void __launch_bounds__(kX1Block, 2) k_pred_x1(const Inst* __restrict_
   }
 }
 
+// Segment and column of lane `lane` of x2 tile `local`: aligned chunks of each
+// segment's columns, or the columns is-2..ie+2 of segment 0, then those of
+// segment 1, ... in one sequence (a wave may end one segment and start the
+// next); x2_aligned says which. False for a lane without a column.
+__device__ __forceinline__ bool x2_lane(const Inst& g, int local, int lane, int seg_len, int& sg,
+                                        int& i) {
+  const int nx1 = uni(g.nx1);
+  if (x2_aligned(nx1)) {
+    const int ncb = dcdiv(nx1 + 6, kX2Block);
+    sg = local / ncb;
+    i = (local - sg * ncb) * kX2Block + lane;
+    return i >= uni(g.is) - 2 && i <= uni(g.ie) + 2;
+  }
+  const int w = nx1 + 4;
+  const int e = local * kX2Block + lane;
+  sg = e / w;
+  i = uni(g.is) - 2 + (e - sg * w);
+  return sg < dcdiv(uni(g.nx2) + 4, seg_len);
+}
+
 // ---------------------------------------------------------------------------
 // Steps 2a-2e (__integrate_2d__.c:189-241): the x2 sweep in the permuted
 // order (d, M2, M3, M1, E, B3c, B1c) with Bx = B2c. Lanes own adjacent
@@ -328,12 +348,8 @@ __global__ void __launch_bounds__(kX2Block) k_pred_x2(const Inst* __restrict__ i
     const Clock* clk = g.clk;
     if (!clk->active) continue;
     const int local = t - g.tile0[K_PRED_X2];
-    // chunks from column 0: each row segment starts on a cache line
-    const int ncb = dcdiv(g.nx1 + 6, kX2Block);
-    const int sg = local / ncb, cb = local - sg * ncb;
-    const int i = cb * kX2Block + lane;
-    if (i < g.is - 2) continue;
-    if (i > g.ie + 2) continue;
+    int sg, i;
+    if (!x2_lane(g, local, lane, seg_len, sg, i)) continue;
     const int jf0 = g.js - 1 + sg * seg_len;
     const int jf1 = min(jf0 + seg_len - 1, g.je + 2);
     const double dt = clk->dts;
@@ -435,7 +451,8 @@ template <bool SAVE, int FLUX, bool STREAM = false>
 __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int ninst, int t,
                                              int seg_len, X2Slots* slots,
                                              double (*aux)[kX2Block], int lane) {
-  // aux rows: B2i of row r at r & 1, s(r) at 2 + (r & 1), M1/d of the newest row
+  // rows are counted from the march's first face row jf0. aux rows: B2i of row
+  // r at r & 1, s(r) at 2 + (r & 1), M1/d of the newest row
   auto b2i_slot = [&](int r) -> double& { return aux[r & 1][lane]; };
   auto src_slot = [&](int r) -> double& { return aux[2 + (r & 1)][lane]; };
   double& v1_carry = aux[4][lane];
@@ -463,14 +480,10 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
   const Clock* clk = g.clk;
   if (!clk->active) return;
   const int local = uni(t - g.tile0[K_PRED_X2]);
-  // chunks from column 0: each row segment starts on a cache line
-  const int ncb = dcdiv(uni(g.nx1) + 6, kX2Block);
-  const int sg = local / ncb, cb = local - sg * ncb;
-  const int i = cb * kX2Block + lane;
-  if (i < uni(g.is) - 2) return;
-  if (i > uni(g.ie) + 2) return;
+  int sg, i;
+  if (!x2_lane(g, local, lane, seg_len, sg, i)) return;
   const int jf0 = uni(g.js) - 1 + sg * seg_len;
-  const int jf1 = min(jf0 + seg_len - 1, uni(g.je) + 2);
+  const int nf = min(seg_len, uni(g.je) + 3 - jf0);
   const double dt = uni(clk->dts);
   const double dx2 = uni(g.dx2);
   const double dtodx2 = dt / dx2;
@@ -481,10 +494,11 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
   double* __restrict__ pw = uni(g.prims);
   const size_t ps = (size_t)uni((int)g.ps);
   const int pitch = uni(g.pitch);
-  // cons->prim of row jj in the permuted order (d, M2, M3, M1, E, B3c, B1c), Bx = B2c;
+  const uint32_t k0 = (uint32_t)(jf0 * pitch + i);
+  // cons->prim of row r in the permuted order (d, M2, M3, M1, E, B3c, B1c), Bx = B2c;
   // with M1/d (the source term's division form) and B2i of the row
-  auto load_row = [&](int jj, int slot, double& v1, double& b2i) {
-    const uint32_t k = (uint32_t)(jj * pitch + i);
+  auto load_row = [&](int r, int slot, double& v1, double& b2i) {
+    const uint32_t k = k0 + (uint32_t)(r * pitch);
     const double d = LD(st + F_D * ps, k), m1 = LD(st + F_M1 * ps, k);
     const Cons7 u{d, LD(st + F_M2 * ps, k), LD(st + F_M3 * ps, k), m1,
                   LD(st + F_E * ps, k), LD(st + F_B3C * ps, k), LD(st + F_B1C * ps, k)};
@@ -492,46 +506,45 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
     v1 = m1 / d;
     b2i = LD(st + F_B2I * ps, k);
   };
-  auto bx_at = [&](int jj) { return LD(st + F_B2C * ps, (uint32_t)(jj * pitch + i)); };
-  // start of the march: rows jf0-2, jf0-1, jf0, the source s(jf0-1) and
-  // the PLM of cell jf0-1
+  auto bx_at = [&](int r) { return LD(st + F_B2C * ps, k0 + (uint32_t)(r * pitch)); };
+  // start of the march: rows -2, -1, 0, the source s(-1) and the PLM of cell -1
   {
     double v1m, b2m, v10, b20, v1u, b2u;
-    load_row(jf0 - 2, 0, v1u, b2u);
-    load_row(jf0 - 1, 1, v1m, b2m);
-    load_row(jf0, 2, v10, b20);
-    src_slot(jf0 - 1) = v1m * (b20 - b2m) / dx2;
-    b2i_slot(jf0) = b20;
+    load_row(-2, 0, v1u, b2u);
+    load_row(-1, 1, v1m, b2m);
+    load_row(0, 2, v10, b20);
+    src_slot(-1) = v1m * (b20 - b2m) / dx2;
+    b2i_slot(0) = b20;
     v1_carry = v10;
   }
   {
     Prim7 wl, wr_unused;
-    plm_cell_s(LdsStencil{&get, 0, 1, 2}, bx_at(jf0 - 1), dtodx2, eos, wl, wr_unused);
+    plm_cell_s(LdsStencil{&get, 0, 1, 2}, bx_at(-1), dtodx2, eos, wl, wr_unused);
     compiler_fence();
     put(0, wl);
   }
   int sP = 1, sQ = 2, sW = 0, sF = 3;  // rows j-1, j; pending Wl(j); free
-  for (int j = jf0; j <= jf1; j++) {
+  for (int r = 0; r < nf; r++) {
     phase_fence();
     {
-      // row j+1; then s(j) = (M1/d)(j) (B2i(j+1) - B2i(j)) / dx2 (:216-224)
+      // row r+1; then s(r) = (M1/d)(r) (B2i(r+1) - B2i(r)) / dx2 (:216-224)
       double v1n, b2n;
-      load_row(j + 1, sF, v1n, b2n);
-      src_slot(j) = v1_carry * (b2n - b2i_slot(j)) / dx2;
-      b2i_slot(j + 1) = b2n;
+      load_row(r + 1, sF, v1n, b2n);
+      src_slot(r) = v1_carry * (b2n - b2i_slot(r)) / dx2;
+      b2i_slot(r + 1) = b2n;
       v1_carry = v1n;
     }
     phase_fence();
     {
       Prim7 wl_next, wr_cur;
       const LdsStencil sten{&get, sP, sQ, sF};
-      plm_cell_s(sten, bx_at(j), dtodx2, eos, wl_next, wr_cur);
+      plm_cell_s(sten, bx_at(r), dtodx2, eos, wl_next, wr_cur);
       compiler_fence();
       put(kWr, wr_cur);
       put(sP, wl_next);
     }
     phase_fence();
-    const uint32_t k = (uint32_t)(j * pitch + i);
+    const uint32_t k = k0 + (uint32_t)(r * pitch);
     const int sw = sW;
     // face states: PLM output + MHD source terms for 1/2 dt (:216-224) +
     // prim->cons (:235-236); rebuilt from LDS for the HLLE fallback
@@ -539,9 +552,9 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
       compiler_fence();
       wl = get(sw);
       wr = get(kWr);
-      b0 = b2i_slot(j);
-      wl.bz = wl.bz + hdt * src_slot(j - 1);
-      wr.bz = wr.bz + hdt * src_slot(j);
+      b0 = b2i_slot(r);
+      wl.bz = wl.bz + hdt * src_slot(r - 1);
+      wr.bz = wr.bz + hdt * src_slot(r);
       ul = prim_to_cons(wl, b0, eos);
       ur = prim_to_cons(wr, b0, eos);
     };
@@ -556,7 +569,7 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
     put7<STREAM>(sc + S_UL2 * ps, ps, k, ul);
     put7<STREAM>(sc + S_UR2 * ps, ps, k, ur);
     put7<STREAM>(sc + S_F2 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
-    // rotate: row j -> j-1, row j+1 -> j, Wl(j+1) pending, Wl(j)'s slot free
+    // rotate: row r -> r-1, row r+1 -> r, Wl(r+1) pending, Wl(r)'s slot free
     const int nP = sQ, nQ = sF, nW = sP, nF = sW;
     sP = nP; sQ = nQ; sW = nW; sF = nF;
   }
@@ -704,12 +717,12 @@ __global__ void __launch_bounds__(kTileX* kTileY) k_corner(const Inst* __restric
     const Inst& g = insts[find_inst(insts, ninst, kind, t)];
     if (!g.clk->active) continue;
     const int local = t - g.tile0[kind];
-    const int w = PRED ? g.nx1 + 4 : g.nx1 + 2;
-    const int ntx = dcdiv(w, kTileX);
-    const int ty = local / ntx, tx = local - ty * ntx;
-    const int i = (PRED ? g.is - 1 : g.is) + tx * kTileX + threadIdx.x;
-    const int j = (PRED ? g.js - 1 : g.js) + ty * kTileY + threadIdx.y;
-    if (i > g.ie + (PRED ? 2 : 1) || j > g.je + (PRED ? 2 : 1)) continue;
+    const int w = PRED ? g.nx1 + 3 : g.nx1 + 1;
+    const int e = local * (kTileX * kTileY) + threadIdx.y * kTileX + threadIdx.x;
+    const int r = e / w;
+    const int i = (PRED ? g.is - 1 : g.is) + (e - r * w);
+    const int j = (PRED ? g.js - 1 : g.js) + r;
+    if (j > g.je + (PRED ? 2 : 1)) continue;
     const size_t ps = g.ps;
     const int pitch = g.pitch;
     double* __restrict__ sc = g.scratch;
@@ -748,11 +761,23 @@ __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ni
   if (!clk->active) return;
   const int local = uni(t - g.tile0[K_CORR]);
   const int gis = uni(g.is), gjs = uni(g.js);
-  int tx, ty;
-  tile_pos(local, dcdiv(uni(g.nx1) + 3, kTileX), dcdiv(uni(g.nx2) + 3, TY), strip, tx, ty);
-  const int i0 = gis - 1 + tx * kTileX, j0 = gjs - 1 + ty * TY;
-  const int i = i0 + threadIdx.x;
-  const int j = j0 + threadIdx.y;
+  int i0, j0, i, j;
+  if (TY == 1 && !CP && strip == 0) {
+    // one row: the cells row after row, 64 to a tile (whole tiles per row left
+    // 10% of the lanes idle at 512^2)
+    const int w = uni(g.nx1) + 2;
+    const int e = local * kTileX + threadIdx.x;
+    const int r = e / w;
+    i0 = i = gis - 1 + (e - r * w);
+    j0 = j = gjs - 1 + r;
+  } else {
+    int tx, ty;
+    tile_pos(local, dcdiv(uni(g.nx1) + 3, kTileX), dcdiv(uni(g.nx2) + 3, TY), strip, tx, ty);
+    i0 = gis - 1 + tx * kTileX;
+    j0 = gjs - 1 + ty * TY;
+    i = i0 + threadIdx.x;
+    j = j0 + threadIdx.y;
+  }
   if (CP) {
     // every thread of the block reaches both barriers: the one before the
     // fill keeps the previous tile's readers ahead of it
@@ -972,8 +997,10 @@ __device__ __forceinline__ int cell_fail_bits(const Inst& g, double d, double M1
   return bits;
 }
 
-// Steps 9, 11a, 11b, 13 (:473-534) over [js,je+1]x[is,ie+1] into the other
-// ping-pong buffer, and the new_dt maximum of the updated interior. The B2c
+// Steps 9, 11a, 11b, 13 (:473-534) over the interior cells and their faces
+// (the last column and row also store their upper faces, so that a 512-cell row is
+// eight tiles, not nine) into the other ping-pong buffer, and the new_dt
+// maximum of the updated interior. The B2c
 // update of 11a and the B1c update of 11b are dropped: Step 13 overwrites them.
 // FUSED: the tile first computes the Step 9 corner emf it reads -- (TY+1)
 // x (kTileX+1) corners -- into LDS from the corrector fluxes, instead of
@@ -999,7 +1026,7 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
     if (!clk->active) continue;
     const int local = t - g.tile0[K_FINAL];
     int tx, ty;
-    tile_pos(local, dcdiv(g.nx1 + 1, kTileX), dcdiv(g.nx2 + 1, TY), strip, tx, ty);
+    tile_pos(local, dcdiv(g.nx1, kTileX), dcdiv(g.nx2, TY), strip, tx, ty);
     const int i0 = g.is + tx * kTileX, j0 = g.js + ty * TY;
     const int i = i0 + threadIdx.x;
     const int j = j0 + threadIdx.y;
@@ -1019,7 +1046,7 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
       __syncthreads();
     }
     double dti = 0.0;
-    if (i <= g.ie + 1 && j <= g.je + 1) {
+    if (i <= g.ie && j <= g.je) {
       const double dt = clk->dts;
       const double dtodx1 = dt / g.dx1, dtodx2 = dt / g.dx2;
       const int cur = clk->cur;
@@ -1034,8 +1061,7 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
       auto corner = [&](int dj, int di) {
         return FUSED ? cemf[cc + dj * kCornerCols + di] : LD(emf, k + dj * pitch + di);
       };
-      const double e00 = corner(0, 0), e10 = corner(1, 0), e01 = corner(0, 1);
-      double b1n = 0.0, b2n = 0.0;
+      const double e00 = corner(0, 0), e10 = corner(1, 0), e01 = corner(0, 1), e11 = corner(1, 1);
       // set_bvals from the source's side: only a tile that reaches the five
       // cells at an edge (four, and the face past them) has ghost images
       const bool edge = fill && (i0 <= g.is + 4 || i0 + kTileX > g.ie - 4 || j0 <= g.js + 4 ||
@@ -1045,28 +1071,32 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
         ix = ghost_images(i, g.is, g.ie, g.bc[0], g.bc[1], false);
         iy = ghost_images(j, g.js, g.je, g.bc[2], g.bc[3], false);
       }
-      if (j <= g.je) {
-        b1n = LD(st + F_B1I * ps, k) - dtodx2 * (e10 - e00);
-        ST(out + F_B1I * ps, k, b1n);
+      // the cell's lower faces, and the upper ones of the last column and row
+      auto put_b1 = [&](int ii, double v) {
+        ST(out + F_B1I * ps, (uint32_t)(j * pitch + ii), v);
         if (edge)
-          for_ghost_images(g, j, i, ghost_images(i, g.is, g.ie, g.bc[0], g.bc[1], true), iy,
+          for_ghost_images(g, j, ii, ghost_images(ii, g.is, g.ie, g.bc[0], g.bc[1], true), iy,
                            [&](int r, int c, bool, bool) {
-                             ST(out + F_B1I * ps, (uint32_t)(r * pitch + c), b1n);
+                             ST(out + F_B1I * ps, (uint32_t)(r * pitch + c), v);
                            });
-      }
-      if (i <= g.ie) {
-        b2n = LD(st + F_B2I * ps, k) + dtodx1 * (e01 - e00);
-        ST(out + F_B2I * ps, k, b2n);
+      };
+      auto put_b2 = [&](int jj, double v) {
+        ST(out + F_B2I * ps, (uint32_t)(jj * pitch + i), v);
         if (edge)
-          for_ghost_images(g, j, i, ix, ghost_images(j, g.js, g.je, g.bc[2], g.bc[3], true),
+          for_ghost_images(g, jj, i, ix, ghost_images(jj, g.js, g.je, g.bc[2], g.bc[3], true),
                            [&](int r, int c, bool, bool) {
-                             ST(out + F_B2I * ps, (uint32_t)(r * pitch + c), b2n);
+                             ST(out + F_B2I * ps, (uint32_t)(r * pitch + c), v);
                            });
-      }
-      if (j <= g.je && i <= g.ie) {
-        const double e11 = corner(1, 1);
-        const double b1p = LD(st + F_B1I * ps, k + 1) - dtodx2 * (e11 - e01);
-        const double b2p = LD(st + F_B2I * ps, k + pitch) + dtodx1 * (e11 - e10);
+      };
+      const double b1n = LD(st + F_B1I * ps, k) - dtodx2 * (e10 - e00);
+      const double b1p = LD(st + F_B1I * ps, k + 1) - dtodx2 * (e11 - e01);
+      const double b2n = LD(st + F_B2I * ps, k) + dtodx1 * (e01 - e00);
+      const double b2p = LD(st + F_B2I * ps, k + pitch) + dtodx1 * (e11 - e10);
+      put_b1(i, b1n);
+      if (i == g.ie) put_b1(i + 1, b1p);
+      put_b2(j, b2n);
+      if (j == g.je) put_b2(j + 1, b2p);
+      {
         const double* F1 = sc + S_F1C * ps;
         const double* F2 = sc + S_F2C * ps;
         double d = LD(st + F_D * ps, k), M1 = LD(st + F_M1 * ps, k), M2 = LD(st + F_M2 * ps, k);

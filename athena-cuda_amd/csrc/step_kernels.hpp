@@ -2,6 +2,8 @@
 // of the CTU+CT step. One "instance" is one 2-D grid (the reference's Grid,
 // athena.h:106-120); the plain step is a batch of one instance.
 #pragma once
+#include <hip/hip_runtime.h>
+
 #include <cmath>
 #include <cstddef>
 #include <cstdint>
@@ -77,14 +79,13 @@ struct Inst {
 // Tile kinds (one per kernel family); tile counts per instance come from
 // tiles_of() below so host and device agree on the decomposition.
 enum KernelKind {
-  K_PRED_X1 = 0,  // rows js-2..je+2, faces is-1..ie+2 in segments of kX1Faces
-  K_PRED_X2,      // columns is-2..ie+2 in chunks of kX2Block from column 0 (row segments
-                  // start on a 128-byte line: the pitch is a multiple of 16), faces
-                  // js-1..je+2 in segments
+  K_PRED_X1 = 0,  // cells is-3..ie+3 of rows js-2..je+2 in one sequence, kX1Faces to a tile
+  K_PRED_X2,      // columns is-2..ie+2 of segments of faces js-1..je+2, kX2Block to a
+                  // tile, in chunks or in one sequence (x2_aligned)
   K_CORR,         // cells [js-1,je+1] x [is-1,ie+1]
   K_CORNER_P,     // corners [js-1,je+2] x [is-1,ie+2]
   K_CORNER_C,     // corners [js,je+1] x [is,ie+1]
-  K_FINAL,        // faces/cells [js,je+1] x [is,ie+1]
+  K_FINAL,        // cells [js,je] x [is,ie]
   K_GHOST,        // ghost cells of all planes
   K_INTERIOR,     // cells [js,je] x [is,ie]
   NKINDS
@@ -106,9 +107,6 @@ inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 // rows of a final-update tile (64 x 4, 8 or 16 cells; anything else: 4)
 inline int final_rows_of(int rows) { return (rows == 8 || rows == 16) ? rows : kTileY; }
 
-// number of tiles of kind k for a grid of nx1 x nx2 zones (x2seg: faces
-// marched per thread by the x2 predictor; corr_rows, final_rows: tile heights
-// of the corrector and the final update)
 // Default faces marched per x2-predictor lane for `cols` lane-columns of x2
 // faces (64-column chunks x rows over the batch): shorter segments give more
 // workgroups (less tail at the end of the launch) for more halo rows per face.
@@ -117,20 +115,6 @@ inline int final_rows_of(int rows) { return (rows == 8 || rows == 16) ? rows : k
 inline int default_x2_seg(long cols) {
   const long s = std::lround(std::sqrt((double)cols) / 50.0);
   return (int)(s < 1 ? 1 : (s > 16 ? 16 : s));
-}
-
-inline int tiles_of(int k, int nx1, int nx2, int x2seg, int corr_rows, int final_rows) {
-  const int sx = nx1 + 8;
-  switch (k) {
-    case K_PRED_X1: return (nx2 + 4) * cdiv(nx1 + 4, kX1Faces);
-    case K_PRED_X2: return cdiv(nx1 + 6, kX2Block) * cdiv(nx2 + 4, x2seg);
-    case K_CORR: return cdiv(nx1 + 3, kTileX) * cdiv(nx2 + 3, corr_rows);
-    case K_CORNER_P: return cdiv(nx1 + 4, kTileX) * cdiv(nx2 + 4, kTileY);
-    case K_CORNER_C: return cdiv(nx1 + 2, kTileX) * cdiv(nx2 + 2, kTileY);
-    case K_FINAL: return cdiv(nx1 + 1, kTileX) * cdiv(nx2 + 1, final_rows_of(final_rows));
-    case K_GHOST: return cdiv(8 * sx + (nx2 + 1) * 8, kGhostBlock);
-    default: return cdiv(nx1, kTileX) * cdiv(nx2, kTileY);
-  }
 }
 
 // whether an instance's set_bvals reads ghosts as they were before it (an
@@ -156,6 +140,38 @@ struct LaunchShape {
                      // s > 0 = strips of s tile columns walked row by row
   int final_rows;    // rows of a final-update tile: 4, 8 or 16 (final_rows_of)
 };
+
+// Whether a grid's x2 tiles start on a cache line: whole chunks of 64 columns
+// from column 0 (the pitch is a multiple of 16), where they leave less than 3%
+// of the lanes idle (HLLE, bound by memory: 3000^2 3303 -> 3255 us a step, 4096^2
+// 6165 -> 6097; Roe within 0.3%); otherwise the columns follow each other across
+// the segments' ends (at 512^2 whole chunks leave 10% of the lanes idle)
+__host__ __device__ inline bool x2_aligned(int nx1) {
+  const int lanes = (nx1 + 6 + kX2Block - 1) / kX2Block * kX2Block;
+  return 100 * (lanes - (nx1 + 4)) < 3 * lanes;
+}
+
+// number of tiles of kind k for a grid of nx1 x nx2 zones
+inline int tiles_of(int k, int nx1, int nx2, const LaunchShape& sh) {
+  const int sx = nx1 + 8;
+  switch (k) {
+    case K_PRED_X1: return cdiv((nx2 + 4) * (nx1 + 6) - 3, kX1Faces);
+    case K_PRED_X2: {
+      const int nseg = cdiv(nx2 + 4, sh.x2_seg);
+      return x2_aligned(nx1) ? cdiv(nx1 + 6, kX2Block) * nseg : cdiv((nx1 + 4) * nseg, kX2Block);
+    }
+    case K_CORR:
+      // tiles of one row without strips follow each other across the rows' ends
+      if (sh.corr_rows == 1 && sh.strip == 0 && sh.fuse_corner < 2)
+        return cdiv((nx1 + 2) * (nx2 + 2), kTileX);
+      return cdiv(nx1 + 3, kTileX) * cdiv(nx2 + 3, sh.corr_rows);
+    case K_CORNER_P: return cdiv((nx1 + 3) * (nx2 + 3), kTileX * kTileY);
+    case K_CORNER_C: return cdiv((nx1 + 1) * (nx2 + 1), kTileX * kTileY);
+    case K_FINAL: return cdiv(nx1, kTileX) * cdiv(nx2, final_rows_of(sh.final_rows));
+    case K_GHOST: return cdiv(8 * sx + (nx2 + 1) * 8, kGhostBlock);
+    default: return cdiv(nx1, kTileX) * cdiv(nx2, kTileY);
+  }
+}
 
 // A list of instances on the device and its tile totals per kernel kind. In
 // device memory the descriptors are followed by the first tiles again, as a

@@ -136,8 +136,8 @@ int athmi_set_shape(athmi_grid *g, int x2_seg, int persist);
 /* Tile order: 1 = each of the 8 XCDs gets one contiguous run of tiles (its L2
  * serves the neighbour rows), 0 = launch order. Results are identical. */
 int athmi_set_tile_order(athmi_grid *g, int xcd_remap);
-/* Rows of a corrector tile (64 x rows faces: 1, 2 or 4; default 2). Results
- * are identical. */
+/* Rows of a corrector tile (64 x rows faces: 1, 2 or 4; default 1: 64 cells
+ * in a row-after-row sequence). Results are identical. */
 int athmi_set_corr_rows(athmi_grid *g, int rows);
 /* Form of the x2 predictor: 0 = each lane marches its column with the PLM
  * stencil in registers (one wave per SIMD), 1 = the stencil and pending face
