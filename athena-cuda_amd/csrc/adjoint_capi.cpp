@@ -39,13 +39,9 @@ const int kSeqRolloutStep[] = {SK_PRED,     SK_CORNER_P,    SK_CORR_BOTH,
                                SK_CORNER_C, SK_FINAL_GHOST, SK_END_ONCE};
 // dt never changes along a rollout: the clock is started once per run of steps
 const int kSeqStart[] = {SK_BEGIN_ONCE};
-// the reverse of one step on two streams: the x1 and x2 halves of Steps 8
-// and 1-2 are independent (their adjoints meet in ain through atomic adds)
-const int kRevHead[] = {AK_FOLD_OUT, AK_ZERO, AK_UPDATE, AK_CORNER_C};  // then fork
-const int kRevMainA[] = {AK_RIEMANN_C1, AK_HALF};                       // || AK_RIEMANN_C2
-const int kRevMid[] = {AK_TRANSVERSE, AK_CORNER_P, AK_EMF_CC};          // after the join
-const int kRevTailA[] = {AK_PRED_X1, AK_PLM_X1, AK_PLMG_X1};            // || x2 tail
-const int kRevTailB[] = {AK_PRED_X2, AK_PLM_X2, AK_PLMG_X2};
+// the reverse of one step
+const int kRevStep[] = {AK_FOLD,    AK_UPDATE, AK_CORRECT,   AK_TRANSVERSE,
+                        AK_PREDICT, AK_PLM,    AK_PLM_GATHER};
 // a slot of the segment's forward scratch: the step's NSCRATCH planes, a copy
 // of its predictor corner emf (used at fusion depth 0, where the corrector's
 // corner kernel overwrites S_EMF) and the predictors' NPRIMS primitive face
@@ -78,9 +74,8 @@ struct athmi_adjoint {
   // first step reads state buffer p is dslot[(2 b + p) K + m] (state buffers
   // seg[b][m], seg[b][m+1], scratch slot [b][m])
   Inst* dslot = nullptr;
-  hipStream_t astream = nullptr, bstream = nullptr;  // the reversal's two streams
+  hipStream_t astream = nullptr;  // the reversal's stream
   hipEvent_t ev_rerun[2] = {nullptr, nullptr}, ev_rev[2] = {nullptr, nullptr}, ev_sync = nullptr;
-  hipEvent_t ev_fork1 = nullptr, ev_join1 = nullptr, ev_fork2 = nullptr, ev_join2 = nullptr;
 
   double* seg_state(int b, int m) const {
     return seg + ((size_t)b * (every + 1) + m) * state_doubles;
@@ -218,12 +213,7 @@ int athmi_adjoint_create(const athmi_desc* desc, double dt, int nsteps, int ever
       athmi_adjoint_destroy(h);
       return fail(ATHMI_EHIP, "athmi_adjoint_create: event creation failed");
     }
-  if (hipStreamCreateWithFlags(&h->bstream, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&h->ev_sync, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&h->ev_fork1, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&h->ev_join1, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&h->ev_fork2, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&h->ev_join2, hipEventDisableTiming) != hipSuccess) {
+  if (hipEventCreateWithFlags(&h->ev_sync, hipEventDisableTiming) != hipSuccess) {
     athmi_adjoint_destroy(h);
     return fail(ATHMI_EHIP, "athmi_adjoint_create: event creation failed");
   }
@@ -269,11 +259,8 @@ int athmi_adjoint_destroy(athmi_adjoint* h) {
     if (h->ev_rerun[b]) (void)hipEventDestroy(h->ev_rerun[b]);
     if (h->ev_rev[b]) (void)hipEventDestroy(h->ev_rev[b]);
   }
-  for (hipEvent_t e : {h->ev_sync, h->ev_fork1, h->ev_join1, h->ev_fork2, h->ev_join2})
-    if (e) (void)hipEventDestroy(e);
-  if (h->bstream) (void)hipStreamSynchronize(h->bstream);
+  if (h->ev_sync) (void)hipEventDestroy(h->ev_sync);
   if (h->astream) (void)hipStreamDestroy(h->astream);
-  if (h->bstream) (void)hipStreamDestroy(h->bstream);
   if (h->g) athmi_destroy(h->g);
   delete h;
   return ATHMI_OK;
@@ -336,7 +323,7 @@ int athmi_adjoint_backward(athmi_adjoint* h, const double* gradN, double* grad0)
   if (!h->have_forward)
     return fail(ATHMI_ESTATE, "athmi_adjoint_backward: run athmi_adjoint_forward first");
   int rc;
-  hipStream_t R = h->g->stream, A = h->astream, B = h->bstream;
+  hipStream_t R = h->g->stream, A = h->astream;
   double* aout = h->adj[0];
   double* ain = h->adj[1];
   if ((rc = dense_to_planes(h, aout, gradN, R))) return rc;
@@ -346,16 +333,9 @@ int athmi_adjoint_backward(athmi_adjoint* h, const double* gradN, double* grad0)
   a.dt = h->dt;
   a.ain = ain;
   a.det = h->det ? 1 : 0;
-  a.color = 0;
-  // the deterministic reverse runs every kernel of a step on one stream, in
-  // the order of the two-stream schedule, with the scatters replaced by
-  // ordered gathers (fold, predictor sources) or disjoint launches (corners)
-  const int fold = h->det ? AK_FOLD_OUT_DET : AK_FOLD_OUT;
-  if (h->det) B = A;
   HIP_TRY(athmi_adjoint_launch(&a, AK_CLEAR, R));
   HIP_TRY(hipEventRecord(h->ev_sync, R));
   HIP_TRY(hipStreamWaitEvent(A, h->ev_sync, 0));
-  HIP_TRY(hipEventRecord(h->ev_join2, A));  // nothing pending on B yet
   const size_t ps = a.g.ps;
   bool rev_pending[2] = {false, false};
   const int blast = (h->nck - 1) % h->nbank;
@@ -374,24 +354,9 @@ int athmi_adjoint_backward(athmi_adjoint* h, const double* gradN, double* grad0)
       a.pw = sc + kSlotPrims * ps;
       a.ain = ain;
       a.aout = aout;
-      // the previous step's x2 tail on B wrote ain planes this step folds
-      HIP_TRY(hipStreamWaitEvent(A, h->ev_join2, 0));
-      for (int k : kRevHead) HIP_TRY(athmi_adjoint_launch(&a, k == AK_FOLD_OUT ? fold : k, A));
-      HIP_TRY(hipEventRecord(h->ev_fork1, A));
-      HIP_TRY(hipStreamWaitEvent(B, h->ev_fork1, 0));
-      HIP_TRY(athmi_adjoint_launch(&a, AK_RIEMANN_C2, B));
-      HIP_TRY(hipEventRecord(h->ev_join1, B));
-      for (int k : kRevMainA) HIP_TRY(athmi_adjoint_launch(&a, k, A));
-      HIP_TRY(hipStreamWaitEvent(A, h->ev_join1, 0));
-      for (int k : kRevMid) HIP_TRY(athmi_adjoint_launch(&a, k, A));
-      HIP_TRY(hipEventRecord(h->ev_fork2, A));
-      HIP_TRY(hipStreamWaitEvent(B, h->ev_fork2, 0));
-      for (int k : kRevTailB) HIP_TRY(athmi_adjoint_launch(&a, k, B));
-      HIP_TRY(hipEventRecord(h->ev_join2, B));
-      for (int k : kRevTailA) HIP_TRY(athmi_adjoint_launch(&a, k, A));
+      for (int k : kRevStep) HIP_TRY(athmi_adjoint_launch(&a, k, A));
       std::swap(ain, aout);
     }
-    HIP_TRY(hipStreamWaitEvent(A, h->ev_join2, 0));
     HIP_TRY(hipEventRecord(h->ev_rev[b], A));
     rev_pending[b] = true;
     // meanwhile re-run segment s-1 into its bank, once that bank's last
@@ -405,7 +370,8 @@ int athmi_adjoint_backward(athmi_adjoint* h, const double* gradN, double* grad0)
   }
   // the set_bvals that precedes the first step
   a.aout = aout;
-  HIP_TRY(athmi_adjoint_launch(&a, fold, A));
+  HIP_TRY(athmi_adjoint_launch(&a, AK_FOLD, A));
+  HIP_TRY(athmi_adjoint_launch(&a, AK_CLEAR_GHOST, A));
   if ((rc = planes_to_dense(h, grad0, aout, A))) return rc;
   HIP_TRY(hipStreamSynchronize(A));
   HIP_TRY(hipStreamSynchronize(R));

@@ -6,17 +6,21 @@
 // conserved and primitive, and fluxes, predictor corner emf, corrector
 // fluxes), the kernels below run the step's stages in reverse and accumulate
 // the adjoint of S^n into ain:
-//   fold        set_bvals: each ghost's adjoint is added to the cell it copies
+//   fold        set_bvals: each cell adds the adjoints of the ghosts that copy it
 //   update      Steps 9, 11a, 11b, 13 -> corrector fluxes, corner emf, identity
-//   corner<C>   Step 9 corner emf -> corrector fluxes' By/Bz, emf3 at t^{n+1/2}
-//   riemann_c   Steps 8b / 8c: corrector Riemann fluxes -> corrected face states
-//   half        Step 7: emf3 at t^{n+1/2} -> half-step face fields, predictor fluxes
+//   correct     Steps 8b / 8c: corrector Riemann fluxes -> corrected face states;
+//               Step 7: emf3 at t^{n+1/2} -> half-step face fields, predictor fluxes
 //   transverse  Steps 5, 6 and the half-step face fields of Step 4
-//   corner<P>   Step 4 corner emf -> predictor fluxes' By/Bz, emf3 at t^n
-//   emf_cc      Step 3
-//   pred<X1/X2> Steps 1c-1e / 2c-2e: sources, prim->cons, predictor fluxes
-//   plm_x1/x2   Steps 1b / 2b: the PLM reconstruction
+//   predict     Steps 1c-1e / 2c-2e: sources, prim->cons, predictor fluxes; Step 3
+//   plm         Steps 1b / 2b: the PLM reconstruction
 //   plm_gather  Steps 1a / 2a: cons->prim
+// The corner emf of Steps 9 and 4 is reversed by its inputs: the corrector and
+// predictor fluxes' By/Bz and the cell-centred emf3 gather their corners'
+// adjoints where their own reverse reads them.
+// One launch holds both sweeps (and Step 7, Step 3 beside them), so a reversed
+// step is seven launches on one stream. The stages that hold few waves per SIMD
+// (correct, predict, plm) run in workgroups of one wave over a row-after-row
+// sequence of cells: at 512^2 whole 64-wide tiles left a tenth of the lanes idle.
 // Nonlinear stages recompute their forward values with the reference's
 // evaluation order (this file is built with -ffp-contract=off, like the exact
 // forward kernels), so every branch is the one the forward pass took. Linear
@@ -53,104 +57,100 @@ __device__ __forceinline__ Prim7 ld7p(const double* base, size_t ps, uint32_t k)
                base[5 * ps + k], base[6 * ps + k]};
 }
 
-// (j, i) of this thread in the range [j0, j1] x [i0, i1] tiled kTileX x kTileY
-__device__ __forceinline__ bool range_ij(int j0, int j1, int i0, int i1, int& j, int& i) {
-  i = i0 + (int)blockIdx.x * kTileX + (int)threadIdx.x;
-  j = j0 + (int)blockIdx.y * kTileY + (int)threadIdx.y;
-  return i <= i1 && j <= j1;
+constexpr int kWave = 64;     // workgroup of the stages with few waves per SIMD
+constexpr int kCells = 256;   // workgroup of the others
+
+// (j, i) of thread `tid` of block b of `n` threads in the range [j0, j1] x
+// [i0, i1], taken row after row
+__device__ __forceinline__ bool range_ij(int b, int n, int j0, int j1, int i0, int i1, int& j,
+                                         int& i) {
+  const int e = b * n + (int)threadIdx.x, w = i1 - i0 + 1, r = e / w;
+  j = j0 + r;
+  i = i0 + (e - r * w);
+  return j <= j1;
 }
 
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kTileX* kTileY) ak_fold(AdjArgs a, int which) {
-  const Inst& g = a.g;
-  const int i = (int)blockIdx.x * kTileX + (int)threadIdx.x;
-  const int j = (int)blockIdx.y * kTileY + (int)threadIdx.y;
-  if (i >= g.sx || j >= g.sy) return;
-  double* A = which ? a.ain : a.aout;
-  const size_t ps = g.ps;
-  const uint32_t k = (uint32_t)(j * g.pitch + i);
-  for (int f = 0; f < NSTATE; f++) {
-    int sj, si;
-    bool neg;
-    if (ghost_src(g, f, j, i, sj, si, neg)) {
-      const double v = A[f * ps + k];
-      if (v != 0.0) ADD(A + f * ps, (uint32_t)(sj * g.pitch + si), neg ? -v : v);
-      A[f * ps + k] = 0.0;
-    }
-  }
+// The adjoint of set_bvals: the thread of a non-ghost cell sums, field by
+// field, the adjoints of the ghosts whose fill copies that cell (in the fixed
+// order of for_ghost_images) and adds them. Only the frame of kFrame cells at
+// each edge can receive (four cells, and the face past them): e numbers its
+// cells, the full rows first.
+constexpr int kFrame = 5;
+__host__ __device__ inline int frame_cells(int nx1, int nx2) {
+  const int w = nx1 + 1, h = nx2 + 1;  // with the faces ie+1, je+1
+  const int hr = h < 2 * kFrame ? h : 2 * kFrame, wc = w < 2 * kFrame ? w : 2 * kFrame;
+  return hr * w + (h - hr) * wc;
 }
-
-// The same fold as an ordered gather (deterministic reverse): the thread of
-// non-ghost cell (j, i) sums, field by field, the adjoints of every ghost
-// whose fill copies that cell -- rows ascending, then columns -- and adds
-// them once. The set_bvals map is separable: ghost row jj maps to a row
-// independently of the column, and ghost column ii to a column, so the
-// candidates are (rows mapping to j or j itself) x (columns mapping to i or i
-// itself). Only cells near an edge can receive; the ghosts are cleared
-// afterwards by ak_fold_clear.
-__global__ void __launch_bounds__(kTileX* kTileY) ak_fold_gather(AdjArgs a) {
+__global__ void __launch_bounds__(kCells) ak_fold(AdjArgs a) {
   const Inst& g = a.g;
-  const int i = (int)blockIdx.x * kTileX + (int)threadIdx.x;
-  const int j = (int)blockIdx.y * kTileY + (int)threadIdx.y;
-  if (i >= g.sx || j >= g.sy) return;
+  const int w = g.nx1 + 1, h = g.nx2 + 1;
+  const int hr = min(h, 2 * kFrame), wc = min(w, 2 * kFrame);
+  const int e = (int)blockIdx.x * kCells + (int)threadIdx.x;
+  if (e >= frame_cells(g.nx1, g.nx2)) return;
+  int r, c;
+  if (e < hr * w) {
+    r = e / w;
+    c = e - r * w;
+    if (r >= kFrame && h > hr) r += h - hr;
+  } else {
+    const int f = e - hr * w;
+    r = f / wc;
+    c = f - r * wc;
+    r += kFrame;
+    if (c >= kFrame && w > wc) c += w - wc;
+  }
+  const int j = g.js + r, i = g.is + c;
   double* A = a.aout;
   const size_t ps = g.ps;
   const int pitch = g.pitch;
-  for (int f = 0; f < NSTATE; f++) {
-    const int ie_x = (f == F_B1I) ? g.ie + 1 : g.ie;
-    const int je_y = (f == F_B2I) ? g.je + 1 : g.je;
-    if (i < g.is || i > ie_x || j < g.js || j > je_y) continue;  // ghosts receive nothing
-    // receivers lie within 4 cells of an edge of the cell-centred range
-    // [js, je] x [is, ie] (face planes: one more cell on the far side)
-    const bool band = (j - g.js < 5) || (je_y - j < 5) || (i - g.is < 5) || (ie_x - i < 5);
-    if (!band) continue;
-    // ascending: ghost rows below, the row itself, ghost rows above
-    int rows[9], cols[9], nr = 0, nc = 0;
-    int sj, si;
-    bool neg;
-    for (int jj = 0; jj < g.js; jj++)
-      if (ghost_src(g, f, jj, g.is, sj, si, neg) && sj == j) rows[nr++] = jj;
-    rows[nr++] = j;
-    for (int jj = je_y + 1; jj < g.sy; jj++)
-      if (ghost_src(g, f, jj, g.is, sj, si, neg) && sj == j) rows[nr++] = jj;
-    for (int ii = 0; ii < g.is; ii++)
-      if (ghost_src(g, f, g.js, ii, sj, si, neg) && si == i) cols[nc++] = ii;
-    cols[nc++] = i;
-    for (int ii = ie_x + 1; ii < g.sx; ii++)
-      if (ghost_src(g, f, g.js, ii, sj, si, neg) && si == i) cols[nc++] = ii;
-    double sum = 0.0;
-    bool any = false;
-    for (int r = 0; r < nr; r++)
-      for (int c = 0; c < nc; c++) {
-        const int jj = rows[r], ii = cols[c];
-        if (jj == j && ii == i) continue;
-        if (ghost_src(g, f, jj, ii, sj, si, neg) && sj == j && si == i) {
-          const double v = A[f * ps + (uint32_t)(jj * pitch + ii)];
-          sum += neg ? -v : v;
-          any = true;
-        }
+  const bool cell_i = i <= g.ie, cell_j = j <= g.je;
+  const unsigned ix = cell_i ? ghost_images(i, g.is, g.ie, g.bc[0], g.bc[1], false) : 0u;
+  const unsigned iy = cell_j ? ghost_images(j, g.js, g.je, g.bc[2], g.bc[3], false) : 0u;
+  const unsigned fx = ghost_images(i, g.is, g.ie, g.bc[0], g.bc[1], true);
+  const unsigned fy = ghost_images(j, g.js, g.je, g.bc[2], g.bc[3], true);
+  // all fields of a class together: their loads are in flight at the same time
+  const uint32_t k = (uint32_t)(j * pitch + i);
+  double v[NSTATE];
+#pragma unroll
+  for (int f = 0; f < NSTATE; f++) v[f] = A[f * ps + k];
+  auto add = [&](int cls, unsigned mx, unsigned my) {
+    for_ghost_images(g, j, i, mx, my, [&](int rr, int cc, bool nx, bool ny) {
+      const uint32_t kg = (uint32_t)(rr * pitch + cc);
+#pragma unroll
+      for (int f = 0; f < NSTATE; f++) {
+        if (ghost_class(f) != cls) continue;
+        const double x = A[f * ps + kg];
+        v[f] += ghost_negates(f, nx, ny) ? -x : x;
       }
-    if (any) A[f * ps + (uint32_t)(j * pitch + i)] += sum;
-  }
+    });
+#pragma unroll
+    for (int f = 0; f < NSTATE; f++)
+      if (ghost_class(f) == cls) A[f * ps + k] = v[f];
+  };
+  if (cell_i && cell_j && (ix | iy)) add(0, ix, iy);
+  if (cell_j && (fx | iy)) add(1, fx, iy);
+  if (cell_i && (ix | fy)) add(2, ix, fy);
 }
-__global__ void __launch_bounds__(kTileX* kTileY) ak_fold_clear(AdjArgs a) {
+__global__ void __launch_bounds__(kCells) ak_clear_ghost(AdjArgs a) {
   const Inst& g = a.g;
-  const int i = (int)blockIdx.x * kTileX + (int)threadIdx.x;
-  const int j = (int)blockIdx.y * kTileY + (int)threadIdx.y;
-  if (i >= g.sx || j >= g.sy) return;
+  int j, i;
+  if (!range_ij(blockIdx.x, kCells, 0, g.sy - 1, 0, g.sx - 1, j, i)) return;
   const uint32_t k = (uint32_t)(j * g.pitch + i);
+  const bool gx = i < g.is || i > g.ie, gy = j < g.js || j > g.je;
+  if (!gx && !gy) return;
   for (int f = 0; f < NSTATE; f++) {
-    int sj, si;
-    bool neg;
-    if (ghost_src(g, f, j, i, sj, si, neg)) a.aout[f * g.ps + k] = 0.0;
+    // the face at ie+1 of B1i (je+1 of B2i) is not a ghost
+    const bool ghost = f == F_B1I   ? (gy || i < g.is || i > g.ie + 1)
+                       : f == F_B2I ? (gx || j < g.js || j > g.je + 1)
+                                    : true;
+    if (ghost) a.aout[f * g.ps + k] = 0.0;
   }
 }
 
-// ALL: every adjoint plane (start of a reverse pass); otherwise ain and the
-// NACC accumulated planes (every step)
-__global__ void __launch_bounds__(256) ak_zero(AdjArgs a, int all) {
-  const size_t n_in = (size_t)NSTATE * a.g.ps;
-  const size_t n_ab = (size_t)(all ? NADJ : NACC) * a.g.ps;
+// every adjoint plane and ain (start of a reverse pass)
+__global__ void __launch_bounds__(256) ak_clear(AdjArgs a) {
+  const size_t n_in = (size_t)NSTATE * a.g.ps, n_ab = (size_t)NADJ * a.g.ps;
   for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n_in + n_ab;
        e += (size_t)gridDim.x * blockDim.x) {
     if (e < n_in) a.ain[e] = 0.0;
@@ -161,11 +161,12 @@ __global__ void __launch_bounds__(256) ak_zero(AdjArgs a, int all) {
 // ---------------------------------------------------------------------------
 // Steps 9, 11a, 11b, 13 (:473-534) over [js,je+1] x [is,ie+1]; the corrector
 // flux adjoints are stored over [js-1,je+1] x [is-1,ie+1], the faces the
-// corrector Riemann reverse reads (zero where no update reads the flux)
-__global__ void __launch_bounds__(kTileX* kTileY) ak_update(AdjArgs a) {
+// corrector Riemann reverse reads (zero where no update reads the flux). The
+// update's identity part starts ain, over the whole padded grid.
+__global__ void __launch_bounds__(kCells) ak_update(AdjArgs a) {
   const Inst& g = a.g;
   int j, i;
-  if (!range_ij(g.js - 1, g.je + 1, g.is - 1, g.ie + 1, j, i)) return;
+  if (!range_ij(blockIdx.x, kCells, 0, g.sy - 1, 0, g.sx - 1, j, i)) return;
   const size_t ps = g.ps;
   const int pitch = g.pitch;
   const double dtodx1 = a.dt / g.dx1, dtodx2 = a.dt / g.dx2;
@@ -180,9 +181,15 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_update(AdjArgs a) {
     if (q == F_B3C) v += ao[F_B3I * ps + kk];
     return v;
   };
-  if (j >= g.js && j <= g.je && i >= g.is && i <= g.ie) {
-    const int q_id[6] = {F_D, F_M1, F_M2, F_M3, F_E, F_B3C};
-    for (int n = 0; n < 6; n++) a.ain[q_id[n] * ps + k] += cb(q_id[n], j, i);
+  const int q_id[6] = {F_D, F_M1, F_M2, F_M3, F_E, F_B3C};
+  for (int n = 0; n < 6; n++) a.ain[q_id[n] * ps + k] = cb(q_id[n], j, i);
+  a.ain[F_B1C * ps + k] = 0.0;
+  a.ain[F_B2C * ps + k] = 0.0;
+  a.ain[F_B3I * ps + k] = 0.0;
+  if (j < g.js - 1 || j > g.je + 1 || i < g.is - 1 || i > g.ie + 1) {
+    a.ain[F_B1I * ps + k] = 0.0;
+    a.ain[F_B2I * ps + k] = 0.0;
+    return;
   }
   // corrector fluxes; the B2c update of 11a and the B1c update of 11b are
   // overwritten by Step 13, so those components get no adjoint there
@@ -198,7 +205,6 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_update(AdjArgs a) {
     for (int n = 0; n < 7; n++)
       F[n * ps + k] = (q2[n] < 0) ? 0.0 : dtodx2 * (cb(q2[n], j, i) - cb(q2[n], j - 1, i));
   }
-  if (j < g.js || i < g.is) return;
   // adjoint of the updated face fields including B1c, B2c = face averages
   auto b1t = [&](int jj, int ii) -> double {
     if (jj < g.js || jj > g.je || ii < g.is || ii > g.ie + 1) return 0.0;
@@ -210,59 +216,49 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_update(AdjArgs a) {
     return ao[F_B2I * ps + (uint32_t)(jj * pitch + ii)] +
            0.5 * (cb(F_B2C, jj, ii) + cb(F_B2C, jj - 1, ii));
   };
-  if (j <= g.je) a.ain[F_B1I * ps + k] += b1t(j, i);
-  if (i <= g.ie) a.ain[F_B2I * ps + k] += b2t(j, i);
+  a.ain[F_B1I * ps + k] = b1t(j, i);
+  a.ain[F_B2I * ps + k] = b2t(j, i);
+  if (j < g.js || i < g.is) return;
   a.ab[A_EMFC * ps + k] = dtodx2 * (b1t(j, i) - b1t(j - 1, i)) + dtodx1 * (b2t(j, i - 1) - b2t(j, i));
 }
 
 // ---------------------------------------------------------------------------
-// integrate_emf3_corner (:632-702) reversed. PRED: Step 4 over
-// [js-1,je+2]x[is-1,ie+2]; otherwise Step 9 over [js,je+1]x[is,ie+1].
+// integrate_emf3_corner (:632-702) reversed, from its inputs' side. Corner K is
+// a quarter of four upwinded estimates, picked by the face mass fluxes
+//   w1 = F1[K-pitch], w2 = F1[K], w3 = F2[K-1], w4 = F2[K]  (1, 0, or 1/2 at 0);
+// each input takes the corners it enters with their weights. The adjoint of a
+// corner outside the range of the reversed step is zero, so no input needs a
+// range test (a weight is 0, 1/2 or 1 whatever the flux there holds).
 __device__ __forceinline__ double upwind_weight(double mass_flux) {
   return (mass_flux > 0.0) ? 1.0 : ((mass_flux < 0.0) ? 0.0 : 0.5);
 }
-
-template <bool PRED>
-__global__ void __launch_bounds__(kTileX* kTileY) ak_corner(AdjArgs a) {
-  const Inst& g = a.g;
-  int j, i;
-  if (PRED) {
-    if (!range_ij(g.js - 1, g.je + 2, g.is - 1, g.ie + 2, j, i)) return;
-  } else {
-    if (!range_ij(g.js, g.je + 1, g.is, g.ie + 1, j, i)) return;
+struct CornerGather {
+  const double *F1, *F2;  // mass fluxes
+  const double* eb;       // adjoint of the corner emf
+  uint32_t p;             // pitch
+  __device__ double q(uint32_t K) const { return 0.25 * eb[K]; }
+  // By of the x1 flux at k: corners k and k + pitch
+  __device__ double f1_by(uint32_t k) const {
+    const double w3 = upwind_weight(F2[k - 1]), w4 = upwind_weight(F2[k]);
+    const double u3 = upwind_weight(F2[k + p - 1]), u4 = upwind_weight(F2[k + p]);
+    return q(k) * (-1.0 - (1.0 - w3) - (1.0 - w4)) + q(k + p) * (-1.0 - u3 - u4);
   }
-  // deterministic reverse: one launch per (j, i) parity class; corners of one
-  // class touch disjoint flux and emf entries, so no entry takes two adds
-  if (a.det && (((j & 1) << 1) | (i & 1)) != a.color) return;
-  const size_t ps = g.ps;
-  const int pitch = g.pitch;
-  const uint32_t k = (uint32_t)(j * pitch + i);
-  const double q = 0.25 * a.ab[(PRED ? A_EMFP : A_EMFC) * ps + k];
-  if (q == 0.0) return;
-  const double* F1 = a.sc + (PRED ? S_F1 : S_F1C) * ps;  // mass fluxes pick the upwind side
-  const double* F2 = a.sc + (PRED ? S_F2 : S_F2C) * ps;
-  double* F1b = a.ab + (PRED ? A_F1 : A_F1C) * ps;
-  double* F2b = a.ab + (PRED ? A_F2 : A_F2C) * ps;
-  double* eb = a.ab + (PRED ? A_ECC : A_ECH) * ps;
-  const uint32_t kjm = k - pitch, kim = k - 1, kjmim = k - pitch - 1;
-  double c_f1jm = 0, c_f1 = 0, c_f2im = 0, c_f2 = 0, c_ejmim = 0, c_ejm = 0, c_eim = 0, c_e00 = 0;
-  double w = upwind_weight(F1[kjm]);  // emf_l2
-  c_f1jm -= 1.0; c_f2im += w; c_ejmim -= w; c_f2 += 1.0 - w; c_ejm -= 1.0 - w;
-  w = upwind_weight(F1[k]);  // emf_r2
-  c_f1 -= 1.0; c_f2im += w; c_eim -= w; c_f2 += 1.0 - w; c_e00 -= 1.0 - w;
-  w = upwind_weight(F2[kim]);  // emf_l1
-  c_f2im += 1.0; c_f1jm -= w; c_ejmim -= w; c_f1 -= 1.0 - w; c_eim -= 1.0 - w;
-  w = upwind_weight(F2[k]);  // emf_r1
-  c_f2 += 1.0; c_f1jm -= w; c_ejm -= w; c_f1 -= 1.0 - w; c_e00 -= 1.0 - w;
-  ADD(F1b + 5 * ps, kjm, q * c_f1jm);
-  ADD(F1b + 5 * ps, k, q * c_f1);
-  ADD(F2b + 6 * ps, kim, q * c_f2im);
-  ADD(F2b + 6 * ps, k, q * c_f2);
-  ADD(eb, kjmim, q * c_ejmim);
-  ADD(eb, kjm, q * c_ejm);
-  ADD(eb, kim, q * c_eim);
-  ADD(eb, k, q * c_e00);
-}
+  // Bz of the x2 flux at k: corners k and k + 1
+  __device__ double f2_bz(uint32_t k) const {
+    const double w1 = upwind_weight(F1[k - p]), w2 = upwind_weight(F1[k]);
+    const double u1 = upwind_weight(F1[k + 1 - p]), u2 = upwind_weight(F1[k + 1]);
+    return q(k) * ((1.0 - w1) + (1.0 - w2) + 1.0) + q(k + 1) * (u1 + u2 + 1.0);
+  }
+  // the cell-centred emf at k: its four corners
+  __device__ double emf_cc(uint32_t k) const {
+    const double q00 = q(k), q01 = q(k + 1), q10 = q(k + p), q11 = q(k + p + 1);
+    if (q00 == 0.0 && q01 == 0.0 && q10 == 0.0 && q11 == 0.0) return 0.0;
+    const double f1 = upwind_weight(F1[k]), f1i = upwind_weight(F1[k + 1]);
+    const double f2 = upwind_weight(F2[k]), f2j = upwind_weight(F2[k + p]);
+    return q00 * (-(1.0 - f1) - (1.0 - f2)) + q01 * (-f1i - (1.0 - f2)) +
+           q10 * (-(1.0 - f1) - f2j) + q11 * (-f1i - f2j);
+  }
+};
 
 // ---------------------------------------------------------------------------
 // Forward values shared by the corrector stages: half-step face fields
@@ -362,18 +358,31 @@ __device__ __forceinline__ CorrCtx corr_ctx(const AdjArgs& a) {
   return CorrCtx{a.g, a.st, a.sc, a.emfp, a.g.ps, a.g.pitch, 0.5 * dtodx1, 0.5 * dtodx2};
 }
 
+// the corners of Step 9 (corrector fluxes) and of Step 4 (predictor fluxes)
+__device__ __forceinline__ CornerGather corner_c(const AdjArgs& a) {
+  const size_t ps = a.g.ps;
+  return CornerGather{a.sc + S_F1C * ps, a.sc + S_F2C * ps, a.ab + A_EMFC * ps,
+                      (uint32_t)a.g.pitch};
+}
+__device__ __forceinline__ CornerGather corner_p(const AdjArgs& a) {
+  const size_t ps = a.g.ps;
+  return CornerGather{a.sc + S_F1 * ps, a.sc + S_F2 * ps, a.ab + A_EMFP * ps,
+                      (uint32_t)a.g.pitch};
+}
+
 // Step 8b (X1: x1 faces [js-1,je+1] x [is,ie+1], :438-447) or 8c (x2 faces
 // [js,je+1] x [is-1,ie+1], :455-464); the two are independent
 template <bool X1, int FLUX>  // FLUX: the grid's Riemann solver
-__global__ void __launch_bounds__(kTileX* kTileY) ak_riemann_c(AdjArgs a) {
+__device__ __forceinline__ void riemann_c(const AdjArgs& a, int block) {
   const Inst& g = a.g;
   int j, i;
   if (X1) {
-    if (!range_ij(g.js - 1, g.je + 1, g.is, g.ie + 1, j, i)) return;
+    if (!range_ij(block, kWave, g.js - 1, g.je + 1, g.is, g.ie + 1, j, i)) return;
   } else {
-    if (!range_ij(g.js, g.je + 1, g.is - 1, g.ie + 1, j, i)) return;
+    if (!range_ij(block, kWave, g.js, g.je + 1, g.is - 1, g.ie + 1, j, i)) return;
   }
   const CorrCtx c = corr_ctx(a);
+  const CornerGather corner = corner_c(a);
   const size_t ps = g.ps;
   const uint32_t k = (uint32_t)(j * g.pitch + i);
   const EosC eos{g.gamma, g.g1, g.g2};
@@ -385,7 +394,9 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_riemann_c(AdjArgs a) {
     Cons7 Lb = zero_cons(), Rb = zero_cons();
     Prim7 Wlb = zero_prim(), Wrb = zero_prim();
     double bxb = 0.0;
-    riemann_b_of<FLUX>(L, R, wl, wr, bx, eos, ld7(a.ab + A_F1C * ps, ps, k), Lb, Rb, Wlb, Wrb, bxb);
+    Cons7 Fb = ld7(a.ab + A_F1C * ps, ps, k);
+    Fb.by += corner.f1_by(k);
+    riemann_b_of<FLUX>(L, R, wl, wr, bx, eos, Fb, Lb, Rb, Wlb, Wrb, bxb);
     cons_to_prim_b(L, bx, eos, Wlb, Lb, bxb);
     cons_to_prim_b(R, bx, eos, Wrb, Rb, bxb);
     st7(a.ab + A_UL1 * ps, ps, k, Lb);
@@ -399,7 +410,9 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_riemann_c(AdjArgs a) {
     Cons7 Lb = zero_cons(), Rb = zero_cons();
     Prim7 Wlb = zero_prim(), Wrb = zero_prim();
     double bxb = 0.0;
-    riemann_b_of<FLUX>(L, R, wl, wr, bx, eos, ld7(a.ab + A_F2C * ps, ps, k), Lb, Rb, Wlb, Wrb, bxb);
+    Cons7 Fb = ld7(a.ab + A_F2C * ps, ps, k);
+    Fb.bz += corner.f2_bz(k);
+    riemann_b_of<FLUX>(L, R, wl, wr, bx, eos, Fb, Lb, Rb, Wlb, Wrb, bxb);
     cons_to_prim_b(L, bx, eos, Wlb, Lb, bxb);
     cons_to_prim_b(R, bx, eos, Wrb, Rb, bxb);
     st7(a.ab + A_UL2 * ps, ps, k, Lb);
@@ -411,14 +424,14 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_riemann_c(AdjArgs a) {
 // Step 7 (:402-431) reversed per cell of [js-1,je+1] x [is-1,ie+1]: stores
 // the adjoints of the cell's half-step d, M1, M2 and B1c, B2c; the transverse
 // reverse hands them on to the predictor fluxes and the half-step face fields.
-__global__ void __launch_bounds__(kTileX* kTileY) ak_half(AdjArgs a) {
+__device__ __forceinline__ void half_step(const AdjArgs& a, int block) {
   const Inst& g = a.g;
   int j, i;
-  if (!range_ij(g.js - 1, g.je + 1, g.is - 1, g.ie + 1, j, i)) return;
+  if (!range_ij(block, kWave, g.js - 1, g.je + 1, g.is - 1, g.ie + 1, j, i)) return;
   const size_t ps = g.ps;
   const int pitch = g.pitch;
   const uint32_t k = (uint32_t)(j * pitch + i);
-  const double Eb = a.ab[A_ECH * ps + k];
+  const double Eb = corner_c(a).emf_cc(k);
   double dhb = 0.0, m1b = 0.0, m2b = 0.0, b1cb = 0.0, b2cb = 0.0;
   if (Eb != 0.0) {
     const CorrCtx c = corr_ctx(a);
@@ -450,6 +463,18 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_half(AdjArgs a) {
   ab[A_HB2 * ps + k] = b2cb;
 }
 
+// Steps 8b, 8c and 7 in one launch: blocks [0, n1) the x1 faces, [n1, n1 + n2)
+// the x2 faces, the rest Step 7 (they write disjoint planes). The Roe reverse
+// holds 512 registers (one wave per SIMD), the HLLE one fits two.
+template <int FLUX>
+__global__ void __launch_bounds__(kWave, FLUX == kFluxHlle ? 2 : 1) ak_correct(AdjArgs a, int n1,
+                                                                              int n2) {
+  const int b = blockIdx.x;
+  if (b < n1) riemann_c<true, FLUX>(a, b);
+  else if (b < n1 + n2) riemann_c<false, FLUX>(a, b - n1);
+  else half_step(a, b - n1 - n2);
+}
+
 // Steps 5, 6 (:284-393), the half-step face fields of Step 4 (:263-275) and
 // the flux part of Step 7, reversed as a gather: each thread owns one cell /
 // face / corner position c of [js-2,je+2] x [is-2,ie+2] and stores the
@@ -463,10 +488,15 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_half(AdjArgs a) {
 // (left at c+1: at c+1-1): with X1(c) = Lb(c+1) + Rb(c) the sources' adjoint
 // is linear in X1(c), and the x2 flux at c receives h2 (X1(c) - X1(c-pitch)).
 // Likewise for x2 faces with X2(c) = Lb(c+pitch) + Rb(c).
+//
+// Tiles of 64 x 4: each position reads its row's and the rows' below values of
+// some 40 planes, which a tile's rows share (in the row-after-row order of the
+// other stages 47 -> 59 us at 512^2).
 __global__ void __launch_bounds__(kTileX* kTileY) ak_transverse(AdjArgs a) {
   const Inst& g = a.g;
-  int j, i;
-  if (!range_ij(g.js - 2, g.je + 2, g.is - 2, g.ie + 2, j, i)) return;
+  const int i = g.is - 2 + (int)blockIdx.x * kTileX + (int)threadIdx.x;
+  const int j = g.js - 2 + (int)blockIdx.y * kTileY + (int)threadIdx.y;
+  if (i > g.ie + 2 || j > g.je + 2) return;
   const size_t ps = g.ps;
   const uint32_t pitch = (uint32_t)g.pitch;
   const uint32_t c = (uint32_t)j * pitch + (uint32_t)i;
@@ -554,13 +584,13 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_transverse(AdjArgs a) {
 }
 
 // Step 3 (:249-255) over [js-2,je+2] x [is-2,ie+2]
-__global__ void __launch_bounds__(kTileX* kTileY) ak_emf_cc(AdjArgs a) {
+__device__ __forceinline__ void emf_cc(const AdjArgs& a, int block) {
   const Inst& g = a.g;
   int j, i;
-  if (!range_ij(g.js - 2, g.je + 2, g.is - 2, g.ie + 2, j, i)) return;
+  if (!range_ij(block, kWave, g.js - 2, g.je + 2, g.is - 2, g.ie + 2, j, i)) return;
   const size_t ps = g.ps;
   const uint32_t k = (uint32_t)(j * g.pitch + i);
-  const double Eb = a.ab[A_ECC * ps + k];
+  const double Eb = corner_p(a).emf_cc(k);
   if (Eb == 0.0) return;
   const double* st = a.st;
   const double d = st[F_D * ps + k], m1 = st[F_M1 * ps + k], m2 = st[F_M2 * ps + k];
@@ -580,13 +610,13 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_emf_cc(AdjArgs a) {
 // stored. X1: faces [js-2,je+2] x [is-1,ie+2]; x2: [js-1,je+2] x [is-2,ie+2].
 // Writes the adjoints of the PLM outputs Wl, Wr (the source only adds to them).
 template <bool X1, int FLUX>  // FLUX: the grid's Riemann solver
-__global__ void __launch_bounds__(kTileX* kTileY) ak_pred(AdjArgs a) {
+__device__ __forceinline__ void predict(const AdjArgs& a, int block) {
   const Inst& g = a.g;
   int j, i;
   if (X1) {
-    if (!range_ij(g.js - 2, g.je + 2, g.is - 1, g.ie + 2, j, i)) return;
+    if (!range_ij(block, kWave, g.js - 2, g.je + 2, g.is - 1, g.ie + 2, j, i)) return;
   } else {
-    if (!range_ij(g.js - 1, g.je + 2, g.is - 2, g.ie + 2, j, i)) return;
+    if (!range_ij(block, kWave, g.js - 1, g.je + 2, g.is - 2, g.ie + 2, j, i)) return;
   }
   const size_t ps = g.ps;
   const uint32_t stride = X1 ? 1u : (uint32_t)g.pitch;
@@ -603,9 +633,12 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_pred(AdjArgs a) {
   {
     const Prim7 wl = ld7p(a.pw + (X1 ? P_WL1 : P_WL2) * ps, ps, k);
     const Prim7 wr = ld7p(a.pw + (X1 ? P_WR1 : P_WR2) * ps, ps, k);
+    Cons7 Fb = ld7(a.ab + (X1 ? A_F1 : A_F2) * ps, ps, k);
+    if (X1) Fb.by += corner_p(a).f1_by(k);
+    else Fb.bz += corner_p(a).f2_bz(k);
     riemann_b_of<FLUX>(ld7(a.sc + (X1 ? S_UL1 : S_UL2) * ps, ps, k),
-              ld7(a.sc + (X1 ? S_UR1 : S_UR2) * ps, ps, k), wl, wr, b0, eos,
-              ld7(a.ab + (X1 ? A_F1 : A_F2) * ps, ps, k), Ulb, Urb, wlb, wrb, b0b);
+                       ld7(a.sc + (X1 ? S_UR1 : S_UR2) * ps, ps, k), wl, wr, b0, eos, Fb, Ulb,
+                       Urb, wlb, wrb, b0b);
     prim_to_cons_b(wl, b0, eos, Ulb, wlb, b0b);
     prim_to_cons_b(wr, b0, eos, Urb, wrb, b0b);
   }
@@ -642,16 +675,33 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_pred(AdjArgs a) {
   st7(a.ab + (X1 ? A_WR1 : A_WR2) * ps, ps, k, wrb);
 }
 
+// Both sweeps' predictor faces and Step 3 in one launch, as ak_correct (ain
+// takes atomic adds from all of them; the deterministic reverse's faces store
+// theirs, and Step 3 alone adds).
+template <int FLUX>
+__global__ void __launch_bounds__(kWave, FLUX == kFluxHlle ? 2 : 1) ak_predict(AdjArgs a, int n1,
+                                                                              int n2) {
+  const int b = blockIdx.x;
+  if (b < n1) predict<true, FLUX>(a, b);
+  else if (b < n1 + n2) predict<false, FLUX>(a, b - n1);
+  else emf_cc(a, b - n1 - n2);
+}
+
 // Steps 1b / 2b reversed for one cell of [js-2,je+2] x [is-2,ie+2]: the PLM
 // of cell k produced Wl at the next face and Wr at its own face. Stores the
 // adjoints of the primitive states of cells k-1, k, k+1 and of Bxc[k] (22
 // planes; zeros where the outputs' adjoints are zero); plm_gather hands them
 // through cons->prim.
+struct PlmSlot {
+  PlmCore c;
+  double pad;
+};
+static_assert((sizeof(PlmSlot) / 8) % 2 == 1, "odd slot stride in doubles");
 template <bool X1>
-__global__ void __launch_bounds__(kTileX* kTileY) ak_plm(AdjArgs a) {
+__device__ __forceinline__ void plm(const AdjArgs& a, int block, PlmSlot* slot) {
   const Inst& g = a.g;
   int j, i;
-  if (!range_ij(g.js - 2, g.je + 2, g.is - 2, g.ie + 2, j, i)) return;
+  if (!range_ij(block, kWave, g.js - 2, g.je + 2, g.is - 2, g.ie + 2, j, i)) return;
   const size_t ps = g.ps;
   const uint32_t stride = X1 ? 1u : (uint32_t)g.pitch;
   const uint32_t k = (uint32_t)(j * g.pitch + i);
@@ -689,13 +739,7 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_plm(AdjArgs a) {
   // A slot is an odd number of doubles long, so that the 8-byte words one
   // field occupies in consecutive lanes' slots fall in distinct LDS banks
   // (68 doubles, an even stride, put lanes 4 or 8 to a bank)
-  struct Slot {
-    PlmCore c;
-    double pad;
-  };
-  static_assert((sizeof(Slot) / 8) % 2 == 1, "odd slot stride in doubles");
-  __shared__ Slot slot[kTileX * kTileY];
-  PlmCore& P = slot[threadIdx.y * kTileX + threadIdx.x].c;
+  PlmCore& P = slot[threadIdx.x].c;
   P.prepare(W[0], W[1], W[2], st[qx * ps + k], a.dt / (X1 ? g.dx1 : g.dx2), eos);
   double wb[3][7];
   for (int c = 0; c < 3; c++)
@@ -707,18 +751,27 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_plm(AdjArgs a) {
   dst[21 * ps + k] = bxcb;
 }
 
+// both sweeps in one launch: blocks [0, n) x1, [n, 2 n) x2. Four one-wave
+// workgroups of 40 KB of slots fill a CU's LDS.
+__global__ void __launch_bounds__(kWave) ak_plm(AdjArgs a, int n) {
+  __shared__ PlmSlot slot[kWave];
+  const int b = blockIdx.x;
+  if (b < n) plm<true>(a, b, slot);
+  else plm<false>(a, b - n, slot);
+}
+
 // Steps 1a / 2a reversed per cell: the primitive-state adjoint of cell c sums
 // the PLM reverses of cells c+1 (its left neighbour slot), c and c-1, and goes
 // through cons->prim once. X1: cells [js-2,je+2] x [is-3,ie+3]; x2:
 // [js-3,je+3] x [is-2,ie+2]. Atomic adds: the two sweeps run concurrently.
 template <bool X1>
-__global__ void __launch_bounds__(kTileX* kTileY) ak_plm_gather(AdjArgs a) {
+__device__ __forceinline__ void plm_gather(const AdjArgs& a, int block) {
   const Inst& g = a.g;
   int j, i;
   if (X1) {
-    if (!range_ij(g.js - 2, g.je + 2, g.is - 3, g.ie + 3, j, i)) return;
+    if (!range_ij(block, kCells, g.js - 2, g.je + 2, g.is - 3, g.ie + 3, j, i)) return;
   } else {
-    if (!range_ij(g.js - 3, g.je + 3, g.is - 2, g.ie + 2, j, i)) return;
+    if (!range_ij(block, kCells, g.js - 3, g.je + 3, g.is - 2, g.ie + 2, j, i)) return;
   }
   const size_t ps = g.ps;
   const uint32_t stride = X1 ? 1u : (uint32_t)g.pitch;
@@ -759,6 +812,14 @@ __global__ void __launch_bounds__(kTileX* kTileY) ak_plm_gather(AdjArgs a) {
   ADD(a.ain + qx * ps, k, bxb);
 }
 
+// blocks [0, n1) x1, the rest x2; `first` skips to the x2 blocks (the
+// deterministic reverse launches the sweeps one after the other)
+__global__ void __launch_bounds__(kCells) ak_plm_gather(AdjArgs a, int first, int n1) {
+  const int b = first + blockIdx.x;
+  if (b < n1) plm_gather<true>(a, b);
+  else plm_gather<false>(a, b - n1);
+}
+
 }  // namespace adjk
 }  // namespace athmi
 
@@ -768,97 +829,55 @@ using namespace athmi::adjk;
 extern "C" hipError_t athmi_adjoint_launch(const AdjArgs* ap, int kernel, hipStream_t s) {
   const AdjArgs& a = *ap;
   const Inst& g = a.g;
-  const dim3 b2(kTileX, kTileY);
-  auto grid2 = [&](int j0, int j1, int i0, int i1) {
-    return dim3((unsigned)cdiv(i1 - i0 + 1, kTileX), (unsigned)cdiv(j1 - j0 + 1, kTileY));
+  // blocks of `threads` over a range of (nx2 + dj) x (nx1 + di) positions
+  auto blocks = [&](int dj, int di, int threads) {
+    return cdiv((g.nx2 + dj) * (g.nx1 + di), threads);
   };
   switch (kernel) {
-    case AK_FOLD_OUT:
-    case AK_FOLD_IN:
-      hipLaunchKernelGGL(ak_fold, grid2(0, g.sy - 1, 0, g.sx - 1), b2, 0, s, a,
-                         kernel == AK_FOLD_IN ? 1 : 0);
-      break;
-    case AK_ZERO:
     case AK_CLEAR:
-      hipLaunchKernelGGL(ak_zero, dim3(2048), dim3(256), 0, s, a, kernel == AK_CLEAR ? 1 : 0);
+      hipLaunchKernelGGL(ak_clear, dim3(2048), dim3(256), 0, s, a);
+      break;
+    case AK_FOLD:
+      hipLaunchKernelGGL(ak_fold, dim3(cdiv(frame_cells(g.nx1, g.nx2), kCells)), dim3(kCells), 0, s,
+                         a);
+      break;
+    case AK_CLEAR_GHOST:
+      hipLaunchKernelGGL(ak_clear_ghost, dim3(blocks(8, 8, kCells)), dim3(kCells), 0, s, a);
       break;
     case AK_UPDATE:
-      hipLaunchKernelGGL(ak_update, grid2(g.js - 1, g.je + 1, g.is - 1, g.ie + 1), b2, 0, s, a);
+      hipLaunchKernelGGL(ak_update, dim3(blocks(8, 8, kCells)), dim3(kCells), 0, s, a);
       break;
-    case AK_CORNER_C:
-      for (int c = 0; c < (a.det ? 4 : 1); c++) {
-        AdjArgs ac = a;
-        ac.color = c;
-        hipLaunchKernelGGL(ak_corner<false>, grid2(g.js, g.je + 1, g.is, g.ie + 1), b2, 0, s, ac);
-      }
+    case AK_CORRECT: {
+      const int n1 = blocks(2, 1, kWave), n2 = blocks(1, 2, kWave), n3 = blocks(2, 2, kWave);
+      const auto fn = g.flux == kFluxHlle ? ak_correct<kFluxHlle> : ak_correct<kFluxRoe>;
+      hipLaunchKernelGGL(fn, dim3(n1 + n2 + n3), dim3(kWave), 0, s, a, n1, n2);
       break;
-    case AK_FOLD_OUT_DET:
-      hipLaunchKernelGGL(ak_fold_gather, grid2(0, g.sy - 1, 0, g.sx - 1), b2, 0, s, a);
-      hipLaunchKernelGGL(ak_fold_clear, grid2(0, g.sy - 1, 0, g.sx - 1), b2, 0, s, a);
-      break;
-    case AK_RIEMANN_C1:
-      if (g.flux == kFluxHlle)
-        hipLaunchKernelGGL((ak_riemann_c<true, kFluxHlle>), grid2(g.js - 1, g.je + 1, g.is, g.ie + 1),
-                           b2, 0, s, a);
-      else
-        hipLaunchKernelGGL((ak_riemann_c<true, kFluxRoe>), grid2(g.js - 1, g.je + 1, g.is, g.ie + 1),
-                           b2, 0, s, a);
-      break;
-    case AK_RIEMANN_C2:
-      if (g.flux == kFluxHlle)
-        hipLaunchKernelGGL((ak_riemann_c<false, kFluxHlle>), grid2(g.js, g.je + 1, g.is - 1, g.ie + 1),
-                           b2, 0, s, a);
-      else
-        hipLaunchKernelGGL((ak_riemann_c<false, kFluxRoe>), grid2(g.js, g.je + 1, g.is - 1, g.ie + 1),
-                           b2, 0, s, a);
-      break;
-    case AK_HALF:
-      hipLaunchKernelGGL(ak_half, grid2(g.js - 1, g.je + 1, g.is - 1, g.ie + 1), b2, 0, s, a);
-      break;
+    }
     case AK_TRANSVERSE:
-      hipLaunchKernelGGL(ak_transverse, grid2(g.js - 2, g.je + 2, g.is - 2, g.ie + 2), b2, 0, s, a);
+      hipLaunchKernelGGL(ak_transverse, dim3(cdiv(g.nx1 + 4, kTileX), cdiv(g.nx2 + 4, kTileY)),
+                         dim3(kTileX, kTileY), 0, s, a);
       break;
-    case AK_CORNER_P:
-      for (int c = 0; c < (a.det ? 4 : 1); c++) {
-        AdjArgs ac = a;
-        ac.color = c;
-        hipLaunchKernelGGL(ak_corner<true>, grid2(g.js - 1, g.je + 2, g.is - 1, g.ie + 2), b2, 0, s,
-                           ac);
+    case AK_PREDICT: {
+      const int n1 = blocks(4, 3, kWave), n2 = blocks(3, 4, kWave), n3 = blocks(4, 4, kWave);
+      const auto fn = g.flux == kFluxHlle ? ak_predict<kFluxHlle> : ak_predict<kFluxRoe>;
+      hipLaunchKernelGGL(fn, dim3(n1 + n2 + n3), dim3(kWave), 0, s, a, n1, n2);
+      break;
+    }
+    case AK_PLM: {
+      const int n = blocks(4, 4, kWave);
+      hipLaunchKernelGGL(ak_plm, dim3(2 * n), dim3(kWave), 0, s, a, n);
+      break;
+    }
+    case AK_PLM_GATHER: {
+      const int n1 = blocks(4, 6, kCells), n2 = blocks(6, 4, kCells);
+      if (a.det) {
+        hipLaunchKernelGGL(ak_plm_gather, dim3(n1), dim3(kCells), 0, s, a, 0, n1);
+        hipLaunchKernelGGL(ak_plm_gather, dim3(n2), dim3(kCells), 0, s, a, n1, n1);
+      } else {
+        hipLaunchKernelGGL(ak_plm_gather, dim3(n1 + n2), dim3(kCells), 0, s, a, 0, n1);
       }
       break;
-    case AK_EMF_CC:
-      hipLaunchKernelGGL(ak_emf_cc, grid2(g.js - 2, g.je + 2, g.is - 2, g.ie + 2), b2, 0, s, a);
-      break;
-    case AK_PRED_X1:
-      if (g.flux == kFluxHlle)
-        hipLaunchKernelGGL((ak_pred<true, kFluxHlle>), grid2(g.js - 2, g.je + 2, g.is - 1, g.ie + 2),
-                           b2, 0, s, a);
-      else
-        hipLaunchKernelGGL((ak_pred<true, kFluxRoe>), grid2(g.js - 2, g.je + 2, g.is - 1, g.ie + 2),
-                           b2, 0, s, a);
-      break;
-    case AK_PLM_X1:
-      hipLaunchKernelGGL(ak_plm<true>, grid2(g.js - 2, g.je + 2, g.is - 2, g.ie + 2), b2, 0, s, a);
-      break;
-    case AK_PRED_X2:
-      if (g.flux == kFluxHlle)
-        hipLaunchKernelGGL((ak_pred<false, kFluxHlle>), grid2(g.js - 1, g.je + 2, g.is - 2, g.ie + 2),
-                           b2, 0, s, a);
-      else
-        hipLaunchKernelGGL((ak_pred<false, kFluxRoe>), grid2(g.js - 1, g.je + 2, g.is - 2, g.ie + 2),
-                           b2, 0, s, a);
-      break;
-    case AK_PLM_X2:
-      hipLaunchKernelGGL(ak_plm<false>, grid2(g.js - 2, g.je + 2, g.is - 2, g.ie + 2), b2, 0, s, a);
-      break;
-    case AK_PLMG_X1:
-      hipLaunchKernelGGL(ak_plm_gather<true>, grid2(g.js - 2, g.je + 2, g.is - 3, g.ie + 3), b2, 0,
-                         s, a);
-      break;
-    case AK_PLMG_X2:
-      hipLaunchKernelGGL(ak_plm_gather<false>, grid2(g.js - 3, g.je + 3, g.is - 2, g.ie + 2), b2, 0,
-                         s, a);
-      break;
+    }
     default:
       return hipErrorInvalidValue;
   }
