@@ -114,18 +114,12 @@ static int copy_state(athmi_adjoint* h, double* dst, const double* src) {
 // dense [NSTATE][Nx2+8][Nx1+8] <-> pitched planes
 static int dense_to_planes(athmi_adjoint* h, double* planes, const double* dense, hipStream_t s) {
   const Inst& I = h->g->hinst[0];
-  for (int q = 0; q < NSTATE; q++)
-    HIP_TRY(hipMemcpy2DAsync(planes + q * I.ps, I.pitch * sizeof(double),
-                             dense + (size_t)q * I.sx * I.sy, I.sx * sizeof(double),
-                             I.sx * sizeof(double), I.sy, hipMemcpyDeviceToDevice, s));
+  HIP_TRY(launch_state_dense(planes, const_cast<double*>(dense), I.ps, I.pitch, I.sx, I.sy, 1, s));
   return ATHMI_OK;
 }
 static int planes_to_dense(athmi_adjoint* h, double* dense, const double* planes, hipStream_t s) {
   const Inst& I = h->g->hinst[0];
-  for (int q = 0; q < NSTATE; q++)
-    HIP_TRY(hipMemcpy2DAsync(dense + (size_t)q * I.sx * I.sy, I.sx * sizeof(double),
-                             planes + q * I.ps, I.pitch * sizeof(double), I.sx * sizeof(double),
-                             I.sy, hipMemcpyDeviceToDevice, s));
+  HIP_TRY(launch_state_dense(const_cast<double*>(planes), dense, I.ps, I.pitch, I.sx, I.sy, 0, s));
   return ATHMI_OK;
 }
 

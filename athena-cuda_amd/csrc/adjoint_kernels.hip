@@ -679,8 +679,7 @@ __device__ __forceinline__ void predict(const AdjArgs& a, int block) {
 // takes atomic adds from all of them; the deterministic reverse's faces store
 // theirs, and Step 3 alone adds).
 template <int FLUX>
-__global__ void __launch_bounds__(kWave, FLUX == kFluxHlle ? 2 : 1) ak_predict(AdjArgs a, int n1,
-                                                                              int n2) {
+__global__ void __launch_bounds__(kWave, 1) ak_predict(AdjArgs a, int n1, int n2) {
   const int b = blockIdx.x;
   if (b < n1) predict<true, FLUX>(a, b);
   else if (b < n1 + n2) predict<false, FLUX>(a, b - n1);

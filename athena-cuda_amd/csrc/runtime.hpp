@@ -44,6 +44,9 @@ hipError_t launch_state_unpack(const double* stage, double* st, size_t ps, int p
                                int sy, hipStream_t s);
 hipError_t launch_state_pack(const double* st, double* stage, size_t ps, int pitch, int sx,
                              int sy, hipStream_t s);
+// dense [NSTATE][sy][sx] on the device <-> the planes of one state buffer
+hipError_t launch_state_dense(double* st, double* dense, size_t ps, int pitch, int sx, int sy,
+                              int to_planes, hipStream_t s);
 }  // namespace athmi
 namespace athmi_rt {
 
