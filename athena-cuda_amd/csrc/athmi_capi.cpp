@@ -43,10 +43,9 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
   }
   if (desc[0].variant != ATHMI_EXACT && desc[0].variant != ATHMI_FAST)
     return fail(ATHMI_EINVAL, "athmi_create: unknown variant");
-  int dev = 0;
+  int dev = 0, ncu = 0;
   HIP_TRY(hipGetDevice(&dev));
-  hipDeviceProp_t prop;
-  HIP_TRY(hipGetDeviceProperties(&prop, dev));
+  HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
 
   athmi_grid* g = new athmi_grid();
   g->n = n;
@@ -55,7 +54,7 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
   g->desc.assign(desc, desc + n);
   g->hinst.resize(n);
   g->cpaw_soln.resize(n);
-  g->bl.ncu = prop.multiProcessorCount;
+  g->bl.ncu = ncu;
   // faces marched per lane by the x2 predictor (1..16)
   long cols = 0;
   for (int k = 0; k < n; k++) cols += (long)cdiv(desc[k].nx1 + 6, kX2Block) * (desc[k].nx2 + 4);
@@ -118,6 +117,10 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
     athmi_destroy(g);
     return fail(ATHMI_ENOMEM, "athmi_create: hipMalloc of the descriptors failed");
   }
+  if (hipHostMalloc(&g->heads, sizeof(ClockHead) * n, hipHostMallocDefault) != hipSuccess) {
+    athmi_destroy(g);
+    return fail(ATHMI_ENOMEM, "athmi_create: hipHostMalloc of the clocks failed");
+  }
   std::vector<Clock> hc(n);
   for (int k = 0; k < n; k++) {
     std::memset(&hc[k], 0, sizeof(Clock));
@@ -160,6 +163,7 @@ int athmi_destroy(athmi_grid* g) {
   if (g->dmem) (void)hipFree(g->dmem);
   if (g->dclk) (void)hipFree(g->dclk);
   if (g->dinst) (void)hipFree(g->dinst);
+  if (g->heads) (void)hipHostFree(g->heads);
   if (g->outbuf) (void)hipFree(g->outbuf);
   if (g->own_stream && g->stream) (void)hipStreamDestroy(g->stream);
   delete g;
@@ -337,10 +341,14 @@ int athmi_integrate(athmi_grid* g) {
   return issue(g, kSeqIntegrate);
 }
 
-static int issue_step(athmi_grid* g) { return issue(g, kSeqStep); }
+static int issue_step(athmi_grid* g) {
+  for (int k : kSeqStep) HIP_TRY(g->launch(&g->bl, k, g->stream));
+  return ATHMI_OK;
+}
 
 int athmi_step(athmi_grid* g) {
   if (!g) return fail(ATHMI_EINVAL, "null handle");
+  g->clocks_change();
   // without the graph every step starts itself: its launches may be captured
   // by the caller and replayed after the host has written the clock
   if (g->clock_written || !g->use_graph) {
@@ -370,17 +378,18 @@ int athmi_run(athmi_grid* g, int max_steps, int* steps) {
   if (!g) return fail(ATHMI_EINVAL, "null handle");
   int issued = 0;
   const int chunk = 16;
-  std::vector<Clock> hc(g->n);
   while (max_steps < 0 || issued < max_steps) {
     // any instance still running?
-    HIP_TRY(hipStreamSynchronize(g->stream));
-    HIP_TRY(hipMemcpy2D(hc.data(), sizeof(Clock), g->dclk, sizeof(Clock),
-                        offsetof(Clock, steps_run), g->n, hipMemcpyDeviceToHost));
+    const int rc = g->fetch_clocks();
+    if (rc) return rc;
     bool running = false;
-    for (const Clock& c : hc)
+    for (int k = 0; k < g->n && !running; k++) {
+      Clock c;
+      std::memcpy(&c, &g->heads[k], sizeof(ClockHead));
       if (c.time < c.tlim && (c.nlim < 0 || c.nstep < c.nlim) && c.time < c.tpause &&
           (c.fail & c.fail_stop) == 0)
         running = true;
+    }
     if (!running) break;
     int m = chunk;
     if (max_steps >= 0) m = std::min(m, max_steps - issued);
@@ -390,7 +399,8 @@ int athmi_run(athmi_grid* g, int max_steps, int* steps) {
     }
     issued += m;
   }
-  HIP_TRY(hipStreamSynchronize(g->stream));
+  const int rc = g->fetch_clocks();
+  if (rc) return rc;
   if (steps) *steps = issued;
   return ATHMI_OK;
 }
@@ -413,6 +423,7 @@ int athmi_profile_steps(athmi_grid* g, int nsteps, double* avg_ms, int nslots) {
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
   for (int k = 0; k < kStepLen; k++) avg_ms[k] = 0.0;
   g->clock_written = true;
+  g->clocks_change();
   for (int s = 0; s < nsteps; s++) {
     HIP_TRY(hipEventRecord(ev[0], g->stream));
     for (int k = 0; k < kStepLen; k++) {
@@ -498,6 +509,7 @@ int athmi_autotune(athmi_grid* g, int steps, int* x2_seg, int* persist, int* xcd
     HIP_TRY(hipMemcpyAsync(g->dclk, hc.data(), sizeof(Clock) * g->n, hipMemcpyHostToDevice,
                            g->stream));
     g->clock_written = true;
+    g->heads_valid = false;
     HIP_TRY(hipStreamSynchronize(g->stream));
     return ATHMI_OK;
   };

@@ -44,6 +44,9 @@ hipError_t launch_state_unpack(const double* stage, double* st, size_t ps, int p
                                int sy, hipStream_t s);
 hipError_t launch_state_pack(const double* st, double* stage, size_t ps, int pitch, int sx,
                              int sy, hipStream_t s);
+// the clocks' heads -> host memory; one head -> the device
+hipError_t launch_clock_publish(const Clock* clk, ClockHead* heads, int n, hipStream_t s);
+hipError_t launch_clock_set(Clock* clk, const ClockHead& head, hipStream_t s);
 // dense [NSTATE][sy][sx] on the device <-> the planes of one state buffer
 hipError_t launch_state_dense(double* st, double* dense, size_t ps, int pitch, int sx, int sy,
                               int to_planes, hipStream_t s);
@@ -89,6 +92,13 @@ struct athmi_grid {
   bool use_graph = true;
   hipGraphExec_t graph = nullptr;
   bool clock_written = true;  // the host wrote a clock since the last main-loop step
+  // the clocks as the host last saw them (pinned memory the device writes), and
+  // whether any work that changes them was queued since
+  ClockHead* heads = nullptr;
+  bool heads_valid = false;
+  // the caller has captured work of this handle, which it may replay at any
+  // time: the heads are then fetched at every read
+  bool caller_captured = false;
   std::vector<std::vector<double>> cpaw_soln;  // initial cpaw2d states (8 planes)
   void* outbuf = nullptr;                      // device staging of the output formats
   size_t outbuf_bytes = 0;
@@ -138,15 +148,32 @@ struct athmi_grid {
     drop_graph();
     return ATHMI_OK;
   }
-  int read_clock(int k, Clock& c) {
+  // before queueing work that changes the clocks
+  void clocks_change() {
+    heads_valid = false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!caller_captured && hipStreamIsCapturing(stream, &st) == hipSuccess &&
+        st != hipStreamCaptureStatusNone)
+      caller_captured = true;
+  }
+  // waits for the stream; the heads are then the device's
+  int fetch_clocks() {
+    if (!heads_valid || caller_captured) HIP_TRY(launch_clock_publish(dclk, heads, n, stream));
     HIP_TRY(hipStreamSynchronize(stream));
-    HIP_TRY(hipMemcpy(&c, dclk + k, offsetof(Clock, divb_bits) + sizeof(unsigned long long),
-                      hipMemcpyDeviceToHost));
+    heads_valid = true;
     return ATHMI_OK;
   }
+  int read_clock(int k, Clock& c) {
+    const int rc = fetch_clocks();
+    if (rc) return rc;
+    std::memcpy(&c, &heads[k], sizeof(ClockHead));
+    return ATHMI_OK;
+  }
+  // after read_clock (which has waited for the stream) of the same instance
   int write_clock_head(int k, const Clock& c) {
     clock_written = true;
-    HIP_TRY(hipMemcpy(dclk + k, &c, offsetof(Clock, divb_bits), hipMemcpyHostToDevice));
+    std::memcpy(&heads[k], &c, offsetof(Clock, divb_bits));
+    HIP_TRY(launch_clock_set(dclk + k, heads[k], stream));
     return ATHMI_OK;
   }
 };
@@ -175,6 +202,7 @@ inline HostGeom geom_of(const athmi_grid* g, int inst) {
 }
 
 inline int issue_seq(athmi_grid* g, const int* seq, size_t n) {
+  g->clocks_change();
   for (size_t k = 0; k < n; k++) HIP_TRY(g->launch(&g->bl, seq[k], g->stream));
   return ATHMI_OK;
 }

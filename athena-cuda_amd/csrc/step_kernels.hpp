@@ -63,6 +63,13 @@ struct Clock {
   unsigned long long dti_slot[kDtSlots];  // bit patterns of non-negative doubles
 };
 
+// a clock without its dt slots, as the host keeps it
+struct ClockHead {
+  unsigned long long w[offsetof(Clock, dti_slot) / 8];
+};
+static_assert(offsetof(Clock, dti_slot) % 8 == 0 && offsetof(Clock, divb_bits) % 8 == 0,
+              "the head is whole words");
+
 struct Inst {
   int nx1, nx2, is, ie, js, je, sx, sy, pitch, flux;
   int bc[4];          // ix1, ox1, ix2, ox2

@@ -129,3 +129,32 @@ def test_static_entry_point_reads_no_earlier_scratch(flux, bc):
         for f in range(11):
             assert np.array_equal(got[f], want[f]), (nx, ny, f)
         g.close()
+
+
+def test_clock_read_between_replays_of_a_captured_step():
+    """Steps the caller has captured change the clocks without a call: every
+    read still gives the device's."""
+    ora, g = start(40, 24, (4, 4, 4, 4), "roe")
+    g.use_graph(False)
+    stream = torch.cuda.Stream()
+    g.set_stream(stream.cuda_stream)
+    g.step()
+    ora.step(1e30)
+    assert g.clock(0) == ora.clock()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        g.step()
+    for n in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        ora.step(1e30)
+        assert g.clock(0) == ora.clock(), n
+        for a, b in zip(g.download(0), ora.get()):
+            assert np.array_equal(a, b), n
+    g.set_limits(1e30, ora.clock()[2] + 1)  # the captured step starts itself
+    for _ in range(3):
+        graph.replay()
+    torch.cuda.synchronize()
+    ora.step(1e30)
+    assert g.clock(0) == ora.clock()
+    g.close()
