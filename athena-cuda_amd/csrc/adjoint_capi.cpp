@@ -35,8 +35,7 @@ const int kSeqForwardScratch[] = {SK_PRED_SAVE, SK_CORNER_P, SK_CORR_BOTH};
 // ghosts
 const int kSeqFinishStep[] = {SK_CORNER_C, SK_FINAL_GHOST, SK_END_ONCE};
 // a whole step so: integrate_2d without the carry, and set_bvals
-const int kSeqRolloutStep[] = {SK_PRED,     SK_CORNER_P,    SK_CORR_BOTH,
-                               SK_CORNER_C, SK_FINAL_GHOST, SK_END_ONCE};
+const int kSeqRolloutStep[] = {SK_PRED, SK_CORNER_P, SK_FINISH, SK_END_ONCE};
 // dt never changes along a rollout: the clock is started once per run of steps
 const int kSeqStart[] = {SK_BEGIN_ONCE};
 // the reverse of one step

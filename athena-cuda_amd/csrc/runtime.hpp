@@ -56,8 +56,7 @@ namespace athmi_rt {
 // kernel sequences of the reference's routines
 // (a main-loop step is started by the k_end before it, or by SK_BEGIN_STEP
 // once the host has written the clock: athmi_grid::clock_written)
-const int kSeqStep[] = {SK_PRED, SK_CORNER_P, SK_CORR_BOTH, SK_CORNER_C, SK_FINAL_GHOST,
-                        SK_END_STEP};
+const int kSeqStep[] = {SK_PRED, SK_CORNER_P, SK_FINISH, SK_END_STEP};
 const int kSeqIntegrate[] = {SK_BEGIN_ONCE, SK_PRED,  SK_CORNER_P_CARRY, SK_CORR_BOTH,
                              SK_CORNER_C,   SK_FINAL, SK_END_ONCE};
 // the step one kernel at a time, as athmi_profile_steps times it

@@ -624,16 +624,13 @@ __global__ void __launch_bounds__(kX1Block, 2) k_pred(const Inst* __restrict__ i
 // x1-flux of B2 is -E3 and the x2-flux of B1 is +E3; each of the four edge
 // estimates is upwinded by the sign of the face mass flux (>0, <0, ==0).
 // F1, F2: Cons1D flux groups (d = 0, By = 5, Bz = 6); ecc: cell-centred emf3.
-__device__ __forceinline__ double corner_emf(const double* F1, const double* F2,
-                                             const double* ecc, size_t ps, int pitch, int j,
-                                             int i) {
-  const uint32_t k = (uint32_t)(j * pitch + i);
-  const uint32_t kjm = k - pitch, kim = k - 1, kjmim = k - pitch - 1;
-  const double f1d_jm = LD(F1, kjm), f1d = LD(F1, k);
-  const double f1by_jm = LD(F1 + 5 * ps, kjm), f1by = LD(F1 + 5 * ps, k);
-  const double f2d_im = LD(F2, kim), f2d = LD(F2, k);
-  const double f2bz_im = LD(F2 + 6 * ps, kim), f2bz = LD(F2 + 6 * ps, k);
-  const double e_jmim = LD(ecc, kjmim), e_jm = LD(ecc, kjm), e_im = LD(ecc, kim), e_00 = LD(ecc, k);
+struct CornerIn {
+  double f1d_jm, f1d, f1by_jm, f1by, f2d_im, f2d, f2bz_im, f2bz, e_jmim, e_jm, e_im, e_00;
+};
+__device__ __forceinline__ double corner_value(const CornerIn& c) {
+  const double f1d_jm = c.f1d_jm, f1d = c.f1d, f1by_jm = c.f1by_jm, f1by = c.f1by;
+  const double f2d_im = c.f2d_im, f2d = c.f2d, f2bz_im = c.f2bz_im, f2bz = c.f2bz;
+  const double e_jmim = c.e_jmim, e_jm = c.e_jm, e_im = c.e_im, e_00 = c.e_00;
   double emf_l1, emf_r1, emf_l2, emf_r2;
   if (f1d_jm > 0.0) emf_l2 = -f1by_jm + (f2bz_im - e_jmim);
   else if (f1d_jm < 0.0) emf_l2 = -f1by_jm + (f2bz - e_jm);
@@ -648,6 +645,15 @@ __device__ __forceinline__ double corner_emf(const double* F1, const double* F2,
   else if (f2d < 0.0) emf_r1 = f2bz + (-f1by - e_00);
   else emf_r1 = f2bz + 0.5 * (-f1by_jm - e_jm - f1by - e_00);
   return 0.25 * (emf_l1 + emf_r1 + emf_l2 + emf_r2);
+}
+__device__ __forceinline__ double corner_emf(const double* F1, const double* F2,
+                                             const double* ecc, size_t ps, int pitch, int j,
+                                             int i) {
+  const uint32_t k = (uint32_t)(j * pitch + i);
+  const uint32_t kjm = k - pitch, kim = k - 1, kjmim = k - pitch - 1;
+  return corner_value(CornerIn{LD(F1, kjm), LD(F1, k), LD(F1 + 5 * ps, kjm), LD(F1 + 5 * ps, k),
+                               LD(F2, kim), LD(F2, k), LD(F2 + 6 * ps, kim), LD(F2 + 6 * ps, k),
+                               LD(ecc, kjmim), LD(ecc, kjm), LD(ecc, kim), LD(ecc, k)});
 }
 
 // ---------------------------------------------------------------------------
@@ -752,6 +758,107 @@ __global__ void __launch_bounds__(kTileX* kTileY) k_corner(const Inst* __restric
 // stores the corners it owns -- together the range [js-1,je+2]x[is-1,ie+2] --
 // in the corner plane for the x2 part (no k_corner<pred> launch).
 constexpr int kCornerCols = kTileX + 1;
+// What the corrector's faces of one instance read
+struct CorrSrc {
+  const double* st;  // state planes
+  const double* sc;  // scratch planes
+  size_t ps;
+  int pitch;
+  double hdtodx1, hdtodx2;
+};
+// corrected x1-face states at k (Steps 5a, 5b)
+__device__ __forceinline__ void corrected_x1(const CorrSrc& s, uint32_t k, Cons7& L, Cons7& R) {
+  const double* const st = s.st;
+  const double* const sc = s.sc;
+  const size_t ps = s.ps;
+  const int pitch = s.pitch;
+  const double hdtodx1 = s.hdtodx1, hdtodx2 = s.hdtodx2;
+  const double* const F2 = sc + S_F2 * ps;
+  const double* const B1i = st + F_B1I * ps;
+  L = get7(sc + S_UL1 * ps, ps, k);
+  R = get7(sc + S_UR1 * ps, ps, k);
+  {  // Step 5a: x2 fluxes at (j+1,i-1),(j,i-1) for L and (j+1,i),(j,i) for R
+    const uint32_t a1 = k + pitch - 1, a0 = k - 1, c1 = k + pitch, c0 = k;
+    L.d = L.d - hdtodx2 * (LD(F2, a1) - LD(F2, a0));
+    L.mx = L.mx - hdtodx2 * (LD(F2 + 3 * ps, a1) - LD(F2 + 3 * ps, a0));
+    L.my = L.my - hdtodx2 * (LD(F2 + 1 * ps, a1) - LD(F2 + 1 * ps, a0));
+    L.mz = L.mz - hdtodx2 * (LD(F2 + 2 * ps, a1) - LD(F2 + 2 * ps, a0));
+    L.e = L.e - hdtodx2 * (LD(F2 + 4 * ps, a1) - LD(F2 + 4 * ps, a0));
+    L.bz = L.bz - hdtodx2 * (LD(F2 + 5 * ps, a1) - LD(F2 + 5 * ps, a0));
+    R.d = R.d - hdtodx2 * (LD(F2, c1) - LD(F2, c0));
+    R.mx = R.mx - hdtodx2 * (LD(F2 + 3 * ps, c1) - LD(F2 + 3 * ps, c0));
+    R.my = R.my - hdtodx2 * (LD(F2 + 1 * ps, c1) - LD(F2 + 1 * ps, c0));
+    R.mz = R.mz - hdtodx2 * (LD(F2 + 2 * ps, c1) - LD(F2 + 2 * ps, c0));
+    R.e = R.e - hdtodx2 * (LD(F2 + 4 * ps, c1) - LD(F2 + 4 * ps, c0));
+    R.bz = R.bz - hdtodx2 * (LD(F2 + 5 * ps, c1) - LD(F2 + 5 * ps, c0));
+  }
+  {  // Step 5b: MHD source terms with the cell-centred field of cells i-1, i
+    double dbx = LD(B1i, k) - LD(B1i, k - 1);
+    double b1 = LD(st + F_B1C * ps, k - 1), b2 = LD(st + F_B2C * ps, k - 1);
+    double b3 = LD(st + F_B3C * ps, k - 1);
+    double v3 = LD(st + F_M3 * ps, k - 1) / LD(st + F_D * ps, k - 1);
+    L.mx = L.mx + hdtodx1 * b1 * dbx;
+    L.my = L.my + hdtodx1 * b2 * dbx;
+    L.mz = L.mz + hdtodx1 * b3 * dbx;
+    L.bz = L.bz + hdtodx1 * v3 * dbx;
+    L.e = L.e + hdtodx1 * b3 * v3 * dbx;
+    dbx = LD(B1i, k + 1) - LD(B1i, k);
+    b1 = LD(st + F_B1C * ps, k); b2 = LD(st + F_B2C * ps, k); b3 = LD(st + F_B3C * ps, k);
+    v3 = LD(st + F_M3 * ps, k) / LD(st + F_D * ps, k);
+    R.mx = R.mx + hdtodx1 * b1 * dbx;
+    R.my = R.my + hdtodx1 * b2 * dbx;
+    R.mz = R.mz + hdtodx1 * b3 * dbx;
+    R.bz = R.bz + hdtodx1 * v3 * dbx;
+    R.e = R.e + hdtodx1 * b3 * v3 * dbx;
+  }
+}
+// corrected x2-face states at k (Steps 6a, 6b)
+__device__ __forceinline__ void corrected_x2(const CorrSrc& s, uint32_t k, Cons7& L, Cons7& R) {
+  const double* const st = s.st;
+  const double* const sc = s.sc;
+  const size_t ps = s.ps;
+  const int pitch = s.pitch;
+  const double hdtodx1 = s.hdtodx1, hdtodx2 = s.hdtodx2;
+  const double* const F1 = sc + S_F1 * ps;
+  const double* const B2i = st + F_B2I * ps;
+  L = get7(sc + S_UL2 * ps, ps, k);
+  R = get7(sc + S_UR2 * ps, ps, k);
+  {  // Step 6a: x1 fluxes at (j-1,i+1),(j-1,i) for L and (j,i+1),(j,i) for R
+    const uint32_t a1 = k - pitch + 1, a0 = k - pitch, c1 = k + 1, c0 = k;
+    L.d = L.d - hdtodx1 * (LD(F1, a1) - LD(F1, a0));
+    L.mx = L.mx - hdtodx1 * (LD(F1 + 2 * ps, a1) - LD(F1 + 2 * ps, a0));
+    L.my = L.my - hdtodx1 * (LD(F1 + 3 * ps, a1) - LD(F1 + 3 * ps, a0));
+    L.mz = L.mz - hdtodx1 * (LD(F1 + 1 * ps, a1) - LD(F1 + 1 * ps, a0));
+    L.e = L.e - hdtodx1 * (LD(F1 + 4 * ps, a1) - LD(F1 + 4 * ps, a0));
+    L.by = L.by - hdtodx1 * (LD(F1 + 6 * ps, a1) - LD(F1 + 6 * ps, a0));
+    R.d = R.d - hdtodx1 * (LD(F1, c1) - LD(F1, c0));
+    R.mx = R.mx - hdtodx1 * (LD(F1 + 2 * ps, c1) - LD(F1 + 2 * ps, c0));
+    R.my = R.my - hdtodx1 * (LD(F1 + 3 * ps, c1) - LD(F1 + 3 * ps, c0));
+    R.mz = R.mz - hdtodx1 * (LD(F1 + 1 * ps, c1) - LD(F1 + 1 * ps, c0));
+    R.e = R.e - hdtodx1 * (LD(F1 + 4 * ps, c1) - LD(F1 + 4 * ps, c0));
+    R.by = R.by - hdtodx1 * (LD(F1 + 6 * ps, c1) - LD(F1 + 6 * ps, c0));
+  }
+  {  // Step 6b: MHD source terms with the cell-centred field of cells j-1, j
+    const uint32_t km = k - pitch;
+    double dby = LD(B2i, k) - LD(B2i, km);
+    double b1 = LD(st + F_B1C * ps, km), b2 = LD(st + F_B2C * ps, km), b3 = LD(st + F_B3C * ps, km);
+    double v3 = LD(st + F_M3 * ps, km) / LD(st + F_D * ps, km);
+    L.mz = L.mz + hdtodx2 * b1 * dby;
+    L.mx = L.mx + hdtodx2 * b2 * dby;
+    L.my = L.my + hdtodx2 * b3 * dby;
+    L.by = L.by + hdtodx2 * v3 * dby;
+    L.e = L.e + hdtodx2 * b3 * v3 * dby;
+    dby = LD(B2i, k + pitch) - LD(B2i, k);
+    b1 = LD(st + F_B1C * ps, k); b2 = LD(st + F_B2C * ps, k); b3 = LD(st + F_B3C * ps, k);
+    v3 = LD(st + F_M3 * ps, k) / LD(st + F_D * ps, k);
+    R.mz = R.mz + hdtodx2 * b1 * dby;
+    R.mx = R.mx + hdtodx2 * b2 * dby;
+    R.my = R.my + hdtodx2 * b3 * dby;
+    R.by = R.by + hdtodx2 * v3 * dby;
+    R.e = R.e + hdtodx2 * b3 * v3 * dby;
+  }
+}
+
 template <int PART, int TY, int FLUX, bool CP>  // TY: rows of a tile of kTileX x TY faces
 __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ninst, int t,
                                           int strip, const LdsPark& park, double* cemf) {
@@ -812,6 +919,7 @@ __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ni
   const size_t ps = (size_t)uni((int)g.ps);
   const int pitch = uni(g.pitch);
   const uint32_t k = (uint32_t)(j * pitch + i);
+  const CorrSrc src{st, sc, ps, pitch, hdtodx1, hdtodx2};
   const double* emf = sc + S_EMF * ps;
   const double* B1i = st + F_B1I * ps;
   const double* B2i = st + F_B2I * ps;
@@ -824,42 +932,7 @@ __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ni
     // rebuilt from memory for the HLLE fallback
     auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
       compiler_fence();
-      L = get7(sc + S_UL1 * ps, ps, k);
-      R = get7(sc + S_UR1 * ps, ps, k);
-      {  // Step 5a: x2 fluxes at (j+1,i-1),(j,i-1) for L and (j+1,i),(j,i) for R
-        const uint32_t a1 = k + pitch - 1, a0 = k - 1, c1 = k + pitch, c0 = k;
-        L.d = L.d - hdtodx2 * (LD(F2, a1) - LD(F2, a0));
-        L.mx = L.mx - hdtodx2 * (LD(F2 + 3 * ps, a1) - LD(F2 + 3 * ps, a0));
-        L.my = L.my - hdtodx2 * (LD(F2 + 1 * ps, a1) - LD(F2 + 1 * ps, a0));
-        L.mz = L.mz - hdtodx2 * (LD(F2 + 2 * ps, a1) - LD(F2 + 2 * ps, a0));
-        L.e = L.e - hdtodx2 * (LD(F2 + 4 * ps, a1) - LD(F2 + 4 * ps, a0));
-        L.bz = L.bz - hdtodx2 * (LD(F2 + 5 * ps, a1) - LD(F2 + 5 * ps, a0));
-        R.d = R.d - hdtodx2 * (LD(F2, c1) - LD(F2, c0));
-        R.mx = R.mx - hdtodx2 * (LD(F2 + 3 * ps, c1) - LD(F2 + 3 * ps, c0));
-        R.my = R.my - hdtodx2 * (LD(F2 + 1 * ps, c1) - LD(F2 + 1 * ps, c0));
-        R.mz = R.mz - hdtodx2 * (LD(F2 + 2 * ps, c1) - LD(F2 + 2 * ps, c0));
-        R.e = R.e - hdtodx2 * (LD(F2 + 4 * ps, c1) - LD(F2 + 4 * ps, c0));
-        R.bz = R.bz - hdtodx2 * (LD(F2 + 5 * ps, c1) - LD(F2 + 5 * ps, c0));
-      }
-      {  // Step 5b: MHD source terms with the cell-centred field of cells i-1, i
-        double dbx = LD(B1i, k) - LD(B1i, k - 1);
-        double b1 = LD(st + F_B1C * ps, k - 1), b2 = LD(st + F_B2C * ps, k - 1);
-        double b3 = LD(st + F_B3C * ps, k - 1);
-        double v3 = LD(st + F_M3 * ps, k - 1) / LD(st + F_D * ps, k - 1);
-        L.mx = L.mx + hdtodx1 * b1 * dbx;
-        L.my = L.my + hdtodx1 * b2 * dbx;
-        L.mz = L.mz + hdtodx1 * b3 * dbx;
-        L.bz = L.bz + hdtodx1 * v3 * dbx;
-        L.e = L.e + hdtodx1 * b3 * v3 * dbx;
-        dbx = LD(B1i, k + 1) - LD(B1i, k);
-        b1 = LD(st + F_B1C * ps, k); b2 = LD(st + F_B2C * ps, k); b3 = LD(st + F_B3C * ps, k);
-        v3 = LD(st + F_M3 * ps, k) / LD(st + F_D * ps, k);
-        R.mx = R.mx + hdtodx1 * b1 * dbx;
-        R.my = R.my + hdtodx1 * b2 * dbx;
-        R.mz = R.mz + hdtodx1 * b3 * dbx;
-        R.bz = R.bz + hdtodx1 * v3 * dbx;
-        R.e = R.e + hdtodx1 * b3 * v3 * dbx;
-      }
+      corrected_x1(src, k, L, R);
       if (CP) {
         const int cc = threadIdx.y * kCornerCols + threadIdx.x;
         bx = LD(B1i, k) - hdtodx2 * (cemf[cc + kCornerCols] - cemf[cc]);
@@ -880,42 +953,7 @@ __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ni
     // corrected x2-face states (Steps 6a, 6b) at the half-step face field
     auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
       compiler_fence();
-      L = get7(sc + S_UL2 * ps, ps, k);
-      R = get7(sc + S_UR2 * ps, ps, k);
-      {  // Step 6a: x1 fluxes at (j-1,i+1),(j-1,i) for L and (j,i+1),(j,i) for R
-        const uint32_t a1 = k - pitch + 1, a0 = k - pitch, c1 = k + 1, c0 = k;
-        L.d = L.d - hdtodx1 * (LD(F1, a1) - LD(F1, a0));
-        L.mx = L.mx - hdtodx1 * (LD(F1 + 2 * ps, a1) - LD(F1 + 2 * ps, a0));
-        L.my = L.my - hdtodx1 * (LD(F1 + 3 * ps, a1) - LD(F1 + 3 * ps, a0));
-        L.mz = L.mz - hdtodx1 * (LD(F1 + 1 * ps, a1) - LD(F1 + 1 * ps, a0));
-        L.e = L.e - hdtodx1 * (LD(F1 + 4 * ps, a1) - LD(F1 + 4 * ps, a0));
-        L.by = L.by - hdtodx1 * (LD(F1 + 6 * ps, a1) - LD(F1 + 6 * ps, a0));
-        R.d = R.d - hdtodx1 * (LD(F1, c1) - LD(F1, c0));
-        R.mx = R.mx - hdtodx1 * (LD(F1 + 2 * ps, c1) - LD(F1 + 2 * ps, c0));
-        R.my = R.my - hdtodx1 * (LD(F1 + 3 * ps, c1) - LD(F1 + 3 * ps, c0));
-        R.mz = R.mz - hdtodx1 * (LD(F1 + 1 * ps, c1) - LD(F1 + 1 * ps, c0));
-        R.e = R.e - hdtodx1 * (LD(F1 + 4 * ps, c1) - LD(F1 + 4 * ps, c0));
-        R.by = R.by - hdtodx1 * (LD(F1 + 6 * ps, c1) - LD(F1 + 6 * ps, c0));
-      }
-      {  // Step 6b: MHD source terms with the cell-centred field of cells j-1, j
-        const uint32_t km = k - pitch;
-        double dby = LD(B2i, k) - LD(B2i, km);
-        double b1 = LD(st + F_B1C * ps, km), b2 = LD(st + F_B2C * ps, km), b3 = LD(st + F_B3C * ps, km);
-        double v3 = LD(st + F_M3 * ps, km) / LD(st + F_D * ps, km);
-        L.mz = L.mz + hdtodx2 * b1 * dby;
-        L.mx = L.mx + hdtodx2 * b2 * dby;
-        L.my = L.my + hdtodx2 * b3 * dby;
-        L.by = L.by + hdtodx2 * v3 * dby;
-        L.e = L.e + hdtodx2 * b3 * v3 * dby;
-        dby = LD(B2i, k + pitch) - LD(B2i, k);
-        b1 = LD(st + F_B1C * ps, k); b2 = LD(st + F_B2C * ps, k); b3 = LD(st + F_B3C * ps, k);
-        v3 = LD(st + F_M3 * ps, k) / LD(st + F_D * ps, k);
-        R.mz = R.mz + hdtodx2 * b1 * dby;
-        R.mx = R.mx + hdtodx2 * b2 * dby;
-        R.my = R.my + hdtodx2 * b3 * dby;
-        R.by = R.by + hdtodx2 * v3 * dby;
-        R.e = R.e + hdtodx2 * b3 * v3 * dby;
-      }
+      corrected_x2(src, k, L, R);
       bx = b2h(k);
       wl = cons_to_prim(L, bx, eos);
       wr = cons_to_prim(R, bx, eos);
@@ -997,6 +1035,80 @@ __device__ __forceinline__ int cell_fail_bits(const Inst& g, double d, double M1
   return bits;
 }
 
+// set_bvals from the source's side: only a tile of w x h cells at (j0, i0) that
+// reaches the five cells at an edge (four, and the face past them) has ghost
+// images
+__device__ __forceinline__ bool near_edge(const Inst& g, int i0, int w, int j0, int h) {
+  return i0 <= g.is + 4 || i0 + w > g.ie - 4 || j0 <= g.js + 4 || j0 + h > g.je - 4;
+}
+
+// The updated faces of interior cell (j, i) (lower: b1n, b2n; upper: b1p, b2p,
+// stored by the last column and row) into the planes `out`, and the ghosts that
+// copy them (edge)
+__device__ __forceinline__ void store_faces(const Inst& g, double* out, int j, int i,
+                                            bool edge, unsigned ix, unsigned iy, double b1n,
+                                            double b1p, double b2n, double b2p) {
+  const size_t ps = g.ps;
+  const int pitch = g.pitch;
+  auto put_b1 = [&](int ii, double v) {
+    ST(out + F_B1I * ps, (uint32_t)(j * pitch + ii), v);
+    if (edge)
+      for_ghost_images(g, j, ii, ghost_images(ii, g.is, g.ie, g.bc[0], g.bc[1], true), iy,
+                       [&](int r, int c, bool, bool) {
+                         ST(out + F_B1I * ps, (uint32_t)(r * pitch + c), v);
+                       });
+  };
+  auto put_b2 = [&](int jj, double v) {
+    ST(out + F_B2I * ps, (uint32_t)(jj * pitch + i), v);
+    if (edge)
+      for_ghost_images(g, jj, i, ix, ghost_images(jj, g.js, g.je, g.bc[2], g.bc[3], true),
+                       [&](int r, int c, bool, bool) {
+                         ST(out + F_B2I * ps, (uint32_t)(r * pitch + c), v);
+                       });
+  };
+  put_b1(i, b1n);
+  if (i == g.ie) put_b1(i + 1, b1p);
+  put_b2(j, b2n);
+  if (j == g.je) put_b2(j + 1, b2p);
+}
+
+// The updated interior cell (j, i) into the planes `out`, with the ghosts that
+// copy it (edge), its failure bits, and its inverse dt
+__device__ __forceinline__ double store_cell(const Inst& g, Clock* clk, double* out,
+                                             int j, int i, bool edge, unsigned ix,
+                                             unsigned iy, double d, double M1, double M2, double M3, double E, double B3c,
+                                             double B1c, double B2c) {
+  const size_t ps = g.ps;
+  const int pitch = g.pitch;
+  const uint32_t k = (uint32_t)(j * pitch + i);
+  ST(out + F_D * ps, k, d);
+  ST(out + F_M1 * ps, k, M1);
+  ST(out + F_M2 * ps, k, M2);
+  ST(out + F_M3 * ps, k, M3);
+  ST(out + F_E * ps, k, E);
+  ST(out + F_B1C * ps, k, B1c);
+  ST(out + F_B2C * ps, k, B2c);
+  ST(out + F_B3C * ps, k, B3c);
+  ST(out + F_B3I * ps, k, B3c);
+  if (edge)
+    for_ghost_images(g, j, i, ix, iy, [&](int r, int c, bool nx, bool ny) {
+      const uint32_t kg = (uint32_t)(r * pitch + c);
+      ST(out + F_D * ps, kg, d);
+      ST(out + F_M1 * ps, kg, nx ? -M1 : M1);
+      ST(out + F_M2 * ps, kg, ny ? -M2 : M2);
+      ST(out + F_M3 * ps, kg, M3);
+      ST(out + F_E * ps, kg, E);
+      ST(out + F_B1C * ps, kg, B1c);
+      ST(out + F_B2C * ps, kg, B2c);
+      ST(out + F_B3C * ps, kg, B3c);
+      ST(out + F_B3I * ps, kg, B3c);
+    });
+  const double dti = inverse_dt(g, d, M1, M2, M3, E);
+  const int bits = cell_fail_bits(g, d, M1, M2, M3, E, B1c, B2c, B3c);
+  if (bits) atomicOr(&clk->fail, bits);
+  return dti;
+}
+
 // Steps 9, 11a, 11b, 13 (:473-534) over the interior cells and their faces
 // (the last column and row also store their upper faces, so that a 512-cell row is
 // eight tiles, not nine) into the other ping-pong buffer, and the new_dt
@@ -1062,40 +1174,17 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
         return FUSED ? cemf[cc + dj * kCornerCols + di] : LD(emf, k + dj * pitch + di);
       };
       const double e00 = corner(0, 0), e10 = corner(1, 0), e01 = corner(0, 1), e11 = corner(1, 1);
-      // set_bvals from the source's side: only a tile that reaches the five
-      // cells at an edge (four, and the face past them) has ghost images
-      const bool edge = fill && (i0 <= g.is + 4 || i0 + kTileX > g.ie - 4 || j0 <= g.js + 4 ||
-                                 j0 + TY > g.je - 4);
+      const double b1n = LD(st + F_B1I * ps, k) - dtodx2 * (e10 - e00);
+      const double b1p = LD(st + F_B1I * ps, k + 1) - dtodx2 * (e11 - e01);
+      const double b2n = LD(st + F_B2I * ps, k) + dtodx1 * (e01 - e00);
+      const double b2p = LD(st + F_B2I * ps, k + pitch) + dtodx1 * (e11 - e10);
+      const bool edge = fill && near_edge(g, i0, kTileX, j0, TY);
       unsigned ix = 0, iy = 0;
       if (edge) {
         ix = ghost_images(i, g.is, g.ie, g.bc[0], g.bc[1], false);
         iy = ghost_images(j, g.js, g.je, g.bc[2], g.bc[3], false);
       }
-      // the cell's lower faces, and the upper ones of the last column and row
-      auto put_b1 = [&](int ii, double v) {
-        ST(out + F_B1I * ps, (uint32_t)(j * pitch + ii), v);
-        if (edge)
-          for_ghost_images(g, j, ii, ghost_images(ii, g.is, g.ie, g.bc[0], g.bc[1], true), iy,
-                           [&](int r, int c, bool, bool) {
-                             ST(out + F_B1I * ps, (uint32_t)(r * pitch + c), v);
-                           });
-      };
-      auto put_b2 = [&](int jj, double v) {
-        ST(out + F_B2I * ps, (uint32_t)(jj * pitch + i), v);
-        if (edge)
-          for_ghost_images(g, jj, i, ix, ghost_images(jj, g.js, g.je, g.bc[2], g.bc[3], true),
-                           [&](int r, int c, bool, bool) {
-                             ST(out + F_B2I * ps, (uint32_t)(r * pitch + c), v);
-                           });
-      };
-      const double b1n = LD(st + F_B1I * ps, k) - dtodx2 * (e10 - e00);
-      const double b1p = LD(st + F_B1I * ps, k + 1) - dtodx2 * (e11 - e01);
-      const double b2n = LD(st + F_B2I * ps, k) + dtodx1 * (e01 - e00);
-      const double b2p = LD(st + F_B2I * ps, k + pitch) + dtodx1 * (e11 - e10);
-      put_b1(i, b1n);
-      if (i == g.ie) put_b1(i + 1, b1p);
-      put_b2(j, b2n);
-      if (j == g.je) put_b2(j + 1, b2p);
+      store_faces(g, out, j, i, edge, ix, iy, b1n, b1p, b2n, b2p);
       {
         const double* F1 = sc + S_F1C * ps;
         const double* F2 = sc + S_F2C * ps;
@@ -1114,37 +1203,204 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
         M3 = M3 - dtodx2 * (LD(F2 + 2 * ps, kp) - LD(F2 + 2 * ps, k));
         E = E - dtodx2 * (LD(F2 + 4 * ps, kp) - LD(F2 + 4 * ps, k));
         B3c = B3c - dtodx2 * (LD(F2 + 5 * ps, kp) - LD(F2 + 5 * ps, k));
-        const double B1c = 0.5 * (b1n + b1p), B2c = 0.5 * (b2n + b2p);
-        ST(out + F_D * ps, k, d);
-        ST(out + F_M1 * ps, k, M1);
-        ST(out + F_M2 * ps, k, M2);
-        ST(out + F_M3 * ps, k, M3);
-        ST(out + F_E * ps, k, E);
-        ST(out + F_B1C * ps, k, B1c);
-        ST(out + F_B2C * ps, k, B2c);
-        ST(out + F_B3C * ps, k, B3c);
-        ST(out + F_B3I * ps, k, B3c);
-        if (edge)
-          for_ghost_images(g, j, i, ix, iy, [&](int r, int c, bool nx, bool ny) {
-            const uint32_t kg = (uint32_t)(r * pitch + c);
-            ST(out + F_D * ps, kg, d);
-            ST(out + F_M1 * ps, kg, nx ? -M1 : M1);
-            ST(out + F_M2 * ps, kg, ny ? -M2 : M2);
-            ST(out + F_M3 * ps, kg, M3);
-            ST(out + F_E * ps, kg, E);
-            ST(out + F_B1C * ps, kg, B1c);
-            ST(out + F_B2C * ps, kg, B2c);
-            ST(out + F_B3C * ps, kg, B3c);
-            ST(out + F_B3I * ps, kg, B3c);
-          });
-        dti = inverse_dt(g, d, M1, M2, M3, E);
-        const int bits = cell_fail_bits(g, d, M1, M2, M3, E, B1c, B2c, B3c);
-        if (bits) atomicOr(&clk->fail, bits);
+        dti = store_cell(g, clk, out, j, i, edge, ix, iy, d, M1, M2, M3, E, B3c, 0.5 * (b1n + b1p),
+                         0.5 * (b2n + b2p));
       }
     }
     const double m = block_max(dti, red);
     if (threadIdx.x == 0 && threadIdx.y == 0) atomic_max_pos(&clk->dti_slot[t % kDtSlots], m);
   }
+}
+
+// ---------------------------------------------------------------------------
+// HLLE: the corrector, Step 9's corners and the final update in one march. A
+// wave takes 64 columns and walks down kCfRows rows. Per row r: the x2 flux at
+// face r (Steps 6, 8c), which finishes the update of row r-1's conserved
+// variables; the x1 flux of row r (Steps 5, 8b), which starts row r's; emf3 at
+// t^{n+1/2} (Step 7); the corner emf of row r from the neighbour lanes; the face
+// fields, cell-centred fields and stores of row r-1. What one row hands to the
+// next stays in the lane's LDS slots, so the corrector fluxes, the cell-centred
+// emf and the corners, 15 planes that k_corr_both writes and k_final reads, never
+// reach memory. Lanes 1..62 finish cells; lanes 0 and 63 hold the neighbours'
+// corner inputs. A march repeats one x2 face row and one x1 row.
+// Bound by the 61 planes it reads and writes once: 4096^2 6.08 -> 5.36 ms a step
+// (this kernel 2.3 ms, 3.6 TB/s), 2048 x 1536 1.157 -> 1.076, 24 grids of 777 x 333
+// 2.34 -> 2.12. Rows: 8, 10, 12, 16 and 24 are within 3% at 4096^2 (more rows repeat
+// less) and 10 is the best at 1200^2 (fewer give more waves). Three waves per
+// SIMD: asked for four, the compiler keeps to 120 registers by issuing each plane's
+// loads behind the last one's use (4096^2 5.7-5.8 ms); with 148 they go out together.
+// Roe, at two waves per SIMD and with its parked values beside the slots, lost
+// (6.95 -> 7.02): it keeps the separate launches.
+enum CfSlot { CF_U = 0, CF_F2 = 6, CF_F1D = 13, CF_F1BY, CF_ECH, CF_E, CF_SLOTS };
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 3)))
+k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
+  __shared__ double lds[CF_SLOTS * 64];
+  const int t = xcd_tile(blockIdx.x, ntiles, remap);
+  const Inst& g = insts[find_inst(insts, ninst, K_CORR_FINAL, t)];
+  Clock* clk = g.clk;
+  if (!clk->active) return;
+  // the lane, formed anew in each phase: addresses derived from it are then
+  // not held across the fluxes, which fill the registers of two waves per SIMD
+  auto fresh_lane = []() {
+    int l = threadIdx.x;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  const int local = uni(t - g.tile0[K_CORR_FINAL]);
+  const int nstrip = dcdiv(uni(g.nx1), kCfCols);
+  const int sg = local / nstrip, s = local - sg * nstrip;
+  const int gis = uni(g.is), gie = uni(g.ie), gje = uni(g.je);
+  const int i0 = gis - 1 + s * kCfCols;
+  const int r0 = uni(g.js) + sg * kCfRows, r1 = min(r0 + kCfRows - 1, gje);
+  const double dt = uni(clk->dts);
+  const double dtodx1 = uni(dt / uni(g.dx1)), dtodx2 = uni(dt / uni(g.dx2));
+  const double hdtodx1 = uni(0.5 * dtodx1), hdtodx2 = uni(0.5 * dtodx2);
+  const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
+  const int cur = uni(clk->cur);
+  const double* __restrict__ st = uni(g.state[cur]);
+  double* __restrict__ out = uni(g.state[cur ^ 1]);
+  const double* __restrict__ sc = uni(g.scratch);
+  const size_t ps = (size_t)uni((int)g.ps);
+  const int pitch = uni(g.pitch);
+  const CorrSrc src{st, sc, ps, pitch, hdtodx1, hdtodx2};
+  const double* emf = sc + S_EMF * ps;
+  const double* B1i = st + F_B1I * ps;
+  const double* B2i = st + F_B2I * ps;
+  const double* F1 = sc + S_F1 * ps;
+  const double* F2 = sc + S_F2 * ps;
+  auto b1h = [&](uint32_t kk) { return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk)); };
+  auto b2h = [&](uint32_t kk) { return LD(B2i, kk) + hdtodx1 * (LD(emf, kk + 1) - LD(emf, kk)); };
+  const bool edge = near_edge(g, i0 + 1, kCfCols, r0, kCfRows);
+  double dti = 0.0;
+#pragma unroll 1
+  for (int r = r0 - 1; r <= r1 + 1; r++) {
+    phase_fence();
+    // lanes past the grid repeat its last column
+    auto cell_of = [&](int lane) { return (uint32_t)(r * pitch + min(i0 + lane, gie + 1)); };
+    if (r >= r0) {
+      const int lane = fresh_lane();
+      const uint32_t k = cell_of(lane);
+      auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
+        compiler_fence();
+        corrected_x2(src, k, L, R);
+        bx = b2h(k);
+        wl = cons_to_prim(L, bx, eos);
+        wr = cons_to_prim(R, bx, eos);
+      };
+      Cons7 L, R;
+      Prim7 wl, wr;
+      double bx;
+      build(L, R, wl, wr, bx);
+      const Cons7 f = riemann_of<kFluxHlle>(L, R, wl, wr, bx, eos, build);
+      compiler_fence();
+      auto slot = [&](int q) -> double& { return lds[q * 64 + lane]; };
+      if (r > r0) {
+        // row r-1: the x2 part of the update (d, M1, M2, M3, E, B3c take the flux
+        // components 0, 3, 1, 2, 4, 5)
+        slot(CF_U + 0) = slot(CF_U + 0) - dtodx2 * (f.d - slot(CF_F2 + 0));
+        slot(CF_U + 1) = slot(CF_U + 1) - dtodx2 * (f.mz - slot(CF_F2 + 3));
+        slot(CF_U + 2) = slot(CF_U + 2) - dtodx2 * (f.mx - slot(CF_F2 + 1));
+        slot(CF_U + 3) = slot(CF_U + 3) - dtodx2 * (f.my - slot(CF_F2 + 2));
+        slot(CF_U + 4) = slot(CF_U + 4) - dtodx2 * (f.e - slot(CF_F2 + 4));
+        slot(CF_U + 5) = slot(CF_U + 5) - dtodx2 * (f.by - slot(CF_F2 + 5));
+      }
+      slot(CF_F2 + 0) = f.d; slot(CF_F2 + 1) = f.mx; slot(CF_F2 + 2) = f.my;
+      slot(CF_F2 + 3) = f.mz; slot(CF_F2 + 4) = f.e; slot(CF_F2 + 5) = f.by;
+      slot(CF_F2 + 6) = f.bz;
+    }
+    phase_fence();
+    Cons7 f1;
+    {
+      const int lane = fresh_lane();
+      const uint32_t k = cell_of(lane);
+      auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
+        compiler_fence();
+        corrected_x1(src, k, L, R);
+        bx = b1h(k);
+        wl = cons_to_prim(L, bx, eos);
+        wr = cons_to_prim(R, bx, eos);
+      };
+      Cons7 L, R;
+      Prim7 wl, wr;
+      double bx;
+      build(L, R, wl, wr, bx);
+      f1 = riemann_of<kFluxHlle>(L, R, wl, wr, bx, eos, build);
+    }
+    phase_fence();
+    const int lane = fresh_lane();
+    const int i = i0 + lane;
+    const uint32_t k = cell_of(lane);
+    const int lm = max(lane - 1, 0), lp = min(lane + 1, 63);
+    const bool fin = lane >= 1 && lane <= kCfCols && i <= gie;
+    auto slot = [&](int q) -> double& { return lds[q * 64 + lane]; };
+    auto slot_at = [&](int q, int l) -> double { return lds[q * 64 + l]; };
+    // Step 7 at (r, i); the slot holds row r-1's until here
+    const double e_jm = slot(CF_ECH), e_jmim = slot_at(CF_ECH, lm);
+    compiler_fence();
+    {
+      const double dhalf = LD(st + F_D * ps, k) - hdtodx1 * (LD(F1, k + 1) - LD(F1, k)) -
+                           hdtodx2 * (LD(F2, k + pitch) - LD(F2, k));
+      const double m1 = LD(st + F_M1 * ps, k) - hdtodx1 * (LD(F1 + 1 * ps, k + 1) - LD(F1 + 1 * ps, k)) -
+                        hdtodx2 * (LD(F2 + 3 * ps, k + pitch) - LD(F2 + 3 * ps, k));
+      const double m2 = LD(st + F_M2 * ps, k) - hdtodx1 * (LD(F1 + 2 * ps, k + 1) - LD(F1 + 2 * ps, k)) -
+                        hdtodx2 * (LD(F2 + 1 * ps, k + pitch) - LD(F2 + 1 * ps, k));
+      const double b1c = 0.5 * (b1h(k) + b1h(k + 1));
+      const double b2c = 0.5 * (b2h(k) + b2h(k + pitch));
+      slot(CF_ECH) = (b1c * m2 - b2c * m1) / dhalf;
+    }
+    compiler_fence();
+    if (r >= r0) {
+      // corner (r, i), lane - 1 for column i-1; the slot holds corner (r-1, i)'s
+      const double e00 = slot(CF_E), e01 = slot_at(CF_E, lp);
+      const double e10 = corner_value(CornerIn{
+          slot(CF_F1D), f1.d, slot(CF_F1BY), f1.by, slot_at(CF_F2 + 0, lm), slot(CF_F2 + 0),
+          slot_at(CF_F2 + 6, lm), slot(CF_F2 + 6), e_jmim, e_jm, slot_at(CF_ECH, lm),
+          slot(CF_ECH)});
+      compiler_fence();
+      slot(CF_E) = e10;
+      compiler_fence();
+      if (r > r0) {
+        const double e11 = slot_at(CF_E, lp);
+        const uint32_t kr = k - pitch;  // row r-1
+        const double b1n = LD(B1i, kr) - dtodx2 * (e10 - e00);
+        const double b1p = LD(B1i, kr + 1) - dtodx2 * (e11 - e01);
+        const double b2n = LD(B2i, kr) + dtodx1 * (e01 - e00);
+        const double b2p = LD(B2i, k) + dtodx1 * (e11 - e10);
+        if (fin) {
+          unsigned ix = 0, iy = 0;
+          if (edge) {
+            ix = ghost_images(i, g.is, g.ie, g.bc[0], g.bc[1], false);
+            iy = ghost_images(r - 1, g.js, g.je, g.bc[2], g.bc[3], false);
+          }
+          store_faces(g, out, r - 1, i, edge, ix, iy, b1n, b1p, b2n, b2p);
+          dti = dmax(dti, store_cell(g, clk, out, r - 1, i, edge, ix, iy, slot(CF_U + 0),
+                                     slot(CF_U + 1), slot(CF_U + 2), slot(CF_U + 3),
+                                     slot(CF_U + 4), slot(CF_U + 5), 0.5 * (b1n + b1p),
+                                     0.5 * (b2n + b2p)));
+        }
+      }
+    }
+    compiler_fence();
+    slot(CF_F1D) = f1.d;
+    slot(CF_F1BY) = f1.by;
+    // row r: the x1 part of the update; the upper face's flux is lane + 1's
+    slot(CF_U + 0) = f1.d; slot(CF_U + 1) = f1.mx; slot(CF_U + 2) = f1.my;
+    slot(CF_U + 3) = f1.mz; slot(CF_U + 4) = f1.e; slot(CF_U + 5) = f1.bz;
+    compiler_fence();
+    const double g0 = slot_at(CF_U + 0, lp), g1 = slot_at(CF_U + 1, lp);
+    const double g2 = slot_at(CF_U + 2, lp), g3 = slot_at(CF_U + 3, lp);
+    const double g4 = slot_at(CF_U + 4, lp), g5 = slot_at(CF_U + 5, lp);
+    compiler_fence();
+    slot(CF_U + 0) = LD(st + F_D * ps, k) - dtodx1 * (g0 - f1.d);
+    slot(CF_U + 1) = LD(st + F_M1 * ps, k) - dtodx1 * (g1 - f1.mx);
+    slot(CF_U + 2) = LD(st + F_M2 * ps, k) - dtodx1 * (g2 - f1.my);
+    slot(CF_U + 3) = LD(st + F_M3 * ps, k) - dtodx1 * (g3 - f1.mz);
+    slot(CF_U + 4) = LD(st + F_E * ps, k) - dtodx1 * (g4 - f1.e);
+    slot(CF_U + 5) = LD(st + F_B3C * ps, k) - dtodx1 * (g5 - f1.bz);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) dti = dmax(dti, __shfl_xor(dti, off, 64));
+  if (threadIdx.x == 0) atomic_max_pos(&clk->dti_slot[t % kDtSlots], dti);
 }
 
 // which = 0: fill the current state buffer; 1: fill the other one (the state
@@ -1386,6 +1642,19 @@ static bool merge_sweeps(const BatchLaunch& b) {
   return b.shape.persist <= 0 && b.shape.x2_kind == 1;
 }
 
+// Whether the HLLE instances take k_corr_final: with the shape settings whose work
+// it replaces at their defaults, where its marches give every CU eight waves
+// (1024^2, seven: 397 -> 399 us a step; 1200 x 1100, eight and a half: 501 -> 485)
+// and its 62-column strips leave at most a third of their lanes idle (400
+// grids of 128^2, 32% idle: 2.78 -> 2.70 ms).
+static bool corr_final(const BatchLaunch& b) {
+  const InstList& l = b.of_flux[kFluxHlle];
+  return merge_sweeps(b) && b.shape.fuse_corner == 1 && !b.thin && l.ninst &&
+         l.ntiles[K_CORR_FINAL] >= 8 * b.ncu &&
+         2.0 * l.ntiles[K_CORR_FINAL] * kCfCols * kCfRows <=
+             3.0 * l.ntiles[K_CORNER_C] * kTileX * kTileY;
+}
+
 static int grid_of(const BatchLaunch& b, const InstList& list, int kind, int per_cu) {
   const int n = list.ntiles[kind];
   if (b.shape.persist <= 0) return n;
@@ -1511,6 +1780,22 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         const int n = l.ntiles[K_CORR];
         hipLaunchKernelGGL(fn, dim3(2 * n), dim3(kTileX, ty), 0, s, l.insts, l.ninst, n,
                            b.shape.xcd_remap, b.shape.strip);
+      }
+      break;
+    }
+    case SK_FINISH: {
+      BatchLaunch rest = b;
+      if (corr_final(b)) {
+        const InstList& l = b.of_flux[kFluxHlle];
+        hipLaunchKernelGGL(k_corr_final, dim3(l.ntiles[K_CORR_FINAL]), dim3(64), 0, s, l.insts,
+                           l.ninst, l.ntiles[K_CORR_FINAL], b.shape.xcd_remap);
+        rest.all = rest.of_flux[kFluxRoe];
+        rest.of_flux[kFluxHlle] = InstList{};
+        if (!rest.all.ninst) break;
+      }
+      for (int q : {SK_CORR_BOTH, SK_CORNER_C, SK_FINAL_GHOST}) {
+        const hipError_t e = ATHMI_FN(launch)(&rest, q, s);
+        if (e != hipSuccess) return e;
       }
       break;
     }

@@ -80,7 +80,7 @@ struct Inst {
   size_t ps;          // plane stride in doubles
   Clock* clk;
   // first global tile of this instance for each kernel kind
-  int tile0[8];
+  int tile0[9];
 };
 
 // Tile kinds (one per kernel family); tile counts per instance come from
@@ -95,6 +95,7 @@ enum KernelKind {
   K_FINAL,        // cells [js,je] x [is,ie]
   K_GHOST,        // ghost cells of all planes
   K_INTERIOR,     // cells [js,je] x [is,ie]
+  K_CORR_FINAL,   // cells [js,je] x [is,ie] in strips of kCfCols columns, kCfRows rows each
   NKINDS
 };
 
@@ -107,6 +108,7 @@ constexpr int kX1Block = 128;
 constexpr int kX1Faces = kX1Block - 3;      // faces produced per x1 tile
 constexpr int kX2Block = 64;                // columns of a predictor-x2 tile
 constexpr int kTileX = 64, kTileY = 4;      // 2-D tiles of the cell/corner kernels
+constexpr int kCfCols = 62, kCfRows = 10;   // cells a corrector-and-final wave finishes
 constexpr int kGhostBlock = 256;
 
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -175,6 +177,7 @@ inline int tiles_of(int k, int nx1, int nx2, const LaunchShape& sh) {
     case K_CORNER_P: return cdiv((nx1 + 3) * (nx2 + 3), kTileX * kTileY);
     case K_CORNER_C: return cdiv((nx1 + 1) * (nx2 + 1), kTileX * kTileY);
     case K_FINAL: return cdiv(nx1, kTileX) * cdiv(nx2, final_rows_of(sh.final_rows));
+    case K_CORR_FINAL: return cdiv(nx1, kCfCols) * cdiv(nx2, kCfRows);
     case K_GHOST: return cdiv(8 * sx + (nx2 + 1) * 8, kGhostBlock);
     default: return cdiv(nx1, kTileX) * cdiv(nx2, kTileY);
   }
@@ -237,6 +240,8 @@ enum StepKernel {
   SK_PRED,            // both predictors, both corrector parts: one launch or two, by the
   SK_PRED_SAVE,       // batch's size
   SK_CORR_BOTH,
+  SK_FINISH,          // SK_CORR_BOTH, SK_CORNER_C and SK_FINAL_GHOST; one launch for the HLLE
+                      // instances of a large batch, which then write no corrector planes
   SK_FINAL_GHOST,     // SK_FINAL and SK_GHOST_NEXT: one launch where every ghost copies a
                       // non-ghost cell
   SK_CORNER_P_CARRY,  // SK_CORNER_P and SK_GHOST_CARRY, in one launch where both are launched

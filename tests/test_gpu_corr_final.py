@@ -1,0 +1,81 @@
+"""The HLLE march that holds the corrector, its corners and the final update:
+taken by batches whose marches (62 columns x 10 rows) give every CU eight waves.
+An ensemble past that line holds grids that end one cell short of, at and past
+a strip and a march, every boundary type and, in one of the two, Roe grids
+beside them; each is checked against the oracle. One large grid is checked
+against the separate launches of a persistent grid."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import OracleGrid, load_pkg
+from test_gpu_merged import desc, state
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [(61, 9), (62, 10), (63, 11), (124, 20), (125, 21), (123, 19), (4, 4), (187, 31), (70, 4),
+         (5, 40)]
+BCS = [(4, 4, 4, 4), (1, 2, 4, 4), (4, 4, 2, 1), (1, 1, 2, 2), (2, 1, 1, 2)]
+FILLER = (248, 40)  # 16 marches
+
+
+def cus():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+@pytest.mark.parametrize("roe", [0, 3])
+def test_ensemble_matches_oracle(roe):
+    pkg = load_pkg()
+    kinds = [(n, b, "hlle") for k, n in enumerate(EDGES) for b in (BCS[k % 5], BCS[(k + 2) % 5])]
+    kinds += [((66, 14), BCS[k], "roe") for k in range(roe)]
+    kinds.append((FILLER, BCS[1], "hlle"))
+    copies = 8 * cus() // 16 + 1
+    of = list(range(len(kinds) - 1)) + [len(kinds) - 1] * copies
+    descs = [desc(*kinds[q][0], kinds[q][2], kinds[q][1]) for q in of]
+    want = []
+    for q, ((nx, ny), bc, flux) in enumerate(kinds):
+        ora = OracleGrid(desc(nx, ny, flux, bc))
+        ora.put(*state(nx, ny, q))
+        ora.set_bvals()
+        ora.set_time(1e-3 / max(nx, ny), 0.0, 1)
+        for _ in range(3):
+            ora.step(1e30)
+        want.append((ora.get(), ora.clock()))
+    g = pkg.Grid(descs)
+    for k, q in enumerate(of):
+        g.upload(k, *state(*kinds[q][0], q))
+    g.set_bvals()
+    for k, q in enumerate(of):
+        g.set_clock(k, 1e-3 / max(kinds[q][0]), 0.0, 1)
+    g.set_limits(1e30, -1)
+    g.run(3)
+    for k, q in enumerate(of):
+        got = g.download(k)
+        for a, b in zip(got, want[q][0]):
+            assert np.array_equal(a, b), (k, kinds[q])
+        assert g.clock(k) == want[q][1], (k, kinds[q])
+    g.close()
+
+
+# fast: the two paths contract different multiplications into FMAs, a few
+# hundred roundings a step of at most 2^-53 of the largest term each
+@pytest.mark.parametrize("variant,tol", [("exact", 0.0), ("fast", 1e-11)])
+@pytest.mark.parametrize("nx,ny,bc", [(1301, 1001, (4, 4, 1, 2)), (1240, 1040, (2, 1, 4, 4))])
+def test_large_grid_matches_separate_launches(nx, ny, bc, variant, tol):
+    pkg = load_pkg()
+    d = desc(nx, ny, "hlle", bc)
+    s0 = state(nx, ny, nx)
+    outs = []
+    for persist in (0, 1):
+        g = pkg.Grid(d, variant=variant)
+        g.upload(0, *s0)
+        g.set_bvals()
+        g.set_clock(0, 1e-3 / max(nx, ny), 0.0, 1)
+        g.set_shape(3, persist)
+        g.set_limits(1e30, -1)
+        g.run(3)
+        outs.append((g.download(0), g.clock(0)))
+        g.close()
+    for a, b in zip(outs[0][0], outs[1][0]):
+        assert np.abs(a - b).max() <= tol * np.abs(b).max()
+    assert abs(outs[0][1][0] - outs[1][1][0]) <= tol * outs[1][1][0]
