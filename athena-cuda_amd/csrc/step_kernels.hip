@@ -1213,7 +1213,7 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
 }
 
 // ---------------------------------------------------------------------------
-// HLLE: the corrector, Step 9's corners and the final update in one march. A
+// The corrector, Step 9's corners and the final update in one march. A
 // wave takes 64 columns and walks down kCfRows rows. Per row r: the x2 flux at
 // face r (Steps 6, 8c), which finishes the update of row r-1's conserved
 // variables; the x1 flux of row r (Steps 5, 8b), which starts row r's; emf3 at
@@ -1223,18 +1223,23 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
 // emf and the corners, 15 planes that k_corr_both writes and k_final reads, never
 // reach memory. Lanes 1..62 finish cells; lanes 0 and 63 hold the neighbours'
 // corner inputs. A march repeats one x2 face row and one x1 row.
-// Bound by the 61 planes it reads and writes once: 4096^2 6.08 -> 5.36 ms a step
-// (this kernel 2.3 ms, 3.6 TB/s), 2048 x 1536 1.157 -> 1.076, 24 grids of 777 x 333
-// 2.34 -> 2.12. Rows: 8, 10, 12, 16 and 24 are within 3% at 4096^2 (more rows repeat
-// less) and 10 is the best at 1200^2 (fewer give more waves). Three waves per
-// SIMD: asked for four, the compiler keeps to 120 registers by issuing each plane's
-// loads behind the last one's use (4096^2 5.7-5.8 ms); with 148 they go out together.
-// Roe, at two waves per SIMD and with its parked values beside the slots, lost
-// (6.95 -> 7.02): it keeps the separate launches.
+// HLLE is bound by the 61 planes it reads and writes once: 4096^2 6.08 -> 5.36 ms a
+// step (this kernel 2.3 ms, 3.6 TB/s), 2048 x 1536 1.157 -> 1.076, 24 grids of
+// 777 x 333 2.34 -> 2.12. Roe, bound by its arithmetic at two waves per SIMD: 4096^2
+// 6.87 -> 6.40, 1240 x 3000 1.688 -> 1.505, 24 grids of 777 x 333 2.65 -> 2.53. Rows: 8,
+// 10, 12, 16 and 24 are within 3% at 4096^2 (more rows repeat less) and 10 is
+// the best at 1200^2 HLLE and 2048^2 Roe (fewer give more waves).
+// Waves per SIMD as a range, not a number: asked for exactly as many waves as fit,
+// or for four HLLE ones, the compiler issues each plane's loads behind
+// the last one's use to save registers (HLLE 5.7-6.4 ms, Roe 7.15); with the
+// lower end below that they go out together (148 and 250 registers).
 enum CfSlot { CF_U = 0, CF_F2 = 6, CF_F1D = 13, CF_F1BY, CF_ECH, CF_E, CF_SLOTS };
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 3)))
+constexpr int CF_PARK = 14;  // the Roe flux's parked values
+template <int FLUX>
+__global__ void __launch_bounds__(64)
+    __attribute__((amdgpu_waves_per_eu(FLUX == kFluxHlle ? 2 : 1, FLUX == kFluxHlle ? 3 : 2)))
 k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
-  __shared__ double lds[CF_SLOTS * 64];
+  __shared__ double lds[(CF_SLOTS + (FLUX == kFluxRoe ? CF_PARK : 0)) * 64];
   const int t = xcd_tile(blockIdx.x, ntiles, remap);
   const Inst& g = insts[find_inst(insts, ninst, K_CORR_FINAL, t)];
   Clock* clk = g.clk;
@@ -1280,6 +1285,7 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
     if (r >= r0) {
       const int lane = fresh_lane();
       const uint32_t k = cell_of(lane);
+      const LdsPark park{lds + CF_SLOTS * 64, 64, lane};
       auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
         compiler_fence();
         corrected_x2(src, k, L, R);
@@ -1291,7 +1297,7 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
       Prim7 wl, wr;
       double bx;
       build(L, R, wl, wr, bx);
-      const Cons7 f = riemann_of<kFluxHlle>(L, R, wl, wr, bx, eos, build);
+      const Cons7 f = riemann_of<FLUX>(L, R, wl, wr, bx, eos, build, park);
       compiler_fence();
       auto slot = [&](int q) -> double& { return lds[q * 64 + lane]; };
       if (r > r0) {
@@ -1313,6 +1319,7 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
     {
       const int lane = fresh_lane();
       const uint32_t k = cell_of(lane);
+      const LdsPark park{lds + CF_SLOTS * 64, 64, lane};
       auto build = [&](Cons7& L, Cons7& R, Prim7& wl, Prim7& wr, double& bx) {
         compiler_fence();
         corrected_x1(src, k, L, R);
@@ -1324,7 +1331,7 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
       Prim7 wl, wr;
       double bx;
       build(L, R, wl, wr, bx);
-      f1 = riemann_of<kFluxHlle>(L, R, wl, wr, bx, eos, build);
+      f1 = riemann_of<FLUX>(L, R, wl, wr, bx, eos, build, park);
     }
     phase_fence();
     const int lane = fresh_lane();
@@ -1642,17 +1649,21 @@ static bool merge_sweeps(const BatchLaunch& b) {
   return b.shape.persist <= 0 && b.shape.x2_kind == 1;
 }
 
-// Whether the HLLE instances take k_corr_final: with the shape settings whose work
-// it replaces at their defaults, where its marches give every CU eight waves
-// (1024^2, seven: 397 -> 399 us a step; 1200 x 1100, eight and a half: 501 -> 485)
-// and its 62-column strips leave at most a third of their lanes idle (400
-// grids of 128^2, 32% idle: 2.78 -> 2.70 ms).
-static bool corr_final(const BatchLaunch& b) {
-  const InstList& l = b.of_flux[kFluxHlle];
+// Whether the instances of solver f take k_corr_final: with the shape settings whose
+// work it replaces at their defaults, where its marches are enough waves per
+// CU and its 62-column strips leave few enough lanes idle. HLLE, eight waves: 1024^2
+// (seven) 397 -> 399 us a step, 1200 x 1100 (eight and a half) 501 -> 485; 400 grids of
+// 128^2 (32% idle) 2.78 -> 2.70 ms. Roe, 21 waves: 1200^2 (nine) 627 -> 696 us,
+// 2048 x 1536 (20.5) 1303 -> 1311, 2048 x 1800 (24) 1533 -> 1467; 400 grids of
+// 128^2 3.08 -> 3.28 ms, 100 of 200 x 300 (19% idle) 2.77 -> 2.72.
+static bool corr_final(const BatchLaunch& b, int f) {
+  const InstList& l = b.of_flux[f];
+  const int waves = f == kFluxHlle ? 8 : 21;
+  const double spare = f == kFluxHlle ? 1.5 : 1.3;  // lanes per cell
+  const double cells = (double)l.ntiles[K_CORNER_C] * kTileX * kTileY;
   return merge_sweeps(b) && b.shape.fuse_corner == 1 && !b.thin && l.ninst &&
-         l.ntiles[K_CORR_FINAL] >= 8 * b.ncu &&
-         2.0 * l.ntiles[K_CORR_FINAL] * kCfCols * kCfRows <=
-             3.0 * l.ntiles[K_CORNER_C] * kTileX * kTileY;
+         l.ntiles[K_CORR_FINAL] >= waves * b.ncu &&
+         (double)l.ntiles[K_CORR_FINAL] * kCfCols * kCfRows <= spare * cells;
 }
 
 static int grid_of(const BatchLaunch& b, const InstList& list, int kind, int per_cu) {
@@ -1783,22 +1794,6 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       }
       break;
     }
-    case SK_FINISH: {
-      BatchLaunch rest = b;
-      if (corr_final(b)) {
-        const InstList& l = b.of_flux[kFluxHlle];
-        hipLaunchKernelGGL(k_corr_final, dim3(l.ntiles[K_CORR_FINAL]), dim3(64), 0, s, l.insts,
-                           l.ninst, l.ntiles[K_CORR_FINAL], b.shape.xcd_remap);
-        rest.all = rest.of_flux[kFluxRoe];
-        rest.of_flux[kFluxHlle] = InstList{};
-        if (!rest.all.ninst) break;
-      }
-      for (int q : {SK_CORR_BOTH, SK_CORNER_C, SK_FINAL_GHOST}) {
-        const hipError_t e = ATHMI_FN(launch)(&rest, q, s);
-        if (e != hipSuccess) return e;
-      }
-      break;
-    }
     case SK_CORNER_C:
       // with the fused final kernel the corners are computed there
       if (b.shape.fuse_corner) break;
@@ -1855,6 +1850,24 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       hipLaunchKernelGGL(k_divb, dim3(grid_of(b, a, K_INTERIOR, 8)), b2, 0, s, a.insts, a.ninst,
                          a.ntiles[K_INTERIOR], b.shape.xcd_remap);
       break;
+    case SK_FINISH: {
+      BatchLaunch rest = b;
+      for (int f = 0; f < 2; f++) {
+        if (!corr_final(b, f)) continue;
+        const InstList& l = b.of_flux[f];
+        hipLaunchKernelGGL(f == kFluxHlle ? k_corr_final<kFluxHlle> : k_corr_final<kFluxRoe>,
+                           dim3(l.ntiles[K_CORR_FINAL]), dim3(64), 0, s, l.insts, l.ninst,
+                           l.ntiles[K_CORR_FINAL], b.shape.xcd_remap);
+        rest.all = rest.of_flux[1 - f];
+        rest.of_flux[f] = InstList{};
+      }
+      if (!rest.all.ninst) break;
+      for (int q : {SK_CORR_BOTH, SK_CORNER_C, SK_FINAL_GHOST}) {
+        const hipError_t e = ATHMI_FN(launch)(&rest, q, s);
+        if (e != hipSuccess) return e;
+      }
+      break;
+    }
     default:
       return hipErrorInvalidValue;
   }

@@ -240,8 +240,8 @@ enum StepKernel {
   SK_PRED,            // both predictors, both corrector parts: one launch or two, by the
   SK_PRED_SAVE,       // batch's size
   SK_CORR_BOTH,
-  SK_FINISH,          // SK_CORR_BOTH, SK_CORNER_C and SK_FINAL_GHOST; one launch for the HLLE
-                      // instances of a large batch, which then write no corrector planes
+  SK_FINISH,          // SK_CORR_BOTH, SK_CORNER_C and SK_FINAL_GHOST; one launch per solver on
+                      // large batches, which then writes no corrector planes
   SK_FINAL_GHOST,     // SK_FINAL and SK_GHOST_NEXT: one launch where every ghost copies a
                       // non-ghost cell
   SK_CORNER_P_CARRY,  // SK_CORNER_P and SK_GHOST_CARRY, in one launch where both are launched

@@ -1,9 +1,10 @@
-"""The HLLE march that holds the corrector, its corners and the final update:
-taken by batches whose marches (62 columns x 10 rows) give every CU eight waves.
-An ensemble past that line holds grids that end one cell short of, at and past
-a strip and a march, every boundary type and, in one of the two, Roe grids
-beside them; each is checked against the oracle. One large grid is checked
-against the separate launches of a persistent grid."""
+"""The march that holds the corrector, its corners and the final update: taken
+by the solver whose marches (62 columns x 10 rows) are enough waves per CU, 8
+with HLLE and 20 with Roe. An ensemble past that line holds grids that end one
+cell short of, at and past a strip and a march and every boundary type, with
+none, a few or as many grids of the other solver beside them; each is checked
+against the oracle. One large grid is checked against the separate launches
+of a persistent grid."""
 import numpy as np
 import pytest
 import torch
@@ -23,14 +24,20 @@ def cus():
     return torch.cuda.get_device_properties(0).multi_processor_count
 
 
-@pytest.mark.parametrize("roe", [0, 3])
-def test_ensemble_matches_oracle(roe):
+def copies_of(flux):
+    return (8 if flux == "hlle" else 21) * cus() // 16 + 1
+
+
+@pytest.mark.parametrize("main,few", [("hlle", 0), ("hlle", 3), ("hlle", 450), ("roe", 0),
+                                      ("roe", 3)])
+def test_ensemble_matches_oracle(main, few):
     pkg = load_pkg()
-    kinds = [(n, b, "hlle") for k, n in enumerate(EDGES) for b in (BCS[k % 5], BCS[(k + 2) % 5])]
-    kinds += [((66, 14), BCS[k], "roe") for k in range(roe)]
-    kinds.append((FILLER, BCS[1], "hlle"))
-    copies = 8 * cus() // 16 + 1
-    of = list(range(len(kinds) - 1)) + [len(kinds) - 1] * copies
+    other = "roe" if main == "hlle" else "hlle"
+    kinds = [(n, b, main) for k, n in enumerate(EDGES) for b in (BCS[k % 5], BCS[(k + 2) % 5])]
+    of = list(range(len(kinds))) + [len(kinds)] * copies_of(main)
+    kinds.append((FILLER, BCS[1], main))
+    of += [len(kinds)] * few
+    kinds.append(((248, 30), BCS[4], other))
     descs = [desc(*kinds[q][0], kinds[q][2], kinds[q][1]) for q in of]
     want = []
     for q, ((nx, ny), bc, flux) in enumerate(kinds):
@@ -60,10 +67,12 @@ def test_ensemble_matches_oracle(roe):
 # fast: the two paths contract different multiplications into FMAs, a few
 # hundred roundings a step of at most 2^-53 of the largest term each
 @pytest.mark.parametrize("variant,tol", [("exact", 0.0), ("fast", 1e-11)])
-@pytest.mark.parametrize("nx,ny,bc", [(1301, 1001, (4, 4, 1, 2)), (1240, 1040, (2, 1, 4, 4))])
-def test_large_grid_matches_separate_launches(nx, ny, bc, variant, tol):
+@pytest.mark.parametrize("nx,ny,flux,bc", [(1301, 1001, "hlle", (4, 4, 1, 2)),
+                                           (1240, 1040, "hlle", (2, 1, 4, 4)),
+                                           (1985, 1701, "roe", (1, 2, 4, 4))])
+def test_large_grid_matches_separate_launches(nx, ny, flux, bc, variant, tol):
     pkg = load_pkg()
-    d = desc(nx, ny, "hlle", bc)
+    d = desc(nx, ny, flux, bc)
     s0 = state(nx, ny, nx)
     outs = []
     for persist in (0, 1):
