@@ -118,10 +118,13 @@ struct athmi_grid {
       for (int k = 0; k < n; k++)
         if (flux < 0 || hinst[k].flux == flux) I[m++] = hinst[k];
       int* first = reinterpret_cast<int*>(I + m);
+      march_of(I, m, I[0].flux == ATHMI_FLUX_HLLE, bl.ncu, L);
+      LaunchShape shape = bl.shape;
+      shape.cf_rows = L.cf_rows;
       for (int k = 0; k < m; k++)
         for (int kind = 0; kind < NKINDS; kind++) {
           first[kind * m + k] = I[k].tile0[kind] = tot[kind];
-          tot[kind] += tiles_of(kind, I[k].nx1, I[k].nx2, bl.shape);
+          tot[kind] += tiles_of(kind, I[k].nx1, I[k].nx2, shape);
         }
       L.insts = reinterpret_cast<const Inst*>(base + used);
       L.ninst = m;

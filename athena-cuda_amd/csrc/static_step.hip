@@ -170,6 +170,7 @@ int athmi_integrate_static(const athmi_desc* desc, double dt, const double* stat
   bl.shape.xcd_remap = 1;
   bl.shape.corr_rows = 1;
   bl.shape.final_rows = 8;
+  bl.shape.cf_rows = 8;  // not launched here: the largest grid the scratch holds is too small
   bl.shape.x2_kind = 1;
   bl.shape.fuse_corner = 1;
   for (int kind = 0; kind < NKINDS; kind++) {

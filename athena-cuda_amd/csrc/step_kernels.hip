@@ -11,9 +11,11 @@
 //   k_corner<P>  Step 4 corner emf (and Step 3 emf3_cc comes from k_pred_x1)
 //   k_corr_both  Steps 4 (half-step face B), 5, 6, 7, 8b, 8c: the tiles of both
 //                parts of k_corr in one launch
-//   k_corner<C>  Step 9 corner emf
+//   k_corner<C>  Step 9 corner emf (fusion depth 0; else k_final computes it)
 //   k_final      Steps 9 (face B), 11a/11b, 13 and the new_dt max, fused
 //                and, from the source's side, set_bvals on the new state
+//   k_corr_final large batches: k_corr_both and k_final in one march, without the
+//                planes between them
 //   k_ghost      set_bvals by itself (a standalone call, grids under 4 cells)
 //   k_end        nstep++, time += dt, dt = min(2 dt, CourNo/max_dti), swap, and the
 //                limits and dt of the next step
@@ -1214,7 +1216,7 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
 
 // ---------------------------------------------------------------------------
 // The corrector, Step 9's corners and the final update in one march. A
-// wave takes 64 columns and walks down kCfRows rows. Per row r: the x2 flux at
+// wave takes 64 columns and walks down `rows` rows. Per row r: the x2 flux at
 // face r (Steps 6, 8c), which finishes the update of row r-1's conserved
 // variables; the x1 flux of row r (Steps 5, 8b), which starts row r's; emf3 at
 // t^{n+1/2} (Step 7); the corner emf of row r from the neighbour lanes; the face
@@ -1223,12 +1225,10 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
 // emf and the corners, 15 planes that k_corr_both writes and k_final reads, never
 // reach memory. Lanes 1..62 finish cells; lanes 0 and 63 hold the neighbours'
 // corner inputs. A march repeats one x2 face row and one x1 row.
-// HLLE is bound by the 61 planes it reads and writes once: 4096^2 6.08 -> 5.36 ms a
-// step (this kernel 2.3 ms, 3.6 TB/s), 2048 x 1536 1.157 -> 1.076, 24 grids of
+// HLLE is bound by the 61 planes it reads and writes once: 4096^2 6.08 -> 5.28 ms a
+// step (this kernel 2.2 ms, 3.7 TB/s), 2048 x 1536 1.152 -> 1.060, 24 grids of
 // 777 x 333 2.34 -> 2.12. Roe, bound by its arithmetic at two waves per SIMD: 4096^2
-// 6.87 -> 6.40, 1240 x 3000 1.688 -> 1.505, 24 grids of 777 x 333 2.65 -> 2.53. Rows: 8,
-// 10, 12, 16 and 24 are within 3% at 4096^2 (more rows repeat less) and 10 is
-// the best at 1200^2 HLLE and 2048^2 Roe (fewer give more waves).
+// 6.87 -> 6.27, 2048 x 1536 1.309 -> 1.248, 24 grids of 777 x 333 2.65 -> 2.53.
 // Waves per SIMD as a range, not a number: asked for exactly as many waves as fit,
 // or for four HLLE ones, the compiler issues each plane's loads behind
 // the last one's use to save registers (HLLE 5.7-6.4 ms, Roe 7.15); with the
@@ -1238,7 +1238,8 @@ constexpr int CF_PARK = 14;  // the Roe flux's parked values
 template <int FLUX>
 __global__ void __launch_bounds__(64)
     __attribute__((amdgpu_waves_per_eu(FLUX == kFluxHlle ? 2 : 1, FLUX == kFluxHlle ? 3 : 2)))
-k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
+k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap,
+                                                        int rows) {
   __shared__ double lds[(CF_SLOTS + (FLUX == kFluxRoe ? CF_PARK : 0)) * 64];
   const int t = xcd_tile(blockIdx.x, ntiles, remap);
   const Inst& g = insts[find_inst(insts, ninst, K_CORR_FINAL, t)];
@@ -1256,7 +1257,7 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
   const int sg = local / nstrip, s = local - sg * nstrip;
   const int gis = uni(g.is), gie = uni(g.ie), gje = uni(g.je);
   const int i0 = gis - 1 + s * kCfCols;
-  const int r0 = uni(g.js) + sg * kCfRows, r1 = min(r0 + kCfRows - 1, gje);
+  const int r0 = uni(g.js) + sg * rows, r1 = min(r0 + rows - 1, gje);
   const double dt = uni(clk->dts);
   const double dtodx1 = uni(dt / uni(g.dx1)), dtodx2 = uni(dt / uni(g.dx2));
   const double hdtodx1 = uni(0.5 * dtodx1), hdtodx2 = uni(0.5 * dtodx2);
@@ -1275,7 +1276,7 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap) {
   const double* F2 = sc + S_F2 * ps;
   auto b1h = [&](uint32_t kk) { return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk)); };
   auto b2h = [&](uint32_t kk) { return LD(B2i, kk) + hdtodx1 * (LD(emf, kk + 1) - LD(emf, kk)); };
-  const bool edge = near_edge(g, i0 + 1, kCfCols, r0, kCfRows);
+  const bool edge = near_edge(g, i0 + 1, kCfCols, r0, rows);
   double dti = 0.0;
 #pragma unroll 1
   for (int r = r0 - 1; r <= r1 + 1; r++) {
@@ -1649,21 +1650,11 @@ static bool merge_sweeps(const BatchLaunch& b) {
   return b.shape.persist <= 0 && b.shape.x2_kind == 1;
 }
 
-// Whether the instances of solver f take k_corr_final: with the shape settings whose
-// work it replaces at their defaults, where its marches are enough waves per
-// CU and its 62-column strips leave few enough lanes idle. HLLE, eight waves: 1024^2
-// (seven) 397 -> 399 us a step, 1200 x 1100 (eight and a half) 501 -> 485; 400 grids of
-// 128^2 (32% idle) 2.78 -> 2.70 ms. Roe, 21 waves: 1200^2 (nine) 627 -> 696 us,
-// 2048 x 1536 (20.5) 1303 -> 1311, 2048 x 1800 (24) 1533 -> 1467; 400 grids of
-// 128^2 3.08 -> 3.28 ms, 100 of 200 x 300 (19% idle) 2.77 -> 2.72.
+// Whether the instances of solver f take k_corr_final: where march_of found it worth
+// it, with the shape settings whose work it replaces at their defaults
 static bool corr_final(const BatchLaunch& b, int f) {
-  const InstList& l = b.of_flux[f];
-  const int waves = f == kFluxHlle ? 8 : 21;
-  const double spare = f == kFluxHlle ? 1.5 : 1.3;  // lanes per cell
-  const double cells = (double)l.ntiles[K_CORNER_C] * kTileX * kTileY;
-  return merge_sweeps(b) && b.shape.fuse_corner == 1 && !b.thin && l.ninst &&
-         l.ntiles[K_CORR_FINAL] >= waves * b.ncu &&
-         (double)l.ntiles[K_CORR_FINAL] * kCfCols * kCfRows <= spare * cells;
+  return merge_sweeps(b) && b.shape.fuse_corner == 1 && !b.thin && b.of_flux[f].ninst &&
+         b.of_flux[f].cf_worth;
 }
 
 static int grid_of(const BatchLaunch& b, const InstList& list, int kind, int per_cu) {
@@ -1857,7 +1848,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         const InstList& l = b.of_flux[f];
         hipLaunchKernelGGL(f == kFluxHlle ? k_corr_final<kFluxHlle> : k_corr_final<kFluxRoe>,
                            dim3(l.ntiles[K_CORR_FINAL]), dim3(64), 0, s, l.insts, l.ninst,
-                           l.ntiles[K_CORR_FINAL], b.shape.xcd_remap);
+                           l.ntiles[K_CORR_FINAL], b.shape.xcd_remap, l.cf_rows);
         rest.all = rest.of_flux[1 - f];
         rest.of_flux[f] = InstList{};
       }

@@ -95,7 +95,7 @@ enum KernelKind {
   K_FINAL,        // cells [js,je] x [is,ie]
   K_GHOST,        // ghost cells of all planes
   K_INTERIOR,     // cells [js,je] x [is,ie]
-  K_CORR_FINAL,   // cells [js,je] x [is,ie] in strips of kCfCols columns, kCfRows rows each
+  K_CORR_FINAL,   // cells [js,je] x [is,ie] in strips of kCfCols columns, cf_rows rows each
   NKINDS
 };
 
@@ -108,7 +108,7 @@ constexpr int kX1Block = 128;
 constexpr int kX1Faces = kX1Block - 3;      // faces produced per x1 tile
 constexpr int kX2Block = 64;                // columns of a predictor-x2 tile
 constexpr int kTileX = 64, kTileY = 4;      // 2-D tiles of the cell/corner kernels
-constexpr int kCfCols = 62, kCfRows = 10;   // cells a corrector-and-final wave finishes
+constexpr int kCfCols = 62;                 // columns a corrector-and-final wave finishes
 constexpr int kGhostBlock = 256;
 
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -148,6 +148,7 @@ struct LaunchShape {
   int strip;         // tile order of the corrector and final kernels: 0 = row by row,
                      // s > 0 = strips of s tile columns walked row by row
   int final_rows;    // rows of a final-update tile: 4, 8 or 16 (final_rows_of)
+  int cf_rows;       // rows a corrector-and-final wave marches (march_of, per list)
 };
 
 // Whether a grid's x2 tiles start on a cache line: whole chunks of 64 columns
@@ -177,7 +178,7 @@ inline int tiles_of(int k, int nx1, int nx2, const LaunchShape& sh) {
     case K_CORNER_P: return cdiv((nx1 + 3) * (nx2 + 3), kTileX * kTileY);
     case K_CORNER_C: return cdiv((nx1 + 1) * (nx2 + 1), kTileX * kTileY);
     case K_FINAL: return cdiv(nx1, kTileX) * cdiv(nx2, final_rows_of(sh.final_rows));
-    case K_CORR_FINAL: return cdiv(nx1, kCfCols) * cdiv(nx2, kCfRows);
+    case K_CORR_FINAL: return cdiv(nx1, kCfCols) * cdiv(nx2, sh.cf_rows);
     case K_GHOST: return cdiv(8 * sx + (nx2 + 1) * 8, kGhostBlock);
     default: return cdiv(nx1, kTileX) * cdiv(nx2, kTileY);
   }
@@ -190,7 +191,42 @@ struct InstList {
   const Inst* insts;
   int ninst;
   int ntiles[NKINDS];
+  int cf_rows;     // rows of a corrector-and-final march
+  bool cf_worth;   // whether it beats the separate launches (march_of)
 };
+
+// The corrector-and-final march of m instances of one solver on ncu CUs. A march
+// of r rows costs about r + 1 (it repeats one row's x1 fluxes and one x2 face row),
+// and waves_per_cu of them run at a time, so the rows are those with the least
+// rounds x (r + 1): a nearly empty last round costs as much as a full one (Roe
+// 2048 x 1536, two rounds of 13 rows 1248 us a step, of 20 rows 1370, three of 10
+// 1313; 1200^2, one round of 12 rows 609, two of 10 697).
+// It is worth it where enough of the lanes' rows in these rounds finish cells; the
+// fewer the rounds, the more, since all waves then load and compute in step. Roe:
+// 1024^2 (0.83 in one round) 462 -> 466 us, 1200^2 (0.87) 629 -> 609, 2048 x 1536 (0.89
+// in two) 1309 -> 1248, 4096^2 (0.92 in eight) 6.87 -> 6.27 ms, 100 grids of 200 x 300
+// (0.70 at 10 rows) 2.77 -> 2.72, 400 of 128^2 (0.60) 3.08 -> 3.28. HLLE: 768^2
+// (0.62 in one) 234 -> 244, 1024^2 (0.79) 396 -> 395, 1200^2 (0.84) 551 -> 513,
+// 2048 x 1536 (0.87) 1152 -> 1060, 4096^2 (0.93 in five) 6.09 -> 5.28 ms, 400 grids of
+// 128^2 (0.52 at 10 rows) 2.78 -> 2.70.
+inline void march_of(const Inst* insts, int m, bool hlle, int ncu, InstList& list) {
+  const long slots = (hlle ? 12L : 8L) * (ncu > 0 ? ncu : 1);
+  double cells = 0.0;
+  for (int k = 0; k < m; k++) cells += (double)insts[k].nx1 * insts[k].nx2;
+  long best = 0, rounds = 0;
+  for (int r = 4; r <= 24; r++) {
+    long t = 0;
+    for (int k = 0; k < m; k++) t += (long)cdiv(insts[k].nx1, kCfCols) * cdiv(insts[k].nx2, r);
+    const long n = (t + slots - 1) / slots;
+    if (r > 4 && n * (r + 1) >= best) continue;
+    best = n * (r + 1);
+    rounds = n;
+    list.cf_rows = r;
+  }
+  const double use = cells / ((double)best * slots * kCfCols);
+  list.cf_worth = use >= (hlle ? 0.55 + 0.25 / rounds : 0.70 + 0.14 / rounds);
+}
+
 inline size_t inst_list_bytes(size_t n) { return n * (sizeof(Inst) + sizeof(int) * NKINDS); }
 
 // Everything a launcher needs for one batch (the instances, the tuned shape
