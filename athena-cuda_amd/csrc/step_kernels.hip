@@ -621,6 +621,112 @@ __global__ void __launch_bounds__(kX1Block, 2) k_pred(const Inst* __restrict__ i
   }
 }
 
+// One x2 face per lane pair, for grids that leave most of the chip empty: a march
+// of one face is two PLMs one after the other (cells j-1 and j) and a flux, and
+// there its latency is the launch's. Here the workgroup's two waves take one cell
+// each, and the first then takes the face: 64^2 Roe 45.0 -> 40.3 us a step, 128 x 64 HLLE
+// 41.7 -> 37.6.
+template <bool SAVE, int FLUX>
+__device__ __forceinline__ void pred_x2_pair(const Inst* __restrict__ insts, int ninst, int t,
+                                             double* lds) {
+  const int lane = threadIdx.x % kX2Block;
+  const int w = uni((int)(threadIdx.x / kX2Block));
+  const Inst& g = insts[find_inst(insts, ninst, K_PRED_X2, t)];
+  const Clock* clk = g.clk;
+  if (!clk->active) return;
+  const int local = uni(t - g.tile0[K_PRED_X2]);
+  int sg, i;
+  const bool in = x2_lane(g, local, lane, 1, sg, i);
+  const double dx2 = uni(g.dx2);
+  const double dt = uni(clk->dts);
+  const double dtodx2 = dt / dx2;
+  const double hdt = 0.5 * dt;
+  const EosC eos{uni(g.gamma), uni(g.g1), uni(g.g2)};
+  const double* __restrict__ st = uni(g.state[clk->cur]);
+  double* __restrict__ sc = uni(g.scratch);
+  double* __restrict__ pw = uni(g.prims);
+  const size_t ps = (size_t)uni((int)g.ps);
+  const int pitch = uni(g.pitch);
+  // rows 0-2: the stencil of the wave's cell, 3: its state at the face
+  auto slots = (X2Slots*)(lds + w * kX2Lds);
+  auto aux = (double (*)[kX2Block])(lds + kX2Slots * 7 * kX2Block);  // the first wave's
+  auto put = [&](X2Slots* s, int q, const Prim7& v) {
+    s[q][0][lane] = v.d; s[q][1][lane] = v.vx; s[q][2][lane] = v.vy; s[q][3][lane] = v.vz;
+    s[q][4][lane] = v.p; s[q][5][lane] = v.by; s[q][6][lane] = v.bz;
+  };
+  auto get_of = [&](X2Slots* s, int q) -> Prim7 {
+    return Prim7{s[q][0][lane], s[q][1][lane], s[q][2][lane], s[q][3][lane],
+                 s[q][4][lane], s[q][5][lane], s[q][6][lane]};
+  };
+  auto get = [&](int q) -> Prim7 { return get_of(slots, q); };
+  typedef decltype(get) Getter;
+  struct Stencil {
+    const Getter* rd;
+    __device__ void get(Prim7& m, Prim7& z, Prim7& p) const {
+      m = (*rd)(0); z = (*rd)(1); p = (*rd)(2);
+    }
+    __device__ void fence() const { compiler_fence(); }
+  };
+  const uint32_t k = (uint32_t)((uni(g.js) - 1 + sg) * pitch + i);  // the face's
+  if (in) {
+    const uint32_t kc = k + (uint32_t)((w - 1) * pitch);  // the wave's cell
+    double v1 = 0.0, bn = 0.0, src = 0.0;
+    for (int q = 0; q < 3; q++) {
+      const uint32_t kr = kc + (uint32_t)((q - 1) * pitch);
+      const double d = LD(st + F_D * ps, kr), m1 = LD(st + F_M1 * ps, kr);
+      const Cons7 u{d, LD(st + F_M2 * ps, kr), LD(st + F_M3 * ps, kr), m1,
+                    LD(st + F_E * ps, kr), LD(st + F_B3C * ps, kr), LD(st + F_B1C * ps, kr)};
+      put(slots, q, cons_to_prim(u, LD(st + F_B2C * ps, kr), eos));
+      if (q == 1) {
+        v1 = m1 / d;
+        bn = LD(st + F_B2I * ps, kr);
+      }
+      if (q == 2) src = v1 * (LD(st + F_B2I * ps, kr) - bn) / dx2;
+    }
+    aux[w][lane] = src;
+    if (w == 1) aux[2][lane] = bn;
+    Prim7 wl, wr;
+    plm_cell_s(Stencil{&get}, LD(st + F_B2C * ps, kc), dtodx2, eos, wl, wr);
+    compiler_fence();
+    put(slots, 3, w == 0 ? wl : wr);
+  }
+  __syncthreads();
+  if (!in || w == 1) return;
+  auto build = [&](Cons7& ul, Cons7& ur, Prim7& wl, Prim7& wr, double& b0) {
+    compiler_fence();
+    wl = get_of((X2Slots*)lds, 3);
+    wr = get_of((X2Slots*)(lds + kX2Lds), 3);
+    b0 = aux[2][lane];
+    wl.bz = wl.bz + hdt * aux[0][lane];
+    wr.bz = wr.bz + hdt * aux[1][lane];
+    ul = prim_to_cons(wl, b0, eos);
+    ur = prim_to_cons(wr, b0, eos);
+  };
+  Cons7 ul, ur;
+  Prim7 wl, wr;
+  double b0;
+  build(ul, ur, wl, wr, b0);
+  if (SAVE) {
+    put7(pw + P_WL2 * ps, ps, k, wl);
+    put7(pw + P_WR2 * ps, ps, k, wr);
+  }
+  put7(sc + S_UL2 * ps, ps, k, ul);
+  put7(sc + S_UR2 * ps, ps, k, ur);
+  put7(sc + S_F2 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
+}
+template <bool SAVE, int FLUX>
+__global__ void __launch_bounds__(kX1Block, 2) k_pred_pair(const Inst* __restrict__ insts,
+                                                           int ninst, int n1, int n2, int remap) {
+  __shared__ double lds[kX2PerBlock * kX2Lds];
+  const int b = blockIdx.x;
+  if (b < n2) {
+    pred_x2_pair<SAVE, FLUX>(insts, ninst, xcd_tile(b, n2, remap), lds);
+  } else {
+    double (*const s)[kX1Block] = (double (*)[kX1Block])lds;
+    pred_x1_tile<SAVE, FLUX>(insts, ninst, xcd_tile(b - n2, n1, remap), s, s + 7, s + 14);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // integrate_emf3_corner (__integrate_2d__.c:632-702) at corner (j, i): the
 // x1-flux of B2 is -E3 and the x2-flux of B1 is +E3; each of the four edge
@@ -1226,7 +1332,7 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
 // reach memory. Lanes 1..62 finish cells; lanes 0 and 63 hold the neighbours'
 // corner inputs. A march repeats one x2 face row and one x1 row.
 // HLLE is bound by the 61 planes it reads and writes once: 4096^2 6.08 -> 5.28 ms a
-// step (this kernel 2.2 ms, 3.7 TB/s), 2048 x 1536 1.152 -> 1.060, 24 grids of
+// step (this kernel 2.56 ms, 3.2 TB/s), 2048 x 1536 1.152 -> 1.060, 24 grids of
 // 777 x 333 2.34 -> 2.12. Roe, bound by its arithmetic at two waves per SIMD: 4096^2
 // 6.87 -> 6.27, 2048 x 1536 1.309 -> 1.248, 24 grids of 777 x 333 2.65 -> 2.53.
 // Waves per SIMD as a range, not a number: asked for exactly as many waves as fit,
@@ -1728,6 +1834,18 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
                                            : (f == kFluxHlle ? k_pred<false, kFluxHlle, false>
                                                              : k_pred<false, kFluxRoe, false>);
         const int n1 = l.ntiles[K_PRED_X1], n2 = l.ntiles[K_PRED_X2];
+        // marches of one face that leave a quarter of the chip empty (Roe, us a step:
+        // 96 x 80, 0.8 workgroups per CU, 44.9 -> 40.8; 180 x 170, three, 53.4 -> 52.2;
+        // 200^2, four, 54.3 -> 54.6)
+        if (b.shape.x2_seg == 1 && n1 + n2 <= 3 * b.ncu) {
+          const auto pair = save ? (f == kFluxHlle ? k_pred_pair<true, kFluxHlle>
+                                                   : k_pred_pair<true, kFluxRoe>)
+                                 : (f == kFluxHlle ? k_pred_pair<false, kFluxHlle>
+                                                   : k_pred_pair<false, kFluxRoe>);
+          hipLaunchKernelGGL(pair, dim3(n1 + n2), dim3(kX1Block), 0, s, l.insts, l.ninst, n1, n2,
+                             b.shape.xcd_remap);
+          continue;
+        }
         const int nb2 = cdiv(n2, kX2PerBlock);
         hipLaunchKernelGGL(fn, dim3(n1 + nb2), dim3(kX1Block), 0, s, l.insts, l.ninst, n1, n2, nb2,
                            b.shape.x2_seg, b.shape.xcd_remap);
