@@ -161,7 +161,10 @@ int athmi_set_strip(athmi_grid *g, int tile_cols);
 int athmi_get_strip(const athmi_grid *g, int *tile_cols);
 /* Rows of a final-update tile (64 x rows cells: 4, 8 or 16; default 8): the
  * taller the tile, the smaller the share of its halo rows read twice.
- * Picked by the autotuner; results are identical. */
+ * Picked by the autotuner; results are identical. This, the strips and the
+ * corrector's tile height have no effect on a batch large enough for the
+ * corrector and the final update to be one kernel (persist 0, x2 form 1,
+ * fusion depth 1). */
 int athmi_set_final_rows(athmi_grid *g, int rows);
 int athmi_get_final_rows(const athmi_grid *g, int *rows);
 /* The current launch shape (any pointer may be NULL) */
@@ -185,7 +188,8 @@ int athmi_autotune(athmi_grid *g, int steps, int *x2_seg, int *persist, int *xcd
 /* Time nsteps main-loop steps kernel by kernel (HIP events on the handle's
  * stream between consecutive launches, no graph); avg_ms[k] receives the mean
  * duration of kernel k of the step (nslots >= 10), named by
- * athmi_step_kernel_name(k). No reference counterpart: measurement hook. */
+ * athmi_step_kernel_name(k): the step's separate kernels, also where athmi_step
+ * runs merged ones. No reference counterpart: measurement hook. */
 int athmi_profile_steps(athmi_grid *g, int nsteps, double *avg_ms, int nslots);
 const char *athmi_step_kernel_name(int k);
 /* Copy nbytes between two fresh device buffers reps times with a plain
