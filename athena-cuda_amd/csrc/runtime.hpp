@@ -57,8 +57,8 @@ namespace athmi_rt {
 // (a main-loop step is started by the k_end before it, or by SK_BEGIN_STEP
 // once the host has written the clock: athmi_grid::clock_written)
 const int kSeqStep[] = {SK_PRED, SK_CORNER_P, SK_FINISH, SK_END_STEP};
-const int kSeqIntegrate[] = {SK_BEGIN_ONCE, SK_PRED,  SK_CORNER_P_CARRY, SK_CORR_BOTH,
-                             SK_CORNER_C,   SK_FINAL, SK_END_ONCE};
+const int kSeqIntegrate[] = {SK_BEGIN_ONCE, SK_PRED, SK_CORNER_P_CARRY, SK_FINISH_BARE,
+                             SK_END_ONCE};
 // the step one kernel at a time, as athmi_profile_steps times it
 const int kSeqProfile[] = {SK_BEGIN_STEP, SK_PRED_X1, SK_PRED_X2, SK_CORNER_P,   SK_CORR,
                            SK_CORR2,      SK_CORNER_C, SK_FINAL,  SK_GHOST_NEXT, SK_END_STEP};

@@ -5,7 +5,8 @@
 // Pipeline of one step (all state in SoA planes, ping-pong buffers):
 //   k_begin      clock: limits, tlim clamp of dt, reset of dt partials (only when the
 //                host has written the clock: k_end starts the next step)
-//   k_pred       both sweeps' predictors in one launch: the tiles of
+//   k_pred       both sweeps' predictors in one launch (k_pred_pair: small grids): the
+//                tiles of
 //     k_pred_x1  Steps 1a-1e: x1 sweep, PLM via an LDS neighbour exchange
 //     k_pred_x2l Steps 2a-2e: x2 sweep, each lane marches down a column
 //   k_corner<P>  Step 4 corner emf (and Step 3 emf3_cc comes from k_pred_x1)
@@ -1345,7 +1346,7 @@ template <int FLUX>
 __global__ void __launch_bounds__(64)
     __attribute__((amdgpu_waves_per_eu(FLUX == kFluxHlle ? 2 : 1, FLUX == kFluxHlle ? 3 : 2)))
 k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap,
-                                                        int rows) {
+                                                        int rows, int fill) {
   __shared__ double lds[(CF_SLOTS + (FLUX == kFluxRoe ? CF_PARK : 0)) * 64];
   const int t = xcd_tile(blockIdx.x, ntiles, remap);
   const Inst& g = insts[find_inst(insts, ninst, K_CORR_FINAL, t)];
@@ -1382,7 +1383,7 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap,
   const double* F2 = sc + S_F2 * ps;
   auto b1h = [&](uint32_t kk) { return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk)); };
   auto b2h = [&](uint32_t kk) { return LD(B2i, kk) + hdtodx1 * (LD(emf, kk + 1) - LD(emf, kk)); };
-  const bool edge = near_edge(g, i0 + 1, kCfCols, r0, rows);
+  const bool edge = fill && near_edge(g, i0 + 1, kCfCols, r0, rows);
   double dti = 0.0;
 #pragma unroll 1
   for (int r = r0 - 1; r <= r1 + 1; r++) {
@@ -1959,19 +1960,22 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       hipLaunchKernelGGL(k_divb, dim3(grid_of(b, a, K_INTERIOR, 8)), b2, 0, s, a.insts, a.ninst,
                          a.ntiles[K_INTERIOR], b.shape.xcd_remap);
       break;
-    case SK_FINISH: {
+    case SK_FINISH:
+    case SK_FINISH_BARE: {
       BatchLaunch rest = b;
       for (int f = 0; f < 2; f++) {
         if (!corr_final(b, f)) continue;
         const InstList& l = b.of_flux[f];
         hipLaunchKernelGGL(f == kFluxHlle ? k_corr_final<kFluxHlle> : k_corr_final<kFluxRoe>,
                            dim3(l.ntiles[K_CORR_FINAL]), dim3(64), 0, s, l.insts, l.ninst,
-                           l.ntiles[K_CORR_FINAL], b.shape.xcd_remap, l.cf_rows);
+                           l.ntiles[K_CORR_FINAL], b.shape.xcd_remap, l.cf_rows,
+                           kernel == SK_FINISH);
         rest.all = rest.of_flux[1 - f];
         rest.of_flux[f] = InstList{};
       }
       if (!rest.all.ninst) break;
-      for (int q : {SK_CORR_BOTH, SK_CORNER_C, SK_FINAL_GHOST}) {
+      const int last = kernel == SK_FINISH ? SK_FINAL_GHOST : SK_FINAL;
+      for (int q : {(int)SK_CORR_BOTH, (int)SK_CORNER_C, last}) {
         const hipError_t e = ATHMI_FN(launch)(&rest, q, s);
         if (e != hipSuccess) return e;
       }

@@ -278,6 +278,7 @@ enum StepKernel {
   SK_CORR_BOTH,
   SK_FINISH,          // SK_CORR_BOTH, SK_CORNER_C and SK_FINAL_GHOST; one launch per solver on
                       // large batches, which then writes no corrector planes
+  SK_FINISH_BARE,     // the same without the ghosts (SK_FINAL)
   SK_FINAL_GHOST,     // SK_FINAL and SK_GHOST_NEXT: one launch where every ghost copies a
                       // non-ghost cell
   SK_CORNER_P_CARRY,  // SK_CORNER_P and SK_GHOST_CARRY, in one launch where both are launched

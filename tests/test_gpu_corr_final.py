@@ -81,3 +81,25 @@ def test_large_grid_matches_separate_launches(nx, ny, flux, bc, variant, tol):
     for a, b in zip(outs[0][0], outs[1][0]):
         assert np.abs(a - b).max() <= tol * np.abs(b).max()
     assert abs(outs[0][1][0] - outs[1][1][0]) <= tol * outs[1][1][0]
+
+
+# integrate_2d alone: the march leaves the ghosts as they were
+@pytest.mark.parametrize("nx,ny,flux,bc", [(1301, 1001, "hlle", (4, 4, 1, 2)),
+                                           (1985, 1701, "roe", (2, 1, 4, 4))])
+def test_large_grid_integrate_alone(nx, ny, flux, bc):
+    pkg = load_pkg()
+    d = desc(nx, ny, flux, bc)
+    s0 = state(nx, ny, nx)
+    outs = []
+    for persist in (0, 1):
+        g = pkg.Grid(d)
+        g.upload(0, *s0)
+        g.set_clock(0, 1e-3 / max(nx, ny), 0.0, 1)
+        g.set_shape(3, persist)
+        for _ in range(2):
+            g.integrate()
+        outs.append((g.download(0), g.clock(0)))
+        g.close()
+    for a, b in zip(outs[0][0], outs[1][0]):
+        assert np.array_equal(a, b)
+    assert outs[0][1] == outs[1][1]
