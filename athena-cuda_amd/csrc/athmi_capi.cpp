@@ -350,10 +350,14 @@ int athmi_step(athmi_grid* g) {
   if (!g) return fail(ATHMI_EINVAL, "null handle");
   g->clocks_change();
   // without the graph every step starts itself: its launches may be captured
-  // by the caller and replayed after the host has written the clock
-  if (g->clock_written || !g->use_graph) {
+  // by the caller and replayed after the host has written the clock. So does
+  // every step once the caller has captured any work of the handle: a replay of
+  // athmi_integrate leaves its own unconditional start in the clock, and a start
+  // launched into a capture has not run
+  const bool always = !g->use_graph || g->caller_captured;
+  if (g->clock_written || always) {
     HIP_TRY(g->launch(&g->bl, SK_BEGIN_STEP, g->stream));
-    g->clock_written = !g->use_graph;
+    g->clock_written = always;
   }
   if (!g->use_graph) return issue_step(g);
   if (!g->graph) {

@@ -96,7 +96,7 @@ struct athmi_grid {
   ClockHead* heads = nullptr;
   bool heads_valid = false;
   // the caller has captured work of this handle, which it may replay at any
-  // time: the heads are then fetched at every read
+  // time: the heads are then fetched at every read, and every step starts itself
   bool caller_captured = false;
   std::vector<std::vector<double>> cpaw_soln;  // initial cpaw2d states (8 planes)
   void* outbuf = nullptr;                      // device staging of the output formats
