@@ -113,7 +113,7 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
     return fail(ATHMI_EHIP, "athmi_create: clearing the state failed");
   }
   if (hipMalloc(&g->dclk, sizeof(Clock) * n) != hipSuccess ||
-      hipMalloc(&g->dinst, 2 * inst_list_bytes(n)) != hipSuccess) {
+      hipMalloc(&g->dinst, inst_lists_bytes(n)) != hipSuccess) {
     athmi_destroy(g);
     return fail(ATHMI_ENOMEM, "athmi_create: hipMalloc of the descriptors failed");
   }

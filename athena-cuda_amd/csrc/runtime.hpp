@@ -109,7 +109,7 @@ struct athmi_grid {
   // the device lists: every instance, and (a batch that mixes the solvers)
   // those of each solver, each with its own tile numbering
   int refresh_tiles() {
-    std::vector<unsigned char> img(2 * inst_list_bytes(n));
+    std::vector<unsigned char> img(inst_lists_bytes(n));
     unsigned char* base = reinterpret_cast<unsigned char*>(dinst);
     size_t used = 0;
     auto add = [&](InstList& L, int flux) {

@@ -227,7 +227,15 @@ inline void march_of(const Inst* insts, int m, bool hlle, int ncu, InstList& lis
   list.cf_worth = use >= (hlle ? 0.55 + 0.25 / rounds : 0.70 + 0.14 / rounds);
 }
 
-inline size_t inst_list_bytes(size_t n) { return n * (sizeof(Inst) + sizeof(int) * NKINDS); }
+// device bytes of a list of n instances, whole descriptors' alignment: the next
+// list starts behind it
+constexpr size_t inst_list_bytes(size_t n) {
+  return (n * (sizeof(Inst) + sizeof(int) * NKINDS) + alignof(Inst) - 1) / alignof(Inst) *
+         alignof(Inst);
+}
+// of the list of all n instances and the two solvers' lists, which share them
+// (two odd shares round up once more than their sum does)
+constexpr size_t inst_lists_bytes(size_t n) { return 2 * inst_list_bytes(n) + alignof(Inst); }
 
 // Everything a launcher needs for one batch (the instances, the tuned shape
 // and the CU count). The kernels that are compiled per Riemann solver take the
