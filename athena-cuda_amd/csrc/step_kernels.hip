@@ -174,9 +174,34 @@ __device__ __forceinline__ Cons7 get7(const double* base, size_t ps, uint32_t k)
                LD(base + 4 * ps, k), LD(base + 5 * ps, k), LD(base + 6 * ps, k)};
 }
 
+// The maximum of inverse time steps, leaving out those that are not a number (a
+// cell of a run told to go on after a non-finite state): the same whatever tile,
+// lane or march a cell falls in. dmax takes its second argument where either is
+// not a number, so a fold with it loses what came before such a cell.
+__device__ __forceinline__ double dti_max(double a, double b) { return fmax(a, b); }
+
+__device__ __forceinline__ double wave_dti_max(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = dti_max(v, __shfl_xor(v, off, 64));
+  return v;
+}
+
+// wave-level max with cross-lane shuffles, then across the block's waves via
+// LDS (red: one slot per wave)
+__device__ __forceinline__ double block_dti_max(double v, double* red) {
+  v = wave_dti_max(v);
+  const int tid = threadIdx.x + threadIdx.y * blockDim.x;
+  if ((tid & 63) == 0) red[tid >> 6] = v;
+  __syncthreads();
+  double m = red[0];
+  const int nw = (blockDim.x * blockDim.y) >> 6;
+  for (int w = 1; w < nw; w++) m = dti_max(m, red[w]);
+  __syncthreads();
+  return m;
+}
+
+// the same with dmax (max |div B|)
 __device__ __forceinline__ double block_max(double v, double* red) {
-  // wave-level max with cross-lane shuffles, then across the block's waves
-  // via LDS (red: one slot per wave)
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = dmax(v, __shfl_xor(v, off, 64));
   const int tid = threadIdx.x + threadIdx.y * blockDim.x;
@@ -1312,11 +1337,11 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
         M3 = M3 - dtodx2 * (LD(F2 + 2 * ps, kp) - LD(F2 + 2 * ps, k));
         E = E - dtodx2 * (LD(F2 + 4 * ps, kp) - LD(F2 + 4 * ps, k));
         B3c = B3c - dtodx2 * (LD(F2 + 5 * ps, kp) - LD(F2 + 5 * ps, k));
-        dti = store_cell(g, clk, out, j, i, edge, ix, iy, d, M1, M2, M3, E, B3c, 0.5 * (b1n + b1p),
-                         0.5 * (b2n + b2p));
+        dti = dti_max(dti, store_cell(g, clk, out, j, i, edge, ix, iy, d, M1, M2, M3, E, B3c,
+                                      0.5 * (b1n + b1p), 0.5 * (b2n + b2p)));
       }
     }
-    const double m = block_max(dti, red);
+    const double m = block_dti_max(dti, red);
     if (threadIdx.x == 0 && threadIdx.y == 0) atomic_max_pos(&clk->dti_slot[t % kDtSlots], m);
   }
 }
@@ -1488,10 +1513,10 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap,
             iy = ghost_images(r - 1, g.js, g.je, g.bc[2], g.bc[3], false);
           }
           store_faces(g, out, r - 1, i, edge, ix, iy, b1n, b1p, b2n, b2p);
-          dti = dmax(dti, store_cell(g, clk, out, r - 1, i, edge, ix, iy, slot(CF_U + 0),
-                                     slot(CF_U + 1), slot(CF_U + 2), slot(CF_U + 3),
-                                     slot(CF_U + 4), slot(CF_U + 5), 0.5 * (b1n + b1p),
-                                     0.5 * (b2n + b2p)));
+          dti = dti_max(dti, store_cell(g, clk, out, r - 1, i, edge, ix, iy, slot(CF_U + 0),
+                                        slot(CF_U + 1), slot(CF_U + 2), slot(CF_U + 3),
+                                        slot(CF_U + 4), slot(CF_U + 5), 0.5 * (b1n + b1p),
+                                        0.5 * (b2n + b2p)));
         }
       }
     }
@@ -1513,8 +1538,7 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap,
     slot(CF_U + 4) = LD(st + F_E * ps, k) - dtodx1 * (g4 - f1.e);
     slot(CF_U + 5) = LD(st + F_B3C * ps, k) - dtodx1 * (g5 - f1.bz);
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) dti = dmax(dti, __shfl_xor(dti, off, 64));
+  dti = wave_dti_max(dti);
   if (threadIdx.x == 0) atomic_max_pos(&clk->dti_slot[t % kDtSlots], dti);
 }
 
@@ -1607,7 +1631,7 @@ __global__ void __launch_bounds__(kDtSlots) k_begin(const Inst* __restrict__ ins
 __device__ __forceinline__ double reduce_slots(Clock* c, double* red) {
   const double m = __longlong_as_double((long long)c->dti_slot[threadIdx.x]);
   c->dti_slot[threadIdx.x] = 0ull;
-  return block_max(m, red);
+  return block_dti_max(m, red);
 }
 
 // mode 0 (end of a main-loop step, main.c:289-292 + new_dt.c:93-97):
@@ -1656,10 +1680,11 @@ __global__ void __launch_bounds__(kTileX* kTileY) k_dti(const Inst* __restrict__
       const double* st = g.state[clk->cur];
       const size_t ps = g.ps;
       const uint32_t k = (uint32_t)(j * g.pitch + i);
-      dti = inverse_dt(g, LD(st + F_D * ps, k), LD(st + F_M1 * ps, k), LD(st + F_M2 * ps, k),
-                       LD(st + F_M3 * ps, k), LD(st + F_E * ps, k));
+      dti = dti_max(dti, inverse_dt(g, LD(st + F_D * ps, k), LD(st + F_M1 * ps, k),
+                                    LD(st + F_M2 * ps, k), LD(st + F_M3 * ps, k),
+                                    LD(st + F_E * ps, k)));
     }
-    const double m = block_max(dti, red);
+    const double m = block_dti_max(dti, red);
     if (threadIdx.x == 0 && threadIdx.y == 0) atomic_max_pos(&clk->dti_slot[t % kDtSlots], m);
   }
 }

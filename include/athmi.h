@@ -110,7 +110,9 @@ int athmi_set_pause(athmi_grid *g, int inst, double t_next);
 
 /* set_bvals(Grid*, 0) (set_bvals.c:114) on every instance */
 int athmi_set_bvals(athmi_grid *g);
-/* new_dt(Grid*) (new_dt.c:25) on every instance; result in the clock's dt */
+/* new_dt(Grid*) (new_dt.c:25) on every instance; result in the clock's dt.
+ * Cells whose inverse time step is not a number (a run told to go on after a
+ * non-finite state) are left out, here and in the step. */
 int athmi_new_dt(athmi_grid *g);
 /* integrate_2d(Grid*) (__integrate_2d__.c:100) on every instance with its
  * clock's dt; the clock's time and nstep are left unchanged */
