@@ -117,10 +117,13 @@ int athmi_create(const athmi_desc* desc, int n, athmi_grid** out) {
     athmi_destroy(g);
     return fail(ATHMI_ENOMEM, "athmi_create: hipMalloc of the descriptors failed");
   }
-  if (hipHostMalloc(&g->heads, sizeof(ClockHead) * n, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&g->heads, sizeof(ClockHead) * n + sizeof(*g->set_done),
+                    hipHostMallocCoherent) != hipSuccess) {
     athmi_destroy(g);
     return fail(ATHMI_ENOMEM, "athmi_create: hipHostMalloc of the clocks failed");
   }
+  g->set_done = reinterpret_cast<unsigned long long*>(g->heads + n);
+  *g->set_done = 0;
   std::vector<Clock> hc(n);
   for (int k = 0; k < n; k++) {
     std::memset(&hc[k], 0, sizeof(Clock));

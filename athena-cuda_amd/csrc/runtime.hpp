@@ -4,9 +4,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "athmi.h"
@@ -44,9 +46,10 @@ hipError_t launch_state_unpack(const double* stage, double* st, size_t ps, int p
                                int sy, hipStream_t s);
 hipError_t launch_state_pack(const double* st, double* stage, size_t ps, int pitch, int sx,
                              int sy, hipStream_t s);
-// the clocks' heads -> host memory; one head -> the device
+// the clocks' heads -> host memory; one head -> the device, then `count` -> host memory
 hipError_t launch_clock_publish(const Clock* clk, ClockHead* heads, int n, hipStream_t s);
-hipError_t launch_clock_set(Clock* clk, const ClockHead& head, hipStream_t s);
+hipError_t launch_clock_set(Clock* clk, const ClockHead& head, unsigned long long* done,
+                            unsigned long long count, hipStream_t s);
 // dense [NSTATE][sy][sx] on the device <-> the planes of one state buffer
 hipError_t launch_state_dense(double* st, double* dense, size_t ps, int pitch, int sx, int sy,
                               int to_planes, hipStream_t s);
@@ -95,6 +98,9 @@ struct athmi_grid {
   // whether any work that changes them was queued since
   ClockHead* heads = nullptr;
   bool heads_valid = false;
+  // writes of clocks queued, and (behind the heads) how many have reached the device
+  unsigned long long set_count = 0;
+  unsigned long long* set_done = nullptr;
   // the caller has captured work of this handle, which it may replay at any
   // time: the heads are then fetched at every read, and every step starts itself
   bool caller_captured = false;
@@ -155,11 +161,16 @@ struct athmi_grid {
     heads_valid = false;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (!caller_captured && hipStreamIsCapturing(stream, &st) == hipSuccess &&
-        st != hipStreamCaptureStatusNone)
+        st != hipStreamCaptureStatusNone) {
+      wait_clock_set();
       caller_captured = true;
+    }
   }
-  // waits for the stream; the heads are then the device's
+  // waits for the stream, and for the null stream as a blocking copy would: the
+  // caller may have replayed captured work there, or written the state's planes.
+  // The heads are then the device's
   int fetch_clocks() {
+    HIP_TRY(hipStreamSynchronize(nullptr));
     if (!heads_valid || caller_captured) HIP_TRY(launch_clock_publish(dclk, heads, n, stream));
     HIP_TRY(hipStreamSynchronize(stream));
     heads_valid = true;
@@ -171,12 +182,25 @@ struct athmi_grid {
     std::memcpy(&c, &heads[k], sizeof(ClockHead));
     return ATHMI_OK;
   }
-  // after read_clock (which has waited for the stream) of the same instance
+  // after read_clock (which has waited for the stream) of the same instance.
+  // Work the caller has captured may be replayed on another stream next: it
+  // must find the clock written
   int write_clock_head(int k, const Clock& c) {
     clock_written = true;
     std::memcpy(&heads[k], &c, offsetof(Clock, divb_bits));
-    HIP_TRY(launch_clock_set(dclk + k, heads[k], stream));
+    HIP_TRY(launch_clock_set(dclk + k, heads[k], set_done, set_count + 1, stream));
+    set_count++;
+    if (caller_captured) HIP_TRY(hipStreamSynchronize(stream));
     return ATHMI_OK;
+  }
+  // until the last write has reached the device. For the first capture, which
+  // forbids a wait for its stream; the bound (far above a launch of one wave) keeps
+  // a lost device from holding the caller
+  void wait_clock_set() const {
+    const auto t0 = std::chrono::steady_clock::now();
+    while (__atomic_load_n(set_done, __ATOMIC_ACQUIRE) != set_count &&
+           std::chrono::steady_clock::now() - t0 < std::chrono::seconds(10))
+      std::this_thread::yield();
   }
 };
 

@@ -86,10 +86,17 @@ __global__ void __launch_bounds__(kXferBlock) k_clock_publish(const Clock* __res
   const int w = e - k * kHeadWords;
   heads[k].w[w] = reinterpret_cast<const unsigned long long*>(clk + k)[w];
 }
-__global__ void __launch_bounds__(64) k_clock_set(Clock* clk, ClockHead head) {
+// (the count of writes that have reached the device follows, for a host that
+// cannot wait for the stream)
+__global__ void __launch_bounds__(64) k_clock_set(Clock* clk, ClockHead head,
+                                                  unsigned long long* done,
+                                                  unsigned long long count) {
   // up to divb_bits, which only the device writes
   for (int w = threadIdx.x; w < (int)(offsetof(Clock, divb_bits) / 8); w += 64)
     reinterpret_cast<unsigned long long*>(clk)[w] = head.w[w];
+  __threadfence_system();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(done, count, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 unsigned blocks_for(size_t n) {
@@ -119,8 +126,9 @@ hipError_t launch_clock_publish(const Clock* clk, ClockHead* heads, int n, hipSt
   return hipGetLastError();
 }
 
-hipError_t launch_clock_set(Clock* clk, const ClockHead& head, hipStream_t s) {
-  hipLaunchKernelGGL(k_clock_set, dim3(1), dim3(64), 0, s, clk, head);
+hipError_t launch_clock_set(Clock* clk, const ClockHead& head, unsigned long long* done,
+                            unsigned long long count, hipStream_t s) {
+  hipLaunchKernelGGL(k_clock_set, dim3(1), dim3(64), 0, s, clk, head, done, count);
   return hipGetLastError();
 }
 
