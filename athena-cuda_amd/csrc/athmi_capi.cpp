@@ -351,7 +351,7 @@ static int issue_step(athmi_grid* g) {
 
 int athmi_step(athmi_grid* g) {
   if (!g) return fail(ATHMI_EINVAL, "null handle");
-  g->clocks_change();
+  const athmi_grid::ClockWork work(g);
   // without the graph every step starts itself: its launches may be captured
   // by the caller and replayed after the host has written the clock. So does
   // every step once the caller has captured any work of the handle: a replay of
@@ -364,6 +364,7 @@ int athmi_step(athmi_grid* g) {
   }
   if (!g->use_graph) return issue_step(g);
   if (!g->graph) {
+    std::lock_guard<std::mutex> lk(g->clk_mu);
     hipGraph_t graph;
     HIP_TRY(hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal));
     int rc = issue_step(g);
@@ -387,15 +388,18 @@ int athmi_run(athmi_grid* g, int max_steps, int* steps) {
   const int chunk = 16;
   while (max_steps < 0 || issued < max_steps) {
     // any instance still running?
-    const int rc = g->fetch_clocks();
-    if (rc) return rc;
     bool running = false;
-    for (int k = 0; k < g->n && !running; k++) {
-      Clock c;
-      std::memcpy(&c, &g->heads[k], sizeof(ClockHead));
-      if (c.time < c.tlim && (c.nlim < 0 || c.nstep < c.nlim) && c.time < c.tpause &&
-          (c.fail & c.fail_stop) == 0)
-        running = true;
+    {
+      std::lock_guard<std::mutex> lk(g->clk_mu);
+      const int rc = g->fetch_clocks();
+      if (rc) return rc;
+      for (int k = 0; k < g->n && !running; k++) {
+        Clock c;
+        std::memcpy(&c, &g->heads[k], sizeof(ClockHead));
+        if (c.time < c.tlim && (c.nlim < 0 || c.nstep < c.nlim) && c.time < c.tpause &&
+            (c.fail & c.fail_stop) == 0)
+          running = true;
+      }
     }
     if (!running) break;
     int m = chunk;
@@ -406,8 +410,11 @@ int athmi_run(athmi_grid* g, int max_steps, int* steps) {
     }
     issued += m;
   }
-  const int rc = g->fetch_clocks();
-  if (rc) return rc;
+  {
+    std::lock_guard<std::mutex> lk(g->clk_mu);
+    const int rc = g->fetch_clocks();
+    if (rc) return rc;
+  }
   if (steps) *steps = issued;
   return ATHMI_OK;
 }
@@ -430,7 +437,7 @@ int athmi_profile_steps(athmi_grid* g, int nsteps, double* avg_ms, int nslots) {
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
   for (int k = 0; k < kStepLen; k++) avg_ms[k] = 0.0;
   g->clock_written = true;
-  g->clocks_change();
+  const athmi_grid::ClockWork work(g);
   for (int s = 0; s < nsteps; s++) {
     HIP_TRY(hipEventRecord(ev[0], g->stream));
     for (int k = 0; k < kStepLen; k++) {
@@ -513,10 +520,10 @@ int athmi_autotune(athmi_grid* g, int steps, int* x2_seg, int* persist, int* xcd
                              hipMemcpyDeviceToDevice, g->stream));
       o += NSTATE * I.ps;
     }
+    const athmi_grid::ClockWork work(g);
     HIP_TRY(hipMemcpyAsync(g->dclk, hc.data(), sizeof(Clock) * g->n, hipMemcpyHostToDevice,
                            g->stream));
     g->clock_written = true;
-    g->heads_valid = false;
     HIP_TRY(hipStreamSynchronize(g->stream));
     return ATHMI_OK;
   };

@@ -4,9 +4,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -95,15 +97,20 @@ struct athmi_grid {
   hipGraphExec_t graph = nullptr;
   bool clock_written = true;  // the host wrote a clock since the last main-loop step
   // the clocks as the host last saw them (pinned memory the device writes), and
-  // whether any work that changes them was queued since
+  // how much work that changes them had been queued by then, of clock_work by now.
+  // clk_mu: the heads and the launches that read or write them, and the capture of
+  // the step graph (a launch beside it would be captured too); a thread may read
+  // the clocks while another steps
   ClockHead* heads = nullptr;
-  bool heads_valid = false;
+  unsigned long long heads_at = ~0ull;
+  std::atomic<unsigned long long> clock_work{0};
+  std::mutex clk_mu;
   // writes of clocks queued, and (behind the heads) how many have reached the device
   unsigned long long set_count = 0;
   unsigned long long* set_done = nullptr;
   // the caller has captured work of this handle, which it may replay at any
   // time: the heads are then fetched at every read, and every step starts itself
-  bool caller_captured = false;
+  std::atomic<bool> caller_captured{false};
   std::vector<std::vector<double>> cpaw_soln;  // initial cpaw2d states (8 planes)
   void* outbuf = nullptr;                      // device staging of the output formats
   size_t outbuf_bytes = 0;
@@ -156,27 +163,36 @@ struct athmi_grid {
     drop_graph();
     return ATHMI_OK;
   }
-  // before queueing work that changes the clocks
-  void clocks_change() {
-    heads_valid = false;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (!caller_captured && hipStreamIsCapturing(stream, &st) == hipSuccess &&
-        st != hipStreamCaptureStatusNone) {
-      wait_clock_set();
-      caller_captured = true;
+  // lives around the queueing of work that changes the clocks. The work counts
+  // once it is queued: a read that another thread began before then does not pass
+  // for one of after
+  struct ClockWork {
+    athmi_grid* g;
+    explicit ClockWork(athmi_grid* g) : g(g) {
+      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+      if (!g->caller_captured && hipStreamIsCapturing(g->stream, &st) == hipSuccess &&
+          st != hipStreamCaptureStatusNone) {
+        g->wait_clock_set();
+        g->caller_captured = true;
+      }
     }
-  }
+    ~ClockWork() { g->clock_work++; }
+    ClockWork(const ClockWork&) = delete;
+  };
   // waits for the stream, and for the null stream as a blocking copy would: the
   // caller may have replayed captured work there, or written the state's planes.
-  // The heads are then the device's
+  // The heads (whose mutex is held) are then the device's
   int fetch_clocks() {
     HIP_TRY(hipStreamSynchronize(nullptr));
-    if (!heads_valid || caller_captured) HIP_TRY(launch_clock_publish(dclk, heads, n, stream));
+    const unsigned long long work = clock_work;
+    if (heads_at != work || caller_captured)
+      HIP_TRY(launch_clock_publish(dclk, heads, n, stream));
     HIP_TRY(hipStreamSynchronize(stream));
-    heads_valid = true;
+    heads_at = work;
     return ATHMI_OK;
   }
   int read_clock(int k, Clock& c) {
+    std::lock_guard<std::mutex> lk(clk_mu);
     const int rc = fetch_clocks();
     if (rc) return rc;
     std::memcpy(&c, &heads[k], sizeof(ClockHead));
@@ -186,6 +202,7 @@ struct athmi_grid {
   // Work the caller has captured may be replayed on another stream next: it
   // must find the clock written
   int write_clock_head(int k, const Clock& c) {
+    std::lock_guard<std::mutex> lk(clk_mu);
     clock_written = true;
     std::memcpy(&heads[k], &c, offsetof(Clock, divb_bits));
     HIP_TRY(launch_clock_set(dclk + k, heads[k], set_done, set_count + 1, stream));
@@ -228,7 +245,7 @@ inline HostGeom geom_of(const athmi_grid* g, int inst) {
 }
 
 inline int issue_seq(athmi_grid* g, const int* seq, size_t n) {
-  g->clocks_change();
+  const athmi_grid::ClockWork work(g);
   for (size_t k = 0; k < n; k++) HIP_TRY(g->launch(&g->bl, seq[k], g->stream));
   return ATHMI_OK;
 }
