@@ -431,32 +431,63 @@ int athmi_divb_max(athmi_grid* g, int inst, double* out) {
 }
 
 int athmi_profile_steps(athmi_grid* g, int nsteps, double* avg_ms, int nslots) {
-  if (!g || !avg_ms || nsteps <= 0 || nslots < kStepLen)
+  if (!g || !avg_ms || nsteps <= 0 || nslots < NSEPARATE)
     return fail(ATHMI_EINVAL, "athmi_profile_steps: bad arguments");
-  std::vector<hipEvent_t> ev(kStepLen + 1);
-  for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
-  for (int k = 0; k < kStepLen; k++) avg_ms[k] = 0.0;
+  // an event after each launch; a step makes at most two per slot (one per solver)
+  struct Marks {
+    hipStream_t stream;
+    std::vector<hipEvent_t> ev;
+    std::vector<int> slot;  // of the launch before event k + 1
+    hipError_t err = hipSuccess;
+    ~Marks() {
+      for (hipEvent_t e : ev) (void)hipEventDestroy(e);
+    }
+    void record() {
+      if (err == hipSuccess && slot.size() == ev.size()) {
+        hipEvent_t e = nullptr;
+        err = hipEventCreate(&e);
+        if (err == hipSuccess) ev.push_back(e);
+      }
+      if (err == hipSuccess) err = hipEventRecord(ev[slot.size()], stream);
+    }
+    static void launched(void* self, int slot) {
+      Marks* m = static_cast<Marks*>(self);
+      m->slot.push_back(slot);
+      m->record();
+    }
+  } marks;
+  marks.stream = g->stream;
+  BatchLaunch bl = g->bl;
+  bl.launched = Marks::launched;
+  bl.launched_arg = &marks;
+  // the step's own launches, or (a caller without their slots) the separate kernels
+  const bool own = nslots >= NSLOTS;
+  const int shown = own ? NSLOTS : NSEPARATE;
+  for (int k = 0; k < shown; k++) avg_ms[k] = 0.0;
   g->clock_written = true;
   const athmi_grid::ClockWork work(g);
   for (int s = 0; s < nsteps; s++) {
-    HIP_TRY(hipEventRecord(ev[0], g->stream));
-    for (int k = 0; k < kStepLen; k++) {
-      HIP_TRY(g->launch(&g->bl, kSeqProfile[k], g->stream));
-      HIP_TRY(hipEventRecord(ev[k + 1], g->stream));
+    marks.slot.clear();
+    marks.record();
+    if (own) {
+      if (s == 0) HIP_TRY(g->launch(&bl, SK_BEGIN_STEP, g->stream));
+      for (int k : kSeqStep) HIP_TRY(g->launch(&bl, k, g->stream));
+    } else {
+      for (int k : kSeqProfile) HIP_TRY(g->launch(&bl, k, g->stream));
     }
-    HIP_TRY(hipEventSynchronize(ev[kStepLen]));
-    for (int k = 0; k < kStepLen; k++) {
+    HIP_TRY(marks.err);
+    HIP_TRY(hipEventSynchronize(marks.ev[marks.slot.size()]));
+    for (size_t k = 0; k < marks.slot.size(); k++) {
       float ms = 0.f;
-      HIP_TRY(hipEventElapsedTime(&ms, ev[k], ev[k + 1]));
-      avg_ms[k] += ms / nsteps;
+      HIP_TRY(hipEventElapsedTime(&ms, marks.ev[k], marks.ev[k + 1]));
+      avg_ms[marks.slot[k]] += ms / nsteps;
     }
   }
-  for (auto& e : ev) (void)hipEventDestroy(e);
   return ATHMI_OK;
 }
 
 const char* athmi_step_kernel_name(int k) {
-  return (k >= 0 && k < kStepLen) ? kStepNames[k] : "";
+  return (k >= 0 && k < NSLOTS) ? kStepNames[k] : "";
 }
 
 int athmi_set_stream(athmi_grid* g, void* s) {

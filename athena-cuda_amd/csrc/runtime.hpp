@@ -64,15 +64,17 @@ namespace athmi_rt {
 const int kSeqStep[] = {SK_PRED, SK_CORNER_P, SK_FINISH, SK_END_STEP};
 const int kSeqIntegrate[] = {SK_BEGIN_ONCE, SK_PRED, SK_CORNER_P_CARRY, SK_FINISH_BARE,
                              SK_END_ONCE};
-// the step one kernel at a time, as athmi_profile_steps times it
+// the step as its separate kernels
 const int kSeqProfile[] = {SK_BEGIN_STEP, SK_PRED_X1, SK_PRED_X2, SK_CORNER_P,   SK_CORR,
                            SK_CORR2,      SK_CORNER_C, SK_FINAL,  SK_GHOST_NEXT, SK_END_STEP};
 const int kSeqNewDt[] = {SK_CLEAR, SK_DTI, SK_DT_FINAL};
 const int kSeqDivb[] = {SK_CLEAR, SK_DIVB};
-const char* const kStepNames[] = {"k_begin",   "k_pred_x1",      "k_pred_x2", "k_corner<pred>",
-                                  "k_corr<1>", "k_corr<2>",      "k_corner<corr>", "k_final",
-                                  "k_ghost",   "k_end"};
-constexpr int kStepLen = sizeof(kSeqProfile) / sizeof(int);
+const char* const kStepNames[] = {"k_begin",   "k_pred_x1",   "k_pred_x2",      "k_corner<pred>",
+                                  "k_corr<1>", "k_corr<2>",   "k_corner<corr>", "k_final",
+                                  "k_ghost",   "k_end",       "k_pred",         "k_pred_pair",
+                                  "k_corr_both", "k_corr_final"};
+static_assert(sizeof(kSeqProfile) / sizeof(int) == NSEPARATE, "a slot per separate kernel");
+static_assert(sizeof(kStepNames) / sizeof(*kStepNames) == NSLOTS, "a name per slot");
 
 inline size_t round_up(size_t a, size_t b) { return (a + b - 1) / b * b; }
 

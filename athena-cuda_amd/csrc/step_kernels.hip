@@ -1812,12 +1812,16 @@ extern "C" {
 hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
   const BatchLaunch& b = *static_cast<const BatchLaunch*>(bl);
   const InstList& a = b.all;
+  auto launched = [&](int slot) {
+    if (b.launched) b.launched(b.launched_arg, slot);
+  };
   const dim3 b2(kTileX, kTileY);
   switch (kernel) {
     case SK_BEGIN_STEP:
     case SK_BEGIN_ONCE:
       hipLaunchKernelGGL(k_begin, dim3(a.ninst), dim3(kDtSlots), 0, s, a.insts,
                          kernel == SK_BEGIN_STEP ? 0 : 1);
+      launched(SLOT_BEGIN);
       break;
     case SK_PRED_X1:
     case SK_PRED_X1_SAVE:
@@ -1827,6 +1831,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         const PredX1Kernel fn = pred_x1_kernel(kernel == SK_PRED_X1_SAVE, f);
         hipLaunchKernelGGL(fn, dim3(grid_of(b, l, K_PRED_X1, kX1PerCu)), dim3(kX1Block), 0, s,
                            l.insts, l.ninst, l.ntiles[K_PRED_X1], b.shape.xcd_remap);
+        launched(SLOT_PRED_X1);
       }
       break;
     case SK_PRED_X2:
@@ -1839,6 +1844,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         hipLaunchKernelGGL(fn, dim3(grid_of(b, l, K_PRED_X2, kind == 1 ? 8 : 16)), dim3(kX2Block),
                            0, s, l.insts,
                            l.ninst, l.ntiles[K_PRED_X2], b.shape.x2_seg, b.shape.xcd_remap);
+        launched(SLOT_PRED_X2);
       }
       break;
     case SK_PRED:
@@ -1870,11 +1876,13 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
                                                    : k_pred_pair<false, kFluxRoe>);
           hipLaunchKernelGGL(pair, dim3(n1 + n2), dim3(kX1Block), 0, s, l.insts, l.ninst, n1, n2,
                              b.shape.xcd_remap);
+          launched(SLOT_PRED_PAIR);
           continue;
         }
         const int nb2 = cdiv(n2, kX2PerBlock);
         hipLaunchKernelGGL(fn, dim3(n1 + nb2), dim3(kX1Block), 0, s, l.insts, l.ninst, n1, n2, nb2,
                            b.shape.x2_seg, b.shape.xcd_remap);
+        launched(SLOT_PRED);
       }
       break;
     }
@@ -1883,6 +1891,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       if (b.shape.fuse_corner >= 2) break;
       hipLaunchKernelGGL(k_corner<true>, dim3(grid_of(b, a, K_CORNER_P, 8)), b2, 0, s, a.insts,
                          a.ninst, a.ntiles[K_CORNER_P], b.shape.xcd_remap, 0);
+      launched(SLOT_CORNER_P);
       break;
     case SK_CORNER_P_CARRY:
       if (b.shape.fuse_corner >= 2) return ATHMI_FN(launch)(bl, SK_GHOST_CARRY, s);
@@ -1904,6 +1913,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         hipLaunchKernelGGL(fn, dim3(grid_of(b, l, K_CORR, 4 * (kTileY / ty))), blk, 0, s,
                            l.insts, l.ninst, l.ntiles[K_CORR],
                            b.shape.xcd_remap, b.shape.strip);
+        launched(x1 ? SLOT_CORR1 : SLOT_CORR2);
       }
       break;
     }
@@ -1926,6 +1936,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
         const int n = l.ntiles[K_CORR];
         hipLaunchKernelGGL(fn, dim3(2 * n), dim3(kTileX, ty), 0, s, l.insts, l.ninst, n,
                            b.shape.xcd_remap, b.shape.strip);
+        launched(SLOT_CORR_BOTH);
       }
       break;
     }
@@ -1934,6 +1945,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       if (b.shape.fuse_corner) break;
       hipLaunchKernelGGL(k_corner<false>, dim3(grid_of(b, a, K_CORNER_C, 8)), b2, 0, s, a.insts,
                          a.ninst, a.ntiles[K_CORNER_C], b.shape.xcd_remap, 0);
+      launched(SLOT_CORNER_C);
       break;
     case SK_FINAL:
     case SK_FINAL_GHOST: {
@@ -1950,6 +1962,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
                                        : (f ? k_final<true, 4> : k_final<false, 4>);
       hipLaunchKernelGGL(fn, dim3(grid_of(b, a, K_FINAL, 32 / ty)), dim3(kTileX, ty), 0, s, a.insts,
                          a.ninst, a.ntiles[K_FINAL], b.shape.xcd_remap, b.shape.strip, fill);
+      launched(SLOT_FINAL);
       break;
     }
     case SK_GHOST_CUR:
@@ -1964,12 +1977,14 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       hipLaunchKernelGGL(k_ghost, dim3(grid_of(b, a, K_GHOST, 8)), dim3(kGhostBlock), 0, s, a.insts,
                          a.ninst, a.ntiles[K_GHOST], which, kernel == SK_GHOST_NEXT ? 1 : 0,
                          b.shape.xcd_remap);
+      launched(SLOT_GHOST);
       break;
     }
     case SK_END_STEP:
     case SK_END_ONCE:
       hipLaunchKernelGGL(k_end, dim3(a.ninst), dim3(kDtSlots), 0, s, a.insts,
                          kernel == SK_END_STEP ? 0 : 1);
+      launched(SLOT_END);
       break;
     case SK_CLEAR:
       hipLaunchKernelGGL(k_clear_slots, dim3(a.ninst), dim3(256), 0, s, a.insts);
@@ -1995,6 +2010,7 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
                            dim3(l.ntiles[K_CORR_FINAL]), dim3(64), 0, s, l.insts, l.ninst,
                            l.ntiles[K_CORR_FINAL], b.shape.xcd_remap, l.cf_rows,
                            kernel == SK_FINISH);
+        launched(SLOT_CORR_FINAL);
         rest.all = rest.of_flux[1 - f];
         rest.of_flux[f] = InstList{};
       }

@@ -251,12 +251,25 @@ struct BatchLaunch {
   bool outgrows_cache;
   LaunchShape shape;
   int ncu;
+  // called (if set) after every launch of a step's kernel, with its StepSlot
+  void (*launched)(void* arg, int slot) = nullptr;
+  void* launched_arg = nullptr;
   // a batch of one: its only list, read through descriptor `ins`
   void single(const Inst* ins, int flux) {
     all.insts = ins;
     of_flux[flux] = all;
     of_flux[1 - flux] = InstList{};
   }
+};
+
+// Kernels of a main-loop step, as athmi_profile_steps numbers them: the separate
+// kernels, then those that hold several stages
+enum StepSlot {
+  SLOT_BEGIN = 0, SLOT_PRED_X1, SLOT_PRED_X2, SLOT_CORNER_P, SLOT_CORR1, SLOT_CORR2, SLOT_CORNER_C,
+  SLOT_FINAL, SLOT_GHOST, SLOT_END,
+  NSEPARATE,
+  SLOT_PRED = NSEPARATE, SLOT_PRED_PAIR, SLOT_CORR_BOTH, SLOT_CORR_FINAL,
+  NSLOTS
 };
 
 // Kernels of the pipeline, launched one at a time by athmi_<variant>_launch

@@ -10,8 +10,8 @@ periodic, Roe flux, PLM, CFL 0.4, FP64, state resident in HBM. The exact
 bar against the reference CPU integrator.
 
 Prints one JSON line with the metric, a roofline object for the dominant kernel
-(the step's algorithmic bytes, 168 B per cell-update, over that kernel's
-HIP-event duration in a kernel-by-kernel pass; its own plane I/O, scratch
+of the step as it is launched (the step's algorithmic bytes, 168 B per
+cell-update, over that kernel's HIP-event duration in a kernel-by-kernel pass; its own plane I/O, scratch
 included, under separate keys), the step-level roofline at 168 algorithmic
 bytes per cell-update, the FP64 work rate, the CPU baseline
 (the reference's own CPU integrator timed on this host on a bounded sample),
@@ -52,6 +52,13 @@ KERNEL_IO = {
     "k_ghost": (11, 11, lambda a, b: 8 * (a + 8) + 8 * (b + 1)),
     "k_begin": (0, 0, lambda a, b: 1),
     "k_end": (0, 0, lambda a, b: 1),
+    # both predictors: U, B1i, B2i -> two times Ul,Ur,F (21), emf3_cc
+    "k_pred": (10, 43, lambda a, b: (a + 5) * (b + 4)),
+    "k_pred_pair": (10, 43, lambda a, b: (a + 5) * (b + 4)),
+    # both correctors: 4 face states (28), 6 components of each flux, U but E, B1i, B2i, emf
+    "k_corr_both": (50, 15, lambda a, b: (a + 3) * (b + 3)),
+    # and the final update, with E as well -> U, B
+    "k_corr_final": (51, 11, lambda a, b: (a + 3) * (b + 3)),
 }
 
 
@@ -426,8 +433,7 @@ def main():
     # kernel-by-kernel pass with HIP events on the handle's stream
     avg = (ctypes.c_double * 16)()
     pkg._check(L.athmi_profile_steps(g._h, args.profile_steps, avg, 16), "profile")
-    kern = {L.athmi_step_kernel_name(k).decode(): avg[k] for k in range(16)
-            if L.athmi_step_kernel_name(k)}
+    kern = {L.athmi_step_kernel_name(k).decode(): avg[k] for k in range(16) if avg[k] > 0.0}
     dom = max(kern, key=kern.get)
     # the metric's algorithmic bytes (168 B per cell-update: the state read
     # once and written once) over one launch of the dominant kernel: the whole

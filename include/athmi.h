@@ -189,9 +189,11 @@ int athmi_autotune(athmi_grid *g, int steps, int *x2_seg, int *persist, int *xcd
                    double *ms_per_step);
 /* Time nsteps main-loop steps kernel by kernel (HIP events on the handle's
  * stream between consecutive launches, no graph); avg_ms[k] receives the mean
- * duration of kernel k of the step (nslots >= 10), named by
- * athmi_step_kernel_name(k): the step's separate kernels, also where athmi_step
- * runs merged ones. No reference counterpart: measurement hook. */
+ * duration per step of kernel k, named by athmi_step_kernel_name(k) ("" past the
+ * last). With nslots >= 14 the step runs as athmi_step launches it, and a kernel
+ * it does not launch has 0; with 10 to 13 it runs as the ten separate kernels,
+ * also where athmi_step runs merged ones. No reference counterpart: measurement
+ * hook. */
 int athmi_profile_steps(athmi_grid *g, int nsteps, double *avg_ms, int nslots);
 const char *athmi_step_kernel_name(int k);
 /* Copy nbytes between two fresh device buffers reps times with a plain
