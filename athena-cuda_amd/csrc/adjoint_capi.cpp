@@ -86,8 +86,8 @@ struct athmi_adjoint {
 static int issue_on(athmi_adjoint* h, const Inst* ins, const int* seq, size_t n) {
   BatchLaunch bl = h->g->bl;
   bl.single(ins, h->g->hinst[0].flux);
-  const athmi_grid::ClockWork work(h->g);
   for (size_t k = 0; k < n; k++) HIP_TRY(h->g->launch(&bl, seq[k], h->g->stream));
+  h->g->clock_work++;  // the handle is the adjoint's own: no caller captures its work
   return ATHMI_OK;
 }
 

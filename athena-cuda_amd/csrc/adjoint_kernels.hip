@@ -23,9 +23,12 @@
 // sequence of cells: at 512^2 whole 64-wide tiles left a tenth of the lanes idle.
 // Nonlinear stages recompute their forward values with the reference's
 // evaluation order (this file is built with -ffp-contract=off, like the exact
-// forward kernels), so every branch is the one the forward pass took. Linear
-// stages scatter with FP64 atomic adds; a value reached through several
-// stencil paths is summed in an unspecified order (roundoff-level).
+// forward kernels), so every branch is the one the forward pass took. The adjoint
+// of the input state takes FP64 atomic adds where several threads of one launch
+// reach a cell: from the predictor faces' sources and Step 3, and from the two
+// sweeps' cons->prim. Their order, and so the last bits, vary from run to run; the
+// deterministic reverse stores the faces' terms, gathers them in order and runs
+// the two sweeps' gathers one after the other.
 #include <hip/hip_runtime.h>
 
 #include "adjoint_device.hpp"
@@ -219,7 +222,8 @@ __global__ void __launch_bounds__(kCells) ak_update(AdjArgs a) {
   a.ain[F_B1I * ps + k] = b1t(j, i);
   a.ain[F_B2I * ps + k] = b2t(j, i);
   if (j < g.js || i < g.is) return;
-  a.ab[A_EMFC * ps + k] = dtodx2 * (b1t(j, i) - b1t(j - 1, i)) + dtodx1 * (b2t(j, i - 1) - b2t(j, i));
+  a.ab[A_EMFC * ps + k] =
+      dtodx2 * (b1t(j, i) - b1t(j - 1, i)) + dtodx1 * (b2t(j, i - 1) - b2t(j, i));
 }
 
 // ---------------------------------------------------------------------------

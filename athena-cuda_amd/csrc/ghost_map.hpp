@@ -125,22 +125,6 @@ __device__ __forceinline__ constexpr bool ghost_negates(int f, bool nx, bool ny)
   return (f == F_M1 && nx) || (f == F_M2 && ny);
 }
 
-// the map of plane f
-__device__ __forceinline__ bool ghost_src(const Inst& g, int f, int j, int i, int& sj, int& si,
-                                          bool& neg, bool& stale) {
-  bool nx, ny;
-  const bool ghost = ghost_chase(g, ghost_class(f), j, i, sj, si, nx, ny, stale);
-  neg = ghost_negates(f, nx, ny);
-  return ghost;
-}
-
-// the map for grids of Nx1, Nx2 >= 4, where no source is stale
-__device__ __forceinline__ bool ghost_src(const Inst& g, int f, int j, int i, int& sj, int& si,
-                                          bool& neg) {
-  bool stale;
-  return ghost_src(g, f, j, i, sj, si, neg, stale);
-}
-
 // The same map from the source's side, for Nx1, Nx2 >= 4 (every ghost copies
 // one non-ghost cell): the ghosts along one direction that copy index c of an
 // interior lo..hi, as a mask -- bit k-1: index lo - k, bit 3+k: hi + k, for

@@ -282,7 +282,8 @@ __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int
   if (in) {
     const double d = LD(st + F_D * ps, k), m1 = LD(st + F_M1 * ps, k), m2 = LD(st + F_M2 * ps, k);
     const double b1c = LD(st + F_B1C * ps, k), b2c = LD(st + F_B2C * ps, k);
-    const Cons7 u{d, m1, m2, LD(st + F_M3 * ps, k), LD(st + F_E * ps, k), b2c, LD(st + F_B3C * ps, k)};
+    const Cons7 u{d,   m1, m2, LD(st + F_M3 * ps, k), LD(st + F_E * ps, k),
+                  b2c, LD(st + F_B3C * ps, k)};
     bxc = b1c;
     lds_put(sw, tid, cons_to_prim(u, bxc, eos));
     // Step 3 (:249-255): emf3 at t^n over [jl,ju] x [il,iu]
@@ -325,14 +326,14 @@ __device__ __forceinline__ void pred_x1_tile(const Inst* __restrict__ insts, int
     put7<STREAM>(sc + S_F1 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
   }
 }
-template <bool SAVE, int FLUX>
+template <int FLUX>
 __global__ void __launch_bounds__(kX1Block, 2) k_pred_x1(const Inst* __restrict__ insts,
                                                          int ninst, int ntiles, int remap) {
   __shared__ double sw[7][kX1Block];
   __shared__ double swl[7][kX1Block];
   __shared__ double swr[7][kX1Block];
   for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x) {
-    pred_x1_tile<SAVE, FLUX>(insts, ninst, xcd_tile(t0, ntiles, remap), sw, swl, swr);
+    pred_x1_tile<false, FLUX>(insts, ninst, xcd_tile(t0, ntiles, remap), sw, swl, swr);
     __syncthreads();
   }
 }
@@ -362,9 +363,9 @@ __device__ __forceinline__ bool x2_lane(const Inst& g, int local, int lane, int 
 // order (d, M2, M3, M1, E, B3c, B1c) with Bx = B2c. Lanes own adjacent
 // columns (coalesced rows); each lane marches down a segment of faces keeping
 // the three-cell PLM stencil and the pending left state in registers.
-// (SAVE and FLUX as for the x1 predictor; the marching stencil keeps this one
-// at one wave per SIMD)
-template <bool SAVE, int FLUX>
+// (FLUX as for the x1 predictor; the marching stencil keeps this one at one wave
+// per SIMD)
+template <int FLUX>
 __global__ void __launch_bounds__(kX2Block) k_pred_x2(const Inst* __restrict__ insts, int ninst,
                                                       int ntiles, int seg_len, int remap) {
   __shared__ double sxl[7][kX2Block];
@@ -444,10 +445,6 @@ __global__ void __launch_bounds__(kX2Block) k_pred_x2(const Inst* __restrict__ i
       Prim7 wl, wr;
       double b0;
       build(ul, ur, wl, wr, b0);
-      if (SAVE) {
-        put7(g.prims + P_WL2 * ps, ps, k, wl);
-        put7(g.prims + P_WR2 * ps, ps, k, wr);
-      }
       put7(sc + S_UL2 * ps, ps, k, ul);
       put7(sc + S_UR2 * ps, ps, k, ur);
       put7(sc + S_F2 * ps, ps, k, riemann_of<FLUX>(ul, ur, wl, wr, b0, eos, build));
@@ -602,24 +599,24 @@ __device__ __forceinline__ void pred_x2_tile(const Inst* __restrict__ insts, int
     sP = nP; sQ = nQ; sW = nW; sF = nF;
   }
 }
-template <bool SAVE, int FLUX>
+template <int FLUX>
 __global__ void __launch_bounds__(kX2Block, 2) k_pred_x2l(const Inst* __restrict__ insts,
                                                           int ninst, int ntiles, int seg_len,
                                                           int remap) {
   __shared__ X2Slots slots[kX2Slots];
   __shared__ double aux[kX2Aux][kX2Block];
   for (int t0 = blockIdx.x; t0 < ntiles; t0 += gridDim.x)
-    pred_x2_tile<SAVE, FLUX>(insts, ninst, xcd_tile(t0, ntiles, remap), seg_len, slots, aux,
-                             threadIdx.x);
+    pred_x2_tile<false, FLUX>(insts, ninst, xcd_tile(t0, ntiles, remap), seg_len, slots, aux,
+                              threadIdx.x);
 }
 
 // Both predictors in one launch (they write disjoint planes). Workgroups
 // [0, nb2) hold two x2 tiles each, one per wave -- the longer marches start
 // first -- and the rest one x1 tile each; both kinds take the 20 KiB of LDS
 // and the registers per wave of two waves per SIMD.
-// STREAM: the 42 output planes are stored past the caches. Where a step's
-// planes outgrow the Infinity Cache the corrector finds them in HBM anyway, and
-// 344 B per cell of stores only push out the state the other sweep and the
+// STREAM: the 42 planes of face states and fluxes are stored past the caches. Where a
+// step's planes outgrow the Infinity Cache the corrector finds them in HBM anyway, and
+// 336 B per cell of stores only push out the state the other sweep and the
 // corrector still read: a step of 1024^2 takes 510 -> 485 us (HLLE 446 -> 411),
 // 2048x1536 1388 -> 1347 (1224 -> 1172), 4096^2 7.07 -> 6.99 ms. Where they fit,
 // the corrector reads them from the cache and streaming costs (512^2 151 -> 157 us).
@@ -1057,7 +1054,9 @@ __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ni
   const double* emf = sc + S_EMF * ps;
   const double* B1i = st + F_B1I * ps;
   const double* B2i = st + F_B2I * ps;
-  auto b1h = [&](uint32_t kk) { return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk)); };
+  auto b1h = [&](uint32_t kk) {
+    return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk));
+  };
   auto b2h = [&](uint32_t kk) { return LD(B2i, kk) + hdtodx1 * (LD(emf, kk + 1) - LD(emf, kk)); };
   const double* F1 = sc + S_F1 * ps;
   const double* F2 = sc + S_F2 * ps;
@@ -1101,9 +1100,11 @@ __device__ __forceinline__ void corr_tile(const Inst* __restrict__ insts, int ni
   // Step 7
   const double dhalf = LD(st + F_D * ps, k) - hdtodx1 * (LD(F1, k + 1) - LD(F1, k)) -
                        hdtodx2 * (LD(F2, k + pitch) - LD(F2, k));
-  const double m1 = LD(st + F_M1 * ps, k) - hdtodx1 * (LD(F1 + 1 * ps, k + 1) - LD(F1 + 1 * ps, k)) -
+  const double m1 = LD(st + F_M1 * ps, k) -
+                    hdtodx1 * (LD(F1 + 1 * ps, k + 1) - LD(F1 + 1 * ps, k)) -
                     hdtodx2 * (LD(F2 + 3 * ps, k + pitch) - LD(F2 + 3 * ps, k));
-  const double m2 = LD(st + F_M2 * ps, k) - hdtodx1 * (LD(F1 + 2 * ps, k + 1) - LD(F1 + 2 * ps, k)) -
+  const double m2 = LD(st + F_M2 * ps, k) -
+                    hdtodx1 * (LD(F1 + 2 * ps, k + 1) - LD(F1 + 2 * ps, k)) -
                     hdtodx2 * (LD(F2 + 1 * ps, k + pitch) - LD(F2 + 1 * ps, k));
   const double b1c = 0.5 * (b1h(k) + b1h(k + 1));
   const double b2c = 0.5 * (b2h(k) + b2h(k + pitch));
@@ -1124,9 +1125,8 @@ __global__ void __launch_bounds__(kTileX* TY, 2) k_corr(const Inst* __restrict__
 // ones): workgroups [0, ntiles) the x2 part with Step 7, the rest the x1 part.
 // HLLE: 132 registers left three waves per SIMD; 128 hold four without spills.
 template <int TY, int FLUX>
-__global__ void __launch_bounds__(kTileX* TY, FLUX == kFluxHlle ? 4 : 2) k_corr_both(const Inst* __restrict__ insts,
-                                                             int ninst, int ntiles, int remap,
-                                                             int strip) {
+__global__ void __launch_bounds__(kTileX* TY, FLUX == kFluxHlle ? 4 : 2)
+k_corr_both(const Inst* __restrict__ insts, int ninst, int ntiles, int remap, int strip) {
   __shared__ double park_lds[14 * kTileX * TY];
   const LdsPark park{park_lds, kTileX * TY, (int)(threadIdx.y * kTileX + threadIdx.x)};
   const int b = blockIdx.x;
@@ -1210,8 +1210,9 @@ __device__ __forceinline__ void store_faces(const Inst& g, double* out, int j, i
 // copy it (edge), its failure bits, and its inverse dt
 __device__ __forceinline__ double store_cell(const Inst& g, Clock* clk, double* out,
                                              int j, int i, bool edge, unsigned ix,
-                                             unsigned iy, double d, double M1, double M2, double M3, double E, double B3c,
-                                             double B1c, double B2c) {
+                                             unsigned iy, double d, double M1, double M2,
+                                             double M3, double E, double B3c, double B1c,
+                                             double B2c) {
   const size_t ps = g.ps;
   const int pitch = g.pitch;
   const uint32_t k = (uint32_t)(j * pitch + i);
@@ -1356,8 +1357,9 @@ __global__ void __launch_bounds__(kTileX* TY) k_final(const Inst* __restrict__ i
 // next stays in the lane's LDS slots, so the corrector fluxes, the cell-centred
 // emf and the corners, 15 planes that k_corr_both writes and k_final reads, never
 // reach memory. Lanes 1..62 finish cells; lanes 0 and 63 hold the neighbours'
-// corner inputs. A march repeats one x2 face row and one x1 row.
-// HLLE is bound by the 61 planes it reads and writes once: 4096^2 6.08 -> 5.28 ms a
+// corner inputs. A march repeats one x2 face row, and the x1 fluxes and emf3 of two
+// rows.
+// HLLE is bound by the 62 planes it reads (51) and writes (11) once: 4096^2 6.08 -> 5.28 ms a
 // step (this kernel 2.56 ms, 3.2 TB/s), 2048 x 1536 1.152 -> 1.060, 24 grids of
 // 777 x 333 2.34 -> 2.12. Roe, bound by its arithmetic at two waves per SIMD: 4096^2
 // 6.87 -> 6.27, 2048 x 1536 1.309 -> 1.248, 24 grids of 777 x 333 2.65 -> 2.53.
@@ -1406,7 +1408,9 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap,
   const double* B2i = st + F_B2I * ps;
   const double* F1 = sc + S_F1 * ps;
   const double* F2 = sc + S_F2 * ps;
-  auto b1h = [&](uint32_t kk) { return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk)); };
+  auto b1h = [&](uint32_t kk) {
+    return LD(B1i, kk) - hdtodx2 * (LD(emf, kk + pitch) - LD(emf, kk));
+  };
   auto b2h = [&](uint32_t kk) { return LD(B2i, kk) + hdtodx1 * (LD(emf, kk + 1) - LD(emf, kk)); };
   const bool edge = fill && near_edge(g, i0 + 1, kCfCols, r0, rows);
   double dti = 0.0;
@@ -1480,9 +1484,11 @@ k_corr_final(const Inst* __restrict__ insts, int ninst, int ntiles, int remap,
     {
       const double dhalf = LD(st + F_D * ps, k) - hdtodx1 * (LD(F1, k + 1) - LD(F1, k)) -
                            hdtodx2 * (LD(F2, k + pitch) - LD(F2, k));
-      const double m1 = LD(st + F_M1 * ps, k) - hdtodx1 * (LD(F1 + 1 * ps, k + 1) - LD(F1 + 1 * ps, k)) -
+      const double m1 = LD(st + F_M1 * ps, k) -
+                        hdtodx1 * (LD(F1 + 1 * ps, k + 1) - LD(F1 + 1 * ps, k)) -
                         hdtodx2 * (LD(F2 + 3 * ps, k + pitch) - LD(F2 + 3 * ps, k));
-      const double m2 = LD(st + F_M2 * ps, k) - hdtodx1 * (LD(F1 + 2 * ps, k + 1) - LD(F1 + 2 * ps, k)) -
+      const double m2 = LD(st + F_M2 * ps, k) -
+                        hdtodx1 * (LD(F1 + 2 * ps, k + 1) - LD(F1 + 2 * ps, k)) -
                         hdtodx2 * (LD(F2 + 1 * ps, k + pitch) - LD(F2 + 1 * ps, k));
       const double b1c = 0.5 * (b1h(k) + b1h(k + 1));
       const double b2c = 0.5 * (b2h(k) + b2h(k + pitch));
@@ -1738,18 +1744,12 @@ constexpr int kX1PerCu = 2 * 4 * 64 / kX1Block;
 
 typedef void (*PredX1Kernel)(const Inst*, int, int, int);
 typedef void (*PredX2Kernel)(const Inst*, int, int, int, int);
-static PredX1Kernel pred_x1_kernel(bool save, int flux) {
-  if (flux == kFluxHlle) return save ? k_pred_x1<true, kFluxHlle> : k_pred_x1<false, kFluxHlle>;
-  return save ? k_pred_x1<true, kFluxRoe> : k_pred_x1<false, kFluxRoe>;
+static PredX1Kernel pred_x1_kernel(int flux) {
+  return flux == kFluxHlle ? k_pred_x1<kFluxHlle> : k_pred_x1<kFluxRoe>;
 }
-static PredX2Kernel pred_x2_kernel(bool save, int flux, int kind) {
-  if (kind == 1) {
-    if (flux == kFluxHlle)
-      return save ? k_pred_x2l<true, kFluxHlle> : k_pred_x2l<false, kFluxHlle>;
-    return save ? k_pred_x2l<true, kFluxRoe> : k_pred_x2l<false, kFluxRoe>;
-  }
-  if (flux == kFluxHlle) return save ? k_pred_x2<true, kFluxHlle> : k_pred_x2<false, kFluxHlle>;
-  return save ? k_pred_x2<true, kFluxRoe> : k_pred_x2<false, kFluxRoe>;
+static PredX2Kernel pred_x2_kernel(int flux, int kind) {
+  if (kind == 1) return flux == kFluxHlle ? k_pred_x2l<kFluxHlle> : k_pred_x2l<kFluxRoe>;
+  return flux == kFluxHlle ? k_pred_x2<kFluxHlle> : k_pred_x2<kFluxRoe>;
 }
 typedef void (*CorrKernel)(const Inst*, int, int, int, int);
 typedef void (*FinalKernel)(const Inst*, int, int, int, int, int);
@@ -1824,23 +1824,21 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
       launched(SLOT_BEGIN);
       break;
     case SK_PRED_X1:
-    case SK_PRED_X1_SAVE:
       for (int f = 0; f < 2; f++) {
         const InstList& l = b.of_flux[f];
         if (!l.ninst) continue;
-        const PredX1Kernel fn = pred_x1_kernel(kernel == SK_PRED_X1_SAVE, f);
+        const PredX1Kernel fn = pred_x1_kernel(f);
         hipLaunchKernelGGL(fn, dim3(grid_of(b, l, K_PRED_X1, kX1PerCu)), dim3(kX1Block), 0, s,
                            l.insts, l.ninst, l.ntiles[K_PRED_X1], b.shape.xcd_remap);
         launched(SLOT_PRED_X1);
       }
       break;
     case SK_PRED_X2:
-    case SK_PRED_X2_SAVE:
       for (int f = 0; f < 2; f++) {
         const InstList& l = b.of_flux[f];
         if (!l.ninst) continue;
         const int kind = b.shape.x2_kind;
-        const PredX2Kernel fn = pred_x2_kernel(kernel == SK_PRED_X2_SAVE, f, kind);
+        const PredX2Kernel fn = pred_x2_kernel(f, kind);
         hipLaunchKernelGGL(fn, dim3(grid_of(b, l, K_PRED_X2, kind == 1 ? 8 : 16)), dim3(kX2Block),
                            0, s, l.insts,
                            l.ninst, l.ntiles[K_PRED_X2], b.shape.x2_seg, b.shape.xcd_remap);
@@ -1850,11 +1848,10 @@ hipError_t ATHMI_FN(launch)(const void* bl, int kernel, hipStream_t s) {
     case SK_PRED:
     case SK_PRED_SAVE: {
       const bool save = kernel == SK_PRED_SAVE;
-      if (!merge_sweeps(b)) {
-        const hipError_t e =
-            ATHMI_FN(launch)(bl, save ? SK_PRED_X1_SAVE : SK_PRED_X1, s);
-        if (e != hipSuccess) return e;
-        return ATHMI_FN(launch)(bl, save ? SK_PRED_X2_SAVE : SK_PRED_X2, s);
+      // (only the adjoint saves, on a handle of its own at the default shape)
+      if (!save && !merge_sweeps(b)) {
+        const hipError_t e = ATHMI_FN(launch)(bl, SK_PRED_X1, s);
+        return e != hipSuccess ? e : ATHMI_FN(launch)(bl, SK_PRED_X2, s);
       }
       for (int f = 0; f < 2; f++) {
         const InstList& l = b.of_flux[f];

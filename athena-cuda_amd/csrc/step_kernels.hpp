@@ -76,7 +76,7 @@ struct Inst {
   double dx1, dx2, gamma, g1, g2;
   double* state[2];   // two ping-pong buffers of NSTATE planes
   double* scratch;    // NSCRATCH planes
-  double* prims;      // NPRIMS planes written by SK_PRED_X1_SAVE / SK_PRED_X2_SAVE
+  double* prims;      // NPRIMS planes written by SK_PRED_SAVE
   size_t ps;          // plane stride in doubles
   Clock* clk;
   // first global tile of this instance for each kernel kind
@@ -196,19 +196,20 @@ struct InstList {
 };
 
 // The corrector-and-final march of m instances of one solver on ncu CUs. A march
-// of r rows costs about r + 1 (it repeats one row's x1 fluxes and one x2 face row),
-// and waves_per_cu of them run at a time, so the rows are those with the least
-// rounds x (r + 1): a nearly empty last round costs as much as a full one (Roe
+// of r rows evaluates r + 1 x2 face rows and the x1 fluxes of r + 2 rows; the times
+// follow r + 1 (measured with 4 to 24 rows at nine sizes). Twelve (HLLE) or eight
+// (Roe) marches run per CU at a time, so the rows are those with the least rounds
+// x (r + 1): a nearly empty last round costs as much as a full one (Roe
 // 2048 x 1536, two rounds of 13 rows 1248 us a step, of 20 rows 1370, three of 10
 // 1313; 1200^2, one round of 12 rows 609, two of 10 697).
 // It is worth it where enough of the lanes' rows in these rounds finish cells; the
 // fewer the rounds, the more, since all waves then load and compute in step. Roe:
 // 1024^2 (0.83 in one round) 462 -> 466 us, 1200^2 (0.87) 629 -> 609, 2048 x 1536 (0.89
-// in two) 1309 -> 1248, 4096^2 (0.92 in eight) 6.87 -> 6.27 ms, 100 grids of 200 x 300
+// in two) 1309 -> 1248, 4096^2 (0.92 in nine) 6.87 -> 6.27 ms, 100 grids of 200 x 300
 // (0.70 at 10 rows) 2.77 -> 2.72, 400 of 128^2 (0.60) 3.08 -> 3.28. HLLE: 768^2
 // (0.62 in one) 234 -> 244, 1024^2 (0.79) 396 -> 395, 1200^2 (0.84) 551 -> 513,
 // 2048 x 1536 (0.87) 1152 -> 1060, 4096^2 (0.93 in five) 6.09 -> 5.28 ms, 400 grids of
-// 128^2 (0.52 at 10 rows) 2.78 -> 2.70.
+// 128^2 (0.52 at 10 rows) 2.78 -> 2.70. Near the lines the two ways differ by 1%.
 inline void march_of(const Inst* insts, int m, bool hlle, int ncu, InstList& list) {
   const long slots = (hlle ? 12L : 8L) * (ncu > 0 ? ncu : 1);
   double cells = 0.0;
@@ -292,11 +293,10 @@ enum StepKernel {
   SK_DTI,             // new_dt partial maxima
   SK_DT_FINAL,        // new_dt.c:93-97
   SK_DIVB,
-  SK_PRED_X1_SAVE,    // predictors that also store their primitive face states
-  SK_PRED_X2_SAVE,    // (Inst::prims), for the adjoint's re-run
-  SK_PRED,            // both predictors, both corrector parts: one launch or two, by the
-  SK_PRED_SAVE,       // batch's size
-  SK_CORR_BOTH,
+  SK_PRED,            // both predictors, in one launch or two by the launch shape
+  SK_PRED_SAVE,       // in one, storing the primitive face states too (Inst::prims), for the
+                      // adjoint's re-run
+  SK_CORR_BOTH,       // both corrector parts, in one launch or two by the launch shape
   SK_FINISH,          // SK_CORR_BOTH, SK_CORNER_C and SK_FINAL_GHOST; one launch per solver on
                       // large batches, which then writes no corrector planes
   SK_FINISH_BARE,     // the same without the ghosts (SK_FINAL)

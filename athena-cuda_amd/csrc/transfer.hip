@@ -121,8 +121,8 @@ hipError_t launch_state_pack(const double* st, double* stage, size_t ps, int pit
 }
 
 hipError_t launch_clock_publish(const Clock* clk, ClockHead* heads, int n, hipStream_t s) {
-  hipLaunchKernelGGL(k_clock_publish, dim3(cdiv(n * kHeadWords, kXferBlock)), dim3(kXferBlock), 0, s,
-                     clk, heads, n);
+  hipLaunchKernelGGL(k_clock_publish, dim3(cdiv(n * kHeadWords, kXferBlock)), dim3(kXferBlock), 0,
+                     s, clk, heads, n);
   return hipGetLastError();
 }
 

@@ -337,6 +337,8 @@ def main():
     ap.add_argument("--size", type=int, default=4096)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--profile-steps", type=int, default=5)
+    ap.add_argument("--separate-kernels", action="store_true",
+                    help="also time the step as its separate kernels")
     ap.add_argument("--batch", type=int, default=256,
                     help="instances of the batched uneven ensemble (0: skip that leg)")
     ap.add_argument("--batch-steps", type=int, default=200)
@@ -458,6 +460,11 @@ def main():
                     "commit": pmc.get("commit"), "workload": pmc.get("workload"),
                     "measured_in_this_run": False},
                 "kernels_ms": kern}
+    if args.separate_kernels:
+        sep = (ctypes.c_double * 10)()
+        pkg._check(L.athmi_profile_steps(g._h, args.profile_steps, sep, 10), "profile")
+        roofline["separate_kernels_ms"] = {L.athmi_step_kernel_name(k).decode(): sep[k]
+                                           for k in range(10)}
     step_bw = ALG_BYTES_PER_CELL * value / 1e9
     out = {
         "metric": "FP64 cell-updates/s at 4096² plain vs batched; adjoint/forward step cost",

@@ -46,10 +46,11 @@ int athmi_adjoint_forward(athmi_adjoint *h, const double *state0, double *stateN
 int athmi_adjoint_backward(athmi_adjoint *h, const double *gradN, double *grad0);
 /* on = 1: the reverse pass sums every adjoint in a fixed order, so two
  * backward passes of one forward pass give bitwise equal gradients: the
- * predictor faces' source terms are stored per face and gathered in order.
- * on = 0 (the default) adds them with FP64 atomics, whose order varies at
- * roundoff level; every other adjoint is gathered in order in both modes. No
- * reference counterpart (the reference has no derivatives). */
+ * predictor faces' source terms are stored per face and gathered in order,
+ * and the two sweeps' cons->prim adjoints are added one sweep after the other.
+ * on = 0 (the default) adds these and Step 3's with FP64 atomics, whose order
+ * varies at roundoff level; every other adjoint is gathered in order in both
+ * modes. No reference counterpart (the reference has no derivatives). */
 int athmi_adjoint_set_deterministic(athmi_adjoint *h, int on);
 /* Number of completed athmi_adjoint_forward calls on the handle. The
  * checkpoints belong to the latest forward pass only: a caller that records
