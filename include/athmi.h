@@ -79,7 +79,9 @@ int athmi_upload(athmi_grid *g, int inst, const double *gas, const double *b1i,
 int athmi_download(athmi_grid *g, int inst, double *gas, double *b1i, double *b2i,
                    double *b3i);
 
-/* Grid.dt / Grid.time / Grid.nstep (athena.h:113-114) of one instance */
+/* Grid.dt / Grid.time / Grid.nstep (athena.h:113-114) of one instance. Reads wait
+ * for the handle's stream and for the null stream (where the caller may replay
+ * work of the handle it has captured); a thread may read while another steps. */
 int athmi_set_clock(athmi_grid *g, int inst, double dt, double time, int nstep);
 int athmi_get_clock(athmi_grid *g, int inst, double *dt, double *time, int *nstep);
 /* Failure word of one instance: the step checks every state it produces and
